@@ -560,9 +560,8 @@ int exh_transcript_proof(exh_transcript h, uint8_t *out, uint64_t cap, uint64_t 
   ApiLock api_lock;
   Transcript *tr = tr_of(h);
   if (!tr) return E_PARAM;
-  std::vector<uint8_t> bytes = tr->encode_proof();
-  *out_len = bytes.size();
-  if (out && cap >= bytes.size()) memcpy(out, bytes.data(), bytes.size());
+  *out_len = tr->proof_size();
+  if (out && cap >= *out_len) tr->encode_proof(out);
   return OK;
 }
 

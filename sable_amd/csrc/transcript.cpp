@@ -162,9 +162,7 @@ int Transcript::send(const uint32_t *vals, int rank, const uint64_t *dims, uint3
   }
   sent_bytes += m->size_bytes();
   if (absorb_it) {
-    std::vector<uint8_t> buf(4 * m->vals.size());
-    for (size_t i = 0; i < m->vals.size(); i++) put_le(m->vals[i], 4, buf.data() + 4 * i);
-    absorb(buf.data(), buf.size());
+    absorb(reinterpret_cast<const uint8_t *>(m->vals.data()), 4 * m->vals.size());  // little-endian words
   }
   if (out) memcpy(out, m->vals.data(), 4 * m->vals.size());
   return OK;
@@ -249,27 +247,36 @@ int Transcript::verify_grind(int bits, uint64_t *nonce) {
 }
 
 // ---- proof bytes: MAGIC | u32 count | messages (src/proofio.lisp:1-9)
-std::vector<uint8_t> Transcript::encode_proof() const {
-  std::vector<uint8_t> out;
+uint64_t Transcript::proof_size() const {
+  uint64_t size = 12;
+  for (const Message &m : messages) size += m.kind == 0 ? 9 + m.bytes.size() : 2 + 8 * m.dims.size() + 4 * m.vals.size();
+  return size;
+}
+
+// (words are little-endian in the proof as they are in this host's memory: whole messages are copied)
+void Transcript::encode_proof(uint8_t *out) const {
   auto put = [&](uint64_t v, int size) {
-    for (int i = 0; i < size; i++) out.push_back((uint8_t)(v >> (8 * i)));
+    put_le(v, size, out);
+    out += size;
   };
-  const char magic[] = "EXACTPF1";
-  out.insert(out.end(), magic, magic + 8);
+  auto copy = [&](const void *from, uint64_t size) {
+    if (size) memcpy(out, from, size);
+    out += size;
+  };
+  copy("EXACTPF1", 8);
   put(messages.size(), 4);
   for (const Message &m : messages) {
     if (m.kind == 0) {
-      out.push_back(0);
+      put(0, 1);
       put(m.bytes.size(), 8);
-      out.insert(out.end(), m.bytes.begin(), m.bytes.end());
+      copy(m.bytes.data(), m.bytes.size());
     } else {
-      out.push_back(1);
-      out.push_back((uint8_t)m.dims.size());
+      put(1, 1);
+      put(m.dims.size(), 1);
       for (uint64_t d : m.dims) put(d, 8);
-      for (uint32_t v : m.vals) put(v, 4);
+      copy(m.vals.data(), 4 * m.vals.size());
     }
   }
-  return out;
 }
 
 int Transcript::load_proof(const uint8_t *octets, uint64_t end) {

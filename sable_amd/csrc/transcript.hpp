@@ -76,7 +76,8 @@ struct Transcript {
   uint64_t grind(int bits);
   int verify_grind(int bits, uint64_t *nonce);
   bool finished() const { return position == messages.size(); }
-  std::vector<uint8_t> encode_proof() const;
+  uint64_t proof_size() const;
+  void encode_proof(uint8_t *out) const;  // proof_size() bytes
 };
 
 bool check_grind(const uint8_t base[32], uint64_t nonce, int bits);
