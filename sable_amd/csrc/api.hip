@@ -1134,17 +1134,17 @@ int exh_basefold_prove_classes(exh_transcript h, int nv, int n_classes, const in
     set_error("invalid-parameter: BaseFold over 1 to 32 classes, 1 <= nv <= 23");
     return E_PARAM;
   }
-  std::vector<const uint32_t *> tables(n_classes);
+  std::vector<BfSource> sources(n_classes);
   for (int k = 0; k < n_classes; k++) {
     DeviceTable *dt = table_of(hs[k]);
     if (!dt || classes[k] < 1 || classes[k] > nv || dt->stride != 8 || dt->n_u32 != ((uint64_t)8 << classes[k])) {
       set_error("invalid-parameter: a class's combined column is 2^c EXT8s");
       return E_PARAM;
     }
-    tables[k] = dt->ptr;
+    sources[k].h = dt->ptr;
   }
-  return basefold_prove_classes(*tr, nv, n_classes, classes, tables.data(), rr, v, grind_bits, queries, out_qs, nullptr,
-                                nullptr, nullptr);
+  return basefold_prove_classes(*tr, nv, n_classes, classes, sources.data(), rr, v, grind_bits, queries, out_qs, nullptr,
+                                nullptr);
 }
 int exh_basefold_prove_encoded(exh_transcript h, int nv, const uint32_t *rr, const uint32_t *v, exh_table table,
                                exh_table codeword, int grind_bits, int queries, uint64_t *out_qs, uint32_t *out_chal,

@@ -361,10 +361,10 @@ struct CombineArgs {
 };
 template <int D>
 __global__ __launch_bounds__(BLOCK) void combine_columns_kernel(const uint32_t *cols, uint64_t len, int ncols,
-                                                                CombineArgs<D> a, uint32_t *out, int accumulate) {
+                                                                CombineArgs<D> a, uint32_t *out, const uint32_t *add) {
   const uint64_t x = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (x >= len) return;
-  Ext<D> g = accumulate ? load_ext<D>(out + x * D) : ext_zero<D>();
+  Ext<D> g = add ? load_ext<D>(add + x * D) : ext_zero<D>();
   for (int k0 = 0; k0 < ncols; k0 += 4) {  // four columns per reduction: 4 p^2 < 2^64
     uint32_t val[4];
 #pragma unroll
@@ -438,21 +438,22 @@ static int combine_many_launch(const uint32_t *d_cols, int ncols, uint64_t len, 
   return OK;
 }
 
+// out = add + sum_k coefficient_k * column_k (add null: zero; it may be `out` itself) for at most COMBINE_COLS columns
+template <int D>
+static void combine_few_launch(const uint32_t *d_cols, int ncols, uint64_t len, const uint32_t *coef, const uint32_t *add,
+                               uint32_t *d_out) {
+  CombineArgs<D> a;
+  memset(&a, 0, sizeof(a));
+  for (int k = 0; k < ncols; k++)
+    for (int cc = 0; cc < D; cc++) a.coef_mont[k][cc] = to_mont(coef[(size_t)k * D + cc] % P);
+  const uint32_t grid = (uint32_t)((len + BLOCK - 1) / BLOCK);
+  hipLaunchKernelGGL((combine_columns_kernel<D>), dim3(grid), dim3(BLOCK), 0, ctx().stream, d_cols, len, ncols, a, d_out,
+                     add);
+}
 template <int D>
 static int combine_launch(const uint32_t *d_cols, int ncols, uint64_t len, const uint32_t *coef, uint32_t *d_out) {
-  Context &c = ctx();
   if (ncols > COMBINE_COLS) return combine_many_launch<D>(d_cols, ncols, len, coef, d_out);
-  for (int first = 0; first < ncols; first += COMBINE_COLS) {
-    const int count = ncols - first < COMBINE_COLS ? ncols - first : COMBINE_COLS;
-    CombineArgs<D> a;
-    memset(&a, 0, sizeof(a));
-    for (int k = 0; k < count; k++)
-      for (int cc = 0; cc < D; cc++) a.coef_mont[k][cc] = to_mont(coef[(size_t)(first + k) * D + cc] % P);
-    const uint32_t *cols = d_cols + (uint64_t)first * len;
-    uint32_t grid = (uint32_t)((len + BLOCK - 1) / BLOCK);
-    hipLaunchKernelGGL((combine_columns_kernel<D>), dim3(grid), dim3(BLOCK), 0, c.stream, cols, len, count, a, d_out,
-                       first > 0 ? 1 : 0);
-  }
+  combine_few_launch<D>(d_cols, ncols, len, coef, nullptr, d_out);
   EXH_HIP(hipGetLastError());
   return OK;
 }
@@ -968,28 +969,6 @@ __global__ __launch_bounds__(BLOCK) void join_coords_kernel(const uint32_t *cols
   store_ext<8>(table + i * 8, e);
 }
 
-// eq(rr, x) for all x of nv bits as one table (weights of the BaseFold sumcheck)
-struct EqOne {
-  int bits;
-};
-__global__ __launch_bounds__(BLOCK) void eq8_kernel(const uint32_t *factors, int bits, uint32_t *out, uint64_t total) {
-  uint64_t x = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (x >= total) return;
-  Ext<8> e = ext_lift<8>(1);
-  for (int b = 0; b < bits; b++)
-    e = ext_mul_mont<8>(e, load_ext<8>(factors + ((size_t)b * 2 + (((x >> b) & 1) ? 0 : 1)) * 8));
-  store_ext<8>(out + x * 8, e);
-}
-
-// copy `count` segments of `words` words each from src + offsets[i] to out
-__global__ void gather_kernel(const uint32_t *src, const uint64_t *offsets, uint32_t words, uint32_t count,
-                              uint32_t *out) {
-  uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (uint64_t)words * count) return;
-  uint32_t seg = (uint32_t)(gid / words), w = (uint32_t)(gid % words);
-  out[gid] = src[offsets[seg] + w];
-}
-
 namespace {
 struct Owned {
   std::vector<void *> ptrs;
@@ -1013,26 +992,6 @@ struct OracleTree {
   int lc;
 };
 }  // namespace
-
-static int gather_to_host(const uint32_t *src, const std::vector<uint64_t> &offsets, uint32_t words,
-                          std::vector<uint32_t> *out) {
-  Context &c = ctx();
-  out->assign((size_t)offsets.size() * words, 0);
-  if (offsets.empty()) return OK;
-  uint64_t *d_off = nullptr;
-  uint32_t *d_out = nullptr;
-  EXH_HIP(hipMalloc((void **)&d_off, offsets.size() * 8));
-  EXH_HIP(hipMalloc((void **)&d_out, out->size() * 4));
-  EXH_HIP(hipMemcpy(d_off, offsets.data(), offsets.size() * 8, hipMemcpyHostToDevice));
-  uint64_t total = out->size();
-  hipLaunchKernelGGL(gather_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, c.stream, src, d_off, words,
-                     (uint32_t)offsets.size(), d_out);
-  EXH_HIP(hipStreamSynchronize(c.stream));
-  EXH_HIP(hipMemcpy(out->data(), d_out, total * 4, hipMemcpyDeviceToHost));
-  EXH_HIP(hipFree(d_off));
-  EXH_HIP(hipFree(d_out));
-  return OK;
-}
 
 // OPEN-QUERIES' two gathers for one (unit, class) (src/pcs.lisp:721-734).  Leaves: out[(q * ncols + k) * 4 + s] =
 // symbol 4 * leaf_q + s of column k (LEAF-ROWS, src/pcs.lisp:275-277, as the (Q, rows, 4) array of
@@ -1129,19 +1088,69 @@ struct BfStepArgs {
   uint64_t cw_m;  // elements after the fold
 };
 
+// The sums of a step's workgroup -> totals -> (last workgroup) pinned host memory.  `mine`: the workgroup's `width`
+// words; host_out receives them and a status word, see BfStepArgs.
+__device__ __forceinline__ void bf_deliver_sums(const RoundTotals &totals, const uint32_t *mine, uint32_t width,
+                                                uint32_t workgroups, unsigned long long *host_out, uint32_t host_seq) {
+  __shared__ uint32_t sums[64];
+  __shared__ uint32_t scratch[TOTALS_POLLS * BLOCK];
+  const uint32_t tid = threadIdx.x;
+  bool ok = true;
+  const uint32_t *from = sums;
+  if (workgroups == 1)
+    from = mine;  // nobody to wait for
+  else if (!add_and_elect(totals, mine, width, scratch, sums, &ok, 0, width, workgroups - 1, workgroups))
+    return;
+  if (tid <= width) {
+    const uint32_t value = tid < width ? (ok ? from[tid] : 0u) : (ok ? 0u : 1u);
+    __hip_atomic_store(host_out + tid, ((unsigned long long)host_seq << 32) | value, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// a step's two weighted sums, accumulated per lane, to their delivery
+__device__ __forceinline__ void bf_finish_sums(const BfStepArgs &a, Acc96 (*acc)[8], uint64_t tile_start) {
+  __shared__ uint32_t lds[BLOCK / 64][16];
+  __shared__ uint32_t mine[16];
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t total = wave_sums_transposed<16>([&](int k) -> uint32_t { return acc_reduce(acc[k / 8][k % 8]); });
+  if (lane < 16) lds[tid >> 6][__brev(lane) >> 28] = total;
+  __syncthreads();
+  if (tid < 2) {  // a workgroup's pairs share one HIGH weight (the tile is |LOW| pairs)
+    Ext<8> t;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      uint32_t v = lds[0][tid * 8 + c];
+#pragma unroll
+      for (int w = 1; w < BLOCK / 64; w++) v = fadd(v, lds[w][tid * 8 + c]);
+      t.c[c] = v;
+    }
+    // times HIGH / R, then times R: the plain product
+    t = ext_mul_mont<8>(t, load_ext<8>(a.high + (tile_start >> a.low_bits) * 8));
+#pragma unroll
+    for (int c = 0; c < 8; c++) mine[tid * 8 + c] = mont_mul(t.c[c], R2);
+  }
+  __syncthreads();
+  bf_deliver_sums(a.totals, mine, 16, a.tt_blocks, a.host_out, a.host_seq);
+}
+
+// RS:FOLD of one element: pair (a, b) at twiddle x: f0 = (a + b)/2, f1 = (a - b)/(2x), f0 + r (f1 - f0)
+__device__ __forceinline__ void bf_fold_codeword(const BfStepArgs &a, const Ext<8> &r, uint64_t s) {
+  if (s >= a.cw_m) return;
+  const Ext<8> x = load_ext<8>(a.cw_in + 2 * s * 8), y = load_ext<8>(a.cw_in + (2 * s + 1) * 8);
+  const Ext<8> f0 = ext_scale_mont<8>(ext_add<8>(x, y), mont_mul(INV2, R2));
+  const Ext<8> f1 = ext_scale_mont<8>(ext_sub<8>(x, y), a.tw_inv2[s]);
+  store_ext<8>(a.cw_out + s * 8, ext_add<8>(f0, ext_mul_mont<8>(r, ext_sub<8>(f1, f0))));
+}
+
 template <bool FOLD>
 __global__ __launch_bounds__(BLOCK) void bf_step_kernel(BfStepArgs a) {
   const uint32_t tid = threadIdx.x;
   Ext<8> r;
 #pragma unroll
   for (int c = 0; c < 8; c++) r.c[c] = a.r_mont[c];
-  if (blockIdx.x >= a.tt_blocks) {  // pair (a, b) at twiddle x: f0 = (a + b)/2, f1 = (a - b)/(2x), f0 + r (f1 - f0)
-    const uint64_t s = (uint64_t)(blockIdx.x - a.tt_blocks) * BLOCK + tid;
-    if (s >= a.cw_m) return;
-    const Ext<8> x = load_ext<8>(a.cw_in + 2 * s * 8), y = load_ext<8>(a.cw_in + (2 * s + 1) * 8);
-    const Ext<8> f0 = ext_scale_mont<8>(ext_add<8>(x, y), mont_mul(INV2, R2));
-    const Ext<8> f1 = ext_scale_mont<8>(ext_sub<8>(x, y), a.tw_inv2[s]);
-    store_ext<8>(a.cw_out + s * 8, ext_add<8>(f0, ext_mul_mont<8>(r, ext_sub<8>(f1, f0))));
+  if (blockIdx.x >= a.tt_blocks) {
+    bf_fold_codeword(a, r, (uint64_t)(blockIdx.x - a.tt_blocks) * BLOCK + tid);
     return;
   }
   const uint64_t tile = (uint64_t)BLOCK * a.pairs_per_thread, tile_start = (uint64_t)blockIdx.x * tile;
@@ -1186,40 +1195,218 @@ __global__ __launch_bounds__(BLOCK) void bf_step_kernel(BfStepArgs a) {
       w = w_ahead;
     }
   }
-  if (!a.do_sums) return;
-  __shared__ uint32_t lds[BLOCK / 64][16];
-  __shared__ uint32_t mine[16], sums[16];
-  __shared__ uint32_t scratch[TOTALS_POLLS * BLOCK];
+  if (a.do_sums) bf_finish_sums(a, acc, tile_start);
+}
+
+// ---- the first rounds from the committed base columns
+// The table that is opened is H = sum_j c_j col_j of few base columns, and its codeword the same combination of
+// theirs.  Neither is formed.  With the first LB variables left open, T[b] = sum_k E[k] H[2^LB k + b] over the weights
+// E of the variables above them, the rounds 0 .. LB - 1 are the host's: a round's h0, h1 are the sums over T folded by
+// the challenges so far, weighted by eq of the open variables above -- one sweep over the base columns (4 bytes an
+// entry) in place of LB passes over tables of 32-byte elements.  T[b] is itself sum_j c_j S_j[b] with base-field
+// columns under the weights, so an entry costs eight multiply-adds.  Level LB's table comes straight from the base
+// columns (2^LB products per column and coordinate: BIND-PREFIX, src/sumcheck.lisp:496-510), and so does the codeword
+// of the first level that anybody looks at (level 2, or 1 when a class joins there): both are linear in H.
+// At nv = 23 and two columns the combination, rounds 0 to 2 and the codeword's folds to level 2 moved 2.3 GB in
+// 720 us of kernels; this way they move 0.55 GB, and the opening (a class of 2^19 joining) went from 1964 to 1290 us
+// with the other changes of this file's opening: no wait before the weights, one gather for all openings.
+// The line at eight columns: their constants fill the kernel's arguments, and each of the two readings of the table
+// costs 4 bytes an entry and column where a combined table costs 32 written once and 32 read twice.
+constexpr int BF_BASE_MAX_COLS = 8;  // columns whose constants travel as kernel arguments
+constexpr int BF_BASE_BITS = 3;      // variables left open at most: 2^3 sums of eight words in registers
+
+struct BfBaseSumsArgs {
+  const uint32_t *cols;  // ncols base columns of len values
+  uint64_t len, n_cells;  // cells of 2^LB consecutive entries
+  const uint32_t *low, *high;
+  uint32_t low_bits, tiles;  // a workgroup takes one column's tile of 2^low_bits cells
+  uint32_t coef[BF_BASE_MAX_COLS][8];  // times R^2
+  RoundTotals totals;
+  unsigned long long *host_out;
+  uint32_t host_seq;
+};
+
+template <int LB>
+__global__ __launch_bounds__(BLOCK) void bf_base_sums_kernel(BfBaseSumsArgs a) {
+  constexpr int B = 1 << LB, WORDS = 8 * B, W = WORDS < 32 ? WORDS : 32, BITS = W == 32 ? 5 : W == 16 ? 4 : 3;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t tile = blockIdx.x % a.tiles, column = blockIdx.x / a.tiles;
+  const uint32_t *col = a.cols + (uint64_t)column * a.len;
+  const uint64_t first = (uint64_t)tile << a.low_bits;
+  const uint64_t left = a.n_cells - first;
+  const uint32_t cells = left < ((uint64_t)1 << a.low_bits) ? (uint32_t)left : 1u << a.low_bits;
+  uint64_t acc[B][8];
 #pragma unroll
-  for (int q = 0; q < 2; q++)
+  for (int b = 0; b < B; b++)
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-      const uint32_t v = wave_sum(acc_reduce(acc[q][c]));
-      if ((tid & 63) == 0) lds[tid >> 6][q * 8 + c] = v;
+    for (int c = 0; c < 8; c++) acc[b][c] = 0;
+  for (uint32_t k = tid; k < cells; k += BLOCK) {
+    uint32_t v[B];
+    const uint32_t *p = col + (first + k) * B;
+    if constexpr (B >= 4) {
+#pragma unroll
+      for (int q = 0; q < B / 4; q++) {
+        const uint4 x = reinterpret_cast<const uint4 *>(p)[q];
+        v[4 * q] = x.x, v[4 * q + 1] = x.y, v[4 * q + 2] = x.z, v[4 * q + 3] = x.w;
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < B; b++) v[b] = p[b];
     }
-  __syncthreads();
-  if (tid < 2) {  // a workgroup's pairs share one HIGH weight (the tile is |LOW| pairs)
-    Ext<8> t;
+    const Ext<8> w = load_ext<8>(a.low + (uint64_t)k * 8);
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-      uint32_t v = lds[0][tid * 8 + c];
+    for (int b = 0; b < B; b++)
 #pragma unroll
-      for (int w = 1; w < BLOCK / 64; w++) v = fadd(v, lds[w][tid * 8 + c]);
-      t.c[c] = v;
-    }
-    // times HIGH / R, then times R: the plain product
-    t = ext_mul_mont<8>(t, load_ext<8>(a.high + (tile_start >> a.low_bits) * 8));
+      for (int c = 0; c < 8; c++) lazy_mad(acc[b][c], w.c[c], v[b]);
+  }
+  __shared__ uint32_t lds[BLOCK / 64][WORDS];
+  __shared__ uint32_t mine[WORDS];
+  uint32_t idx = 0;
 #pragma unroll
-    for (int c = 0; c < 8; c++) mine[tid * 8 + c] = mont_mul(t.c[c], R2);
+  for (int b = 0; b < BITS; b++) idx |= ((lane >> b) & 1u) << (BITS - 1 - b);
+#pragma unroll
+  for (int at = 0; at < WORDS; at += W) {
+    const uint32_t total =
+        wave_sums_transposed<W>([&](int k) -> uint32_t { return lazy_reduce(acc[(at + k) / 8][(at + k) % 8]); });
+    if (lane < W) lds[wave][at + idx] = total;
   }
   __syncthreads();
-  bool ok;
-  if (!add_and_elect(a.totals, mine, 16, scratch, sums, &ok, 0, 16, a.tt_blocks - 1, a.tt_blocks)) return;
-  if (tid < 17) {
-    const uint32_t value = tid < 16 ? (ok ? sums[tid] : 0u) : (ok ? 0u : 1u);
-    __hip_atomic_store(a.host_out + tid, ((unsigned long long)a.host_seq << 32) | value, __ATOMIC_RELAXED,
+  if (tid < B) {  // times the tile's HIGH weight and the column's coefficient
+    Ext<8> t, c;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      uint32_t v = lds[0][tid * 8 + k];
+#pragma unroll
+      for (int w = 1; w < BLOCK / 64; w++) v = fadd(v, lds[w][tid * 8 + k]);
+      t.c[k] = v;
+      c.c[k] = a.coef[column][k];
+    }
+    t = ext_mul_mont<8>(ext_mul_mont<8>(t, load_ext<8>(a.high + (uint64_t)tile * 8)), c);
+#pragma unroll
+    for (int k = 0; k < 8; k++) mine[tid * 8 + k] = t.c[k];
+  }
+  __syncthreads();
+  bf_deliver_sums(a.totals, mine, WORDS, gridDim.x, a.host_out, a.host_seq);
+}
+
+struct BfBaseArgs {
+  BfStepArgs s;  // the table's part with tt_in unused; the codeword's part with cw_in, tw_inv2 when it is a plain fold
+  const uint32_t *cols, *cws;  // ncols base columns of col_len values, their codewords of cw_len symbols
+  uint64_t col_len, cw_len;
+  uint32_t ncols;
+  const uint32_t *tw0, *tw1;  // 1 / (2x) of the codeword's levels 0 and 1
+  uint32_t tt_coef[BF_BASE_MAX_COLS][1 << BF_BASE_BITS][8];  // c_j eq((x_0, x_1, ..), b), times R
+  uint32_t cw_coef[BF_BASE_MAX_COLS][4][8];                  // c_j {1, x_0, x_1, x_0 x_1}, times R
+};
+static_assert(sizeof(BfBaseArgs) <= 4096, "kernel arguments");
+
+// sum over b of coef[b][c] v[b] / R for N = 2, 4 or 8 products
+template <int N>
+__device__ __forceinline__ uint32_t mont_dot(const uint32_t (*coef)[8], int c, const uint32_t *v) {
+  uint64_t t = 0;
+#pragma unroll
+  for (int b = 0; b < N; b++) {
+    // four products below p^2 fit 64 bits; from then on, two at a time above a sum brought below p 2^32
+    if (b >= 4 && b % 2 == 0) t = mont_lazy(t);
+    t += (uint64_t)coef[b][c] * v[b];
+  }
+  return mont_reduce4(t);
+}
+
+// TT: the table of level TT from the base columns, with the next round's sums (0: no table part).
+// CW: the codeword of level CW = 1 or 2 from the base codewords; 3: a plain fold of a codeword of elements.
+template <int TT, int CW>
+__global__ __launch_bounds__(BLOCK) void bf_base_kernel(BfBaseArgs a) {
+  const uint32_t tid = threadIdx.x;
+  if (TT == 0 || blockIdx.x >= a.s.tt_blocks) {
+    const uint64_t s = (uint64_t)(blockIdx.x - a.s.tt_blocks) * BLOCK + tid;
+    if constexpr (CW == 3) {
+      Ext<8> r;
+#pragma unroll
+      for (int c = 0; c < 8; c++) r.c[c] = a.s.r_mont[c];
+      bf_fold_codeword(a.s, r, s);
+    } else {
+      if (s >= a.s.cw_m) return;
+      const uint32_t half = mont_mul(INV2, R2);
+      Ext<8> out = ext_zero<8>();
+      uint32_t t0[2], t2 = 0;
+      if constexpr (CW == 1)
+        t0[0] = a.tw0[s];
+      else
+        t0[0] = a.tw0[2 * s], t0[1] = a.tw0[2 * s + 1], t2 = a.tw1[s];
+      for (uint32_t j = 0; j < a.ncols; j++) {
+        const uint32_t *cw = a.cws + (uint64_t)j * a.cw_len;
+        uint32_t q[4];  // the base values that go with 1, x_0, x_1, x_0 x_1
+        if constexpr (CW == 1) {
+          const uint2 e = *reinterpret_cast<const uint2 *>(cw + 2 * s);
+          q[0] = mont_mul(fadd(e.x, e.y), half);
+          q[1] = fsub(mont_mul(fsub(e.x, e.y), t0[0]), q[0]);
+        } else {
+          const uint4 e = *reinterpret_cast<const uint4 *>(cw + 4 * s);
+          // level 1's two elements u + x_0 v; their fold at level 1's twiddle
+          const uint32_t u0 = mont_mul(fadd(e.x, e.y), half), v0 = fsub(mont_mul(fsub(e.x, e.y), t0[0]), u0);
+          const uint32_t u1 = mont_mul(fadd(e.z, e.w), half), v1 = fsub(mont_mul(fsub(e.z, e.w), t0[1]), u1);
+          q[0] = mont_mul(fadd(u0, u1), half), q[1] = mont_mul(fadd(v0, v1), half);
+          q[2] = fsub(mont_mul(fsub(u0, u1), t2), q[0]), q[3] = fsub(mont_mul(fsub(v0, v1), t2), q[1]);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) out.c[c] = fadd(out.c[c], mont_dot<CW == 1 ? 2 : 4>(a.cw_coef[j], c, q));
+      }
+      store_ext<8>(a.s.cw_out + s * 8, out);
+    }
+    return;
+  }
+  if constexpr (TT > 0) {
+    constexpr int B = 1 << TT;
+    const uint64_t tile = (uint64_t)BLOCK * a.s.pairs_per_thread, tile_start = (uint64_t)blockIdx.x * tile;
+    const uint64_t low_mask = ((uint64_t)1 << a.s.low_bits) - 1;
+    Acc96 acc[2][8];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+      for (int c = 0; c < 8; c++) acc_zero(acc[q][c]);
+    for (uint32_t k = 0; k < a.s.pairs_per_thread; k++) {
+      const uint64_t i = tile_start + (uint64_t)k * BLOCK + tid;
+      if (i >= a.s.n_pairs) break;
+      Ext<8> lo = ext_zero<8>(), hi = ext_zero<8>(), w = ext_zero<8>();
+      if (a.s.do_sums) w = load_ext<8>(a.s.low + (i & low_mask) * 8);
+      for (uint32_t j = 0; j < a.ncols; j++) {
+        const uint4 *p = reinterpret_cast<const uint4 *>(a.cols + (uint64_t)j * a.col_len + 2 * B * i);
+        uint32_t v[2 * B];
+#pragma unroll
+        for (int q = 0; q < B / 2; q++) {
+          const uint4 x = p[q];
+          v[4 * q] = x.x, v[4 * q + 1] = x.y, v[4 * q + 2] = x.z, v[4 * q + 3] = x.w;
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+          lo.c[c] = fadd(lo.c[c], mont_dot<B>(a.tt_coef[j], c, v));
+          hi.c[c] = fadd(hi.c[c], mont_dot<B>(a.tt_coef[j], c, v + B));
+        }
+      }
+      store_ext<8>(a.s.tt_out + 2 * i * 8, lo);
+      store_ext<8>(a.s.tt_out + (2 * i + 1) * 8, hi);
+      if (a.s.do_sums) {
+        ext_mul_acc<8>(acc[0], lo, w);
+        ext_mul_acc<8>(acc[1], hi, w);
+      }
+    }
+    if (a.s.do_sums) bf_finish_sums(a.s, acc, tile_start);
+  }
+}
+
+// `count` quads (16 bytes each) from anywhere in device memory into pinned host memory, every word as a 64-bit word
+// (seq << 32 | value); `src` lies in pinned memory as well
+__global__ __launch_bounds__(BLOCK) void gather_quads_kernel(const uint32_t *const *src, uint32_t count,
+                                                             unsigned long long *host_dst, uint32_t seq) {
+  const uint32_t gid = blockIdx.x * BLOCK + threadIdx.x;
+  if (gid >= count) return;
+  const uint4 v = *reinterpret_cast<const uint4 *>(src[gid]);
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    __hip_atomic_store(host_dst + 4 * (uint64_t)gid + k, ((unsigned long long)seq << 32) | w[k], __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
-  }
 }
 
 // `words` words from device memory into pinned host memory as 64-bit words (seq << 32 | value), each its own flag
@@ -1228,18 +1415,6 @@ __global__ __launch_bounds__(BLOCK) void deliver_kernel(const uint32_t *src, uin
   for (uint32_t u = threadIdx.x; u < words; u += BLOCK)
     __hip_atomic_store(host_dst + u, ((unsigned long long)seq << 32) | src[u], __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// segments of 8 words from anywhere in device memory, side by side into out
-__global__ __launch_bounds__(BLOCK) void gather8_kernel(const uint32_t *const *src, uint32_t count, uint32_t *out) {
-  const uint64_t gid = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (gid >= (uint64_t)count * 8) return;
-  out[gid] = src[gid / 8][gid % 8];
-}
-
-__global__ __launch_bounds__(BLOCK) void zero_words_kernel(uint32_t *p, uint64_t words) {
-  const uint64_t gid = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (gid < words) p[gid] = 0;
 }
 
 // the host's side of such words in pinned memory: true once all n carry seq (their low halves then go to out);
@@ -1264,25 +1439,60 @@ static bool await_words(Context &c, const volatile unsigned long long *w, size_t
   return true;
 }
 
-// regions of the context's pinned host buffer BaseFold's rounds use (in 32-bit words): a slot of 17 64-bit words
-// per round, then a slot of 128 * 8 64-bit words per oracle cap
+// regions of the context's pinned host buffer BaseFold uses (in 32-bit words): a slot of 17 64-bit words per round,
+// a slot of 128 * 8 64-bit words per oracle cap, and above the first 2^16 words a slot of 65 64-bit words per class's
+// sums, the point's factors, and a gather's addresses and words
 constexpr size_t BF_PIN = 32768, BF_ROUND_SLOT = 40, BF_MAX_ROUNDS = 40, BF_CAP_SLOT = 2048, BF_MAX_ORACLES = 14;
 static_assert(CAP_PIN == BF_PIN + BF_MAX_ROUNDS * BF_ROUND_SLOT, "a commitment's cap lands in the first cap slot");
-static_assert(BF_PIN + BF_MAX_ROUNDS * BF_ROUND_SLOT + BF_MAX_ORACLES * BF_CAP_SLOT <= 65536, "the pinned buffer");
-constexpr uint32_t BF_GROUPS = 32;  // rows of totals of a round's sums (16 words each)
+static_assert(BF_PIN + BF_MAX_ROUNDS * BF_ROUND_SLOT + BF_MAX_ORACLES * BF_CAP_SLOT <= 65536, "the rounds' part");
+constexpr size_t BF_CLASS_PIN = 65536, BF_CLASS_SLOT = 136, BF_MAX_CLASSES = 32;
+constexpr size_t BF_FACTOR_PIN = BF_CLASS_PIN + BF_MAX_CLASSES * BF_CLASS_SLOT, BF_FACTOR_WORDS = 512;
+constexpr size_t GATHER_PIN = BF_FACTOR_PIN + BF_FACTOR_WORDS, GATHER_QUADS = 8192;
+static_assert(GATHER_PIN + 10 * GATHER_QUADS <= ((size_t)1 << 18), "the pinned buffer");
+static_assert(GATHER_PIN % 2 == 0 && BF_CLASS_SLOT % 2 == 0, "64-bit words");
+constexpr uint32_t BF_GROUPS = 32;  // rows of totals of a round's sums (16 words each) and of a class's (64 words)
 
-// BASEFOLD (src/pcs.lisp:581-657) over ncls size classes, ascending, the last one nv: class c's table d_h[k]
-// (2^c EXT8s) joins the message table and the codeword at level nv - c (:590-600, :635-639).  d_cws (optional, and
-// optional per class): the class's codeword ENCODE-EXT(H_c) (2^(c+1) EXT8s) when the caller has it already --
-// encoding is linear, so the codeword of a combination of committed columns is the same combination of their
-// committed codewords (COMBINE-COLUMNS over the codewords) -- else it is encoded here, coordinate by coordinate.
-int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, const uint32_t *const *d_hs,
-                           const uint32_t *rr, const uint32_t *v, int grind_bits, int queries, uint64_t *out_qs,
-                           uint32_t *out_chal, uint32_t *out_final, const uint32_t *const *d_cws) {
+// `quads` (addresses of 16 bytes each in device memory) to the host, four words a quad: the addresses go out and the
+// words come back through pinned memory, one launch and one poll per GATHER_QUADS of them, where a copy of the
+// addresses, a copy of the words and a wait on the stream are 50 us
+static int gather_quads(const std::vector<const uint32_t *> &quads, uint32_t *out) {
+  Context &c = ctx();
+  for (size_t at = 0; at < quads.size(); at += GATHER_QUADS) {
+    const size_t n = std::min(quads.size() - at, GATHER_QUADS);
+    memcpy(c.host_pinned + GATHER_PIN, quads.data() + at, n * sizeof(quads[0]));
+    if (++c.log_seq == 0) ++c.log_seq;
+    constexpr size_t words_at = GATHER_PIN + 2 * GATHER_QUADS;
+    hipLaunchKernelGGL(gather_quads_kernel, dim3((uint32_t)((n + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, c.stream,
+                       reinterpret_cast<const uint32_t *const *>(c.host_pinned_dev + GATHER_PIN), (uint32_t)n,
+                       reinterpret_cast<unsigned long long *>(c.host_pinned_dev + words_at), c.log_seq);
+    EXH_HIP(hipGetLastError());
+    if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(c.host_pinned + words_at), 4 * n, c.log_seq,
+                     out + 4 * at)) {
+      set_error("device-error: an opening's words did not arrive");
+      return E_DEVICE;
+    }
+  }
+  return OK;
+}
+
+bool bf_base_source(const uint32_t *columns, const uint32_t *codewords, int ncols, int c) {
+  // (whole quads are read: a column of 2^c values and its codeword begin on 16 bytes)
+  return columns && codewords && ncols >= 1 && ncols <= BF_BASE_MAX_COLS && c >= 3 &&
+         ((reinterpret_cast<uintptr_t>(columns) | reinterpret_cast<uintptr_t>(codewords)) & 15) == 0;
+}
+
+// BASEFOLD (src/pcs.lisp:581-657) over ncls size classes, ascending, the last one nv: class c's table (2^c EXT8s)
+// joins the message table and the codeword at level nv - c (:590-600, :635-639).  A class given as a table without its
+// codeword is encoded here, coordinate by coordinate (ENCODE-EXT); one given by base columns (BfSource) is read from
+// them where it is needed: encoding is linear, so the codeword of a combination of committed columns is the same
+// combination of their committed codewords.
+int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, const BfSource *src, const uint32_t *rr,
+                           const uint32_t *v, int grind_bits, int queries, uint64_t *out_qs, uint32_t *out_chal,
+                           uint32_t *out_final, BfMore *more_words) {
   Context &c = ctx();
   int status = c.require();
   if (status) return status;
-  if (ncls < 1 || cls[ncls - 1] != nv || queries < 1 || nv > 30) {
+  if (ncls < 1 || ncls > (int)BF_MAX_CLASSES || cls[ncls - 1] != nv || queries < 1 || nv > 30) {
     set_error("invalid-parameter: basefold takes its classes in ascending order, the largest being nv <= 30");
     return E_PARAM;
   }
@@ -1291,174 +1501,318 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
       set_error("invalid-parameter: basefold classes must ascend");
       return E_PARAM;
     }
-  const uint32_t *d_h = d_hs[ncls - 1];
+  const BfSource &top = src[ncls - 1];
   const int fl = nv - 5 > 0 ? nv - 5 : 0;
+  if (fl > (int)BF_MAX_ROUNDS) {
+    set_error("invalid-parameter: basefold rounds beyond the buffers");
+    return E_PARAM;
+  }
   const uint64_t len = (uint64_t)1 << nv;
   Owned mem;
+  auto grid_of = [](uint64_t n) { return dim3((uint32_t)((n + BLOCK - 1) / BLOCK)); };
+  // ENCODE-EXT of a table of 2^cc EXT8s
+  auto encode_ext = [&](const uint32_t *h, int cc) -> uint32_t * {
+    const uint64_t n = (uint64_t)1 << cc;
+    uint32_t *cols = mem.alloc(n * 8), *cwcols = mem.alloc(2 * n * 8), *cw = mem.alloc(2 * n * 8);
+    if (!cols || !cwcols || !cw) {
+      status = E_NOMEM;
+      return nullptr;
+    }
+    hipLaunchKernelGGL(split_coords_kernel, grid_of(n), dim3(BLOCK), 0, c.stream, h, cols, n);
+    if ((status = rs_encode_columns(cols, 8, cc, cwcols))) return nullptr;
+    hipLaunchKernelGGL(join_coords_kernel, grid_of(2 * n), dim3(BLOCK), 0, c.stream, cwcols, cw, 2 * n);
+    return cw;
+  };
+  // The largest class from its base columns: BB variables are left open (see bf_base_sums_kernel), up to the first
+  // level a class joins at, since there the table has to exist; the codeword is formed at level CB.
+  const bool base = !top.h && fl > 0;
+  const int first_join = ncls > 1 ? nv - cls[ncls - 2] : BF_BASE_BITS;
+  const int BB = base ? std::min({BF_BASE_BITS, first_join, fl}) : 0, CB = base ? std::min(BB, 2) : 0;
+  const uint32_t *tt = top.h, *cw = top.cw;
+  if (!base) {
+    if (!tt) {  // (no rounds: the table itself goes out)
+      uint32_t *h = mem.alloc(len * 8);
+      if (!h) return E_NOMEM;
+      combine_few_launch<8>(top.columns, top.ncols, len, top.coef, nullptr, h);
+      tt = h;
+    }
+    if (fl > 0 && !cw && !(cw = encode_ext(tt, nv))) return status;
+  }
   // the folded message tables ping-pong between two buffers (the class's own table is read in round 0 and never
   // written); so do the folded codewords, except that a level with an oracle tree keeps a buffer of its own
-  uint32_t *tt_a = mem.alloc(len * 4 + 8), *tt_b = mem.alloc(len * 2 + 8);
-  uint32_t *cw_b = mem.alloc(len * 8), *cw_c = mem.alloc(len * 4 + 8);
-  uint32_t *cw0 = nullptr, *cols = nullptr, *cwcols = nullptr;
-  const bool given = d_cws && d_cws[ncls - 1];
-  if (!given) {
-    cw0 = mem.alloc(2 * len * 8), cols = mem.alloc(len * 8), cwcols = mem.alloc(2 * len * 8);
-    if (!cw0 || !cols || !cwcols) return E_NOMEM;
-  } else if (ncls > 1) {  // the joining classes add their codewords into the working one
-    cols = mem.alloc(len * 4), cwcols = mem.alloc(len * 8);
-    if (!cols || !cwcols) return E_NOMEM;
-  }
-  const uint32_t max_grid = 1024;
-  uint32_t *partials = mem.alloc((uint64_t)max_grid * 24 + 24), *factors = mem.alloc((uint64_t)nv * 16 + 16);
-  if (!tt_a || !tt_b || !cw_b || !cw_c || !partials || !factors) return E_NOMEM;
-  uint32_t *sums = partials + (uint64_t)max_grid * 24;
-  const uint32_t grid_len = (uint32_t)((len + BLOCK - 1) / BLOCK);
-  // cw = ENCODE-EXT(H) unless given
-  const uint32_t *cw = given ? d_cws[ncls - 1] : cw0;
-  if (!given) {
-    hipLaunchKernelGGL(split_coords_kernel, dim3(grid_len), dim3(BLOCK), 0, c.stream, d_h, cols, len);
-    if ((status = rs_encode_columns(cols, 8, nv, cwcols))) return status;
-    hipLaunchKernelGGL(join_coords_kernel, dim3(2 * grid_len), dim3(BLOCK), 0, c.stream, cwcols, cw0, 2 * len);
-  }
-  // ---- the rounds' split weights: round i sums over the pairs k of variables i+1 .. nv-1; LOW covers a workgroup's
-  // tile, HIGH the rest
-  std::vector<int> low_bits(std::max(fl, 1), 0);
-  std::vector<uint64_t> low_off(std::max(fl, 1), 0), high_off(std::max(fl, 1), 0);
-  uint32_t *weights = nullptr;
-  {
-    std::vector<uint32_t> f((size_t)nv * 16);
-    for (int b = 0; b < nv; b++)
-      for (int k = 0; k < 8; k++) {
-        uint32_t r = rr[(size_t)b * 8 + k] % P;
-        f[((size_t)b * 2) * 8 + k] = to_mont(r);
-        f[((size_t)b * 2 + 1) * 8 + k] = to_mont(fsub(k == 0 ? 1u : 0u, r));
-      }
-    EXH_HIP(hipMemcpyAsync(factors, f.data(), f.size() * 4, hipMemcpyHostToDevice, c.stream));
-    EXH_HIP(hipStreamSynchronize(c.stream));  // `f` is pageable
-    if (fl > BF_MAX_ROUNDS || 2 * fl > 64) {
-      set_error("invalid-parameter: basefold rounds beyond the buffers");
-      return E_PARAM;
+  const uint64_t tt_words = base ? (len >> BB) * 8 : len * 4 + 8, cw_words = base ? (2 * len >> CB) * 8 : len * 8;
+  uint32_t *tt_a = mem.alloc(tt_words + 8), *tt_b = mem.alloc(tt_words / 2 + 8);
+  uint32_t *cw_b = mem.alloc(cw_words), *cw_c = mem.alloc(cw_words / 2 + 8), *factors = mem.alloc((uint64_t)nv * 16 + 16);
+  if (!tt_a || !tt_b || !cw_b || !cw_c || !factors) return E_NOMEM;
+  // ---- the point's factors, staged in pinned memory for the launch that builds the weights
+  uint32_t *pin_factors = c.host_pinned + BF_FACTOR_PIN;
+  static_assert(30 * 16 <= BF_FACTOR_WORDS, "the factors' room");
+  for (int b = 0; b < nv; b++)
+    for (int k = 0; k < 8; k++) {
+      uint32_t r = rr[(size_t)b * 8 + k] % P;
+      pin_factors[((size_t)b * 2) * 8 + k] = to_mont(r);
+      pin_factors[((size_t)b * 2 + 1) * 8 + k] = to_mont(fsub(k == 0 ? 1u : 0u, r));
     }
-    std::vector<int> first, bits;
-    std::vector<uint64_t> off;
-    uint64_t pos = 0;
-    for (int i = 0; i < fl; i++) {
-      const int rest = nv - 1 - i;  // variables of the pairs
-      // (tiles of 2^10 to 2^12 pairs, at least a thousand of them while the table is that large: long tiles in few
-      // workgroups trail their loads one after another, short ones pay the reduction and the atomics per tile)
-      low_bits[i] = std::min(rest, std::min(std::max(rest - 10, 10), 12));
-      low_off[i] = pos, first.push_back(i + 1), bits.push_back(low_bits[i]), off.push_back(pos);
-      pos += (uint64_t)1 << low_bits[i];
-      high_off[i] = pos, first.push_back(i + 1 + low_bits[i]), bits.push_back(rest - low_bits[i]), off.push_back(pos);
-      pos += (uint64_t)1 << (rest - low_bits[i]);
+  // ---- split weights: round i sums over the pairs k of variables i+1 .. nv-1; LOW covers a workgroup's tile, HIGH the
+  // rest.  A class's sums over base columns leave its first bits open and go over the variables above those.
+  struct Split {
+    int low_bits = 0, rest = 0;
+    uint64_t low = 0, high = 0;
+  };
+  std::vector<int> first, bits;
+  std::vector<uint64_t> off;
+  uint64_t pos = 0;
+  auto split = [&](int from, int low_bits) {
+    Split w;
+    w.rest = nv - from, w.low_bits = std::min(w.rest, low_bits);
+    w.low = pos, first.push_back(from), bits.push_back(w.low_bits), off.push_back(pos);
+    pos += (uint64_t)1 << w.low_bits;
+    w.high = pos, first.push_back(from + w.low_bits), bits.push_back(w.rest - w.low_bits), off.push_back(pos);
+    pos += (uint64_t)1 << (w.rest - w.low_bits);
+    return w;
+  };
+  std::vector<Split> round_w(std::max(fl, 1)), class_w(ncls);
+  for (int i = BB; i < fl; i++)
+    // (tiles of 2^10 to 2^12 pairs, at least a thousand of them while the table is that large: long tiles in few
+    // workgroups trail their loads one after another, short ones pay the reduction and the atomics per tile)
+    round_w[i] = split(i + 1, std::min(std::max(nv - 1 - i - 10, 10), 12));
+  auto open_bits = [&](int k) { return k + 1 == ncls ? BB : BF_BASE_BITS; };
+  for (int k = 0; k < ncls; k++)
+    if (!src[k].h && (k + 1 < ncls || base)) {
+      const int rest = cls[k] - open_bits(k);
+      class_w[k] = split(nv - rest, std::min(std::max(rest - 8, 10), 13));
     }
-    if (fl > 0) {
-      weights = mem.alloc(pos * 8);
-      if (!weights) return E_NOMEM;
-      if ((status = eq_tables_launch(8, (int)first.size(), first.data(), bits.data(), off.data(), factors, nv, weights)))
-        return status;
-    }
+  // ---- the sums' totals, cleared by the launch that builds the weights, and the pinned slots
+  const uint64_t round_totals = (uint64_t)std::max(fl, 1) * BF_GROUPS * 16, class_totals = (uint64_t)ncls * BF_GROUPS * 64;
+  const uint64_t total_words = 2 * (round_totals + class_totals) + std::max(fl, 1) + ncls;
+  uint32_t *totals_mem = mem.alloc(total_words), *weights = mem.alloc(pos * 8 + 8);
+  if (!totals_mem || !weights) return E_NOMEM;
+  unsigned long long *totals64 = reinterpret_cast<unsigned long long *>(totals_mem);
+  uint32_t *arrivals = totals_mem + 2 * (round_totals + class_totals);
+  for (size_t t = 0; t < first.size(); t += 64) {
+    const int count = (int)std::min<size_t>(64, first.size() - t);
+    status = eq_tables_launch(8, count, first.data() + t, bits.data() + t, off.data() + t, factors, nv, weights,
+                              t == 0 ? c.host_pinned_dev + BF_FACTOR_PIN : nullptr, totals_mem, t == 0 ? total_words : 0);
+    if (status) return status;
   }
-  EXH_HIP(hipGetLastError());
-  Domain *dom;
-  if ((status = get_domain(nv + 1, &dom))) return status;
-
-  hf::E prf = hf::lift(1, 8), claim = hf::from(v, 8);
-  // y_c = H_c at the point's last c coordinates, for the classes still to join; ysum their sum (:593-595)
-  const uint32_t one8[8] = {1, 0, 0, 0, 0, 0, 0, 0};
-  std::vector<hf::E> yc(ncls, hf::zero(8));
-  hf::E ysum = hf::zero(8);
-  for (int k = 0; k + 1 < ncls; k++) {
-    const uint64_t clen = (uint64_t)1 << cls[k], n_pairs = clen / 2;
-    uint32_t *eqc = tt_a;  // the eq table of the point's tail (at most half of the buffer's room)
-    hipLaunchKernelGGL(eq8_kernel, dim3((uint32_t)((clen + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, c.stream,
-                       factors + (size_t)(nv - cls[k]) * 16, cls[k], eqc, clen);
-    uint32_t grid = (uint32_t)std::min<uint64_t>((n_pairs + BLOCK - 1) / BLOCK, max_grid);
-    hipLaunchKernelGGL(dot_pairs_kernel, dim3(grid), dim3(BLOCK), 0, c.stream, d_hs[k], eqc, n_pairs, partials);
-    hipLaunchKernelGGL(sum_columns_kernel, dim3(24), dim3(BLOCK), 0, c.stream, partials, grid, 24u, sums);
-    uint32_t dots[24];
-    EXH_HIP(hipMemcpyAsync(dots, sums, 96, hipMemcpyDeviceToHost, c.stream));
-    EXH_HIP(hipStreamSynchronize(c.stream));
-    yc[k] = hf::add(hf::from(dots, 8), hf::from(dots + 8, 8));  // even entries' products + odd entries' products
-    ysum = hf::add(ysum, yc[k]);
-  }
-  // ---- the rounds' totals (cleared by a kernel: callers may record this path) and the pinned slots
-  const uint64_t total_words = (uint64_t)std::max(fl, 1) * BF_GROUPS * 16 * 2 + std::max(fl, 1) + 1;
-  uint32_t *totals_mem = mem.alloc(total_words + (total_words & 1));
-  if (!totals_mem) return E_NOMEM;
-  hipLaunchKernelGGL(zero_words_kernel, dim3((uint32_t)((total_words + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, c.stream,
-                     totals_mem, total_words);
-  uint32_t *arrivals = totals_mem + (uint64_t)std::max(fl, 1) * BF_GROUPS * 16 * 2;
   volatile uint32_t *pin = c.host_pinned + BF_PIN;
   uint32_t *pin_dev = c.host_pinned_dev + BF_PIN;
   if (++c.log_seq == 0) ++c.log_seq;  // (a word of an earlier proof carries an earlier number)
   const uint32_t seq = c.log_seq;
-
-  std::vector<OracleTree> oracles;
-  const uint32_t *tt = d_h;  // the table the next step reads
-  uint32_t x[8] = {0};
-  // the launch of round i: fold the table by x (the challenge of round i - 1) when i > 0, sum round i's h0, h1;
-  // with_cw: fold the codeword of level i - 1 as well, into cw_out
-  auto launch_step = [&](int i, bool fold, bool do_sums, uint32_t *cw_out) -> int {
-    BfStepArgs a;
-    memset(&a, 0, sizeof(a));
-    const uint64_t entries = fold ? len >> i : len >> i;  // entries of the table summed (after the fold)
-    (void)entries;
-    const uint64_t n_pairs = (len >> i) / 2;
-    a.tt_in = tt, a.fold = fold ? 1 : 0, a.do_sums = do_sums ? 1 : 0, a.n_pairs = n_pairs;
-    if (fold) a.tt_out = (tt == tt_a) ? tt_b : tt_a;
-    uint32_t tile = 1;
-    if (do_sums) {
-      a.low = weights + low_off[i] * 8, a.high = weights + high_off[i] * 8, a.low_bits = (uint32_t)low_bits[i];
-      tile = (uint32_t)1 << low_bits[i];  // |LOW| pairs: one HIGH weight per workgroup
-    } else {
-      tile = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(n_pairs, 1), 4 * BLOCK);
+  auto groups_of = [](uint32_t workgroups) {
+    uint32_t groups = 1;
+    while (groups * 2 <= BF_GROUPS && groups * 2 <= workgroups) groups *= 2;
+    return groups;
+  };
+  auto class_slot = [&](int k) { return BF_CLASS_PIN + (size_t)k * BF_CLASS_SLOT; };
+  // the sums of class k over its base columns, or h0 and h1 of its table under round nv - c's weights
+  auto launch_class_sums = [&](int k) -> int {
+    unsigned long long *host_out = reinterpret_cast<unsigned long long *>(c.host_pinned_dev + class_slot(k));
+    RoundTotals t{totals64 + round_totals + (uint64_t)k * BF_GROUPS * 64, arrivals + std::max(fl, 1) + k, 1, 64, 200000};
+    if (src[k].h) {
+      const Split &w = round_w[nv - cls[k]];
+      BfStepArgs a;
+      memset(&a, 0, sizeof(a));
+      a.tt_in = src[k].h, a.do_sums = 1, a.n_pairs = (uint64_t)1 << (cls[k] - 1);
+      a.low = weights + w.low * 8, a.high = weights + w.high * 8, a.low_bits = (uint32_t)w.low_bits;
+      const uint64_t tile = (uint64_t)1 << w.low_bits;
+      a.pairs_per_thread = std::max<uint32_t>(1, (uint32_t)(tile / BLOCK));
+      a.tt_blocks = (uint32_t)((a.n_pairs + tile - 1) / tile);
+      t.groups = groups_of(a.tt_blocks), a.totals = t, a.host_out = host_out, a.host_seq = seq;
+      hipLaunchKernelGGL(bf_step_kernel<false>, dim3(a.tt_blocks), dim3(BLOCK), 0, c.stream, a);
+      EXH_HIP(hipGetLastError());
+      return OK;
     }
-    a.pairs_per_thread = std::max<uint32_t>(1, tile / BLOCK);
-    a.tt_blocks = n_pairs ? (uint32_t)((n_pairs + tile - 1) / tile) : 0;
-    for (int k = 0; k < 8; k++) a.r_mont[k] = to_mont(x[k]);
-    if (do_sums) {
-      uint32_t groups = 1;
-      while (groups * 2 <= BF_GROUPS && groups * 2 <= a.tt_blocks) groups *= 2;
-      a.totals.totals = reinterpret_cast<unsigned long long *>(totals_mem) + (uint64_t)i * BF_GROUPS * 16;
-      a.totals.arrivals = arrivals + i;
-      a.totals.groups = groups, a.totals.pstride = 16, a.totals.spin_limit = 200000;
+    BfBaseSumsArgs a;
+    memset(&a, 0, sizeof(a));
+    const int lb = open_bits(k);
+    const Split &w = class_w[k];
+    a.cols = src[k].columns, a.len = (uint64_t)1 << cls[k], a.n_cells = a.len >> lb;
+    a.low = weights + w.low * 8, a.high = weights + w.high * 8, a.low_bits = (uint32_t)w.low_bits;
+    a.tiles = 1u << (w.rest - w.low_bits);
+    for (int j = 0; j < src[k].ncols; j++)
+      for (int q = 0; q < 8; q++) a.coef[j][q] = to_mont(to_mont(src[k].coef[(size_t)j * 8 + q] % P));
+    const uint32_t grid = a.tiles * (uint32_t)src[k].ncols;
+    t.groups = groups_of(grid), a.totals = t, a.host_out = host_out, a.host_seq = seq;
+    c.prof_begin("basefold_base_sums", k, 4 * (uint64_t)src[k].ncols * a.len);
+    hipLaunchKernelGGL(lb == 1 ? bf_base_sums_kernel<1> : lb == 2 ? bf_base_sums_kernel<2> : bf_base_sums_kernel<3>,
+                       dim3(grid), dim3(BLOCK), 0, c.stream, a);
+    c.prof_end();
+    EXH_HIP(hipGetLastError());
+    return OK;
+  };
+  auto await_class = [&](int k, int words, uint32_t *out) -> int {
+    if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(c.host_pinned + class_slot(k)), words + 1,
+                     seq, out) ||
+        out[words]) {
+      set_error("device-error: a basefold class's sums did not arrive");
+      return E_DEVICE;
+    }
+    return OK;
+  };
+  // sum_b eq(r, b) T[b]
+  auto eq_fold = [&](std::vector<hf::E> t, const uint32_t *r) {
+    for (int b = 0; t.size() > 1; b++) {
+      const hf::E rb = hf::from(r + 8 * (size_t)b, 8);
+      for (size_t q = 0; q < t.size() / 2; q++) t[q] = hf::add(hf::mul(rb, hf::sub(t[2 * q + 1], t[2 * q])), t[2 * q]);
+      t.resize(t.size() / 2);
+    }
+    return t[0];
+  };
+  std::vector<uint32_t> class_words(65);
+  auto open_sums = [&](int k, std::vector<hf::E> *t) -> int {
+    const int n = 1 << open_bits(k);
+    if ((status = await_class(k, 8 * n, class_words.data()))) return status;
+    t->clear();
+    for (int b = 0; b < n; b++) t->push_back(hf::from(class_words.data() + 8 * b, 8));
+    return OK;
+  };
+
+  // the launch of round i (level i): fold the table by the challenges it awaits, sum round i's h0, h1; with cw_out
+  // fold the codeword to level i as well
+  std::vector<hf::E> xs;  // the challenges
+  const Domain *dom = nullptr;
+  if (fl > 0) {
+    Domain *d;
+    if ((status = get_domain(nv + 1, &d))) return status;
+    dom = d;
+  }
+  std::vector<OracleTree> oracles;
+  auto launch_step = [&](int i, bool fold, bool do_sums, uint32_t *cw_out) -> int {
+    BfBaseArgs b;
+    memset(&b, 0, sizeof(b));
+    BfStepArgs &a = b.s;
+    const uint64_t n_pairs = (len >> i) / 2;
+    const bool tt_base = base && i <= BB, tt_part = !tt_base || i == BB;  // (below level BB the base columns stand)
+    const bool from_base = fold && tt_base, cw_base = from_base && cw_out && i == CB;
+    a.tt_in = tt, a.fold = fold ? 1 : 0, a.do_sums = do_sums && tt_part ? 1 : 0, a.n_pairs = n_pairs;
+    if (fold && tt_part) a.tt_out = (tt == tt_a) ? tt_b : tt_a;
+    uint64_t tile = std::min<uint64_t>(std::max<uint64_t>(n_pairs, 1), 4 * BLOCK);
+    if (a.do_sums) {
+      const Split &w = round_w[i];
+      a.low = weights + w.low * 8, a.high = weights + w.high * 8, a.low_bits = (uint32_t)w.low_bits;
+      tile = (uint64_t)1 << w.low_bits;  // |LOW| pairs: one HIGH weight per workgroup
+    }
+    a.pairs_per_thread = std::max<uint32_t>(1, (uint32_t)(tile / BLOCK));
+    a.tt_blocks = tt_part ? (uint32_t)((n_pairs + tile - 1) / tile) : 0;
+    if (!xs.empty())
+      for (int k = 0; k < 8; k++) a.r_mont[k] = to_mont(xs.back()[k]);
+    if (a.do_sums) {
+      a.totals = RoundTotals{totals64 + (uint64_t)i * BF_GROUPS * 16, arrivals + i, groups_of(a.tt_blocks), 16, 200000};
       a.host_out = reinterpret_cast<unsigned long long *>(pin_dev + (size_t)i * BF_ROUND_SLOT), a.host_seq = seq;
     }
     uint32_t cw_blocks = 0;
     if (cw_out) {
-      const uint64_t m = (len >> (i - 1));  // elements of the folded codeword: half of level i - 1's 2^(nv + 2 - i)
-      a.cw_in = cw, a.cw_out = cw_out, a.cw_m = m, a.tw_inv2 = dom->tw_inv2 + dom->off[i - 1];
-      cw_blocks = (uint32_t)((m + BLOCK - 1) / BLOCK);
+      a.cw_in = cw, a.cw_out = cw_out, a.cw_m = 2 * len >> i;  // elements of the folded codeword
+      a.tw_inv2 = dom->tw_inv2 + dom->off[i - 1];
+      cw_blocks = (uint32_t)((a.cw_m + BLOCK - 1) / BLOCK);
     }
-    if (a.tt_blocks + cw_blocks == 0) return OK;
-    c.prof_begin("basefold_step", i, (fold ? 3 : 2) * n_pairs * 32 * (do_sums || fold ? 1 : 0) + (cw_out ? 3 * a.cw_m * 32 : 0));
-    if (fold)
-      hipLaunchKernelGGL(bf_step_kernel<true>, dim3(a.tt_blocks + cw_blocks), dim3(BLOCK), 0, c.stream, a);
-    else
-      hipLaunchKernelGGL(bf_step_kernel<false>, dim3(a.tt_blocks + cw_blocks), dim3(BLOCK), 0, c.stream, a);
+    if (from_base) {
+      b.cols = top.columns, b.cws = top.codewords, b.col_len = len, b.cw_len = 2 * len, b.ncols = (uint32_t)top.ncols;
+      b.tw0 = dom->tw_inv2 + dom->off[0], b.tw1 = i >= 2 ? dom->tw_inv2 + dom->off[1] : nullptr;
+      const hf::E one = hf::lift(1, 8);
+      for (int j = 0; j < top.ncols; j++) {
+        const hf::E cj = hf::from(top.coef + 8 * (size_t)j, 8);
+        std::vector<hf::E> eqs{cj};
+        for (int q = 0; q < i; q++) {  // entry b of 2^i: bit q of b goes with challenge q
+          std::vector<hf::E> next(eqs.size() * 2);
+          for (size_t e = 0; e < eqs.size(); e++) {
+            next[e + eqs.size()] = hf::mul(eqs[e], xs[q]);
+            next[e] = hf::sub(eqs[e], next[e + eqs.size()]);
+          }
+          eqs.swap(next);
+        }
+        for (size_t e = 0; e < eqs.size(); e++)
+          for (int k = 0; k < 8; k++) b.tt_coef[j][e][k] = to_mont(eqs[e][k]);
+        if (cw_base) {
+          const hf::E x1 = i >= 2 ? xs[1] : one;
+          const hf::E prods[4] = {cj, hf::mul(cj, xs[0]), hf::mul(cj, x1), hf::mul(hf::mul(cj, xs[0]), x1)};
+          for (int e = 0; e < 4; e++)
+            for (int k = 0; k < 8; k++) b.cw_coef[j][e][k] = to_mont(prods[e][k]);
+        }
+      }
+    }
+    const dim3 grid(a.tt_blocks + cw_blocks);
+    if (grid.x == 0) return OK;
+    c.prof_begin("basefold_step", i,
+                 (tt_part ? (from_base ? 4 * (uint64_t)top.ncols * len + 64 * n_pairs : (fold ? 3 : 2) * n_pairs * 32) : 0) +
+                     (cw_out ? (cw_base ? 8 * (uint64_t)top.ncols * len + 32 * a.cw_m : 3 * a.cw_m * 32) : 0));
+    if (from_base) {
+      if (i == 1)
+        hipLaunchKernelGGL((bf_base_kernel<1, 1>), grid, dim3(BLOCK), 0, c.stream, b);
+      else if (i == 2 && tt_part)
+        hipLaunchKernelGGL((bf_base_kernel<2, 2>), grid, dim3(BLOCK), 0, c.stream, b);
+      else if (i == 2)
+        hipLaunchKernelGGL((bf_base_kernel<0, 2>), grid, dim3(BLOCK), 0, c.stream, b);
+      else
+        hipLaunchKernelGGL((bf_base_kernel<3, 3>), grid, dim3(BLOCK), 0, c.stream, b);
+    } else if (fold) {
+      hipLaunchKernelGGL(bf_step_kernel<true>, grid, dim3(BLOCK), 0, c.stream, a);
+    } else {
+      hipLaunchKernelGGL(bf_step_kernel<false>, grid, dim3(BLOCK), 0, c.stream, a);
+    }
     c.prof_end();
     EXH_HIP(hipGetLastError());
-    if (fold) tt = a.tt_out;
+    if (fold && tt_part) tt = a.tt_out;
     if (cw_out) cw = cw_out;
     return OK;
   };
-  if (fl > 0 && (status = launch_step(0, false, true, nullptr))) return status;
+  if (base) {
+    if ((status = launch_class_sums(ncls - 1))) return status;
+  } else if (fl > 0 && (status = launch_step(0, false, true, nullptr))) {
+    return status;
+  }
+  // y_c = H_c at the point's last c coordinates, for the classes still to join; ysum their sum (:593-595)
+  std::vector<hf::E> yc(ncls, hf::zero(8));
+  hf::E ysum = hf::zero(8);
+  auto small_table = [&](int k) { return src[k].h && nv - cls[k] >= fl; };  // no round has its weights: 2^5 elements at most
+  for (int k = 0; k + 1 < ncls; k++)
+    if (!small_table(k) && (status = launch_class_sums(k))) return status;
+  for (int k = 0; k + 1 < ncls; k++) {
+    const uint32_t *point = rr + 8 * (size_t)(nv - cls[k]);
+    if (small_table(k)) {
+      const uint64_t n = (uint64_t)1 << cls[k];
+      std::vector<uint32_t> h(n * 8);
+      std::vector<const uint32_t *> quads;
+      for (uint64_t q = 0; q < 2 * n; q++) quads.push_back(src[k].h + 4 * q);
+      if ((status = gather_quads(quads, h.data()))) return status;
+      yc[k] = hf::mle_eval(h.data(), cls[k], point, 8);
+    } else if (src[k].h) {
+      if ((status = await_class(k, 16, class_words.data()))) return status;
+      yc[k] = eq_fold({hf::from(class_words.data(), 8), hf::from(class_words.data() + 8, 8)}, point);
+    } else {
+      std::vector<hf::E> t;
+      if ((status = open_sums(k, &t))) return status;
+      yc[k] = eq_fold(t, point);
+    }
+    ysum = hf::add(ysum, yc[k]);
+  }
+
+  hf::E prf = hf::lift(1, 8), claim = hf::from(v, 8);
+  std::vector<hf::E> open_t;  // the sums over the open variables, folded by the challenges so far
+  if (base && (status = open_sums(ncls - 1, &open_t))) return status;
   size_t cap_slots = 0;
   for (int i = 0; i < fl; i++) {
     // ---- the round's message from h0, h1
-    uint32_t hh[17];
-    if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(pin + (size_t)i * BF_ROUND_SLOT), 17, seq,
-                     hh) ||
-        hh[16]) {
-      set_error("device-error: a basefold round's sums did not arrive");
-      return E_DEVICE;
+    hf::E h0, h1;
+    if (i < BB) {
+      std::vector<hf::E> even, odd;
+      for (size_t q = 0; q < open_t.size(); q += 2) even.push_back(open_t[q]), odd.push_back(open_t[q + 1]);
+      h0 = eq_fold(even, rr + 8 * (size_t)(i + 1)), h1 = eq_fold(odd, rr + 8 * (size_t)(i + 1));
+    } else {
+      uint32_t hh[17];
+      if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(pin + (size_t)i * BF_ROUND_SLOT), 17, seq,
+                       hh) ||
+          hh[16]) {
+        set_error("device-error: a basefold round's sums did not arrive");
+        return E_DEVICE;
+      }
+      h0 = hf::from(hh, 8), h1 = hf::from(hh + 8, 8);
     }
-    const hf::E h0 = hf::from(hh, 8), h1 = hf::from(hh + 8, 8);
     const hf::E ri = hf::from(rr + 8 * (size_t)i, 8), one_r = hf::sub(hf::lift(1, 8), ri);
     const hf::E eqx[3] = {one_r, ri, hf::sub(hf::scale(ri, 2), one_r)};
     const hf::E hx[3] = {h0, h1, hf::sub(hf::scale(h1, 2), h0)};
-    uint32_t ev[24];
+    uint32_t ev[24], x[8];
     const hf::E a_term = ncls > 1 ? hf::mul(prf, ysum) : hf::zero(8);  // the classes still to join, :607-612
     for (int parity = 0; parity < 3; parity++) {
       hf::E t = hf::mul(hf::mul(prf, eqx[parity]), hx[parity]);
@@ -1472,9 +1826,15 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
       return E_REJECT;
     }
     tr.challenge(8, x);
+    xs.push_back(hf::from(x, 8));
     if (out_chal) memcpy(out_chal + 8 * i, x, 32);
-    claim = hf::lagrange({hf::from(ev, 8), hf::from(ev + 8, 8), hf::from(ev + 16, 8)}, hf::from(x, 8));
-    prf = hf::mul(prf, hf::eq1(hf::from(rr + 8 * i, 8), hf::from(x, 8)));
+    claim = hf::lagrange({hf::from(ev, 8), hf::from(ev + 8, 8), hf::from(ev + 16, 8)}, xs.back());
+    prf = hf::mul(prf, hf::eq1(hf::from(rr + 8 * i, 8), xs.back()));
+    if (i < BB) {
+      for (size_t q = 0; q < open_t.size() / 2; q++)
+        open_t[q] = hf::add(open_t[2 * q], hf::mul(xs.back(), hf::sub(open_t[2 * q + 1], open_t[2 * q])));
+      open_t.resize(open_t.size() / 2);
+    }
     // ---- level l: fold the table and the codeword by x; an oracle tree over the folded codeword; the joins
     const int l = i + 1;
     const uint64_t cur = len >> i;  // elements of the folded codeword
@@ -1482,7 +1842,7 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     bool joins = false;
     for (int k = 0; k + 1 < ncls; k++) joins = joins || nv - cls[k] == l;
     uint32_t *cw_out = nullptr;
-    if (l < fl) {  // (the last level's codeword is never looked at)
+    if (l < fl && l >= CB) {  // (the last level's codeword is never looked at)
       if (oracle) {
         if (oracles.size() >= BF_MAX_ORACLES) {
           set_error("invalid-parameter: basefold oracle levels beyond the buffers");
@@ -1492,7 +1852,7 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
         if (!cw_out) return E_NOMEM;
       } else {
         cw_out = (cw == cw_b) ? cw_c : cw_b;
-        if (cur * 8 > (cw_out == cw_b ? len * 8 : len * 4)) cw_out = cw_b;  // (only level 1 needs the larger one)
+        if (cur * 8 > (cw_out == cw_b ? cw_words : cw_words / 2)) cw_out = cw_b;  // (only the first needs the larger one)
       }
     }
     // the next round's sums ride on the fold unless a class joins in between
@@ -1520,36 +1880,32 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
         set_error("device-error: a basefold oracle's cap did not arrive");
         return E_DEVICE;
       }
-      std::vector<uint8_t> cap(32 * rows);
-      memcpy(cap.data(), cap_words.data(), 32 * rows);
-      if ((status = tr.send_bytes(cap.data(), (int64_t)(32 * rows), nullptr))) return status;
+      if ((status = tr.send_bytes(reinterpret_cast<const uint8_t *>(cap_words.data()), (int64_t)(32 * rows), nullptr)))
+        return status;
       oracles.push_back(o);
     }
     if (joins) {
+      static const uint32_t one8[8] = {1, 0, 0, 0, 0, 0, 0, 0};
       for (int k = 0; k + 1 < ncls; k++)  // the classes that join at this level, :635-639
         if (nv - cls[k] == l) {
           const uint64_t clen = (uint64_t)1 << cls[k];
-          const uint32_t gl = (uint32_t)((clen + BLOCK - 1) / BLOCK);
-          uint32_t *tt_w = const_cast<uint32_t *>(tt), *cw_w = const_cast<uint32_t *>(cw);  // folded: ours to write
-          scale_add_launch<8>(tt_w, d_hs[k], tt_w, clen, one8);
+          uint32_t *tt_w = const_cast<uint32_t *>(tt);  // folded: ours to write
+          if (src[k].h)
+            scale_add_launch<8>(tt_w, src[k].h, tt_w, clen, one8);
+          else
+            combine_few_launch<8>(src[k].columns, src[k].ncols, clen, src[k].coef, tt_w, tt_w);
           if (l < fl) {
-            const uint32_t *cwk = d_cws ? d_cws[k] : nullptr;
-            if (!cwk) {  // ENCODE-EXT of the class's table, into a buffer of its own
-              uint32_t *joined = mem.alloc(2 * clen * 8);
-              if (!joined) return E_NOMEM;
-              hipLaunchKernelGGL(split_coords_kernel, dim3(gl), dim3(BLOCK), 0, c.stream, d_hs[k], cols, clen);
-              if ((status = rs_encode_columns(cols, 8, cls[k], cwcols))) return status;
-              hipLaunchKernelGGL(join_coords_kernel, dim3(2 * gl), dim3(BLOCK), 0, c.stream, cwcols, joined, 2 * clen);
-              cwk = joined;
-            }
-            if (oracle) {  // the oracle keeps the codeword it hashed: the sum goes to a buffer of its own
-              uint32_t *sum = mem.alloc(2 * clen * 8);
-              if (!sum) return E_NOMEM;
-              scale_add_launch<8>(cw, cwk, sum, 2 * clen, one8);
-              cw = sum;
+            // (an oracle keeps the codeword it hashed: the sum goes to a buffer of its own then)
+            uint32_t *cw_w = oracle ? mem.alloc(2 * clen * 8) : const_cast<uint32_t *>(cw);
+            if (!cw_w) return E_NOMEM;
+            if (src[k].h) {
+              const uint32_t *cwk = src[k].cw ? src[k].cw : encode_ext(src[k].h, cls[k]);
+              if (!cwk) return status;
+              scale_add_launch<8>(cw, cwk, cw_w, 2 * clen, one8);
             } else {
-              scale_add_launch<8>(cw_w, cwk, cw_w, 2 * clen, one8);
+              combine_few_launch<8>(src[k].codewords, src[k].ncols, 2 * clen, src[k].coef, cw, cw_w);
             }
+            cw = cw_w;
           }
           ysum = hf::sub(ysum, yc[k]);
         }
@@ -1560,8 +1916,9 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
   // the final table in the clear, the final claim, grinding, the query positions
   uint64_t mlen = len >> fl;
   std::vector<uint32_t> m(mlen * 8);
-  EXH_HIP(hipMemcpyAsync(m.data(), tt, mlen * 32, hipMemcpyDeviceToHost, c.stream));
-  EXH_HIP(hipStreamSynchronize(c.stream));
+  std::vector<const uint32_t *> quads;
+  for (uint64_t q = 0; q < 2 * mlen; q++) quads.push_back(tt + 4 * q);
+  if ((status = gather_quads(quads, m.data()))) return status;
   uint64_t dims[2] = {mlen, 8};
   if ((status = tr.send(m.data(), 2, dims, nullptr))) return status;
   if (out_final) memcpy(out_final, m.data(), mlen * 32);
@@ -1575,52 +1932,48 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
   tr.challenge_bits(nv - 1, queries, qs.data());
   if (out_qs) memcpy(out_qs, qs.data(), 8 * (size_t)queries);
   // ---- the oracle openings, recorded (src/pcs.lisp:651-655): every queried leaf's four symbols and every path's
-  // siblings of every oracle in one gather of 8-word segments and one copy back
-  if (!oracles.empty()) {
-    std::vector<const uint32_t *> segs;
-    for (const OracleTree &o : oracles)
-      for (int q = 0; q < queries; q++) {
-        const uint64_t li = qs[q] >> o.level;
-        for (int s = 0; s < 4; s++) segs.push_back(o.cw + (4 * li + s) * 8);
-        uint64_t level_start = 0, n = o.nleaves, idx = li;
-        for (int d = 0; d < o.lc; d++) {
-          segs.push_back(o.levels + (level_start + (idx ^ 1)) * 8);
-          level_start += n;
-          n /= 2;
-          idx >>= 1;
-        }
+  // siblings of every oracle, and whatever else the caller opens at these positions, in one gather
+  quads.clear();
+  auto digest_quads = [&](const uint32_t *d) { quads.push_back(d), quads.push_back(d + 4); };
+  for (const OracleTree &o : oracles)
+    for (int q = 0; q < queries; q++) {
+      const uint64_t li = qs[q] >> o.level;
+      for (int sy = 0; sy < 4; sy++) digest_quads(o.cw + (4 * li + sy) * 8);
+      uint64_t level_start = 0, n = o.nleaves, idx = li;
+      for (int d = 0; d < o.lc; d++) {
+        digest_quads(o.levels + (level_start + (idx ^ 1)) * 8);
+        level_start += n;
+        n /= 2;
+        idx >>= 1;
       }
-    const size_t nseg = segs.size();
-    uint32_t *d_ptrs = mem.alloc(nseg * 2 + 2), *d_out = mem.alloc(nseg * 8);
-    if (!d_ptrs || !d_out) return E_NOMEM;
-    std::vector<uint32_t> got(nseg * 8);
-    EXH_HIP(hipMemcpyAsync(d_ptrs, segs.data(), nseg * 8, hipMemcpyHostToDevice, c.stream));
-    hipLaunchKernelGGL(gather8_kernel, dim3((uint32_t)((nseg * 8 + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, c.stream,
-                       reinterpret_cast<const uint32_t *const *>(d_ptrs), (uint32_t)nseg, d_out);
-    EXH_HIP(hipGetLastError());
-    EXH_HIP(hipMemcpyAsync(got.data(), d_out, nseg * 32, hipMemcpyDeviceToHost, c.stream));
-    EXH_HIP(hipStreamSynchronize(c.stream));
-    size_t at = 0;
-    for (const OracleTree &o : oracles) {
-      std::vector<uint32_t> leaves((size_t)queries * 32);  // (Q, 8 rows, 4 symbols): row d holds coordinate d
-      std::vector<uint32_t> path;
-      for (int q = 0; q < queries; q++) {
-        for (int s = 0; s < 4; s++, at++)
-          for (int d = 0; d < 8; d++) leaves[((size_t)q * 8 + d) * 4 + s] = got[at * 8 + d];
-        for (int d = 0; d < o.lc; d++, at++) path.insert(path.end(), got.begin() + at * 8, got.begin() + at * 8 + 8);
-      }
-      uint64_t d3[3] = {(uint64_t)queries, 8, 4};
-      if ((status = tr.send(leaves.data(), 3, d3, nullptr, false))) return status;
-      if ((status = tr.send_bytes((const uint8_t *)path.data(), (int64_t)path.size() * 4, nullptr, false))) return status;
     }
+  const size_t oracle_quads = quads.size();
+  if (more_words) more_words->segments(qs.data(), &quads);
+  std::vector<uint32_t> got(quads.size() * 4);
+  if ((status = gather_quads(quads, got.data()))) return status;
+  const uint32_t *at = got.data();
+  for (const OracleTree &o : oracles) {
+    std::vector<uint32_t> leaves((size_t)queries * 32);  // (Q, 8 rows, 4 symbols): row d holds coordinate d
+    std::vector<uint32_t> path;
+    for (int q = 0; q < queries; q++) {
+      for (int sy = 0; sy < 4; sy++, at += 8)
+        for (int d = 0; d < 8; d++) leaves[((size_t)q * 8 + d) * 4 + sy] = at[d];
+      path.insert(path.end(), at, at + 8 * (size_t)o.lc);
+      at += 8 * (size_t)o.lc;
+    }
+    uint64_t d3[3] = {(uint64_t)queries, 8, 4};
+    if ((status = tr.send(leaves.data(), 3, d3, nullptr, false))) return status;
+    if ((status = tr.send_bytes((const uint8_t *)path.data(), (int64_t)path.size() * 4, nullptr, false))) return status;
   }
+  if (more_words) more_words->words.assign(got.begin() + 4 * oracle_quads, got.end());
   return OK;
 }
 
 int basefold_prove(Transcript &tr, int nv, const uint32_t *rr, const uint32_t *v, const uint32_t *d_h, int grind_bits,
                    int queries, uint64_t *out_qs, uint32_t *out_chal, uint32_t *out_final, const uint32_t *d_cw) {
-  return basefold_prove_classes(tr, nv, 1, &nv, &d_h, rr, v, grind_bits, queries, out_qs, out_chal, out_final,
-                                d_cw ? &d_cw : nullptr);
+  BfSource src;
+  src.h = d_h, src.cw = d_cw;
+  return basefold_prove_classes(tr, nv, 1, &nv, &src, rr, v, grind_bits, queries, out_qs, out_chal, out_final);
 }
 
 // The final opening over several size classes, one key per class, each a unit of its own with its own tree:
@@ -1637,49 +1990,65 @@ int pcs_open(Transcript &tr, int nv, int nkeys, const OpenClass *keys, const uin
     return E_PARAM;
   }
   Owned mem;
-  std::vector<int> cls(nkeys);
-  std::vector<const uint32_t *> hs(nkeys), cws(nkeys, nullptr);
+  std::vector<int> cls(nkeys), depth(nkeys, 0);
+  std::vector<BfSource> src(nkeys);
   for (int k = 0; k < nkeys; k++) {
-    cls[k] = keys[k].c;
-    if (keys[k].c < 1 || keys[k].c > 30 || keys[k].ncols < 1) {
+    const OpenClass &key = keys[k];
+    cls[k] = key.c;
+    if (key.c < 1 || key.c > 30 || key.ncols < 1) {
       set_error("invalid-parameter: opening key");
       return E_PARAM;
     }
-    uint32_t *h = mem.alloc(((uint64_t)8) << keys[k].c);
+    if (key.d_levels) depth[k] = cap_level_of((uint64_t)1 << (key.c - 1));
+    if (bf_base_source(key.d_columns, key.d_codewords, key.ncols, key.c)) {
+      src[k].columns = key.d_columns, src[k].codewords = key.d_codewords, src[k].coef = key.coef, src[k].ncols = key.ncols;
+      continue;
+    }
+    uint32_t *h = mem.alloc(((uint64_t)8) << key.c);
     if (!h) return E_NOMEM;
-    if ((status = combine_columns_device(8, keys[k].d_columns, keys[k].ncols, (uint64_t)1 << keys[k].c, keys[k].coef, h)))
-      return status;
-    hs[k] = h;
+    if ((status = combine_columns_device(8, key.d_columns, key.ncols, (uint64_t)1 << key.c, key.coef, h))) return status;
+    src[k].h = h;
     // ENCODE-EXT of the combined column by the encoder's linearity: the same combination of the committed
     // codewords (2^(c+1) symbols per column), no transform
-    if (keys[k].d_codewords) {
-      uint32_t *cwk = mem.alloc(((uint64_t)16) << keys[k].c);
+    if (key.d_codewords) {
+      uint32_t *cwk = mem.alloc(((uint64_t)16) << key.c);
       if (!cwk) return E_NOMEM;
-      if ((status = combine_columns_device(8, keys[k].d_codewords, keys[k].ncols, (uint64_t)2 << keys[k].c,
-                                           keys[k].coef, cwk)))
+      if ((status = combine_columns_device(8, key.d_codewords, key.ncols, (uint64_t)2 << key.c, key.coef, cwk)))
         return status;
-      cws[k] = cwk;
+      src[k].cw = cwk;
     }
   }
   std::vector<uint64_t> qs(queries > 0 ? queries : 1);
-  if ((status = basefold_prove_classes(tr, nv, nkeys, cls.data(), hs.data(), rr, v, grind_bits, queries, qs.data(),
-                                       nullptr, nullptr, cws.data())))
+  // OPEN-QUERIES rides on BaseFold's own gather: per key the queried leaves' rows, then their paths' siblings
+  BfMore more;
+  more.segments = [&](const uint64_t *at, std::vector<const uint32_t *> *quads) {
+    for (int k = 0; k < nkeys; k++) {
+      const OpenClass &key = keys[k];
+      const uint64_t nleaves = (uint64_t)1 << (key.c - 1);
+      for (int q = 0; q < queries; q++)
+        for (int j = 0; j < key.ncols; j++)
+          quads->push_back(key.d_codewords + (uint64_t)j * ((uint64_t)2 << key.c) + 4 * (at[q] >> (nv - key.c)));
+      for (int q = 0; q < queries; q++)
+        for (int d = 0; d < depth[k]; d++) {
+          const uint64_t start = 2 * nleaves - 2 * (nleaves >> d);
+          const uint32_t *digest = key.d_levels + (start + (((at[q] >> (nv - key.c)) >> d) ^ 1)) * 8;
+          quads->push_back(digest), quads->push_back(digest + 4);
+        }
+    }
+  };
+  if ((status = basefold_prove_classes(tr, nv, nkeys, cls.data(), src.data(), rr, v, grind_bits, queries, qs.data(),
+                                       nullptr, nullptr, &more)))
     return status;
   if (out_qs) memcpy(out_qs, qs.data(), 8 * (size_t)queries);
+  const uint32_t *at = more.words.data();
   for (int k = 0; k < nkeys; k++) {
-    const OpenClass &key = keys[k];
-    std::vector<uint64_t> leaves(queries);
-    for (int q = 0; q < queries; q++) leaves[q] = qs[q] >> (nv - key.c);
-    const int max_depth = cap_level_of((uint64_t)1 << (key.c - 1));
-    std::vector<uint32_t> rows((size_t)queries * key.ncols * 4);
-    std::vector<uint8_t> paths((size_t)queries * max_depth * 32 + 1);
-    int depth = 0;
-    if ((status = open_queries_device(key.d_codewords, key.ncols, key.c, key.d_levels, leaves.data(), queries,
-                                      rows.data(), paths.data(), &depth)))
+    uint64_t d3[3] = {(uint64_t)queries, (uint64_t)keys[k].ncols, 4};
+    if ((status = tr.send(at, 3, d3, nullptr, false))) return status;
+    at += (size_t)queries * keys[k].ncols * 4;
+    const size_t path_words = (size_t)queries * depth[k] * 8;
+    if ((status = tr.send_bytes(reinterpret_cast<const uint8_t *>(at), (int64_t)path_words * 4, nullptr, false)))
       return status;
-    uint64_t d3[3] = {(uint64_t)queries, (uint64_t)key.ncols, 4};
-    if ((status = tr.send(rows.data(), 3, d3, nullptr, false))) return status;
-    if ((status = tr.send_bytes(paths.data(), (int64_t)queries * depth * 32, nullptr, false))) return status;
+    at += path_words;
   }
   return OK;
 }

@@ -4,6 +4,9 @@
 #pragma once
 #include <stdint.h>
 
+#include <functional>
+#include <vector>
+
 #include "transcript.hpp"
 
 namespace exh {
@@ -43,11 +46,25 @@ int basefold_prove(Transcript &tr, int nv, const uint32_t *rr, const uint32_t *v
                    const uint32_t *d_cw = nullptr);
 int basefold_verify(Transcript &tr, int nv, const uint32_t *rr, const uint32_t *v, int grind_bits, int queries,
                     uint64_t *out_qs);
-// BASEFOLD over several size classes (ascending, the last one nv): class c's table d_hs[k] joins at level nv - c
-// d_cws (optional): per class its codeword as for basefold_prove, or null entries
-int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, const uint32_t *const *d_hs,
-                           const uint32_t *rr, const uint32_t *v, int grind_bits, int queries, uint64_t *out_qs,
-                           uint32_t *out_chal, uint32_t *out_final, const uint32_t *const *d_cws = nullptr);
+// What a size class brings to BASEFOLD: its table of 2^c EXT8s on the device (h), with its codeword (cw, 2^(c+1) EXT8s)
+// when the caller has it; or the few base columns, their committed codewords and the EXT8 coefficients (host) whose
+// combination that table is, which is then never formed in full (bf_base_source says when that is possible).
+struct BfSource {
+  const uint32_t *h = nullptr, *cw = nullptr;
+  const uint32_t *columns = nullptr, *codewords = nullptr, *coef = nullptr;
+  int ncols = 0;
+};
+bool bf_base_source(const uint32_t *columns, const uint32_t *codewords, int ncols, int c);
+// more device words the opened positions call for: `segments` appends addresses of 16-byte quads once the positions
+// are known, `words` receives their contents (four words a quad, in order)
+struct BfMore {
+  std::function<void(const uint64_t *qs, std::vector<const uint32_t *> *quads)> segments;
+  std::vector<uint32_t> words;
+};
+// BASEFOLD over several size classes (ascending, the last one nv): class c's table joins at level nv - c
+int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, const BfSource *src, const uint32_t *rr,
+                           const uint32_t *v, int grind_bits, int queries, uint64_t *out_qs, uint32_t *out_chal,
+                           uint32_t *out_final, BfMore *more = nullptr);
 // one key of the final opening: a size class, a unit of its own with its own tree
 struct OpenClass {
   int c = 0, ncols = 0;

@@ -11,7 +11,7 @@ Context &ctx() { return t_ctx ? *t_ctx : g_ctx; }
 void use_context(Context *c) { t_ctx = c; }
 
 static int pinned_buffer(Context &c) {
-  c.host_pinned_words = 1 << 16;
+  c.host_pinned_words = 1 << 18;
   // coherent and mapped: a kernel writes a sumcheck's logs into it directly and the host polls for them
   EXH_HIP(hipHostMalloc((void **)&c.host_pinned, c.host_pinned_words * 4, hipHostMallocMapped | hipHostMallocCoherent));
   EXH_HIP(hipHostGetDevicePointer((void **)&c.host_pinned_dev, c.host_pinned, 0));

@@ -78,6 +78,12 @@ EXH_HD uint32_t mont_reduce4(uint64_t t) {
   return umin32(r, r + P);
 }
 EXH_HD uint32_t mont_mul(uint32_t a, uint32_t b) { return mont_reduce((uint64_t)a * b); }
+// Between the products of a longer sum: a sum t < 2^64 whose high word is below 2 p brought below p 2^32 (the same
+// residue).  Two more products below p^2 then keep it below p 2^32 + 2 p^2 < 2^64 with a high word below 2 p again.
+EXH_HD uint64_t mont_lazy(uint64_t t) {
+  const uint32_t hi = (uint32_t)(t >> 32);
+  return (uint64_t)umin32(hi, hi - P) << 32 | (uint32_t)t;
+}
 // exact a b mod p (two reductions; host-side helpers and rare device paths)
 EXH_HD uint32_t fmul(uint32_t a, uint32_t b) { return mont_mul(mont_mul(a, b), R2); }
 EXH_HD uint32_t to_mont(uint32_t a) { return mont_mul(a, R2); }

@@ -446,9 +446,10 @@ int eq_table_device(int D, int k, const uint32_t *r, uint32_t *d_out) {
 
 // Eq tables over ranges of a point's variables, one launch: table k covers the variables [first[k], first[k] +
 // bits[k]) and lands at d_out + off[k] * D (2^bits[k] elements); d_factors holds (r_v R, (1 - r_v) R) per variable,
-// 2 n_vars D words.  At most 64 tables.  Enqueued on the context's stream; nothing is waited for.
-int eq_tables_launch(int D, int count, const int *first, const int *bits, const uint64_t *off,
-                     const uint32_t *d_factors, int n_vars, uint32_t *d_out) {
+// 2 n_vars D words.  At most 64 tables.  Enqueued on the context's stream; nothing is waited for.  With `staged` the
+// factors are taken from there (pinned host memory) and left at d_factors; the launch also clears zero_words words.
+int eq_tables_launch(int D, int count, const int *first, const int *bits, const uint64_t *off, uint32_t *d_factors,
+                     int n_vars, uint32_t *d_out, const uint32_t *staged, uint32_t *zero, uint64_t zero_words) {
   Context &c = ctx();
   if (count < 1 || count > 64 || n_vars > MAXROUNDS || (D != 4 && D != 8)) {
     set_error("invalid-parameter: eq tables (at most 64 tables over at most 48 variables)");
@@ -462,13 +463,13 @@ int eq_tables_launch(int D, int count, const int *first, const int *bits, const 
     eqt.off[k] = off[k], eqt.first[k] = first[k], eqt.bits[k] = bits[k];
     total += (uint64_t)1 << bits[k];
   }
-  const uint32_t grid = (uint32_t)((total + BLOCK - 1) / BLOCK);
+  const uint32_t grid = (uint32_t)((std::max(total, zero_words / 4) + BLOCK - 1) / BLOCK), words = (uint32_t)(2 * n_vars * D);
   if (D == 4)
-    hipLaunchKernelGGL(eq_tables_kernel<4>, dim3(grid), dim3(BLOCK), 0, c.stream, eqt, d_factors,
-                       (uint32_t)(2 * n_vars * D), d_out, total, nullptr, (uint64_t)0);
+    hipLaunchKernelGGL(eq_tables_kernel<4>, dim3(grid), dim3(BLOCK), 0, c.stream, eqt, d_factors, words, d_out, total,
+                       zero, zero_words, staged, words, d_factors);
   else
-    hipLaunchKernelGGL(eq_tables_kernel<8>, dim3(grid), dim3(BLOCK), 0, c.stream, eqt, d_factors,
-                       (uint32_t)(2 * n_vars * D), d_out, total, nullptr, (uint64_t)0);
+    hipLaunchKernelGGL(eq_tables_kernel<8>, dim3(grid), dim3(BLOCK), 0, c.stream, eqt, d_factors, words, d_out, total,
+                       zero, zero_words, staged, words, d_factors);
   EXH_HIP(hipGetLastError());
   return OK;
 }

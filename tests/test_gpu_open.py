@@ -159,3 +159,15 @@ def test_mixed_height_trees(height, inject_at):
             assert not sa.check_path(leaves[i], np.array(path).reshape(-1, 32), i, root)
     for t in [tl, levels] + ti:
         t.free()
+
+
+@pytest.mark.parametrize("classes", [[(6, 1)], [(7, 3)], [(8, 8)], [(9, 9)], [(10, 3), (13, 2)], [(11, 1), (13, 8)],
+                                     [(5, 3), (9, 4)], [(9, 12), (12, 2)], [(9, 2), (12, 12)], [(5, 9), (8, 2)],
+                                     [(12, 1), (13, 1)], [(4, 1), (5, 2)]])
+def test_openings_from_base_columns(classes):
+    """The opening whose first rounds are answered from the base columns: one, two and three open variables (as many
+    as there are rounds, and up to the first level a class joins at), the most columns that take that way and one
+    more, classes given one way joining a largest class given the other, and the sizes without any round."""
+    if max(c for c, _ in classes) <= 5:  # (no round: nothing joins, so only the largest class is opened)
+        classes = classes[-1:]
+    test_opening_matches_the_oracle_and_verifies(classes)
