@@ -45,7 +45,7 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "231e5e376de79cc5846c1066f523eebba93af71672a4413b12058045d92f2105",
+    "kernel_sources_sha256": "cf29373c05cd0362b530efea8ede22474ab9d02e96d71e4fbb5537d908d9df26",
     "traffic": {("round_nodes_base", 24): 204058883, ("round_fold2_base", 24): 404005645},
     # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), 272 multiply-adds and 96 multiplies of
     # the reductions in the extension rounds (2^21 + 2^20 + ... pairs)

@@ -1114,7 +1114,7 @@ __device__ __forceinline__ void bf_finish_sums(const BfStepArgs &a, Acc96 (*acc)
   __shared__ uint32_t mine[16];
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t total = wave_sums_transposed<16>([&](int k) -> uint32_t { return acc_reduce(acc[k / 8][k % 8]); });
-  if (lane < 16) lds[tid >> 6][__brev(lane) >> 28] = total;
+  if (transposed_writer<16>(lane)) lds[tid >> 6][transposed_word<16>(lane)] = total;
   __syncthreads();
   if (tid < 2) {  // a workgroup's pairs share one HIGH weight (the tile is |LOW| pairs)
     Ext<8> t;
@@ -1228,7 +1228,7 @@ struct BfBaseSumsArgs {
 
 template <int LB>
 __global__ __launch_bounds__(BLOCK) void bf_base_sums_kernel(BfBaseSumsArgs a) {
-  constexpr int B = 1 << LB, WORDS = 8 * B, W = WORDS < 32 ? WORDS : 32, BITS = W == 32 ? 5 : W == 16 ? 4 : 3;
+  constexpr int B = 1 << LB, WORDS = 8 * B, W = WORDS < 32 ? WORDS : 32;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t tile = blockIdx.x % a.tiles, column = blockIdx.x / a.tiles;
   const uint32_t *col = a.cols + (uint64_t)column * a.len;
@@ -1261,14 +1261,11 @@ __global__ __launch_bounds__(BLOCK) void bf_base_sums_kernel(BfBaseSumsArgs a) {
   }
   __shared__ uint32_t lds[BLOCK / 64][WORDS];
   __shared__ uint32_t mine[WORDS];
-  uint32_t idx = 0;
-#pragma unroll
-  for (int b = 0; b < BITS; b++) idx |= ((lane >> b) & 1u) << (BITS - 1 - b);
 #pragma unroll
   for (int at = 0; at < WORDS; at += W) {
     const uint32_t total =
         wave_sums_transposed<W>([&](int k) -> uint32_t { return lazy_reduce(acc[(at + k) / 8][(at + k) % 8]); });
-    if (lane < W) lds[wave][at + idx] = total;
+    if (transposed_writer<W>(lane)) lds[wave][at + transposed_word<W>(lane)] = total;
   }
   __syncthreads();
   if (tid < B) {  // times the tile's HIGH weight and the column's coefficient

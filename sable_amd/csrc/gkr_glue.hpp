@@ -48,7 +48,8 @@ __device__ inline void dev_absorb_bytes(RunB3S &s, const uint32_t *words, uint32
   for (uint32_t base = 0; base < total; base += 64) {
     const uint32_t g = base + lane;
     uint32_t word = g < 4 ? len : (g < 8 || g >= total) ? 0 : words[(g - 8) >> 2];
-    rb3s_append_bytes(s, (word >> (8 * (g & 3))) & 0xff, total - base < 64 ? total - base : 64);
+    if (g < total) rb3s_put_byte(s, lane, word >> (8 * (g & 3)));
+    rb3s_advance(s, total - base < 64 ? total - base : 64);
   }
 }
 

@@ -36,6 +36,14 @@ struct StmtDesc {
 #define EXH_DESC_FN
 #endif
 
+// the largest number of factors in a group
+template <class Desc>
+EXH_DESC_FN constexpr int desc_maxdeg(const Desc &d) {
+  int m = 1;
+  for (int g = 0; g < d.G; g++) m = d.deg[g] > m ? d.deg[g] : m;
+  return m;
+}
+
 // ---- the slots of the base-field sweep that serves rounds 0 and 1 (the kernels and their generator agree here)
 // the index of X among group g's evaluation points, or -1
 template <class Desc>

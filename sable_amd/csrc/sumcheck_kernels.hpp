@@ -498,58 +498,70 @@ __device__ __forceinline__ void pair_from_raw(const Desc &d, const uint4 (*raw)[
   }
 }
 
-// the value of lane (l ^ M) of the wavefront
+// A lane's values meet those of the lane that differs from it in lane bit M: x and y become, in the lanes with the
+// bit clear, the two lanes' values of the first, in the others those of the second.  Bits 5 and 4 take one exchange of
+// half registers; for the others the value the partner keeps is fetched by a permutation within a row of 16: the
+// opposite lane of a group of 8 for bit 2 (so bits 0 and 1 come after it: until then all of a group's lanes still hold
+// the same words), eight lanes on for bit 3, within quads for bits 1 and 0.  None goes through LDS.
 template <int M>
-__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
-  if constexpr (M == 1)
-    return EXH_DPP(v, 0xB1);  // quad_perm [1,0,3,2]
-  else if constexpr (M == 2)
-    return EXH_DPP(v, 0x4E);  // quad_perm [2,3,0,1]
-  else if constexpr (M == 8)
-    return EXH_DPP(v, 0x128);  // row_ror:8
-  else if constexpr (M == 4 || M == 16)
-    return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (M << 10) | 0x1f);  // xor within 32 lanes
-  else
-    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(((threadIdx.x & 63) ^ 32) << 2), (int)v);
+__device__ __forceinline__ uint32_t lane_partner(uint32_t v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "bits within a row");
+  return M == 1 ? EXH_DPP(v, 0xB1) : M == 2 ? EXH_DPP(v, 0x4E) : M == 4 ? EXH_DPP(v, 0x141) : EXH_DPP(v, 0x128);
 }
-
-// One step of the transposing reduction: the 2 * H values a lane holds become H, each the sum over
-// the lane pair (l, l ^ M); lanes with bit M clear keep the lower half of the values, the others the
-// upper half.
-template <int M, int H>
-__device__ __forceinline__ void halve_step(uint32_t *a) {
-  const bool upper = (threadIdx.x & M) != 0;
-#pragma unroll
-  for (int k = 0; k < H; k++) {
-    uint32_t keep = upper ? a[k + H] : a[k], send = upper ? a[k] : a[k + H];
-    a[k] = fadd(keep, lane_xor<M>(send));
+template <int M>
+__device__ __forceinline__ uint32_t lane_sum(uint32_t v) {  // v plus the partner's v
+  if constexpr (M >= 16) {
+    const auto p = M == 32 ? __builtin_amdgcn_permlane32_swap(v, v, false, false) : __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return fadd(p[0], p[1]);
+  } else {
+    return fadd(v, lane_partner<M>(v));
+  }
+}
+template <int M>
+__device__ __forceinline__ uint32_t lane_halve(uint32_t x, uint32_t y) {  // the sum of x (bit clear) or of y (bit set)
+  if constexpr (M >= 16) {
+    const auto p = M == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false) : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    return fadd(p[0], p[1]);
+  } else {
+    const bool upper = (threadIdx.x & M) != 0;
+    return fadd(upper ? y : x, lane_partner<M>(upper ? x : y));
   }
 }
 
-// The wavefront's sums of W = 8, 16 or 32 values per lane, value k given by val(k): afterwards lane l
-// holds the sum over all 64 lanes of value bitrev(l mod W).  About 2 W cross-lane operations instead of
-// the 6 W of one reduction tree per value.  The first step consumes the values as they are produced, so
-// only W / 2 are live at once.
+// The wavefront's sums of W = 8, 16 or 32 values per lane, value k given by val(k): the values are halved over lane
+// bits 5, 4, 3, .. until each lane holds one (about 2 W operations instead of the 6 W of a tree per value), then summed
+// over the bits that are left.  Lane l ends with the sum of value transposed_word<W>(l); val is called for two values
+// at a time, so only W / 2 are live at once.
+template <int W>
+__device__ __forceinline__ uint32_t transposed_word(uint32_t lane) {
+  const uint32_t b5 = (lane >> 5) & 1, b4 = (lane >> 4) & 1, b3 = (lane >> 3) & 1, b2 = (lane >> 2) & 1, b1 = (lane >> 1) & 1;
+  return W == 32 ? 16 * b5 + 8 * b4 + 4 * b3 + 2 * b2 + b1 : W == 16 ? 8 * b5 + 4 * b4 + 2 * b3 + b2 : 4 * b5 + 2 * b4 + b3;
+}
+template <int W>
+__device__ __forceinline__ bool transposed_writer(uint32_t lane) {  // one lane per value
+  return (lane & (64 / W - 1)) == 0;
+}
 template <int W, class F>
 __device__ __forceinline__ uint32_t wave_sums_transposed(F val) {
+  static_assert(W == 8 || W == 16 || W == 32, "three to five halvings");
   uint32_t a[W / 2];
-  const bool upper = (threadIdx.x & 1) != 0;
 #pragma unroll
   for (int k = 0; k < W / 2; k++) {
-    uint32_t lo = val(k), hi = val(k + W / 2);
-    a[k] = fadd(upper ? hi : lo, lane_xor<1>(upper ? lo : hi));
+    const uint32_t x = val(k), y = val(k + W / 2);
+    a[k] = lane_halve<32>(x, y);
   }
-  if constexpr (W == 32) {
-    halve_step<2, 8>(a), halve_step<4, 4>(a), halve_step<8, 2>(a), halve_step<16, 1>(a);
-  } else if constexpr (W == 16) {
-    halve_step<2, 4>(a), halve_step<4, 2>(a), halve_step<8, 1>(a);
-    a[0] = fadd(a[0], lane_xor<16>(a[0]));
+#pragma unroll
+  for (int k = 0; k < W / 4; k++) a[k] = lane_halve<16>(a[k], a[k + W / 4]);
+#pragma unroll
+  for (int k = 0; k < W / 8; k++) a[k] = lane_halve<8>(a[k], a[k + W / 8]);
+  if constexpr (W >= 16) {
+#pragma unroll
+    for (int k = 0; k < W / 16; k++) a[k] = lane_halve<4>(a[k], a[k + W / 16]);
   } else {
-    halve_step<2, 2>(a), halve_step<4, 1>(a);
-    a[0] = fadd(a[0], lane_xor<8>(a[0]));
-    a[0] = fadd(a[0], lane_xor<16>(a[0]));
+    a[0] = lane_sum<4>(a[0]);
   }
-  return fadd(a[0], lane_xor<32>(a[0]));
+  a[0] = W == 32 ? lane_halve<2>(a[0], a[1 % (W / 2)]) : lane_sum<2>(a[0]);
+  return lane_sum<1>(a[0]);
 }
 
 // accumulator words [first, first + W) of the lane, reduced mod p (zero beyond the statement's), summed
@@ -560,12 +572,8 @@ __device__ __forceinline__ void chunk_sums(const Desc &d, Acc96 (*acc)[D], int f
     const int o = first + k;
     return o < d.nacc * D ? acc_reduce(acc[o / D][o % D]) : 0u;
   });
-  const uint32_t l = threadIdx.x & 63;
-  constexpr int BITS = W == 32 ? 5 : W == 16 ? 4 : 3;
-  uint32_t idx = 0;
-#pragma unroll
-  for (int b = 0; b < BITS; b++) idx |= ((l >> b) & 1u) << (BITS - 1 - b);
-  if (l < W && first + idx < (uint32_t)d.nacc * D) lds_row[first + idx] = total;
+  const uint32_t l = threadIdx.x & 63, o = first + transposed_word<W>(l);
+  if (transposed_writer<W>(l) && o < (uint32_t)d.nacc * D) lds_row[o] = total;
 }
 
 // The workgroup's sums of every accumulator, reduced mod p, into sums[nacc * D] (LDS); all threads call.
@@ -617,13 +625,8 @@ __device__ __forceinline__ void part_chunk_sums(const Desc &d, Acc96 (*acc)[D], 
     const int o = first + k, q = o / D;
     return PARTS * q + PART < MAXACC && q < count ? acc_reduce(acc[(PARTS * q + PART) % MAXACC][o % D]) : 0u;
   });
-  const uint32_t l = threadIdx.x & 63;
-  constexpr int BITS = W == 32 ? 5 : W == 16 ? 4 : 3;
-  uint32_t idx = 0;
-#pragma unroll
-  for (int b = 0; b < BITS; b++) idx |= ((l >> b) & 1u) << (BITS - 1 - b);
-  const uint32_t o = first + idx;
-  if (l < W && o < (uint32_t)count * D) sums[(PARTS * (o / D) + PART) * D + o % D] = total;
+  const uint32_t l = threadIdx.x & 63, o = first + transposed_word<W>(l);
+  if (transposed_writer<W>(l) && o < (uint32_t)count * D) sums[(PARTS * (o / D) + PART) * D + o % D] = total;
 }
 template <int D, int PART, int PARTS, class Desc>
 __device__ __forceinline__ void part_wave_sums(const Desc &d, Acc96 (*acc)[D], uint32_t *sums) {
@@ -640,13 +643,13 @@ __device__ __forceinline__ void part_wave_sums(const Desc &d, Acc96 (*acc)[D], u
   }
 }
 
-// From the round's accumulator sums (LDS, nacc * D words, scaled as the kernels leave them) to the round
-// message, through the transcript, to the next challenge: rows = mtilde * sums + c0
-// (ROUND-MESSAGE, src/sumcheck.lisp:313-317), send = absorb the rows (src/transcript.lisp:116-128),
-// r = challenge (src/transcript.lisp:174-176).  All threads of the workgroup call; scratch is LDS.
+// From the round's accumulator sums (LDS, scaled as the kernels leave them) to the round message, through the
+// transcript, to the next challenge: rows = mtilde * sums + c0 (ROUND-MESSAGE, src/sumcheck.lisp:313-317), send =
+// absorb the rows (src/transcript.lisp:116-128), r = challenge (src/transcript.lisp:174-176).  The workgroup's first
+// wavefront does it alone: the message's words lie across its lanes and go from there straight into the transcript's
+// pending block, with no barrier and no trip through LDS in between.
 struct EpilogueLds {
-  alignas(16) uint32_t prod[MAXPTS * MAXACC * 8];
-  uint32_t msg[MAXPTS * 8];
+  alignas(16) uint32_t prod[MAXPTS * MAXACC * 8];  // the totals' words of the groups, before they are added up
   uint32_t chal[8];
   uint32_t r_mont[8];
   uint32_t ring[RING_WORDS];
@@ -657,60 +660,108 @@ struct EpilogueLds {
   alignas(16) uint32_t c0[MAXPTS * 8];
 };
 
+// Which part of the message a lane computes: word o = lane / parts (row o / D, coordinate o % D), and of its sum over
+// the accumulators every parts-th term from `part` on; parts is as large as the message leaves lanes for, up to 8.
 template <int D>
-__device__ __forceinline__ void round_message(const uint32_t *sums, uint32_t nacc, uint32_t points,
-                                              const uint32_t *mtilde, const uint32_t *c0, EpilogueLds *e) {
-  const uint32_t tid = threadIdx.x, nthreads = blockDim.x;
-  for (uint32_t u = tid; u < points * nacc; u += nthreads) {
-    uint32_t a = u % nacc;
-    Ext<D> m = load_ext<D>(mtilde + (size_t)u * D), sv;
+struct MessageLane {
+  uint32_t o, part, parts;
+  uint32_t at[D];  // the word of an accumulator's sum that goes with coordinate w^i of the map's element, or of its triple
+};
+constexpr uint32_t TRIPLED = MAXACC * 8;  // sums[TRIPLED + o] = 3 sums[o]: the products that wrap, w^D = 3
+template <int D>
+__device__ __forceinline__ MessageLane<D> message_lane(uint32_t points) {
+  const uint32_t lane = threadIdx.x & 63, words = points * D;
+  MessageLane<D> ml;
+  ml.parts = words <= 8 ? 8 : words <= 16 ? 4 : words <= 32 ? 2 : 1;
+  ml.o = lane / ml.parts, ml.part = lane % ml.parts;
+  const uint32_t c = ml.o % D, e = D == 8 ? __brev(c) >> 29 : __brev(c) >> 30;
 #pragma unroll
-    for (int c = 0; c < D; c++) sv.c[c] = sums[a * D + c];
-    Ext<D> pr = ext_mul_mont<D>(m, sv);
-#pragma unroll
-    for (int c = 0; c < D; c++) e->prod[u * D + c] = pr.c[c];
+  for (int i = 0; i < D; i++) {
+    const uint32_t j = (e - i) & (D - 1), tower = D == 8 ? __brev(j) >> 29 : __brev(j) >> 30;
+    ml.at[i] = tower + ((uint32_t)i > e ? TRIPLED : 0u);
   }
-  lds_barrier();
-  for (uint32_t o = tid; o < points * D; o += nthreads) {
-    uint32_t k = o / D, c = o % D, v = c0[o];
-    for (uint32_t a = 0; a < nacc; a++) v = fadd(v, e->prod[(k * nacc + a) * D + c]);
-    e->msg[o] = v;
-  }
-  lds_barrier();
+  return ml;
 }
 
-// the first wavefront's part: send the message, draw the challenge, log both (every lane the same steps)
-// With `publish` (an LDS word), the challenge times R is in e->r_mont and *publish = round + 1 as soon as it is
-// drawn, before the transcript absorbs the squeeze's bytes: the workgroup's other wavefronts wait for that word
-// instead of a barrier and begin the fold while this one finishes the transcript's bookkeeping.
+// the lane's message word (every lane of a word's group has it); sums with their triples, mtilde and c0 in LDS
 template <int D>
-__device__ __forceinline__ void transcript_step(RunB3S &tr, Ctrl *ctrl, uint32_t round, uint32_t points,
-                                                EpilogueLds *e, bool log = true, uint32_t *publish = nullptr,
-                                                PendingAppend *pending = nullptr) {
-  const uint32_t tid = threadIdx.x;
-  if (pending) rb3s_flush(tr, *pending);
-  dev_absorb_words(tr, e->msg, points * D);
-  dev_challenge(tr, D, e->chal, [&] {
-    if (tid < (uint32_t)D) e->r_mont[tid] = to_mont(e->chal[tid]);
-    __builtin_amdgcn_wave_barrier();
-    if (publish && tid == 0) __hip_atomic_store(publish, round + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }, pending);
-  if (log)
-    for (uint32_t o = tid; o < points * D; o += 64) ctrl->msg[round][o] = e->msg[o];
-  if (log && tid < (uint32_t)D) ctrl->chal[round][tid] = e->chal[tid], ctrl->r_mont[tid] = e->r_mont[tid];
+__device__ __forceinline__ uint32_t round_message_word(const uint32_t *sums, uint32_t nacc, uint32_t points,
+                                                       const uint32_t *mtilde, const uint32_t *c0, const MessageLane<D> &ml) {
+  const uint32_t o = ml.o < points * D ? ml.o : points * D - 1;
+  uint64_t t = 0;
+  for (uint32_t a = ml.part; a < nacc; a += ml.parts) {
+    const Ext<D> m = load_ext<D>(mtilde + (size_t)((o / D) * nacc + a) * D);
+#pragma unroll
+    for (int i = 0; i < D; i++) {
+      if (i % 2 == 0) t = mont_lazy(t);
+      t += (uint64_t)m.c[brev(i, D)] * sums[a * D + ml.at[i]];
+    }
+  }
+  uint32_t v = mont_reduce4(t);
+  if (ml.parts >= 2) v = fadd(v, EXH_DPP(v, 0xB1));
+  if (ml.parts >= 4) v = fadd(v, EXH_DPP(v, 0x4E));
+  if (ml.parts >= 8) v = fadd(v, EXH_DPP(v, 0x141));
+  return fadd(v, c0[o]);
 }
 
+// the triples beside the sums (the first wavefront)
+__device__ __forceinline__ void triple_sums(uint32_t *sums, uint32_t width) {
+  for (uint32_t o = threadIdx.x & 63; o < width; o += 64) sums[TRIPLED + o] = times3(sums[o]);
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The first wavefront's step: send the message whose words the lanes hold (what the last squeeze left to absorb and
+// the message's length go first, unless `prefixed` says that they went already), draw the challenge into e->chal and,
+// times R, e->r_mont, call `ready`, then log both.  What this squeeze leaves to absorb stays in `pending`.
+template <int D, class F>
+__device__ __forceinline__ void transcript_step(RunB3S &tr, Ctrl *ctrl, uint32_t round, uint32_t points, EpilogueLds *e,
+                                                const MessageLane<D> &ml, uint32_t word, PendingAppend &pending,
+                                                bool prefixed, bool log, F ready) {
+  const uint32_t lane = threadIdx.x & 63, words = points * D;
+  if (!prefixed) rb3s_flush(tr, pending, words);
+  for (uint32_t base = 0; base < words; base += 16) {  // sixteen words at a time, a word's bytes shared by its lanes
+    const uint32_t o = ml.o - base;
+    if (ml.o >= base && o < 16 && ml.o < words) {
+      if (ml.parts >= 4) {
+        if (ml.part < 4) rb3s_put_byte(tr, 4 * o + ml.part, word >> (8 * ml.part));
+      } else if (ml.parts == 2) {
+        rb3s_put_byte(tr, 4 * o + 2 * ml.part, word >> (16 * ml.part));
+        rb3s_put_byte(tr, 4 * o + 2 * ml.part + 1, word >> (16 * ml.part + 8));
+      } else {
+        rb3s_put_word(tr, 4 * o, word);
+      }
+    }
+    rb3s_advance(tr, 4 * (words - base < 16 ? words - base : 16));
+  }
+  dev_challenge(
+      tr, D,
+      [&](uint32_t at, uint32_t v) {
+        e->chal[at] = v;
+        e->r_mont[at] = to_mont(v);
+      },
+      ready, &pending);
+  if (log) {
+    if (ml.part == 0 && ml.o < words) ctrl->msg[round][ml.o] = word;
+    if (lane < (uint32_t)D) ctrl->chal[round][lane] = e->chal[lane], ctrl->r_mont[lane] = e->r_mont[lane];
+  }
+}
+
+// (all threads of the workgroup may call; the first wavefront works)
 template <int D>
-__device__ __forceinline__ void round_epilogue(Ctrl *ctrl, const uint32_t *sums, uint32_t nacc, uint32_t points,
+__device__ __forceinline__ void round_epilogue(Ctrl *ctrl, uint32_t *sums, uint32_t nacc, uint32_t points,
                                                const uint32_t *mtilde, const uint32_t *c0, EpilogueLds *e,
                                                bool staged = false) {
   const uint32_t tid = threadIdx.x;
-  round_message<D>(sums, nacc, points, mtilde, c0, e);
   if (tid < 64) {
     const uint32_t round = staged ? e->round : ctrl->round;
     RunB3S tr;
+    PendingAppend pending{0, 0, 0};
     rb3s_load(tr, e->ring, staged ? reinterpret_cast<const DevB3S *>(e->state) : &ctrl->tr);
-    transcript_step<D>(tr, ctrl, round, points, e);
+    const MessageLane<D> ml = message_lane<D>(points);
+    triple_sums(sums, nacc * D);
+    const uint32_t word = round_message_word<D>(sums, nacc, points, mtilde, c0, ml);
+    transcript_step<D>(tr, ctrl, round, points, e, ml, word, pending, false, true, [] {});
+    rb3s_flush(tr, pending);
     rb3s_store(tr, &ctrl->tr);
     if (tid == 0) ctrl->round = round + 1;
   }
@@ -861,7 +912,7 @@ __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const 
   if (!sh.do_sums) return;
 
   __shared__ uint32_t lds[BLOCK / 64][MAXACC * D];
-  __shared__ uint32_t sums[MAXACC * D];
+  __shared__ uint32_t sums[2 * TRIPLED];
   // a device-driven round: what the elected workgroup's serial part reads from memory (the transcript's state, the
   // message map, the constant terms) is requested by every workgroup here, ahead of the reduction that hides the
   // trip; the one elected later finds it in its LDS
@@ -994,7 +1045,7 @@ constexpr int EPI_BLOCK = 1024;
 template <int D>
 __global__ __launch_bounds__(EPI_BLOCK) void epilogue_kernel(EpilogueArgs args) {
   __shared__ uint32_t scratch[EPI_BLOCK];
-  __shared__ uint32_t sums[MAXACC * D];
+  __shared__ uint32_t sums[2 * TRIPLED];
   __shared__ EpilogueLds epi;
   const uint32_t tid = threadIdx.x, width = args.nacc * D, ps = args.pstride;
   // everything the serial part needs from global memory is requested first, so that its latency
@@ -1021,6 +1072,20 @@ __device__ __forceinline__ void small_round_sums(const Desc &d, const Ext<D> *lo
   part_wave_sums<D, PART, PARTS>(d, acc, sums);
 }
 
+// An accumulator as a lane walks it in a spread round (see tail_body): its degree, its evaluation point, and where in
+// LDS its factors' tables begin.
+constexpr int SPREAD_FACTORS = MAXDEG;
+struct SpreadUnit {
+  uint32_t deg, x, table[SPREAD_FACTORS];
+};
+__device__ __forceinline__ uint32_t lane_bits(uint32_t n) {  // 2^bits: the next power of two from n up
+  return n <= 1 ? 0 : 32 - __builtin_clz(n - 1);
+}
+template <int M>
+struct LaneBit {
+  static constexpr int value = M;
+};
+
 // Load (folding or lifting on the way in) into LDS, then per round sums -> message -> challenge -> fold
 // on the slice this workgroup holds: entries [w * E, (w + 1) * E) of every table, E = entries / grid.
 // A grid launch ends when its rounds are done and leaves the slices in `out` for the one-workgroup
@@ -1029,17 +1094,23 @@ template <int D, class Desc>
 __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args) {
   extern __shared__ __align__(16) uint32_t tail_tables[];  // [T][capacity][D]
   __shared__ uint32_t lds[BLOCK / 64][MAXACC * D];
-  __shared__ uint32_t sums[MAXACC * D];
+  __shared__ uint32_t sums[2 * TRIPLED];
   __shared__ EpilogueLds epi;
   __shared__ uint32_t c0s[MAXTAIL * MAXPTS * D];
-  __shared__ uint32_t ready_round;  // rounds whose challenge the first wavefront has published, counted from the proof's first
+  // (a statement in direct form, or with linear forms among its factors, keeps a pair's accumulators on one lane)
+  constexpr bool SPREAD = !is_direct<Desc>::value;
+  __shared__ SpreadUnit units[SPREAD ? MAXACC : 1];
   const uint32_t tid = threadIdx.x, cap = args.capacity, G = gridDim.x, wg = blockIdx.x;
-  if (tid == 0) ready_round = 0;
   const uint32_t width = (uint32_t)d.nacc * D;
   if (args.ctrl->round != args.first_round) return;  // an earlier launch gave up: leave the count as it is
   RunB3S tr;
-  PendingAppend pending{0, 0};  // (the first wavefront's)
-  if (tid < 64) rb3s_load(tr, epi.ring, &args.ctrl->tr);
+  PendingAppend pending{0, 0, 0};  // (the first wavefront's)
+  MessageLane<D> ml;
+  bool prefixed = false;
+  if (tid < 64) {
+    rb3s_load(tr, epi.ring, &args.ctrl->tr);
+    ml = message_lane<D>(args.points);
+  }
   uint32_t entries = (args.first_fold ? args.entries / 2 : args.entries) / G;  // of this workgroup's slice
   {
     Ext<D> r = ext_zero<D>();
@@ -1073,6 +1144,16 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     }
     for (uint32_t u = tid; u < args.points * width; u += BLOCK) epi.mtilde[u] = args.mtilde[u];
     for (uint32_t u = tid; u < args.rounds * args.points * D; u += BLOCK) c0s[u] = args.c0[u];
+  }
+  if (SPREAD && tid < (uint32_t)d.nacc) {
+    uint32_t a = 0;
+    for (int g = 0; g < d.G; g++)
+      for (int k = 0; k < d.nev[g]; k++, a++)
+        if (a == tid) {
+          units[tid].deg = (uint32_t)d.deg[g], units[tid].x = (uint32_t)d.ev[g][k];
+          for (int j = 0; j < SPREAD_FACTORS; j++)
+            units[tid].table[j] = (uint32_t)d.tab[g][j < d.deg[g] ? j : 0] * cap * D;
+        }
   }
   // The session's own weight tables (see TailArgs::factors), in LDS behind the tables: the factors first, then
   // per round its LOW and its HIGH table.  An entry is a chain of at most n_vars products, one entry per thread
@@ -1131,9 +1212,19 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     wl = load_ext<D>(args.weights + (args.low_off[jj] + (i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
     wh = load_ext<D>(args.weights + (args.high_off[jj] + (i >> args.low_bits[jj])) * D);
   };
-  // a fold of `count` outputs by r, a table per wavefront, in place: the lanes run in lockstep, so every read of
-  // a chunk of 64 comes before its writes, and those land below what later chunks read
-  auto fold_small = [&](const Ext<D> &r, uint32_t count) {
+  // A fold of `count` outputs by r, in place: the lanes run in lockstep, so every read of a chunk of 64 comes before
+  // its writes, and those land below what later chunks read.  `spread`: wavefronts 1 to 3, an output per lane (a
+  // table's outputs in as many lanes as the next power of two, so in one wavefront); else a table per wavefront.
+  auto fold_small = [&](const Ext<D> &r, uint32_t count, bool spread) {
+    if (spread) {
+      const uint32_t u = tid - 64, bits = lane_bits(count), t = u >> bits, x = u & ((1u << bits) - 1);
+      if (tid >= 64 && t < (uint32_t)d.T && x < count) {
+        const uint32_t *p = tail_tables + ((size_t)t * cap + 2 * x) * D;
+        const Ext<D> folded = fold_ext<D>(load_ext<D>(p), load_ext<D>(p + D), r);
+        store_ext<D>(tail_tables + ((size_t)t * cap + x) * D, folded);
+      }
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < MAXT; t++)
       if (t < d.T && (uint32_t)((t + 1) & 3) == wave) {  // (the first wavefront, late from the transcript, last)
@@ -1144,13 +1235,120 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
         }
       }
   };
-  fetch_weight(0, entries / 2);
+  // Rounds whose (accumulator, pair) units fit the 192 lanes of wavefronts 1 to 3 run spread: a unit per lane, which
+  // walks the accumulator's factors (their tables and its evaluation point come from LDS) instead of every wavefront
+  // computing a third of the accumulators of a pair per lane; a unit is a few products where a third of a GKR layer's
+  // accumulators is four, and the sum over the pairs halves its words over the lanes first.
+  // (with several blocks the pairs are no power of two: a unit's lanes are the next one)
+  auto spreads = [&](uint32_t pairs) {
+    return SPREAD && BLOCK == 256 && d.NV == 0 && pairs <= 64 && ((uint32_t)d.nacc << lane_bits(pairs)) <= 192;
+  };
+  uint32_t unit_a = 0, unit_pair = 0, unit_deg = 0, unit_x = 0, unit_table[SPREAD_FACTORS];
+  Ext<D> unit_w = ext_zero<D>();
+  // a lane's unit of a round and its weight, which wait for nothing that the round before computes
+  auto prepare_unit = [&](uint32_t jj, uint32_t pairs) {
+    const uint32_t u = tid < 64 ? 0 : tid - 64;
+    const uint32_t bits = lane_bits(pairs);
+    unit_a = u >> bits, unit_pair = u & ((1u << bits) - 1);
+    const bool on = unit_pair < pairs;  // (a lane without a pair takes the last one with no weight)
+    const SpreadUnit &unit = units[unit_a < (uint32_t)d.nacc ? unit_a : 0];
+    unit_deg = unit.deg, unit_x = unit.x;
+#pragma unroll
+    for (int j = 0; j < SPREAD_FACTORS; j++) unit_table[j] = unit.table[j];
+    const uint64_t i = (uint64_t)wg * pairs + (on ? unit_pair : pairs - 1);
+    const uint32_t *low = own_weights ? own_tables + (size_t)own_at(jj, false) * D : args.weights + args.low_off[jj] * D;
+    const uint32_t *high = own_weights ? own_tables + (size_t)own_at(jj, true) * D : args.weights + args.high_off[jj] * D;
+    const Ext<D> l = load_ext<D>(low + (i & (((uint64_t)1 << args.low_bits[jj]) - 1)) * D);
+    const Ext<D> h = load_ext<D>(high + (i >> args.low_bits[jj]) * D);
+    unit_w = ext_scale_mont<D>(ext_mul_mont<D>(l, h), on ? R2 : 0u);  // (times R for the product that takes it in below)
+  };
+  // the round's sums from the units (wavefronts 1 to 3), with their triples
+  auto unit_sums = [&](uint32_t pairs) {
+    const int maxx = d.maxx, maxdeg = desc_maxdeg(d);
+    auto factor = [&](uint32_t table) {  // the factor's line at the unit's evaluation point
+      const uint32_t *p = tail_tables + table + 2 * (unit_pair < pairs ? unit_pair : pairs - 1) * D;
+      const Ext<D> lo = load_ext<D>(p), hi = load_ext<D>(p + D);
+      Ext<D> v;
+#pragma unroll
+      for (int c = 0; c < D; c++) {
+        const uint32_t slope = fsub(hi.c[c], lo.c[c]);
+        uint32_t at = unit_x >= 1 ? hi.c[c] : lo.c[c], next = hi.c[c];
+#pragma unroll
+        for (int x = 2; x <= MAXX; x++)
+          if (x <= maxx) {
+            next = fadd(next, slope);
+            at = unit_x >= (uint32_t)x ? next : at;
+          }
+        v.c[c] = at;
+      }
+      return v;
+    };
+    Ext<D> f = factor(unit_table[0]);
+#pragma unroll
+    for (int j = 1; j < SPREAD_FACTORS; j++)
+      if (j < maxdeg) {
+        if ((uint32_t)j < unit_deg) f = ext_mul_mont<D>(f, factor(unit_table[j]));
+      }
+    f = ext_mul_mont<D>(f, unit_w);
+    // Over the pairs, the low lane bits of a unit: the words are halved as long as there are several.  Bit 2 comes first:
+    // its partner is the opposite lane of a group of 8, which still holds the same words then (see lane_partner).
+    const uint32_t lanes = 1u << lane_bits(pairs);
+    uint32_t v[D], word = 0, count = D, keys = 0;
+#pragma unroll
+    for (int c = 0; c < D; c++) v[c] = f.c[c];
+    auto step = [&](auto bit) {
+      constexpr int M = decltype(bit)::value;
+      if (lanes <= (uint32_t)M) return;
+      auto halve = [&](auto half) {
+        constexpr int H = decltype(half)::value;
+#pragma unroll
+        for (int k = 0; k < H; k++) v[k] = lane_halve<M>(v[k], v[k + H]);
+        word = 2 * word + ((lane & M) ? 1 : 0), count = H, keys |= M;
+      };
+      if constexpr (M <= 4) {
+        if (D == 8 && count == 8)
+          halve(LaneBit<D / 2>{});
+        else if (count == 4)
+          halve(LaneBit<2>{});
+        else if (count == 2)
+          halve(LaneBit<1>{});
+        else
+          v[0] = lane_sum<M>(v[0]);
+      } else {
+        v[0] = lane_sum<M>(v[0]);
+      }
+    };
+    step(LaneBit<4>{}), step(LaneBit<1>{}), step(LaneBit<2>{}), step(LaneBit<8>{}), step(LaneBit<16>{}), step(LaneBit<32>{});
+    if (tid >= 64 && unit_a < (uint32_t)d.nacc && (unit_pair & ~keys) == 0) {
+#pragma unroll
+      for (int k = 0; k < D; k++)
+        if (k < (int)count) {
+          const uint32_t o = unit_a * D + word * count + k;
+          sums[o] = v[k], sums[TRIPLED + o] = times3(v[k]);
+        }
+    }
+  };
+  if (spreads(entries / 2)) {
+    __syncthreads();  // (the units and the session's own weights)
+    if (tid >= 64) prepare_unit(0, entries / 2);
+  } else {
+    fetch_weight(0, entries / 2);
+  }
   __syncthreads();
   for (uint32_t jj = 0; jj < args.rounds; jj++) {
     const uint32_t pairs = entries / 2;
-    const bool small = pairs <= 64 && BLOCK == 256;
+    const bool small = pairs <= 64 && BLOCK == 256, spread = spreads(pairs), more = jj + 1 < args.rounds;
+    const bool next_spread = more && spreads(pairs / 2);
     {  // the round's sums
-      if (small) {  // each wavefront its own share of the pair's accumulators, in code of its own
+      if (spread) {
+        // the first wavefront, which ran the transcript, meanwhile absorbs what the last squeeze left to absorb and
+        // the length of the message to come (a compression every other round): nobody waits for that any more
+        if (wave == 0)
+          rb3s_flush(tr, pending, args.points * D), prefixed = true;
+        else
+          unit_sums(pairs);
+        lds_barrier();
+      } else if (small) {  // each wavefront its own share of the pair's accumulators, in code of its own
         Ext<D> lo[MAXT], hi[MAXT];
         const uint32_t at = lane < pairs ? lane : 0;
 #pragma unroll
@@ -1162,11 +1360,10 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
           }
         Ext<D> ww = ext_mul_mont<D>(wl, wh);
         if (lane >= pairs) ww = ext_zero<D>();  // lanes without a pair add nothing
-        if (jj + 1 < args.rounds) fetch_weight(jj + 1, pairs / 2);
-        // three wavefronts share the accumulators; the first, which ran the transcript, meanwhile absorbs what the
-        // last squeeze left to absorb (a compression every other round): nobody waits for that any more
+        if (more && !next_spread) fetch_weight(jj + 1, pairs / 2);
+        // three wavefronts share the accumulators; the first as above
         if (wave == 0)
-          rb3s_flush(tr, pending);
+          rb3s_flush(tr, pending, args.points * D), prefixed = true;
         else if (wave == 1)
           small_round_sums<D, 0, 3>(d, lo, hi, ww, sums, args.consts);
         else if (wave == 2)
@@ -1197,7 +1394,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
           }
           accumulate_pair<D, Ext<D>>(d, lo, hi, ext_mul_mont<D>(wl, wh), acc, args.consts);
         }
-        if (jj + 1 < args.rounds) fetch_weight(jj + 1, pairs / 2);
+        if (more && !next_spread) fetch_weight(jj + 1, pairs / 2);
         block_sums<D, true>(d, acc, lds, sums);
       }
       if (G > 1) {
@@ -1234,27 +1431,30 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
         for (uint32_t o = tid; o < width; o += BLOCK) {
           uint32_t v = 0;
           for (uint32_t g = 0; g < NG; g++) v = fadd(v, epi.prod[g * width + o]);
-          sums[o] = v;
+          sums[o] = v, sums[TRIPLED + o] = times3(v);
         }
         lds_barrier();
       }
     }
     {  // the message, the challenge, the fold
-      round_message<D>(sums, (uint32_t)d.nacc, args.points, epi.mtilde, c0s + (size_t)jj * args.points * D, &epi);
-      // the first wavefront publishes the challenge the moment it is drawn and finishes the transcript's step while
-      // the others, which wait for that word alone, are already folding
-      if (tid < 64) {
-        transcript_step<D>(tr, args.ctrl, args.first_round + jj, args.points, &epi, wg == 0, &ready_round, &pending);
+      // The first wavefront goes on alone, up to the barrier at which the others, which meanwhile prepare what of the
+      // next round they can, wait for the challenge; it finishes the transcript's step behind that barrier.
+      if (wave == 0) {
+        if (G == 1 && !spread) triple_sums(sums, width);
+        const uint32_t word = round_message_word<D>(sums, (uint32_t)d.nacc, args.points, epi.mtilde,
+                                                    c0s + (size_t)jj * args.points * D, ml);
+        transcript_step<D>(tr, args.ctrl, args.first_round + jj, args.points, &epi, ml, word, pending, prefixed, wg == 0,
+                           [] { lds_barrier(); });
+        prefixed = false;
       } else {
-        while (__hip_atomic_load(&ready_round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != args.first_round + jj + 1)
-          __builtin_amdgcn_s_sleep(1);
+        if (next_spread) prepare_unit(jj + 1, pairs / 2);
+        lds_barrier();
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       Ext<D> r;
 #pragma unroll
       for (int c = 0; c < D; c++) r.c[c] = epi.r_mont[c];
       if (small) {
-        fold_small(r, pairs);
+        fold_small(r, pairs, ((uint32_t)d.T << lane_bits(pairs)) <= 192);
         lds_barrier();
       }
       // fold in place, 256 entries at a time in ascending order: a chunk's reads come before its writes,
@@ -1372,7 +1572,7 @@ __device__ __forceinline__ uint32_t lazy_reduce(uint64_t acc) {
 template <int D>
 struct NodesEpilogueLds {
   uint32_t slot_sums[MAXACC * D];
-  uint32_t sums[MAXACC * D];
+  uint32_t sums[2 * TRIPLED];
   uint32_t basis[(MAXDEG + 1) * (MAXDEG + 1) * D];  // [deg][node]: Lagrange basis at r0, Montgomery form
   // the statement's shape: indexed by lane-dependent values out of the kernel's arguments, every access would be
   // a load from memory with the next one waiting behind it
@@ -1441,11 +1641,18 @@ __device__ __forceinline__ void nodes_epilogue_body(const NodesEpilogueArgs &arg
     for (int c = 0; c < D; c++) L.sums[tid * D + c] = total.c[c];
   }
   __syncthreads();
-  round_message<D>(L.sums, nacc, points, epi.mtilde, epi.c0, &epi);
   RunB3S tr;
+  PendingAppend pending{0, 0, 0};
+  MessageLane<D> ml;
+  auto send_round = [&](uint32_t round) {  // (the first wavefront)
+    triple_sums(L.sums, nacc * D);
+    const uint32_t word = round_message_word<D>(L.sums, nacc, points, epi.mtilde, epi.c0, ml);
+    transcript_step<D>(tr, args.e.ctrl, round, points, &epi, ml, word, pending, false, true, [] {});
+  };
   if (tid < 64) {
     rb3s_load(tr, epi.ring, reinterpret_cast<const DevB3S *>(epi.state));
-    transcript_step<D>(tr, args.e.ctrl, 0, points, &epi);
+    ml = message_lane<D>(points);
+    send_round(0);
   }
   __syncthreads();
   // ---- round 1: the basis of nodes 0..deg at r0, L_m = prod_{q != m} (r0 - q) / (m - q)
@@ -1482,9 +1689,9 @@ __device__ __forceinline__ void nodes_epilogue_body(const NodesEpilogueArgs &arg
     for (int c = 0; c < D; c++) L.sums[tid * D + c] = total.c[c];
   }
   __syncthreads();
-  round_message<D>(L.sums, nacc, points, epi.mtilde, epi.c0, &epi);
   if (tid < 64) {
-    transcript_step<D>(tr, args.e.ctrl, 1, points, &epi);
+    send_round(1);
+    rb3s_flush(tr, pending);
     rb3s_store(tr, &args.e.ctrl->tr);
     if (tid == 0) args.e.ctrl->round = 2;
   }
@@ -1624,16 +1831,14 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
   const uint32_t lane = tid & 63, wave = tid >> 6;
   nodes_epilogue_stage<D>(args.epi, L);  // (the loads' trip hides behind the reduction below)
   {  // the wavefront's sums, 32 words at a time by the transposing reduction
-    uint32_t idx = 0;
-#pragma unroll
-    for (int b = 0; b < 5; b++) idx |= ((lane >> b) & 1u) << (4 - b);
+    const uint32_t idx = transposed_word<32>(lane);
 #pragma unroll
     for (int first = 0; first < WORDS; first += 32) {
       const uint32_t total = wave_sums_transposed<32>([&](int k) -> uint32_t {
         const int o = first + k;
         return o < WORDS ? lazy_reduce(acc[o / D][o % D]) : 0u;
       });
-      if (lane < 32) lds[wave][first + idx] = total;
+      if (transposed_writer<32>(lane)) lds[wave][first + idx] = total;
     }
   }
   __syncthreads();

@@ -520,3 +520,19 @@ def test_wide_forms_of_other_shapes_in_direct_form(form, nt, cnames, d, n, mixed
     assert len([name for name in names_launched if name.startswith("round_")]) < n, names_launched
     for t in dev:
         t.free()
+
+
+@pytest.mark.parametrize("d,K,n", [(4, 1, 9), (8, 1, 8), (4, 3, 7), (8, 5, 5), (4, 7, 6), (4, 48, 3)])
+@pytest.mark.parametrize("form,nt", [
+    ("(* t0 t1)", 2),                                    # two accumulators: 64 pairs fit the lanes
+    ("(* t0 t1 t2 t0 t1 t2)", 3),                        # the most factors and points, one group
+    ("(+ (* 7 t0) (* t0 t1) (* t1 t2 t3))", 4),          # groups of one, two and three factors on one wavefront
+    ("(+ (* t0 t1) (* t2 t3) (* t4 t5) (* t0 t5) (* t1 t4) (* t2 t2))", 6),  # twelve accumulators: 16 pairs
+], ids=["pair", "degree-six", "mixed-degrees", "six-groups"])
+def test_rounds_spread_over_the_lanes(form, nt, d, K, n):
+    """The last rounds, an accumulator of one pair per lane: every number of pairs down to one (and an odd number of
+    blocks, whose lanes are the next power of two), with the accumulators' words halved over 0 to 3 lane bits."""
+    rng = np.random.default_rng(K * 100 + n * 10 + nt)
+    tables = [rand_ext(rng, (K << n,), d) for _ in range(nt)]
+    bw = rand_ext(rng, (K,), d) if K > 1 else None
+    prove_both("spread", d, n, form, ["t%d" % t for t in range(nt)], tables, eq=rand_ext(rng, (n,), d), block_weights=bw)
