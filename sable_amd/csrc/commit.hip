@@ -539,9 +539,12 @@ __device__ __forceinline__ void load_digest(const uint32_t *p, uint32_t h[8]) {
 // (level k + 1 starts 8 * n_k words after level k) and carried to the next step through LDS.
 // LEAVES 0: `level` holds digests; 1: the bottom nodes are the leaf digests of ncols codewords
 // (written too); 2: of an oracle codeword.
+// With cap_out the last level is the cap: its words go to pinned host memory as 64-bit words (seq << 32 | value)
+// too, eight lanes to a digest.  Height 0 (one workgroup, at most BLOCK / 2 leaves): the leaves are the cap.
 template <int LEAVES>
 __global__ __launch_bounds__(BLOCK) void subtree_kernel(uint32_t *level, uint64_t n, int height, const uint32_t *cw,
-                                                        int ncols, uint64_t cw_len) {
+                                                        int ncols, uint64_t cw_len, unsigned long long *cap_out,
+                                                        uint32_t seq) {
   __shared__ uint32_t lds[BLOCK][9];  // a digest per row, padded against bank conflicts
   const uint32_t t = threadIdx.x;
   uint64_t first = (uint64_t)blockIdx.x * BLOCK;  // this workgroup's first node of the level being written
@@ -564,12 +567,18 @@ __global__ __launch_bounds__(BLOCK) void subtree_kernel(uint32_t *level, uint64_
       store_digest(level + 8 * c0, left);
       store_digest(level + 8 * (c0 + 1), right);
     }
-    b3_node(left, right, h);
-    store_digest(out + 8 * (first + t), h);
+    if (height > 0) {
+      b3_node(left, right, h);
+      store_digest(out + 8 * (first + t), h);
 #pragma unroll
-    for (int i = 0; i < 8; i++) lds[t][i] = h[i];
+      for (int i = 0; i < 8; i++) lds[t][i] = h[i];
+    } else if (2 * t + 1 < BLOCK) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) lds[2 * t][i] = left[i], lds[2 * t + 1][i] = right[i];
+    }
   }
   uint32_t width = BLOCK;  // nodes of the current level held by this workgroup (when full)
+  if (height == 0) count = n;
   for (int s = 1; s < height; s++) {
     __syncthreads();
     out += 8 * count;
@@ -586,6 +595,13 @@ __global__ __launch_bounds__(BLOCK) void subtree_kernel(uint32_t *level, uint64_
 #pragma unroll
       for (int i = 0; i < 8; i++) lds[t][i] = h[i];
     }
+  }
+  if (cap_out) {
+    __syncthreads();
+    for (uint32_t w = t; w < 8 * width; w += BLOCK)
+      if (first + w / 8 < count)
+        __hip_atomic_store(cap_out + 8 * first + w, ((unsigned long long)seq << 32) | lds[w / 8][w % 8], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -610,8 +626,14 @@ static int cap_level_of(uint64_t leaves) {  // src/pcs.lisp:57-59
 // Every level of the tree at d_levels (leaves first), a few launches of up to nine levels each; the
 // leaf digests are computed by the first launch (leaves 1: ncols codewords, 2: an oracle codeword) or
 // already there (0).  A single leaf (no node above it) is hashed by the same kernel's bottom step.
+// With cap_out (an oracle's tree, of two leaves or more) the tree ends at its cap, and the launch that reaches it
+// writes the cap to the host, see subtree_kernel: nobody reads the levels above.  Seven levels of one compression's
+// latency and one or two launches less per oracle: an opening at nv = 23 (eight oracles) 1312 -> 1207 us.  Not for a
+// tree that is handed out: the words arrive before the launch has ended, when a reader on another stream may not yet
+// look at the levels.
 static int merkle_tree_launch(uint32_t *d_levels, uint64_t nleaves, int leaves, const uint32_t *cw, int ncols,
-                              uint64_t cw_len, uint64_t *cap_rows, uint64_t *cap_off_words) {
+                              uint64_t cw_len, uint64_t *cap_rows, uint64_t *cap_off_words,
+                              unsigned long long *cap_out = nullptr, uint32_t seq = 0) {
   Context &c = ctx();
   uint32_t *level = d_levels;
   uint64_t n = nleaves;
@@ -622,24 +644,30 @@ static int merkle_tree_launch(uint32_t *d_levels, uint64_t nleaves, int leaves, 
     hipLaunchKernelGGL(single_leaf_kernel<1>, dim3(1), dim3(64), 0, c.stream, level, cw, ncols, cw_len);
   if (nleaves == 1 && leaves == 2)
     hipLaunchKernelGGL(single_leaf_kernel<2>, dim3(1), dim3(64), 0, c.stream, level, cw, ncols, cw_len);
-  while (n > 1) {
+  const uint64_t stop = cap_out ? nleaves >> lc : 1;
+  while (n > stop || (cap_out && leaves != 0)) {
     int height = 0;
     // The launch that hashes the leaves climbs few levels: above the leaves every level halves the threads at work
     // and costs a whole compression's latency, so a workgroup of a tall launch idles most of its life (measured at
     // 2^22 leaves: 246 us with nine levels in the first launch, 198 us with five, 175 us with three; five leaves the
     // fewest launches above -- over digests only, nine levels each -- and the shortest commit, 0.51 against 0.55 ms).
     static const int leaf_height = getenv("EXH_MERKLE_LEAF_HEIGHT") ? atoi(getenv("EXH_MERKLE_LEAF_HEIGHT")) : 5;
-    const int max_height = leaves != 0 ? leaf_height : 9;
-    for (uint64_t v = n; v > 1 && height < max_height; v >>= 1) height++;
+    // (a workgroup to a compute unit or fewer leave no other work to idle beside: one launch climbs all it can)
+    const int max_height = leaves != 0 && !(cap_out && n / 2 <= 128 * BLOCK) ? leaf_height : 9;
+    for (uint64_t v = n; v > stop && height < max_height; v >>= 1) height++;
+    unsigned long long *const out = n >> height == stop ? cap_out : nullptr;
     uint32_t grid = (uint32_t)((n / 2 + BLOCK - 1) / BLOCK);
     c.prof_begin(leaves == 1 ? "merkle_leaves" : leaves == 2 ? "merkle_oracle_leaves" : "merkle_levels", 0,
                  (leaves == 1 ? (uint64_t)ncols * 16 * n : leaves == 2 ? 128 * n : 0) + 64 * n);
     if (leaves == 1)
-      hipLaunchKernelGGL(subtree_kernel<1>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len);
+      hipLaunchKernelGGL(subtree_kernel<1>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len, out,
+                         seq);
     else if (leaves == 2)
-      hipLaunchKernelGGL(subtree_kernel<2>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len);
+      hipLaunchKernelGGL(subtree_kernel<2>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len, out,
+                         seq);
     else
-      hipLaunchKernelGGL(subtree_kernel<0>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len);
+      hipLaunchKernelGGL(subtree_kernel<0>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len, out,
+                         seq);
     c.prof_end();
     leaves = 0;
     for (int s = 0; s < height; s++) {
@@ -1865,11 +1893,10 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
       o.levels = mem.alloc((2 * o.nleaves) * 8);
       if (!o.levels) return E_NOMEM;
       uint64_t rows = 0, cap_off = 0;
-      if ((status = merkle_tree_launch(o.levels, o.nleaves, 2, o.cw, 1, o.cw_len, &rows, &cap_off))) return status;
       const size_t cap_at = BF_MAX_ROUNDS * BF_ROUND_SLOT + cap_slots * BF_CAP_SLOT;
-      hipLaunchKernelGGL(deliver_kernel, dim3(1), dim3(BLOCK), 0, c.stream, o.levels + cap_off, (uint32_t)(8 * rows),
-                         reinterpret_cast<unsigned long long *>(pin_dev + cap_at), seq);
-      EXH_HIP(hipGetLastError());
+      if ((status = merkle_tree_launch(o.levels, o.nleaves, 2, o.cw, 1, o.cw_len, &rows, &cap_off,
+                                       reinterpret_cast<unsigned long long *>(pin_dev + cap_at), seq)))
+        return status;
       cap_slots++;
       std::vector<uint32_t> cap_words(8 * rows);
       if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(pin + cap_at), 8 * rows, seq,

@@ -171,3 +171,10 @@ def test_openings_from_base_columns(classes):
     if max(c for c, _ in classes) <= 5:  # (no round: nothing joins, so only the largest class is opened)
         classes = classes[-1:]
     test_opening_matches_the_oracle_and_verifies(classes)
+
+
+@pytest.mark.parametrize("c", [8, 10, 11, 12, 19, 20])
+def test_oracle_trees_that_end_at_their_cap(c):
+    """The first oracle has 2^(c - 3) leaves: at most 128, where the leaves are the cap, one and two levels below it,
+    the most that one launch climbs (nine) and one more, which takes two."""
+    test_opening_matches_the_oracle_and_verifies([(c, 1)])
