@@ -1325,19 +1325,6 @@ struct BfBaseArgs {
 };
 static_assert(sizeof(BfBaseArgs) <= 4096, "kernel arguments");
 
-// sum over b of coef[b][c] v[b] / R for N = 2, 4 or 8 products
-template <int N>
-__device__ __forceinline__ uint32_t mont_dot(const uint32_t (*coef)[8], int c, const uint32_t *v) {
-  uint64_t t = 0;
-#pragma unroll
-  for (int b = 0; b < N; b++) {
-    // four products below p^2 fit 64 bits; from then on, two at a time above a sum brought below p 2^32
-    if (b >= 4 && b % 2 == 0) t = mont_lazy(t);
-    t += (uint64_t)coef[b][c] * v[b];
-  }
-  return mont_reduce4(t);
-}
-
 // TT: the table of level TT from the base columns, with the next round's sums (0: no table part).
 // CW: the codeword of level CW = 1 or 2 from the base codewords; 3: a plain fold of a codeword of elements.
 template <int TT, int CW>

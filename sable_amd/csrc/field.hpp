@@ -68,11 +68,13 @@ EXH_HD uint32_t mont_reduce(uint64_t t) {
   uint32_t r = (uint32_t)(t >> 32) - u;  // low words cancel exactly
   return umin32(r, r + P);
 }
-// t / R mod p for any t < 4 p^2 < 2^64 (a sum of four products): result in [0, p)
+// t / R mod p for any t < 2^64 whose high word is below 2 p: result in [0, p).  That holds for a sum of four products
+// (below 4 p^2, high word below 1.985 p) and for what mont_lazy leaves plus two products (below p 2^32 + 2 p^2, high word
+// below 1.993 p).
 EXH_HD uint32_t mont_reduce4(uint64_t t) {
   uint32_t m = (uint32_t)t * PINV;
   uint32_t u = (uint32_t)(((uint64_t)m * P) >> 32);  // < p
-  uint32_t hi = (uint32_t)(t >> 32);                 // < 1.99 p
+  uint32_t hi = (uint32_t)(t >> 32);                 // < 2 p
   hi = umin32(hi, hi - P);                           // < p (the wrapped alternative is the larger unsigned value)
   uint32_t r = hi - u;                               // in (-p, p): no comparison, no select
   return umin32(r, r + P);
@@ -83,6 +85,18 @@ EXH_HD uint32_t mont_mul(uint32_t a, uint32_t b) { return mont_reduce((uint64_t)
 EXH_HD uint64_t mont_lazy(uint64_t t) {
   const uint32_t hi = (uint32_t)(t >> 32);
   return (uint64_t)umin32(hi, hi - P) << 32 | (uint32_t)t;
+}
+// sum over b of coef[b][c] v[b] / R for N = 2, 4 or 8 products
+template <int N>
+EXH_HD uint32_t mont_dot(const uint32_t (*coef)[8], int c, const uint32_t *v) {
+  uint64_t t = 0;
+#pragma unroll
+  for (int b = 0; b < N; b++) {
+    // four products below p^2 fit 64 bits; from then on, two at a time above a sum brought below p 2^32
+    if (b >= 4 && b % 2 == 0) t = mont_lazy(t);
+    t += (uint64_t)coef[b][c] * v[b];
+  }
+  return mont_reduce4(t);
 }
 // exact a b mod p (two reductions; host-side helpers and rare device paths)
 EXH_HD uint32_t fmul(uint32_t a, uint32_t b) { return mont_mul(mont_mul(a, b), R2); }

@@ -203,3 +203,54 @@ def test_the_bench_constants_go_with_the_present_kernel_sources():
     bench = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(bench)
     assert bench.MEASURED["kernel_sources_sha256"] == bench.kernel_sources_sha256()
+
+
+SUMS = r"""
+#include <stdio.h>
+#include "field.hpp"
+using namespace exh;
+template <int N> void dots(const uint32_t *a, const uint32_t *b) {
+  uint32_t coef[N][8];
+  for (int k = 0; k < N; k++) for (int c = 0; c < 8; c++) coef[k][c] = a[k];
+  printf("%d %u\n", N, mont_dot<N>(coef, 5, b));
+}
+int main() {
+  uint32_t a[64], b[64];
+  int n;
+  while (scanf("%d", &n) == 1) {
+    for (int k = 0; k < n; k++) if (scanf("%u %u", a + k, b + k) != 2) return 1;
+    if (n == 2) dots<2>(a, b);
+    if (n == 4) dots<4>(a, b);
+    if (n == 8) dots<8>(a, b);
+    // a round message's word: two products at a time above a sum brought down
+    uint64_t t = 0;
+    for (int k = 0; k < n; k++) {
+      if (k % 2 == 0) t = mont_lazy(t);
+      t += (uint64_t)a[k] * b[k];
+    }
+    printf("%d %u\n", n, mont_reduce4(t));
+  }
+}
+"""
+
+
+def test_lazily_reduced_sums_of_products(tmp_path):
+    """field.hpp's sums of products between reductions, on the host: every operand p - 1 (the largest sums, a high word
+    just below 2 p), sums that end at a multiple of p 2^32 and random ones, against Python's integers."""
+    import subprocess
+    P, rng = sa.P, np.random.default_rng(3)
+    (tmp_path / "sums.cpp").write_text(SUMS)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-w", "-I", os.path.join(ROOT, "sable_amd", "csrc"), "-o",
+                    str(tmp_path / "sums"), str(tmp_path / "sums.cpp")], check=True, timeout=120)
+    cases = []
+    for n in (2, 4, 6, 8, 16, 64):
+        cases += [[(P - 1, P - 1)] * n, [(P - 1, 1)] * n, [(0, P - 1)] * n,
+                  [(P - 1, P - 1)] * (n - 1) + [(1, pow(2, 32, P))]]
+        cases += [[(int(x), int(y)) for x, y in rng.integers(0, P, (n, 2))] for _ in range(50)]
+    text = "\n".join("%d %s" % (len(c), " ".join("%d %d" % p for p in c)) for c in cases)
+    got = subprocess.run([str(tmp_path / "sums")], input=text, capture_output=True, text=True, check=True, timeout=60)
+    want = []
+    for c in cases:
+        word = "%d %d" % (len(c), sum(x * y for x, y in c) * pow(2, -32, P) % P)
+        want += [word] * (2 if len(c) in (2, 4, 8) else 1)
+    assert got.stdout.split("\n")[:-1] == want
