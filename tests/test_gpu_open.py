@@ -178,3 +178,25 @@ def test_oracle_trees_that_end_at_their_cap(c):
     """The first oracle has 2^(c - 3) leaves: at most 128, where the leaves are the cap, one and two levels below it,
     the most that one launch climbs (nine) and one more, which takes two."""
     test_opening_matches_the_oracle_and_verifies([(c, 1)])
+
+
+@pytest.mark.parametrize("classes,queries", [
+    ([(8, 70)], 130),                      # 9100 quads of leaves and the oracles': two launches of the gather
+    ([(9, 3), (12, 70)], 130),             # and with paths behind the launches' border
+    ([(c, 1) for c in range(5, 23)], 5),   # 68 weight tables, of which one launch builds 64
+], ids=["leaves", "leaves-and-paths", "many-classes"])
+def test_openings_beyond_one_launch_of_a_kind(classes, queries):
+    nv = max(c for c, _ in classes)
+    both = [committed(c, ncols, 700 + 10 * c + ncols) for c, ncols in classes]
+    dev, host = [d for d, _ in both], [h for _, h in both]
+    rr = orc.splitmix_field(29 + nv, nv * 8).reshape(nv, 8)
+    v = np.zeros(8, np.uint32)
+    for key in host:
+        v = orc.ext_add(v, orc.mle_eval(key["h"], rr[nv - key["c"]:], 8))
+    for _ in range(2):  # (the second proof's words land where the first one's lie)
+        tr, otr = sa.Transcript("open", 4), orc.Transcript("open", 4)
+        assert sa.pcs_open(tr, nv, dev, rr, v, queries=queries) == orc.pcs_open(otr, nv, host, rr, v, queries=queries)
+        assert tr.proof() == otr.proof(), "opening: proof bytes differ from the oracle's"
+    vtr = sa.Transcript("open", 4, proof=tr.proof())
+    assert sa.pcs_verify_opening(vtr, nv, dev, rr, v, queries=queries) and vtr.finished()
+    free(dev)
