@@ -1240,6 +1240,10 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // computing a third of the accumulators of a pair per lane; a unit is a few products where a third of a GKR layer's
   // accumulators is four, and the sum over the pairs halves its words over the lanes first.
   // (with several blocks the pairs are no power of two: a unit's lanes are the next one)
+  // 192 is what three wavefronts hold: a round beyond that takes the shares below.  With the rule and without it, us:
+  // the interpreter gains most (six groups, n = 12: 497 and 683; one group of six factors, n = 10: 428 and 767), the
+  // kernels of a statement's own are about even (a launch over GKR layers: one lookup 28.2 and 27.6, two 34.2 and 34.7,
+  // three 52.6 and 53.4 with the glue, 57.0 and 51.2 without; over the blocks of two lookups 21.5 and 25.3).
   auto spreads = [&](uint32_t pairs) {
     return SPREAD && BLOCK == 256 && d.NV == 0 && pairs <= 64 && ((uint32_t)d.nacc << lane_bits(pairs)) <= 192;
   };
