@@ -45,8 +45,8 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "cf29373c05cd0362b530efea8ede22474ab9d02e96d71e4fbb5537d908d9df26",
-    "traffic": {("round_nodes_base", 24): 204058883, ("round_fold2_base", 24): 404005645},
+    "kernel_sources_sha256": "d2cfeb9f4b755f3b43f82258767dea9734521640e7cc63880e7391a67ce17059",
+    "traffic": {("round_nodes_base", 24): 204044940, ("round_fold2_base", 24): 404016799},
     # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), 272 multiply-adds and 96 multiplies of
     # the reductions in the extension rounds (2^21 + 2^20 + ... pairs)
     "int32_mul_per_prove": 76 * (1 << 22) + 368 * ((1 << 21) + (1 << 20) + (1 << 19) + (1 << 19)),
