@@ -1235,9 +1235,9 @@ __global__ __launch_bounds__(BLOCK) void bf_step_kernel(BfStepArgs a) {
 // columns under the weights, so an entry costs eight multiply-adds.  Level LB's table comes straight from the base
 // columns (2^LB products per column and coordinate: BIND-PREFIX, src/sumcheck.lisp:496-510), and so does the codeword
 // of the first level that anybody looks at (level 2, or 1 when a class joins there): both are linear in H.
-// At nv = 23 and two columns the combination, rounds 0 to 2 and the codeword's folds to level 2 moved 2.3 GB; this way
-// they move 0.55 GB, and an opening of 2^23 x 2 takes 918 us in place of 1517 (the same library with every class
-// combined; 2^23 x 8: 1151 and 1589).
+// At nv = 23 and two columns the combinations and the folds to the table of level 3 and the codeword of level 2 are
+// 3.2 GB; this way they are 0.49 GB (by the counters), and an opening of 2^23 x 2 takes 918 us in place of 1517 (the same
+// library with every class combined; 2^23 x 8: 1151 and 1589).
 // The line at eight columns: their constants (384 bytes a column) fill the 4 KiB of a kernel's arguments.  The two ways
 // meet there at 2^20 (base columns and combined, us: 588 / 656 at one column, 618 / 660 at four, 639 / 668 at six, 666 / 668
 // at eight), at 2^16 (401 / 449 at one, 450 / 446 at eight) and below (2^13 x 8 305 / 318, 2^10 x 8 211 / 215); above 2^20
