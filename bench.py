@@ -45,7 +45,7 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "d2cfeb9f4b755f3b43f82258767dea9734521640e7cc63880e7391a67ce17059",
+    "kernel_sources_sha256": "f61b985680ef3d6123ac81708d7da1438b9195d220fb0da110c0b8e035ac4d81",
     "traffic": {("round_nodes_base", 24): 204044940, ("round_fold2_base", 24): 404016799},
     # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), 272 multiply-adds and 96 multiplies of
     # the reductions in the extension rounds (2^21 + 2^20 + ... pairs)

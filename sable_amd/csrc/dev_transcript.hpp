@@ -3,8 +3,9 @@
 // transcript operations a prover round needs (src/transcript.lisp:95-100, 116-128, 152-176).  It absorbs
 // and squeezes exactly the bytes the host transcript would.
 //
-// One wavefront runs it, every lane executing the same (uniform) steps, and a lone wavefront issues an instruction
-// every 4.3 cycles (5.2 in the longer encoding) whatever it depends on: what counts is the number of instructions.
+// One wavefront runs it, every lane executing the same (uniform) steps.  A lone wavefront issues dependent instructions
+// 8.0 cycles apart and independent ones 5.0 (256 of a kind in a row between two clock readings), so a step costs its
+// longest chain first and its number of instructions second.
 // The compression function is spread over the four lanes of each quad: lane i holds column i of the 4x4 state, so the
 // four G functions of a half-round run side by side.  The chaining value stays in registers, where the compression
 // takes and leaves it (lane i: words i and 4 + i); the pending block is a 128-byte ring in LDS (two 64-byte halves
