@@ -45,11 +45,11 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "f61b985680ef3d6123ac81708d7da1438b9195d220fb0da110c0b8e035ac4d81",
-    "traffic": {("round_nodes_base", 24): 204044940, ("round_fold2_base", 24): 404016799},
-    # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), 272 multiply-adds and 96 multiplies of
-    # the reductions in the extension rounds (2^21 + 2^20 + ... pairs)
-    "int32_mul_per_prove": 76 * (1 << 22) + 368 * ((1 << 21) + (1 << 20) + (1 << 19) + (1 << 19)),
+    "kernel_sources_sha256": "1cb6e57b07c3d638bf21f5ef80d8a0aea69d847fa3430f3fec99865772392b6f",
+    "traffic": {("round_nodes_base", 24): 204089568, ("round_fold2_base", 24): 202987904, ("round_fold3_base", 24): 303140608},
+    # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), and multiply-adds and multiplies of the
+    # reductions of 344 in round 2 (2^21 pairs), 440 in round 3 (2^20) and 368 in the extension rounds (2^19 + 2^18 + ...)
+    "int32_mul_per_prove": 76 * (1 << 22) + 344 * (1 << 21) + 440 * (1 << 20) + 368 * (1 << 20),
 }
 KERNEL_SOURCES = ["sumcheck_kernels.hpp", "field.hpp", "dev_transcript.hpp", "blake3.hpp", "stmtdesc.hpp"]
 

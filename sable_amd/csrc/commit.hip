@@ -786,7 +786,7 @@ int merkle_levels_injected_device(const uint32_t *d_leaves, uint64_t nleaves, in
 // pick(tt) pick(et), pick = even entry, odd entry, 2 odd - even.  Partials per workgroup.
 __global__ __launch_bounds__(BLOCK) void dot_pairs_kernel(const uint32_t *tt, const uint32_t *et, uint64_t n_pairs,
                                                           uint32_t *partials) {
-  Acc96 acc[3][8];
+  AccLazy acc[3][8];
 #pragma unroll
   for (int k = 0; k < 3; k++)
 #pragma unroll
@@ -1137,7 +1137,7 @@ __device__ __forceinline__ void bf_deliver_sums(const RoundTotals &totals, const
 }
 
 // a step's two weighted sums, accumulated per lane, to their delivery
-__device__ __forceinline__ void bf_finish_sums(const BfStepArgs &a, Acc96 (*acc)[8], uint64_t tile_start) {
+__device__ __forceinline__ void bf_finish_sums(const BfStepArgs &a, AccLazy (*acc)[8], uint64_t tile_start) {
   __shared__ uint32_t lds[BLOCK / 64][16];
   __shared__ uint32_t mine[16];
   const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -1183,7 +1183,7 @@ __global__ __launch_bounds__(BLOCK) void bf_step_kernel(BfStepArgs a) {
   }
   const uint64_t tile = (uint64_t)BLOCK * a.pairs_per_thread, tile_start = (uint64_t)blockIdx.x * tile;
   const uint64_t low_mask = ((uint64_t)1 << a.low_bits) - 1;
-  Acc96 acc[2][8];
+  AccLazy acc[2][8];
 #pragma unroll
   for (int q = 0; q < 2; q++)
 #pragma unroll
@@ -1374,7 +1374,7 @@ __global__ __launch_bounds__(BLOCK) void bf_base_kernel(BfBaseArgs a) {
     constexpr int B = 1 << TT;
     const uint64_t tile = (uint64_t)BLOCK * a.s.pairs_per_thread, tile_start = (uint64_t)blockIdx.x * tile;
     const uint64_t low_mask = ((uint64_t)1 << a.s.low_bits) - 1;
-    Acc96 acc[2][8];
+    AccLazy acc[2][8];
 #pragma unroll
     for (int q = 0; q < 2; q++)
 #pragma unroll

@@ -80,11 +80,24 @@ EXH_HD uint32_t mont_reduce4(uint64_t t) {
   return umin32(r, r + P);
 }
 EXH_HD uint32_t mont_mul(uint32_t a, uint32_t b) { return mont_reduce((uint64_t)a * b); }
+// A sum of products on its way, kept as it is written: the compiler otherwise adds two products up by themselves and the
+// sum to that, and splits a sum whose high word has been brought down into its two words (one and three instructions
+// more a time; a product into the sum is one).
+EXH_HD void keep_sum(uint64_t &t) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+v"(t));
+#endif
+}
 // Between the products of a longer sum: a sum t < 2^64 whose high word is below 2 p brought below p 2^32 (the same
 // residue).  Two more products below p^2 then keep it below p 2^32 + 2 p^2 < 2^64 with a high word below 2 p again.
 EXH_HD uint64_t mont_lazy(uint64_t t) {
   const uint32_t hi = (uint32_t)(t >> 32);
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef uint32_t words __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint64_t, words{(uint32_t)t, umin32(hi, hi - P)});
+#else
   return (uint64_t)umin32(hi, hi - P) << 32 | (uint32_t)t;
+#endif
 }
 // sum over b of coef[b][c] v[b] / R for N = 2, 4 or 8 products
 template <int N>
@@ -185,11 +198,12 @@ EXH_HD Ext<D> ext_scale_mont(const Ext<D> &a, uint32_t s) {
   return o;
 }
 
-// The D unreduced coefficient sums of a * b in F_p[w]/(w^D - 3), each a sum of D products with the
-// wrapping b's tripled first (src/field.lisp:220-234); emit(e_tower, group, sum) receives them in
-// groups of at most four products.
-template <int D, class F>
-EXH_HD void ext_mul_sums(const Ext<D> &a, const Ext<D> &b, F emit) {
+// The D coefficient sums of a * b in F_p[w]/(w^D - 3), each a sum of D products with the wrapping b's tripled first
+// (src/field.lisp:220-234): start(e) gives what coefficient e (tower order) starts from and emit(e, sum) takes the sum.
+// CARRIED: a sum starts below p 2^32, else at zero; it is brought below p 2^32 again (mont_lazy) whenever two more products
+// could take its high word to 2 p, so that mont_reduce4 and mont_lazy take what is emitted.
+template <int D, bool CARRIED, class Start, class Emit>
+EXH_HD void ext_mul_sums(const Ext<D> &a, const Ext<D> &b, Start start, Emit emit) {
   uint32_t pa[D], pb[D], pb3[D];
 #pragma unroll
   for (int e = 0; e < D; e++) {
@@ -201,27 +215,24 @@ EXH_HD void ext_mul_sums(const Ext<D> &a, const Ext<D> &b, F emit) {
   for (int j = 1; j < D; j++) pb3[j] = times3(pb[j]);
 #pragma unroll
   for (int e = 0; e < D; e++) {
+    uint64_t t = start(brev(e, D));
 #pragma unroll
-    for (int g = 0; g < D; g += 4) {
-      uint64_t t = 0;
-#pragma unroll
-      for (int i = g; i < g + 4; i++) {
-        int j = (e - i) & (D - 1);
-        t += (uint64_t)pa[i] * (i > e ? pb3[j] : pb[j]);
-      }
-      emit(brev(e, D), g / 4, t);
+    for (int i = 0; i < D; i++) {
+      const int j = (e - i) & (D - 1);
+      if (i % 2 == 0 && i >= (CARRIED ? 2 : 4)) t = mont_lazy(t);
+      t += (uint64_t)pa[i] * (i > e ? pb3[j] : pb[j]);
+      if (i % 2 == 0 && i >= (CARRIED ? 0 : 4)) keep_sum(t);
     }
+    emit(brev(e, D), t);
   }
 }
 
-// a b / R
+// a b / R: one reduction per coefficient.  (At D = 8, with the two halves' sums reduced by themselves and added up, and the
+// sums in the compiler's order, a pair of a four-factor statement's fold round was 5870 instructions; 5030 this way.)
 template <int D>
 EXH_HD Ext<D> ext_mul_mont(const Ext<D> &a, const Ext<D> &b) {
   Ext<D> o;
-  ext_mul_sums<D>(a, b, [&](int e, int g, uint64_t t) {
-    uint32_t r = mont_reduce4(t);
-    o.c[e] = g == 0 ? r : fadd(o.c[e], r);
-  });
+  ext_mul_sums<D, false>(a, b, [](int) { return (uint64_t)0; }, [&](int e, uint64_t t) { o.c[e] = mont_reduce4(t); });
   return o;
 }
 // exact a b (host-side helpers)
@@ -233,10 +244,19 @@ EXH_HD Ext<D> ext_mul(const Ext<D> &a, const Ext<D> &b) {
   return o;
 }
 
-// acc += a b, unreduced (D 96-bit accumulators in tower order)
+// A sum of any number of extension products: a 64-bit word per coefficient, kept below p 2^32 by mont_lazy.
+struct AccLazy {
+  uint64_t v;
+};
+EXH_HD void acc_zero(AccLazy &a) { a.v = 0; }
+EXH_HD uint32_t acc_reduce(const AccLazy &a) {  // mod p, exactly
+  return mont_reduce4((a.v >> 32) * (uint64_t)R2 + (uint64_t)(uint32_t)a.v * R1);  // < 4 p^2
+}
+// acc += a b (D sums in tower order).  Eight registers at D = 4 where 96-bit sums take twelve, sixteen for twenty-four at
+// D = 8, for the same number of instructions.
 template <int D>
-EXH_HD void ext_mul_acc(Acc96 *acc, const Ext<D> &a, const Ext<D> &b) {
-  ext_mul_sums<D>(a, b, [&](int e, int, uint64_t t) { acc_add(acc[e], t); });
+EXH_HD void ext_mul_acc(AccLazy *acc, const Ext<D> &a, const Ext<D> &b) {
+  ext_mul_sums<D, true>(a, b, [&](int e) { return acc[e].v; }, [&](int e, uint64_t t) { acc[e].v = mont_lazy(t); });
 }
 // acc += a * s for a base value s
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -270,13 +290,6 @@ EXH_HD void ext_scale_acc(Acc96 *acc, const Ext<D> &a, uint32_t s) {
   for (int i = 0; i < D; i++) acc_mad(acc[i], a.c[i], s);
 }
 #endif
-template <int D>
-EXH_HD Ext<D> acc_reduce_ext(const Acc96 *acc) {
-  Ext<D> o;
-#pragma unroll
-  for (int i = 0; i < D; i++) o.c[i] = acc_reduce(acc[i]);
-  return o;
-}
 
 #if defined(__HIPCC__)
 // ---- KoalaBear in double precision, for the products of base-field values that are sums and differences of

@@ -535,16 +535,17 @@ static uint32_t tile_pairs_per_thread(uint64_t n_pairs, uint64_t max_grid, uint6
   return ppt;
 }
 
+// `folds`: the folds before the sums, 0 or 1, or 2 or 3 of base tables at once; outs: the folded tables (empty: not kept)
 template <int D>
-static int launch_round(SumcheckSession &s, bool fold, bool do_sums, const std::vector<uint32_t *> &outs,
-                        uint64_t n_pairs, int j, bool double_fold = false) {
+static int launch_round(SumcheckSession &s, int folds, bool do_sums, const std::vector<uint32_t *> &outs,
+                        uint64_t n_pairs, int j) {
   Context &c = ctx();
   RoundArgs<D> a;
   memset(&a, 0, sizeof(a));
   int T = s.st.T();
   for (int t = 0; t < T; t++) {
     a.in[t] = s.cur[t];
-    a.out[t] = fold ? outs[t] : nullptr;
+    a.out[t] = folds && !outs.empty() ? outs[t] : nullptr;
   }
   a.n_pairs = n_pairs;
   a.do_sums = do_sums ? 1 : 0;
@@ -559,7 +560,6 @@ static int launch_round(SumcheckSession &s, bool fold, bool do_sums, const std::
   a.deferred = do_sums && ((uint64_t)BLOCK * ppt <= ((uint64_t)1 << a.low_bits)) ? 1 : 0;
   a.partials = s.d_partials;
   a.pstride = s.pstride;
-  a.double_fold = double_fold ? 1 : 0;
   if (s.device_loop) a.ctrl = s.d_ctrl;
   a.consts = s.d_direct;
   uint32_t grid = (uint32_t)((n_pairs + (uint64_t)BLOCK * ppt - 1) / ((uint64_t)BLOCK * ppt));
@@ -580,23 +580,23 @@ static int launch_round(SumcheckSession &s, bool fold, bool do_sums, const std::
       EXH_HIP(hipMemsetAsync(a.arrivals, 0, 4, c.stream));
     }
   }
-  if (fold && !s.device_loop)
+  if (folds && !s.device_loop)
     for (int k = 0; k < D; k++) a.r_mont[k] = to_mont(s.pending_r[k]);
   {
     // bytes this launch must move: every table read once, the folded tables written once
-    uint64_t in_words = (double_fold ? 8 : fold ? 4 : 2) * n_pairs * (s.cur_base ? 1 : D),
-             out_words = fold ? 2 * n_pairs * D : 0;
-    const char *name = double_fold ? "round_fold2_base"
-                       : fold      ? (s.cur_base ? "round_fold_base" : "round_fold_ext")
-                                   : (s.cur_base ? "round_base" : "round_ext");
+    uint64_t in_words = ((uint64_t)2 << folds) * n_pairs * (s.cur_base ? 1 : D), out_words = a.out[0] ? 2 * n_pairs * D : 0;
+    const char *name = folds == 3   ? "round_fold3_base"
+                       : folds == 2 ? "round_fold2_base"
+                       : folds      ? (s.cur_base ? "round_fold_base" : "round_fold_ext")
+                                    : (s.cur_base ? "round_base" : "round_ext");
     c.prof_begin(name, j, (uint64_t)T * 4 * (in_words + out_words));
   }
-  if (double_fold)
-    s.kernels->launch_fold2(&a, grid, c.stream);
+  if (folds >= 2)
+    s.kernels->launch_bind(&a, folds, grid, c.stream);
   else if (s.generated)
-    s.kernels->launch(&a, s.cur_base, fold, grid, c.stream);
+    s.kernels->launch(&a, s.cur_base, folds != 0, grid, c.stream);
   else
-    launch_interp<D>(a, s.desc, s.cur_base, fold, grid, c.stream);
+    launch_interp<D>(a, s.desc, s.cur_base, folds != 0, grid, c.stream);
   c.prof_end();
   if (do_sums && s.device_loop && !own_epilogue) {
     EpilogueArgs e;
@@ -746,8 +746,8 @@ int SumcheckSession::round_sums(uint32_t *out) {
     out_buf.assign(T, nullptr);
     for (int t = 0; t < T; t++) out_buf[t] = (uint32_t *)dst.ptr + (uint64_t)t * out_size * D;
     n_pairs = out_size / 2;
-    status = D == 4 ? launch_round<4>(*this, true, true, out_buf, n_pairs, j)
-                    : launch_round<8>(*this, true, true, out_buf, n_pairs, j);
+    status = D == 4 ? launch_round<4>(*this, 1, true, out_buf, n_pairs, j)
+                    : launch_round<8>(*this, 1, true, out_buf, n_pairs, j);
     if (status) return status;
     for (int t = 0; t < T; t++) cur[t] = out_buf[t];
     cur_base = false;
@@ -756,8 +756,8 @@ int SumcheckSession::round_sums(uint32_t *out) {
     pending_fold = false;
   } else {
     n_pairs = size / 2;
-    status = D == 4 ? launch_round<4>(*this, false, true, out_buf, n_pairs, j)
-                    : launch_round<8>(*this, false, true, out_buf, n_pairs, j);
+    status = D == 4 ? launch_round<4>(*this, 0, true, out_buf, n_pairs, j)
+                    : launch_round<8>(*this, 0, true, out_buf, n_pairs, j);
     if (status) return status;
   }
   size_t words = (size_t)st.nacc * D;
@@ -1056,22 +1056,40 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   int status = OK, j = 0;
   int folds_due = 0;  // folds by the last challenges drawn that the tables still await (2 after the base-field sweep for rounds 0 and 1)
   const char *no_nodes = getenv("EXACTA_HIP_NO_BASE_ROUND1");
+  uint64_t slice_max = SLICE_LDS_BYTES / ((uint64_t)T * 2 * D * 4);
+  if (const char *cap = getenv("EXACTA_HIP_MAX_SLICE_PAIRS"))  // tests: keep more rounds on the streaming kernels
+    slice_max = std::min<uint64_t>(slice_max, strtoull(cap, nullptr, 10));
+  // (proofs running side by side share the device: each one's grid takes its part, a power of two)
+  const uint64_t grid_max = std::min<uint64_t>(256, c.compute_units > 0 ? c.compute_units : 1) / (c.share > 1 ? 2 : 1);
+  // pairs that the grid of LDS-resident slices can take, and the one-workgroup launch: more of them are a streaming round
+  auto slices_max = [&]() { return std::max(slice_max * grid_max, tail_pairs(T, D)); };
   for (; j < n && status == OK; j++) {
     const bool fold_due = folds_due > 0;
     uint64_t n_pairs = (size >> folds_due) / 2;  // pairs summed in round j (after the pending folds)
-    if (folds_due == 2) {  // round 2 after the base-field sweep: both folds at once, then the sums
+    // Rounds 2 and 3 after the base-field sweep read the base tables once more, bound by two and by three challenges at
+    // once.  When round 3 is a streaming round too, nothing of generation 2 is written: generation 3 comes from as many
+    // bytes of the base tables as generation 2 has (half as many at F_p^8), and takes fewer instructions than a fold.
+    // A proof this way and with generation 2 kept, us: four tables of 2^26 at F_p^8 3508 and 4004, of 2^23 765 and 822;
+    // three of 2^24 at F_p^4 479 and 503.  (Where the rounds from 3 on run on slices they take generation 2 as it is.)
+    if (folds_due >= 2) {
       round = j;
-      uint64_t out_size = size / 4;
-      Arena &dst = ((generation + 1) % 2 == 0) ? arena_a() : arena_b();
-      out_buf.assign(T, nullptr);
-      for (int t = 0; t < T; t++) out_buf[t] = (uint32_t *)dst.ptr + (uint64_t)t * out_size * D;
-      status = D == 4 ? launch_round<4>(*this, true, true, out_buf, n_pairs, j, true)
-                      : launch_round<8>(*this, true, true, out_buf, n_pairs, j, true);
-      for (int t = 0; t < T; t++) cur[t] = out_buf[t];
-      cur_base = false;
-      size = out_size;
-      generation += 2;
-      folds_due = 1;
+      const bool keep = folds_due == 3 || n_pairs / 2 <= slices_max();
+      if (keep) {
+        const uint64_t out_size = size >> folds_due;
+        Arena &dst = ((generation + folds_due - 1) % 2 == 0) ? arena_a() : arena_b();
+        out_buf.assign(T, nullptr);
+        for (int t = 0; t < T; t++) out_buf[t] = (uint32_t *)dst.ptr + (uint64_t)t * out_size * D;
+        status = D == 4 ? launch_round<4>(*this, folds_due, true, out_buf, n_pairs, j)
+                        : launch_round<8>(*this, folds_due, true, out_buf, n_pairs, j);
+        for (int t = 0; t < T; t++) cur[t] = out_buf[t];
+        cur_base = false;
+        size = out_size;
+        generation += folds_due;
+        folds_due = 1;
+      } else {
+        status = D == 4 ? launch_round<4>(*this, 2, true, {}, n_pairs, j) : launch_round<8>(*this, 2, true, {}, n_pairs, j);
+        folds_due = 3;
+      }
       tail_done = false;
       continue;
     }
@@ -1085,12 +1103,6 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
     // slice need not lie in one block)
     uint64_t odd = n_pairs;
     while (odd > 1 && odd % 2 == 0) odd /= 2;
-    uint64_t slice_max = SLICE_LDS_BYTES / ((uint64_t)T * 2 * D * 4);
-    if (const char *cap = getenv("EXACTA_HIP_MAX_SLICE_PAIRS"))  // tests: keep more rounds on the streaming kernels
-      slice_max = std::min<uint64_t>(slice_max, strtoull(cap, nullptr, 10));
-    // (proofs running side by side share the device: each one's grid takes its part, a power of two)
-    const uint64_t grid_max =
-        std::min<uint64_t>(256, c.compute_units > 0 ? c.compute_units : 1) / (c.share > 1 ? 2 : 1);
     if (odd > 1) {  // (EXACTA_HIP_NO_BLOCK_SLICES=1: tables of several blocks stay on the streaming kernels)
       const char *no_block_slices = getenv("EXACTA_HIP_NO_BLOCK_SLICES");
       if (no_block_slices && no_block_slices[0] == '1') odd = 17;
@@ -1145,15 +1157,15 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
       continue;
     }
     if (!fold_due) {
-      status = D == 4 ? launch_round<4>(*this, false, true, out_buf, n_pairs, j)
-                      : launch_round<8>(*this, false, true, out_buf, n_pairs, j);
+      status = D == 4 ? launch_round<4>(*this, 0, true, out_buf, n_pairs, j)
+                      : launch_round<8>(*this, 0, true, out_buf, n_pairs, j);
     } else {
       uint64_t out_size = size / 2;
       Arena &dst = (generation % 2 == 0) ? arena_a() : arena_b();
       out_buf.assign(T, nullptr);
       for (int t = 0; t < T; t++) out_buf[t] = (uint32_t *)dst.ptr + (uint64_t)t * out_size * D;
-      status = D == 4 ? launch_round<4>(*this, true, true, out_buf, n_pairs, j)
-                      : launch_round<8>(*this, true, true, out_buf, n_pairs, j);
+      status = D == 4 ? launch_round<4>(*this, 1, true, out_buf, n_pairs, j)
+                      : launch_round<8>(*this, 1, true, out_buf, n_pairs, j);
       for (int t = 0; t < T; t++) cur[t] = out_buf[t];
       cur_base = false;
       size = out_size;

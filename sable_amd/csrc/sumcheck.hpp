@@ -17,8 +17,8 @@ namespace exh {
 struct KernelSet {  // the launchers generated for one statement and one degree D, at build time or at run time
   std::function<void(const void *args, bool in_base, bool fold, uint32_t grid, hipStream_t stream)> launch;
   std::function<void(const void *args, uint32_t grid, hipStream_t stream)> launch_tail;
-  // base tables folded twice at once (round 2 after the base-field sweep), and that sweep's slot sums
-  std::function<void(const void *args, uint32_t grid, hipStream_t stream)> launch_fold2;
+  // base tables folded two or three times at once (rounds 2 and 3 after the base-field sweep), and that sweep's slot sums
+  std::function<void(const void *args, int folds, uint32_t grid, hipStream_t stream)> launch_bind;
   std::function<void(const void *args, int pass, uint32_t grid, hipStream_t stream)> launch_nodes;
   int nodes_passes = 0;  // launches of launch_nodes per round (0: not available)
   // workgroups of the tail kernel a compute unit holds at once with that much dynamic LDS (-1: unknown)

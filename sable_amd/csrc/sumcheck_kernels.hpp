@@ -48,7 +48,7 @@ struct Ctrl {
 template <int D>
 struct RoundArgs {
   const uint32_t *in[MAXT];  // the tables read: 4 entries per pair when folding, else 2
-  uint32_t *out[MAXT];       // folded tables written (FOLD)
+  uint32_t *out[MAXT];       // folded tables written (after a fold; null after two or three at once: only the sums)
   const uint32_t *low;       // |LOW| = 2^low_bits EXTs
   const uint32_t *high;      // n_high EXTs
   uint32_t *partials;        // [gridDim.x][nacc][D]
@@ -60,7 +60,6 @@ struct RoundArgs {
   uint32_t r_mont[D];        // the fold challenge, times R (host-driven rounds)
   Ctrl *ctrl;                // device-driven rounds: the fold challenge is read from here (else null)
   uint32_t pstride;          // words per workgroup partial (a power of two >= nacc * D)
-  uint32_t double_fold;      // base tables, folded by challenges 0 and 1 at once (8 entries -> 2 per pair)
   // device-driven rounds: the round's sums meet in counted totals and the last workgroup to arrive sends the
   // message and draws the challenge itself (see RoundTotals); totals null: one partial row per workgroup
   unsigned long long *totals;  // [groups][pstride], zero before the launch
@@ -174,10 +173,6 @@ template <int D>
 __device__ __forceinline__ Ext<D> v_mul(const Ext<D> &a, const Ext<D> &b) { return ext_mul_mont<D>(a, b); }
 template <int D>
 __device__ __forceinline__ void v_weigh(Acc96 *acc, const Ext<D> &w, uint32_t v) { ext_scale_acc<D>(acc, w, v); }
-template <int D>
-__device__ __forceinline__ void v_weigh(Acc96 *acc, const Ext<D> &w, const Ext<D> &v) {
-  ext_mul_acc<D>(acc, v, w);  // the weight second: its tripled wrap coefficients are shared by the pair's points
-}
 
 // integer multiples and integer offsets, for the linear forms
 template <int D>
@@ -210,7 +205,7 @@ __device__ __forceinline__ V v_of(const Ext<D> &w) {
 template <int D>
 __device__ __forceinline__ void v_mul_acc(Acc96 *acc, uint32_t a, uint32_t b) { acc_mad(acc[0], a, b); }
 template <int D>
-__device__ __forceinline__ void v_mul_acc(Acc96 *acc, const Ext<D> &a, const Ext<D> &b) { ext_mul_acc<D>(acc, a, b); }
+__device__ __forceinline__ void v_mul_acc(AccLazy *acc, const Ext<D> &a, const Ext<D> &b) { ext_mul_acc<D>(acc, a, b); }
 
 // A statement too wide for accumulators per table group comes in direct form: its descriptor's type carries an
 // evaluator of the written form (generated code) and a flag, and the accumulators are the wire points.
@@ -223,6 +218,13 @@ struct is_direct {
   static constexpr bool value = sizeof(test<T>(nullptr)) == sizeof(char);
 };
 
+// The accumulators of a pair's words: sums of products of extension elements, or of a weight and a base value (whose two
+// instructions a word the 96-bit sum is cheaper for); a statement in direct form evaluates in the extension either way.
+template <class V, class Desc>
+struct AccOf {
+  typedef typename std::conditional<std::is_same<V, uint32_t>::value && !is_direct<Desc>::value, Acc96, AccLazy>::type type;
+};
+
 // The pair's contribution for a statement in direct form: the tables' lines in Montgomery form (so that sums and
 // products of any shape stay in one scale), the form evaluated at each wire point X = 0, 2, 3, ..., and w times
 // that value added to the point's accumulator.  The loop over the points is kept a loop: the evaluator is long,
@@ -230,7 +232,7 @@ struct is_direct {
 // because each is named by a constant inside the switch.
 template <int D, class V, class Desc, int PARTS, int PART>
 __device__ __forceinline__ void accumulate_direct(const Desc &d, const V *lo, const V *hi, const Ext<D> &w,
-                                                  Acc96 (*acc)[D], const uint32_t *kc) {
+                                                  AccLazy (*acc)[D], const uint32_t *kc) {
   Ext<D> at0[MAXT], slope[MAXT];
 #pragma unroll
   for (int t = 0; t < MAXT; t++)
@@ -267,13 +269,8 @@ __device__ __forceinline__ void accumulate_direct(const Desc &d, const V *lo, co
 // the accumulators by it, and they move from registers to scratch memory): the last rounds, with a pair per lane
 // and lanes to spare, give each of a workgroup's wavefronts a share of a pair's accumulators, so that a round
 // waits for a quarter of the products.
-template <int D, class V, class Desc, int PARTS = 1, int PART = 0>
-__device__ __forceinline__ void accumulate_pair(const Desc &d, const V *lo, const V *hi, const Ext<D> &w,
-                                                Acc96 (*acc)[D], const uint32_t *kc = nullptr) {
-  if constexpr (is_direct<Desc>::value) {
-    accumulate_direct<D, V, Desc, PARTS, PART>(d, lo, hi, w, acc, kc);
-    return;
-  }
+template <int D, class V, class Desc, int PARTS, int PART, class Acc>
+__device__ __forceinline__ void accumulate_groups(const Desc &d, const V *lo, const V *hi, const Ext<D> &w, Acc (*acc)[D]) {
   V cur[MAXT], slope[MAXT];
 #pragma unroll
   for (int t = 0; t < MAXT; t++)
@@ -351,6 +348,15 @@ __device__ __forceinline__ void accumulate_pair(const Desc &d, const V *lo, cons
   }
 }
 
+template <int D, class V, class Desc, int PARTS = 1, int PART = 0, class Acc>
+__device__ __forceinline__ void accumulate_pair(const Desc &d, const V *lo, const V *hi, const Ext<D> &w,
+                                                Acc (*acc)[D], const uint32_t *kc = nullptr) {
+  if constexpr (is_direct<Desc>::value)
+    accumulate_direct<D, V, Desc, PARTS, PART>(d, lo, hi, w, acc, kc);
+  else
+    accumulate_groups<D, V, Desc, PARTS, PART>(d, lo, hi, w, acc);
+}
+
 // A workgroup barrier that orders LDS traffic only: what the threads of a workgroup hand each other in these
 // kernels lives in LDS, and a full barrier would also wait for every global access in flight (the weights fetched
 // a round ahead, the rows on their way to the host).
@@ -369,47 +375,81 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
   return fadd(fadd(a, b), fadd(c, d));
 }
 
-// eq((r0, r1), b) for b = 0..3 (bit 0 of b goes with r0), in Montgomery form: the weights that bind two
-// variables of a base table at once, entry <- sum_b e[b] * T[4 x + b] (BIND-PREFIX, src/sumcheck.lisp:496-510)
-template <int D>
+// eq((r0, .., r_(F-1)), b) for b < 2^F, F = 2 or 3 (bit k of b goes with r_k), in Montgomery form: the weights that bind
+// the first F variables of a base table at once, entry <- sum_b e[b] * T[2^F x + b] (BIND-PREFIX, src/sumcheck.lisp:496-510)
+template <int D, int F>
 struct BindWeights {
-  Ext<D> e[4];
+  Ext<D> e[1 << F];
 };
-template <int D>
-__device__ __forceinline__ BindWeights<D> bind_weights(const Ext<D> &r0_mont, const Ext<D> &r1_mont) {
-  BindWeights<D> w;
-  w.e[3] = ext_mul_mont<D>(r0_mont, r1_mont);  // r0 r1 R
-  w.e[1] = ext_sub<D>(r0_mont, w.e[3]);        // r0 (1 - r1) R
-  w.e[2] = ext_sub<D>(r1_mont, w.e[3]);        // (1 - r0) r1 R
-  Ext<D> one = ext_lift<D>(R1);
-  w.e[0] = ext_add<D>(ext_sub<D>(ext_sub<D>(one, r0_mont), r1_mont), w.e[3]);
+// The weights of challenges 0 to F - 1 (the last one also lies in ctrl->r_mont), a coefficient a lane: every workgroup
+// forms them for itself, and as straight code on values that are the same for all lanes the 2 or 6 products run on the
+// scalar unit, some 1,200 dependent instructions at D = 8 and F = 2 before a workgroup's first pair.  All threads call;
+// the words end up in scalar registers.
+template <int D, int F>
+__device__ __forceinline__ BindWeights<D, F> bind_weights(const Ctrl *ctrl) {
+  __shared__ uint32_t r[F][2 * D];           // the challenges in powers of w, times R; then their triples
+  __shared__ uint32_t e[(1 << F) * D];       // the weights, in powers of w
+  const uint32_t tid = threadIdx.x, k = tid % D;
+  if (tid < (uint32_t)(F * D)) {
+    const uint32_t v = to_mont(ctrl->chal[tid / D][brev(k, D)]);
+    r[tid / D][k] = v, r[tid / D][D + k] = times3(v);
+    if (tid < (uint32_t)D) {
+      const uint32_t one = k == 0 ? R1 : 0u;
+      e[D + k] = v, e[k] = fsub(one, v);  // bound by r_0 alone: r_0 and 1 - r_0
+    }
+  }
+#pragma unroll
+  for (int f = 1; f < F; f++) {  // e[b + 2^f] = e[b] r_f, e[b] -= that
+    __syncthreads();
+    uint32_t at = 0, v = 0, rest = 0;
+    if (tid < (uint32_t)(D << f)) {
+      at = tid / D * D;
+      uint64_t t = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < (uint32_t)D; i++) {
+        const uint32_t j = (k - i) & (D - 1);
+        if (i >= 4 && i % 2 == 0) t = mont_lazy(t);
+        t += (uint64_t)e[at + i] * r[f][i > k ? D + j : j];
+      }
+      v = mont_reduce4(t), rest = fsub(e[at + k], v);
+    }
+    __syncthreads();
+    if (tid < (uint32_t)(D << f)) e[at + k] = rest, e[(D << f) + at + k] = v;
+  }
+  __syncthreads();
+  BindWeights<D, F> w;
+#pragma unroll
+  for (int b = 0; b < 1 << F; b++)
+#pragma unroll
+    for (int c = 0; c < D; c++) w.e[b].c[c] = (uint32_t)__builtin_amdgcn_readfirstlane((int)e[b * D + brev(c, D)]);
   return w;
 }
-// sum_b e[b] * v[b], exact: four products per coordinate, one reduction
-template <int D>
-__device__ __forceinline__ Ext<D> bind4(const BindWeights<D> &w, uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
+// sum_b e[b] * v[b], exact: one reduction per coordinate
+template <int D, int F>
+__device__ __forceinline__ Ext<D> bind(const BindWeights<D, F> &w, const uint32_t *v) {
   Ext<D> o;
 #pragma unroll
-  for (int c = 0; c < D; c++)
-    o.c[c] = mont_reduce4((uint64_t)w.e[0].c[c] * v0 + (uint64_t)w.e[1].c[c] * v1 + (uint64_t)w.e[2].c[c] * v2 +
-                          (uint64_t)w.e[3].c[c] * v3);
+  for (int c = 0; c < D; c++) {
+    uint64_t t = 0;
+#pragma unroll
+    for (int b = 0; b < 1 << F; b++) {
+      if (b >= 4 && b % 2 == 0) t = mont_lazy(t);
+      t += (uint64_t)w.e[b].c[c] * v[b];
+      if (b >= 4 && b % 2 == 0) keep_sum(t);
+    }
+    o.c[c] = mont_reduce4(t);
+  }
   return o;
 }
 
-// the pair (lo, hi) of every table at pair index i, folding first when FOLD (FOLD2: base tables folded
-// twice at once by the bind weights)
-template <int D, bool IN_BASE, bool FOLD, class V, class Desc, bool FOLD2 = false>
+// the pair (lo, hi) of every table at pair index i, folding first when FOLD
+template <int D, bool IN_BASE, bool FOLD, class V, class Desc>
 __device__ __forceinline__ void load_pair(const Desc &d, const uint32_t *const *in, uint32_t *const *out, uint64_t i,
-                                          const Ext<D> &r, V *lo, V *hi, const BindWeights<D> *bw = nullptr) {
+                                          const Ext<D> &r, V *lo, V *hi) {
 #pragma unroll
   for (int t = 0; t < MAXT; t++) {
     if (t < d.T) {
-      if constexpr (FOLD2) {
-        const uint4 *p = reinterpret_cast<const uint4 *>(in[t] + 8 * i);
-        uint4 e = p[0], f = p[1];
-        lo[t] = bind4<D>(*bw, e.x, e.y, e.z, e.w);
-        hi[t] = bind4<D>(*bw, f.x, f.y, f.z, f.w);
-      } else if constexpr (FOLD && IN_BASE) {
+      if constexpr (FOLD && IN_BASE) {
         uint4 e = *reinterpret_cast<const uint4 *>(in[t] + 4 * i);
         lo[t] = fold_base<D>(e.x, e.y, r);
         hi[t] = fold_base<D>(e.z, e.w, r);
@@ -434,27 +474,23 @@ __device__ __forceinline__ void load_pair(const Desc &d, const uint32_t *const *
   }
 }
 
-// The same in two steps, so that a pair's loads can be issued one pair ahead of its arithmetic: the words as
-// they lie in memory (QUADS 16-byte quads per table), then the pair from them.
-template <int D, bool IN_BASE, bool FOLD, bool FOLD2>
+// The same in two steps, so that a table's loads can be issued ahead of their arithmetic: the words as they lie in memory
+// (QUADS 16-byte quads per table), then the pair from them.  FOLDS: the folds before the pair, 0 or 1, or 2 or 3 of base
+// tables at once by the bind weights.
+template <int D, bool IN_BASE, int FOLDS>
 constexpr int raw_quads() {
-  return FOLD2 ? 2 : (FOLD && IN_BASE) ? 1 : FOLD ? D : IN_BASE ? 1 : D / 2;
+  return IN_BASE ? (FOLDS == 3 ? 4 : FOLDS == 2 ? 2 : 1) : FOLDS == 1 ? D : D / 2;
 }
-template <int D, bool IN_BASE, bool FOLD, bool FOLD2, int Q, class Desc>
-__device__ __forceinline__ void fetch_raw(const Desc &d, const uint32_t *const *in, uint64_t i, uint4 (*raw)[Q]) {
+template <int D, bool IN_BASE, int FOLDS, int Q>
+__device__ __forceinline__ void fetch_raw(const uint32_t *in, uint64_t i, uint4 *raw) {
+  if constexpr (FOLDS == 0 && IN_BASE) {
+    uint2 e = *reinterpret_cast<const uint2 *>(in + 2 * i);
+    raw[0] = make_uint4(e.x, e.y, 0u, 0u);
+  } else {
+    // words per pair: 16 (three folds), 8 (two), 4 (base, folding), 4 D (extension, folding), 2 D (extension)
+    const uint4 *p = reinterpret_cast<const uint4 *>(in) + (uint64_t)Q * i;
 #pragma unroll
-  for (int t = 0; t < MAXT; t++) {
-    if (t < d.T) {
-      if constexpr (!FOLD2 && !FOLD && IN_BASE) {
-        uint2 e = *reinterpret_cast<const uint2 *>(in[t] + 2 * i);
-        raw[t][0] = make_uint4(e.x, e.y, 0u, 0u);
-      } else {
-        // words per pair: 8 (FOLD2), 4 (base, folding), 4 D (extension, folding), 2 D (extension)
-        const uint4 *p = reinterpret_cast<const uint4 *>(in[t]) + (uint64_t)Q * i;
-#pragma unroll
-        for (int q = 0; q < Q; q++) raw[t][q] = p[q];
-      }
-    }
+    for (int q = 0; q < Q; q++) raw[q] = p[q];
   }
 }
 template <int D>
@@ -464,37 +500,30 @@ __device__ __forceinline__ Ext<D> ext_from_quads(const uint4 *q) {
   if constexpr (D == 8) e.c[4] = q[1].x, e.c[5] = q[1].y, e.c[6] = q[1].z, e.c[7] = q[1].w;
   return e;
 }
-template <int D, bool IN_BASE, bool FOLD, class V, bool FOLD2, int Q, class Desc>
-__device__ __forceinline__ void pair_from_raw(const Desc &d, const uint4 (*raw)[Q], uint32_t *const *out, uint64_t i,
-                                              const Ext<D> &r, V *lo, V *hi, const BindWeights<D> *bw) {
+template <int D, bool IN_BASE, int FOLDS, class V>
+__device__ __forceinline__ void pair_from_raw(const uint4 *raw, const Ext<D> &r, V &lo, V &hi,
+                                              const BindWeights<D, FOLDS == 3 ? 3 : 2> *bw) {
+  if constexpr (FOLDS >= 2) {
+    constexpr int H = FOLDS == 3 ? 2 : 1;  // quads per entry
+    uint32_t v[8 * H];
 #pragma unroll
-  for (int t = 0; t < MAXT; t++) {
-    if (t < d.T) {
-      if constexpr (FOLD2) {
-        const uint4 e = raw[t][0], f = raw[t][1];
-        lo[t] = bind4<D>(*bw, e.x, e.y, e.z, e.w);
-        hi[t] = bind4<D>(*bw, f.x, f.y, f.z, f.w);
-      } else if constexpr (FOLD && IN_BASE) {
-        const uint4 e = raw[t][0];
-        lo[t] = fold_base<D>(e.x, e.y, r);
-        hi[t] = fold_base<D>(e.z, e.w, r);
-      } else if constexpr (FOLD) {
-        constexpr int E = D / 4;  // quads per element
-        lo[t] = fold_ext<D>(ext_from_quads<D>(raw[t]), ext_from_quads<D>(raw[t] + E), r);
-        hi[t] = fold_ext<D>(ext_from_quads<D>(raw[t] + 2 * E), ext_from_quads<D>(raw[t] + 3 * E), r);
-      } else if constexpr (IN_BASE) {
-        lo[t] = raw[t][0].x;
-        hi[t] = raw[t][0].y;
-      } else {
-        constexpr int E = D / 4;
-        lo[t] = ext_from_quads<D>(raw[t]);
-        hi[t] = ext_from_quads<D>(raw[t] + E);
-      }
-      if constexpr (FOLD) {
-        store_ext<D>(out[t] + 2 * i * D, lo[t]);
-        store_ext<D>(out[t] + (2 * i + 1) * D, hi[t]);
-      }
-    }
+    for (int q = 0; q < 2 * H; q++) v[4 * q] = raw[q].x, v[4 * q + 1] = raw[q].y, v[4 * q + 2] = raw[q].z, v[4 * q + 3] = raw[q].w;
+    lo = bind<D>(*bw, v);
+    hi = bind<D>(*bw, v + 4 * H);
+  } else if constexpr (FOLDS == 1 && IN_BASE) {
+    lo = fold_base<D>(raw[0].x, raw[0].y, r);
+    hi = fold_base<D>(raw[0].z, raw[0].w, r);
+  } else if constexpr (FOLDS == 1) {
+    constexpr int E = D / 4;  // quads per element
+    lo = fold_ext<D>(ext_from_quads<D>(raw), ext_from_quads<D>(raw + E), r);
+    hi = fold_ext<D>(ext_from_quads<D>(raw + 2 * E), ext_from_quads<D>(raw + 3 * E), r);
+  } else if constexpr (IN_BASE) {
+    lo = raw[0].x;
+    hi = raw[0].y;
+  } else {
+    constexpr int E = D / 4;
+    lo = ext_from_quads<D>(raw);
+    hi = ext_from_quads<D>(raw + E);
   }
 }
 
@@ -566,8 +595,8 @@ __device__ __forceinline__ uint32_t wave_sums_transposed(F val) {
 
 // accumulator words [first, first + W) of the lane, reduced mod p (zero beyond the statement's), summed
 // over the wavefront and left in lds_row[first ..]
-template <int D, int W, class Desc>
-__device__ __forceinline__ void chunk_sums(const Desc &d, Acc96 (*acc)[D], int first, uint32_t *lds_row) {
+template <int D, int W, class Desc, class Acc>
+__device__ __forceinline__ void chunk_sums(const Desc &d, Acc (*acc)[D], int first, uint32_t *lds_row) {
   const uint32_t total = wave_sums_transposed<W>([&](int k) -> uint32_t {
     const int o = first + k;
     return o < d.nacc * D ? acc_reduce(acc[o / D][o % D]) : 0u;
@@ -580,8 +609,8 @@ __device__ __forceinline__ void chunk_sums(const Desc &d, Acc96 (*acc)[D], int f
 // TRANSPOSED picks the cross-lane scheme: the transposing reduction is the shorter path (the latency-bound
 // LDS-resident rounds use it), one tree per value keeps fewer registers live (the streaming round kernels,
 // whose occupancy it would cost, use that).
-template <int D, bool TRANSPOSED, class Desc>
-__device__ __forceinline__ void block_sums(const Desc &d, Acc96 (*acc)[D], uint32_t (*lds)[MAXACC * D],
+template <int D, bool TRANSPOSED, class Desc, class Acc>
+__device__ __forceinline__ void block_sums(const Desc &d, Acc (*acc)[D], uint32_t (*lds)[MAXACC * D],
                                            uint32_t *sums) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if constexpr (TRANSPOSED) {
@@ -620,7 +649,7 @@ __device__ __forceinline__ void block_sums(const Desc &d, Acc96 (*acc)[D], uint3
 // on the wavefront that has this part), reduced mod p, into sums[a * D ..] (LDS).  Every word of sums is written
 // by one wavefront.
 template <int D, int PART, int PARTS, int W, class Desc>
-__device__ __forceinline__ void part_chunk_sums(const Desc &d, Acc96 (*acc)[D], int first, int count, uint32_t *sums) {
+__device__ __forceinline__ void part_chunk_sums(const Desc &d, AccLazy (*acc)[D], int first, int count, uint32_t *sums) {
   const uint32_t total = wave_sums_transposed<W>([&](int k) -> uint32_t {
     const int o = first + k, q = o / D;
     return PARTS * q + PART < MAXACC && q < count ? acc_reduce(acc[(PARTS * q + PART) % MAXACC][o % D]) : 0u;
@@ -629,7 +658,7 @@ __device__ __forceinline__ void part_chunk_sums(const Desc &d, Acc96 (*acc)[D], 
   if (transposed_writer<W>(l) && o < (uint32_t)count * D) sums[(PARTS * (o / D) + PART) * D + o % D] = total;
 }
 template <int D, int PART, int PARTS, class Desc>
-__device__ __forceinline__ void part_wave_sums(const Desc &d, Acc96 (*acc)[D], uint32_t *sums) {
+__device__ __forceinline__ void part_wave_sums(const Desc &d, AccLazy (*acc)[D], uint32_t *sums) {
   const int count = (d.nacc - PART + PARTS - 1) / PARTS;  // accumulators of this part
   if (count <= 0) return;
   if (count * D <= 8)
@@ -834,6 +863,7 @@ __device__ __forceinline__ bool add_and_elect(const RoundTotals &rt, const uint3
 
 // One workgroup's share of a round: pairs [block * tile, (block + 1) * tile) with tile = BLOCK *
 // pairs_per_thread, folded first when FOLD, summed into the workgroup's partial row.
+constexpr int FETCH_QUADS = 16;  // 16-byte quads of tables' words that a lane holds ahead of their arithmetic
 template <int D>
 struct RoundShape {
   const uint32_t *low, *high;
@@ -848,52 +878,68 @@ struct RoundShape {
   const uint32_t *consts;
 };
 
-template <int D, bool IN_BASE, bool FOLD, class Desc, bool FOLD2 = false, bool GENERATED = false>
+template <int D, bool IN_BASE, int FOLDS, class Desc, bool GENERATED = false>
 __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const *in, uint32_t *const *out,
                                            const RoundShape<D> &sh, const Ext<D> &r, uint32_t block,
-                                           uint32_t *partial_row, const BindWeights<D> *bw = nullptr) {
-  constexpr bool BASE_MODE = IN_BASE && !FOLD;  // the pair's values are base-field
+                                           uint32_t *partial_row, const BindWeights<D, FOLDS == 3 ? 3 : 2> *bw = nullptr) {
+  constexpr bool BASE_MODE = IN_BASE && FOLDS == 0;  // the pair's values are base-field
   using V = typename std::conditional<BASE_MODE, uint32_t, Ext<D>>::type;
   const uint32_t tid = threadIdx.x;
   const uint64_t tile = (uint64_t)BLOCK * sh.pairs_per_thread;
   const uint64_t tile_start = (uint64_t)block * tile;
   const uint64_t low_mask = ((uint64_t)1 << sh.low_bits) - 1;
 
-  Acc96 acc[MAXACC][D];
+  typename AccOf<V, Desc>::type acc[MAXACC][D];
 #pragma unroll
   for (int a = 0; a < MAXACC; a++)
 #pragma unroll
     for (int c = 0; c < D; c++) acc_zero(acc[a][c]);
 
-  // With a statement known at compile time and D = 4 the next pair's words are fetched before this pair's
-  // arithmetic (two workgroups per compute unit leave the registers for it, and too few wavefronts to hide the
-  // loads behind one another); the interpreter and D = 8 keep the plain order.
-  // (nor does a statement in direct form: it is wide, and its tables' words ahead would not fit the registers)
-  constexpr bool AHEAD = GENERATED && D == 4 && !is_direct<Desc>::value;
+  // With a statement known at compile time a table's words are fetched well before their arithmetic (two workgroups per
+  // compute unit leave the registers for it, and too few wavefronts to hide the loads behind one another): SLOTS tables'
+  // words are held, table t in slot t % SLOTS, and a slot is filled again as soon as its words are used, with the next
+  // table that goes there -- of this pair, or of the next one, whose first SLOTS tables then arrive under the sums.
+  // (64 registers of words: two tables at a time of extension elements at D = 8, four at D = 4, all of them in base tables.
+  // Without it, at D = 8, a table's loads waited behind the store of the table before: the largest fold round of a
+  // four-table statement, 1.6 GB, took 530 us, 440 this way; more or fewer slots, 32 or 96 registers, make no difference
+  // beyond the runs'.  Whole pairs held twice, as D = 4 did, are 96 registers for three tables and spill for eight.
+  // A lane without a next pair fetches the tile's first one: a load under a condition would have to be merged with
+  // what the slot held as soon as it is issued.)
+  // The interpreter, and a statement in direct form, which is wide and calls its evaluator in a loop, keep the plain order.
+  constexpr bool AHEAD = GENERATED && !is_direct<Desc>::value;
   if constexpr (AHEAD) {
-    constexpr int Q = raw_quads<D, IN_BASE, FOLD, FOLD2>();
-    uint4 raw[MAXT][Q], ahead[MAXT][Q];
-    if (tile_start + tid < sh.n_pairs) fetch_raw<D, IN_BASE, FOLD, FOLD2, Q>(d, in, tile_start + tid, raw);
+    constexpr int Q = raw_quads<D, IN_BASE, FOLDS>(), SLOTS = FETCH_QUADS / Q < MAXT ? FETCH_QUADS / Q : MAXT;
+    const bool store = FOLDS == 1 || (FOLDS >= 2 && out[0] != nullptr);
+    uint4 raw[SLOTS][Q];
+    const uint64_t first = tile_start + tid < sh.n_pairs ? tile_start + tid : tile_start;
+#pragma unroll
+    for (int t = 0; t < SLOTS; t++)
+      if (t < d.T) fetch_raw<D, IN_BASE, FOLDS, Q>(in[t], first, raw[t]);
     for (uint32_t k = 0; k < sh.pairs_per_thread; k++) {
       const uint64_t i = tile_start + (uint64_t)k * BLOCK + tid;
       if (i >= sh.n_pairs) break;
-      const bool more = k + 1 < sh.pairs_per_thread && i + BLOCK < sh.n_pairs;
-      if (more) fetch_raw<D, IN_BASE, FOLD, FOLD2, Q>(d, in, i + BLOCK, ahead);
+      const uint64_t next = k + 1 < sh.pairs_per_thread && i + BLOCK < sh.n_pairs ? i + BLOCK : tile_start;
       Ext<D> w;
       if (sh.do_sums) w = load_ext<D>(sh.low + (i & low_mask) * D);
       V lo[MAXT], hi[MAXT];
-      pair_from_raw<D, IN_BASE, FOLD, V, FOLD2, Q>(d, raw, out, i, r, lo, hi, bw);
+#pragma unroll
+      for (int t = 0; t < MAXT; t++)
+        if (t < d.T) {
+          pair_from_raw<D, IN_BASE, FOLDS, V>(raw[t % SLOTS], r, lo[t], hi[t], bw);
+          if (t + SLOTS < d.T)
+            fetch_raw<D, IN_BASE, FOLDS, Q>(in[t + SLOTS < MAXT ? t + SLOTS : 0], i, raw[t % SLOTS]);
+          else
+            fetch_raw<D, IN_BASE, FOLDS, Q>(in[t % SLOTS], next, raw[t % SLOTS]);
+          if constexpr (FOLDS > 0) {
+            if (store) {
+              store_ext<D>(out[t] + 2 * i * D, lo[t]);
+              store_ext<D>(out[t] + (2 * i + 1) * D, hi[t]);
+            }
+          }
+        }
       if (sh.do_sums) {
         if (!sh.deferred) w = ext_mul_mont<D>(w, load_ext<D>(sh.high + (i >> sh.low_bits) * D));
         accumulate_pair<D, V>(d, lo, hi, w, acc, sh.consts);
-      }
-      if (more) {
-#pragma unroll
-        for (int t = 0; t < MAXT; t++)
-          if (t < d.T) {
-#pragma unroll
-            for (int q = 0; q < Q; q++) raw[t][q] = ahead[t][q];
-          }
       }
     }
   } else {
@@ -901,7 +947,7 @@ __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const 
       const uint64_t i = tile_start + (uint64_t)k * BLOCK + tid;
       if (i >= sh.n_pairs) break;
       V lo[MAXT], hi[MAXT];
-      load_pair<D, IN_BASE, FOLD, V, Desc, FOLD2>(d, in, out, i, r, lo, hi, bw);
+      load_pair<D, IN_BASE, FOLDS == 1, V, Desc>(d, in, out, i, r, lo, hi);
       if (sh.do_sums) {
         Ext<D> w = load_ext<D>(sh.low + (i & low_mask) * D);
         if (!sh.deferred) w = ext_mul_mont<D>(w, load_ext<D>(sh.high + (i >> sh.low_bits) * D));
@@ -967,31 +1013,24 @@ __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const 
   round_epilogue<D>(sh.ctrl, sums, (uint32_t)d.nacc, sh.points, epi.mtilde, epi.c0, &epi, true);
 }
 
-template <int D, bool IN_BASE, bool FOLD, class Desc, bool FOLD2 = false, bool GENERATED = false>
+template <int D, bool IN_BASE, int FOLDS, class Desc, bool GENERATED = false>
 __device__ __forceinline__ void round_body(const Desc &d, const RoundArgs<D> &args) {
-  Ext<D> r = ext_zero<D>();
-  if constexpr (FOLD2) {  // challenge 0 from the log, challenge 1 is the latest
-    Ext<D> r0, r1;
-#pragma unroll
-    for (int c = 0; c < D; c++) r0.c[c] = to_mont(args.ctrl->chal[0][c]), r1.c[c] = args.ctrl->r_mont[c];
-    BindWeights<D> bw = bind_weights<D>(r0, r1);
-    RoundShape<D> sh{args.low, args.high, args.n_pairs, args.low_bits, args.pairs_per_thread, args.deferred != 0,
-                     args.do_sums != 0, RoundTotals{args.totals, args.arrivals, args.groups, args.pstride, args.spin_limit},
-                     args.points, args.mtilde, args.c0, args.ctrl, args.consts};
-    round_core<D, true, true, Desc, true, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x,
-                                          args.partials + (uint64_t)blockIdx.x * args.pstride, &bw);
-    return;
-  }
-  if constexpr (FOLD) {
-    const uint32_t *rp = args.ctrl ? args.ctrl->r_mont : args.r_mont;
-#pragma unroll
-    for (int c = 0; c < D; c++) r.c[c] = rp[c];
-  }
   RoundShape<D> sh{args.low, args.high, args.n_pairs, args.low_bits, args.pairs_per_thread, args.deferred != 0,
                    args.do_sums != 0, RoundTotals{args.totals, args.arrivals, args.groups, args.pstride, args.spin_limit},
                    args.points, args.mtilde, args.c0, args.ctrl, args.consts};
-  round_core<D, IN_BASE, FOLD, Desc, false, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x,
-                               args.partials + (uint64_t)blockIdx.x * args.pstride);
+  uint32_t *const partial_row = args.partials + (uint64_t)blockIdx.x * args.pstride;
+  Ext<D> r = ext_zero<D>();
+  if constexpr (FOLDS >= 2) {
+    const BindWeights<D, FOLDS> bw = bind_weights<D, FOLDS>(args.ctrl);
+    round_core<D, true, FOLDS, Desc, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x, partial_row, &bw);
+  } else {
+    if constexpr (FOLDS == 1) {
+      const uint32_t *rp = args.ctrl ? args.ctrl->r_mont : args.r_mont;
+#pragma unroll
+      for (int c = 0; c < D; c++) r.c[c] = rp[c];
+    }
+    round_core<D, IN_BASE, FOLDS, Desc, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x, partial_row);
+  }
 }
 
 // The round's second launch when the device drives the loop: one workgroup adds the partials, forms the
@@ -1063,7 +1102,7 @@ __global__ __launch_bounds__(EPI_BLOCK) void epilogue_kernel(EpilogueArgs args) 
 template <int D, int PART, int PARTS, class Desc>
 __device__ __forceinline__ void small_round_sums(const Desc &d, const Ext<D> *lo, const Ext<D> *hi, const Ext<D> &w,
                                                  uint32_t *sums, const uint32_t *kc) {
-  Acc96 acc[MAXACC][D];
+  AccLazy acc[MAXACC][D];
 #pragma unroll
   for (int a = 0; a < MAXACC; a++)
 #pragma unroll
@@ -1376,7 +1415,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
           small_round_sums<D, 2, 3>(d, lo, hi, ww, sums, args.consts);
         lds_barrier();
       } else {
-        Acc96 acc[MAXACC][D];
+        AccLazy acc[MAXACC][D];
 #pragma unroll
         for (int a = 0; a < MAXACC; a++)
 #pragma unroll
@@ -1889,7 +1928,7 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
 // a kernel generated for one statement: S::d is its descriptor, known at compile time
 template <int D, bool IN_BASE, bool FOLD, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel(RoundArgs<D> args) {
-  round_body<D, IN_BASE, FOLD, decltype(S::d), false, true>(S::d, args);
+  round_body<D, IN_BASE, FOLD ? 1 : 0, decltype(S::d), true>(S::d, args);
 }
 template <int D, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(1, 1))) void tail_kernel(TailArgs<D> args) {
@@ -1902,9 +1941,11 @@ template <int D, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void tail_kernel_narrow(TailArgs<D> args) {
   tail_body<D>(S::d, args);
 }
-template <int D, class S>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel_fold2(RoundArgs<D> args) {
-  round_body<D, true, true, decltype(S::d), true, true>(S::d, args);
+// base tables folded by the first FOLDS = 2 or 3 challenges at once, see round_core; without tables to write (out[0] null)
+// only the sums are taken
+template <int D, class S, int FOLDS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel_bind(RoundArgs<D> args) {
+  round_body<D, true, FOLDS, decltype(S::d), true>(S::d, args);
 }
 template <int D, class S, int PASS, int SPP>
 __global__ __launch_bounds__(BLOCK) void nodes_kernel(NodesArgs<D> args) {
@@ -1914,7 +1955,7 @@ __global__ __launch_bounds__(BLOCK) void nodes_kernel(NodesArgs<D> args) {
 // the interpreter: the same bodies over a run-time descriptor
 template <int D, bool IN_BASE, bool FOLD>
 __global__ __launch_bounds__(BLOCK) void round_kernel_interp(RoundArgs<D> args, StmtDesc d) {
-  round_body<D, IN_BASE, FOLD>(d, args);
+  round_body<D, IN_BASE, FOLD ? 1 : 0>(d, args);
 }
 template <int D>
 __global__ __launch_bounds__(BLOCK) void tail_kernel_interp(TailArgs<D> args, StmtDesc d) {

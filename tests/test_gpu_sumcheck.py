@@ -309,6 +309,49 @@ def test_round_one_in_the_base_field_and_the_double_fold(form, names, cnames, d,
         t.free()
 
 
+GKR2 = ("(+ (* a p0 q1) (* a p1 q0) (* al q0 q1) (* b r0 s1) (* b r1 s0) (* bl s0 s1))",
+        ["p0", "p1", "q0", "q1", "r0", "r1", "s0", "s1"], ["a", "al", "b", "bl"])
+
+
+@pytest.mark.parametrize("form,names,cnames,d,n", [
+    # (the rounds after the sweep stream down to 256 or 128 pairs here: from these sizes on round 3 is one of them)
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 12),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 13),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 11),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 12),
+    ("(* t0 t1 t2)", ["t0", "t1", "t2"], [], 8, 13),
+])
+def test_round_three_from_the_base_tables(form, names, cnames, d, n, monkeypatch):
+    """Where round 3 after the base-field sweep streams as well, round 2 writes no folded tables and round 3 binds three
+    variables of the base tables at once: same proof bytes, finals and folded tables as the oracle, on either side of
+    that line."""
+    monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
+    rng = np.random.default_rng(n * 17 + d)
+    tables = [rng.integers(0, P, 1 << n, dtype=np.uint32) for _ in names]
+    tables[0][:] = P - 1  # the largest values: every product and sum at its bound
+    eq = rand_ext(rng, (n,), d)
+    consts = rand_ext(rng, (len(cnames),), d) if cnames else None
+    prove_both("bind3", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames)
+
+
+@pytest.mark.parametrize("form,names,cnames,d,n,K,base", [
+    (*GKR2, 4, 8, 3, False),  # eight tables, four held ahead; 384 and 192 pairs: a last workgroup with half its lanes
+    (*GKR2, 4, 10, 1, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 8, 3, False),  # four tables, two held ahead
+    ("(* t0 t1)", ["t0", "t1"], [], 8, 9, 5, False),
+])
+def test_streaming_rounds_with_tables_fetched_ahead(form, names, cnames, d, n, K, base, monkeypatch):
+    """More tables than a lane holds ahead of its arithmetic, and lanes without a next pair."""
+    monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
+    rng = np.random.default_rng(n * 19 + d)
+    tables = [rng.integers(0, P, K << n, dtype=np.uint32) if base else rand_ext(rng, (K << n,), d) for _ in names]
+    consts = rand_ext(rng, (len(cnames),), d) if cnames else None
+    bw = rand_ext(rng, (K,), d) if K > 1 else None
+    st, *_ = prove_both("ahead", d, n, form, names, tables, eq=rand_ext(rng, (n,), d), constants=consts, cnames=cnames,
+                        block_weights=bw)
+    assert st.has_generated_kernel(d)
+
+
 @pytest.mark.parametrize("K,n,d,with_eq", [(2, 8, 4, True), (4, 10, 4, False), (2, 6, 8, True)])
 def test_base_field_sweep_with_block_weights(K, n, d, with_eq, monkeypatch):
     """The same opening sweep when block weights are the HIGH factor (K a power of two, base tables)."""
