@@ -32,33 +32,49 @@ __global__ __launch_bounds__(BLOCK) void gkr_reduce_kernel(const uint32_t *p, co
   store_ext<D>(qq + o * D, ext_mul_mont<D>(q0, q1r));
 }
 
-// The layers m_top .. 0 of one lookup's tree with one block, in one workgroup: layer m has 2^m <= BLOCK parents,
-// a thread takes one, and the workgroup's barrier stands between a layer's writes and the next one's reads.  (A
-// launch per layer is 4 us each for a few hundred products.)
-constexpr int REDUCE_TOP_LAYERS = 9;  // m_top <= 8: 256 parents
+// The layers m_top .. 0 of a block of a lookup's tree, in one workgroup (block blockIdx.x of lookup blockIdx.y): layer m
+// has 2^m <= BLOCK parents, a thread takes one, and the workgroup's barrier stands between a layer's writes and the next
+// one's reads.  (A launch per layer is 4 us each for a few hundred products.)
+constexpr int REDUCE_TOP_LAYERS = 9;     // m_top <= 8: 256 parents
+constexpr int REDUCE_MAXL = MAXT / 4;    // lookups: four tables each
 struct ReduceTopArgs {
-  const uint32_t *p, *q;  // layer m_top + 1
-  uint32_t *pp[REDUCE_TOP_LAYERS], *qq[REDUCE_TOP_LAYERS];
+  // layer m_top + 1; where the tree over the block index begins, `valid` roots (the others are 0 / 1) that go to pad_p,
+  // pad_q with them (else null: every child is there)
+  const uint32_t *p[REDUCE_MAXL], *q[REDUCE_MAXL];
+  uint32_t *pad_p[REDUCE_MAXL], *pad_q[REDUCE_MAXL];
+  uint32_t *pp[REDUCE_MAXL][REDUCE_TOP_LAYERS], *qq[REDUCE_MAXL][REDUCE_TOP_LAYERS];
   int m_top;
+  uint32_t valid;
 };
 template <int D>
 __global__ __launch_bounds__(BLOCK) void gkr_reduce_top_kernel(ReduceTopArgs a) {
   static_assert((1 << (REDUCE_TOP_LAYERS - 1)) <= BLOCK, "a thread per parent");
-  const uint32_t *p = a.p, *q = a.q;
-  for (int m = a.m_top; m >= 0; m--) {
-    const uint32_t o = threadIdx.x, half = 1u << m;
-    if (o < half) {
-      Ext<D> p0 = load_ext<D>(p + o * D), p1 = load_ext<D>(p + (o + half) * D);
-      Ext<D> q0 = load_ext<D>(q + o * D), q1 = load_ext<D>(q + (o + half) * D);
-      Ext<D> q1r, q0r;
-#pragma unroll
-      for (int c = 0; c < D; c++) q1r.c[c] = mont_mul(q1.c[c], R2), q0r.c[c] = mont_mul(q0.c[c], R2);
-      store_ext<D>(a.pp[m] + o * D, ext_add<D>(ext_mul_mont<D>(p0, q1r), ext_mul_mont<D>(p1, q0r)));
-      store_ext<D>(a.qq[m] + o * D, ext_mul_mont<D>(q0, q1r));
+  const uint32_t b = blockIdx.x, l = blockIdx.y;
+  const uint32_t *p = a.p[l], *q = a.q[l];
+  if (a.pad_p[l]) {
+    for (uint32_t o = threadIdx.x; o < 2u << a.m_top; o += BLOCK) {
+      store_ext<D>(a.pad_p[l] + o * D, o < a.valid ? load_ext<D>(p + o * D) : ext_zero<D>());
+      store_ext<D>(a.pad_q[l] + o * D, o < a.valid ? load_ext<D>(q + o * D) : ext_lift<D>(1));
     }
     __threadfence();
     __syncthreads();
-    p = a.pp[m], q = a.qq[m];
+    p = a.pad_p[l], q = a.pad_q[l];
+  }
+  for (int m = a.m_top; m >= 0; m--) {
+    const uint32_t half = 1u << m, x = threadIdx.x;
+    const uint64_t o = ((uint64_t)b << m) + x, c0 = ((uint64_t)b << (m + 1)) + x;
+    if (x < half) {
+      Ext<D> p0 = load_ext<D>(p + c0 * D), p1 = load_ext<D>(p + (c0 + half) * D);
+      Ext<D> q0 = load_ext<D>(q + c0 * D), q1 = load_ext<D>(q + (c0 + half) * D);
+      Ext<D> q1r, q0r;
+#pragma unroll
+      for (int c = 0; c < D; c++) q1r.c[c] = mont_mul(q1.c[c], R2), q0r.c[c] = mont_mul(q0.c[c], R2);
+      store_ext<D>(a.pp[l][m] + o * D, ext_add<D>(ext_mul_mont<D>(p0, q1r), ext_mul_mont<D>(p1, q0r)));
+      store_ext<D>(a.qq[l][m] + o * D, ext_mul_mont<D>(q0, q1r));
+    }
+    __threadfence();
+    __syncthreads();
+    p = a.pp[l][m], q = a.qq[l][m];
   }
 }
 
@@ -97,6 +113,21 @@ __global__ __launch_bounds__(BLOCK) void halves_kernel(HalvesArgs a) {
   store_ext<D>(upper + o * D, load_ext<D>(v + (b * 2 * size + size + x) * D));
 }
 
+// The same for every layer of a tree at once, in the order in which the tree's one allocation holds them: layer m, from
+// n - 1 down to 0, has `vectors` vectors (p and q of each lookup) of K 2^m entries.  The halves of layer l + 1's vector i
+// are tables 2 i and 2 i + 1 of layer l's sumcheck, at out + (2 vectors K (2^l - 1) + t K 2^l) D.  blockIdx.y: the vector.
+template <int D>
+__global__ __launch_bounds__(BLOCK) void all_halves_kernel(const uint32_t *tree, uint32_t *out, uint32_t K, int n,
+                                                           uint64_t entries) {
+  const uint64_t o = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+  if (o >= entries) return;  // K (2^(n-1) - 1): layers 0 .. n - 2 one after the other
+  const uint32_t layer = 31 - __clz((uint32_t)(o / K) + 1), vectors = gridDim.y;
+  const uint64_t size = (uint64_t)1 << layer, at = o - K * (size - 1), b = at >> layer, x = at & (size - 1);
+  const uint32_t *v = tree + (vectors * K * (((uint64_t)1 << n) - 4 * size) + blockIdx.y * K * 2 * size) * D;
+  uint32_t *lower = out + (2 * vectors * K * (size - 1) + 2 * blockIdx.y * K * size) * D;
+  store_ext<D>(lower + at * D, load_ext<D>(v + (b * 2 * size + x) * D));
+  store_ext<D>(lower + (K * size + at) * D, load_ext<D>(v + (b * 2 * size + size + x) * D));
+}
 
 namespace {
 
@@ -207,6 +238,12 @@ struct DeviceBuffers {  // frees what it allocated when the proof ends
 
 constexpr size_t GKR_BW_PIN = 8192, GKR_BW_PIN_WORDS = 1024;  // words of the context's pinned buffer (see below)
 
+// a layer of K blocks can be chained: see gkr_prove_upper
+bool blocks_chain(int K, int L, int D) {
+  const uint64_t pairs = SumcheckSession::one_workgroup_pairs(4 * L, D), block_pairs = SumcheckSession::one_workgroup_pairs(4 * L + 1, D);
+  return K > 1 && K <= GLUE_MAXBLOCKS && (uint64_t)K <= pairs && ((uint64_t)1 << block_bits(K)) / 2 <= block_pairs;
+}
+
 // what the chain's sticky word means for the proof (host side)
 int chain_outcome(uint32_t failed) {
   if (!failed) return OK;
@@ -237,24 +274,54 @@ static int launch_glue(const GlueArgs<D> &a, std::vector<uint8_t> *held = nullpt
   return OK;
 }
 
+// The tables of the layers' sumchecks, on the device: of the tree over the block index (several blocks; lk layers), and of
+// the layers in the blocks (n - 1).
+struct ChainTables {
+  std::vector<const uint32_t *> roots;  // p and q of every lookup
+  std::vector<std::vector<const uint32_t *>> top, layers;
+};
+
 template <int D>
-static int prove_upper_chained(Transcript &tr, int n, int L, const std::vector<std::vector<const uint32_t *>> &layers,
-                               const std::string &label, uint32_t *out_ri, uint32_t *out_cp, uint32_t *out_cq) {
+static int prove_upper_chained(Transcript &tr, int n, int K, int lk, int L, const ChainTables &tables,
+                               const std::string &label, uint32_t *out_ri, uint32_t *out_rb, uint32_t *out_cp,
+                               uint32_t *out_cq) {
   Context &c = ctx();
   const int NT = 4 * L;
-  Statement st = layer_statement(L, false);
-  // the log: the roots, then per layer its round messages, challenges, finals and fresh point
-  std::vector<size_t> log_off(n - 1);
+  const Statement st = layer_statement(L, false), st_blk = K > 1 ? layer_statement(L, true) : Statement();
+  // The sumchecks in their order, and where each one's messages, challenges and -- unless it is a layer's own with several
+  // blocks -- finals and fresh point lie in the log, behind the roots.
+  enum Kind { TOP, LAYER, BLOCKS };
+  struct Step {
+    Kind kind;
+    int layer, rounds, points;
+    bool finals;
+    size_t log_at;
+    std::string header;
+    const std::vector<const uint32_t *> *tabs;  // (BLOCKS: what the layer's rounds leave)
+  };
+  std::vector<Step> steps;
   size_t words = (size_t)2 * L * D;
-  for (int layer = 0; layer < n - 1; layer++) {
-    const int points = layer > 0 ? 2 : 1;
-    log_off[layer] = words;
-    words += (size_t)layer * points * D + (size_t)layer * D + (size_t)NT * D + D;
+  auto add_step = [&](Kind kind, int layer, const std::string &name, int rounds, int degree, int blocks,
+                      const std::vector<const uint32_t *> *tabs) {
+    Step s{kind, layer, rounds, degree > 1 ? degree : 1, kind != LAYER || K == 1, words,
+           header_bytes(name, rounds, degree, blocks), tabs};
+    words += (size_t)rounds * s.points * D + (size_t)rounds * D + (s.finals ? (size_t)NT * D + D : 0);
+    steps.push_back(s);
+  };
+  for (size_t j = 0; j < tables.top.size(); j++) add_step(TOP, (int)j, label + "-top", (int)j, j > 0 ? 2 : 0, 1, &tables.top[j]);
+  for (size_t j = 0; j < tables.layers.size(); j++) {
+    add_step(LAYER, (int)j, label, (int)j, j > 0 ? 2 : 0, K, &tables.layers[j]);
+    if (K > 1) add_step(BLOCKS, (int)j, label + "-blk", lk, st_blk.degree, 1, nullptr);
   }
+  for (const Step &s : steps)
+    if (s.header.size() > 64) {
+      set_error("invalid-parameter: label too long for the chained layers");
+      return E_PARAM;
+    }
   DeviceBuffers bufs;
   GkrChainState *chain = reinterpret_cast<GkrChainState *>(bufs.alloc((sizeof(GkrChainState) + 3) / 4));
-  uint32_t *d_log = bufs.alloc(words);
-  if (!chain || !d_log) {
+  uint32_t *d_log = bufs.alloc(words), *d_bw = K > 1 ? bufs.alloc((size_t)K * D) : nullptr;
+  if (!chain || !d_log || (K > 1 && !d_bw)) {
     set_error("device-out-of-memory: the GKR chain's log");
     return E_NOMEM;
   }
@@ -262,98 +329,101 @@ static int prove_upper_chained(Transcript &tr, int n, int L, const std::vector<s
   EXH_HIP(hipMemcpyAsync(&chain->tr, &first, sizeof(first), hipMemcpyHostToDevice, c.stream));
   // (a fill kernel would do as well; the chain is never captured into a graph)
   EXH_HIP(hipMemsetAsync(&chain->failed, 0, sizeof(chain->failed), c.stream));
-  const std::vector<int> strides(NT, D);
-  const std::vector<uint32_t> no_point((size_t)n * D, 0), no_consts((size_t)2 * L * D, 0);
-  auto layer_tables = [&](int layer) {  // with one block the halves are views (LAYER-TABLES, src/gkr.lisp:199-206)
-    std::vector<const uint32_t *> tabs(NT);
-    const uint64_t size = (uint64_t)1 << layer;
-    for (int l = 0; l < L; l++)
-      for (int w = 0; w < 2; w++) {
-        const uint32_t *v = layers[layer + 1][2 * l + w];
-        tabs[4 * l + 2 * w] = v;
-        tabs[4 * l + 2 * w + 1] = v + size * D;
-      }
-    return tabs;
+  const std::vector<int> strides(NT + 1, D);
+  const std::vector<uint32_t> no_point((size_t)std::max(n, lk) * D, 0), no_consts((size_t)2 * L * D, 0), no_bw((size_t)K * D, 0);
+  std::vector<const uint32_t *> blk_tabs(NT + 1, nullptr);
+  auto begin_step = [&](SumcheckSession &s, const Step &step) {
+    if (step.kind == BLOCKS)
+      return s.begin(st_blk, D, lk, blk_tabs.data(), strides.data(), nullptr, nullptr, 1, no_consts.data(), -1, false, true);
+    const bool blocks = step.kind == LAYER && K > 1;
+    return s.begin(st, D, step.rounds, step.tabs->data(), strides.data(), no_point.data(), blocks ? no_bw.data() : nullptr,
+                   blocks ? K : 1, no_consts.data(), step.rounds > 0 ? 2 : 0, false, true);
   };
   int status;
-  {  // the largest layer first, for its buffers alone: the arenas then never grow (and never wait) mid-chain
+  // the largest sumchecks first, for their buffers alone: the arenas then never grow (and never wait) mid-chain
+  for (size_t i = steps.size() - 1, kinds = 0; kinds < 2 && i < steps.size(); i--, kinds++) {
     SumcheckSession widest;
-    std::vector<const uint32_t *> tabs = layer_tables(n - 2);
-    if ((status = widest.begin(st, D, n - 2, tabs.data(), strides.data(), no_point.data(), nullptr, 1, no_consts.data(),
-                               n - 2 > 0 ? 2 : 0, false, true)))
-      return status;
+    if ((status = begin_step(widest, steps[i]))) return status;
+  }
+  if (!tables.top.empty()) {
+    SumcheckSession widest;
+    if ((status = begin_step(widest, steps[tables.top.size() - 1]))) return status;
   }
   const Ctrl *prev_ctrl = nullptr;
   std::vector<const uint32_t *> prev_tabs;
   const DevB3S unused_state = first;
-  // a layer's last launch waits here for the next step, which rides on it (EXACTA_HIP_NO_GKR_FUSE=1: never)
+  // a sumcheck's last launch waits here for the next step, which rides on it (EXACTA_HIP_NO_GKR_FUSE=1: never)
   std::vector<uint8_t> held;
   const KernelSet *held_kernels = nullptr;
   const char *no_fuse = getenv("EXACTA_HIP_NO_GKR_FUSE");
   const bool fuse = !(no_fuse && no_fuse[0] == '1');
-  for (int layer = 0; layer <= n - 1; layer++) {  // launch `layer` closes layer - 1 and opens `layer`; the last only closes
+  for (size_t i = 0; i <= steps.size(); i++) {  // launch i closes sumcheck i - 1 and opens sumcheck i; the last only closes
     GlueArgs<D> a;
     memset(&a, 0, sizeof(a));
-    a.chain = chain, a.L = L, a.NT = NT;
-    if (layer == 0) {
+    a.chain = chain, a.L = L, a.NT = NT, a.K = 1;
+    if (i == 0) {
       a.close_kind = 1, a.log = d_log;
-      for (int i = 0; i < 2 * L; i++) a.tabs[i] = layers[0][i];
-    } else if (layer == 1) {  // layer 0 has no rounds: its finals are its tables' single entries
-      a.close_kind = 3, a.prev_rounds = 0, a.prev_points = 1, a.log = d_log + log_off[0];
-      for (int t = 0; t < NT; t++) a.tabs[t] = prev_tabs[t];
+      for (int t = 0; t < 2 * L; t++) a.tabs[t] = tables.roots[t];
     } else {
-      a.close_kind = 2, a.prev_ctrl = prev_ctrl, a.prev_rounds = layer - 1, a.prev_points = 2;
-      a.log = d_log + log_off[layer - 1];
+      const Step &prev = steps[i - 1];
+      a.prev_rounds = prev.rounds, a.prev_points = prev.points, a.log = d_log + prev.log_at;
+      if (prev.rounds > 0) {
+        a.close_kind = prev.finals ? 2 : 4, a.prev_ctrl = prev_ctrl;
+      } else if (prev.finals) {  // no rounds: its finals are its tables' single entries
+        a.close_kind = 3;
+        for (int t = 0; t < NT; t++) a.tabs[t] = prev_tabs[t];
+      }
+      if (prev.kind == BLOCKS) a.fin_skip = 1, a.blocks_closed = 1, a.tt_at = prev.layer;
     }
-    if (layer == n - 1) {
+    if (i == steps.size()) {
       if ((status = launch_glue<D>(a, &held, held_kernels))) return status;
       break;
     }
-    const int degree = layer > 0 ? 2 : 0;
-    const std::string header = header_bytes(label, layer, degree, 1);
-    if (header.size() > 64) {
-      set_error("invalid-parameter: label too long for the chained layers");
+    const Step &step = steps[i];
+    a.open = step.kind == BLOCKS ? 2 : 1, a.n = step.rounds, a.header_len = (int)step.header.size();
+    for (size_t k = 0; k < step.header.size(); k++) a.header[k / 4] |= (uint32_t)(uint8_t)step.header[k] << (8 * (k % 4));
+    if (step.kind != TOP) a.K = K, a.lk = lk, a.bw_table = d_bw;
+    if (step.kind == BLOCKS) {
+      blk_tabs[0] = d_bw;
+      for (int t = 0; t < NT; t++) blk_tabs[t + 1] = prev_tabs[t];
+    }
+    if (step.rounds == 0) {
+      if ((status = launch_glue<D>(a, &held, held_kernels))) return status;
+      prev_tabs = *step.tabs;
+      continue;
+    }
+    SumcheckSession s;
+    if ((status = begin_step(s, step))) return status;
+    std::vector<uint32_t> lagfix;
+    std::vector<int> acc_group;
+    s.message_map_scalars(&lagfix, &acc_group);
+    a.points = s.points, a.nacc = std::max(s.st.nacc, 1), a.c0_words = step.rounds * s.points * D;
+    if ((int)lagfix.size() > MAXPTS * MAXACC || !s.setup_deferred || s.points != step.points) {
+      set_error("invalid-parameter: layer statement beyond the chained layers' limits");
       return E_PARAM;
     }
-    a.open = 1, a.n = layer, a.header_len = (int)header.size();
-    for (size_t i = 0; i < header.size(); i++) a.header[i / 4] |= (uint32_t)(uint8_t)header[i] << (8 * (i % 4));
-    std::vector<const uint32_t *> tabs = layer_tables(layer);
-    if (layer == 0) {
-      if ((status = launch_glue<D>(a))) return status;
-    } else {
-      SumcheckSession s;
-      if ((status = s.begin(st, D, layer, tabs.data(), strides.data(), no_point.data(), nullptr, 1, no_consts.data(),
-                            degree, false, true)))
-        return status;
-      std::vector<uint32_t> lagfix;
-      std::vector<int> acc_group;
-      s.message_map_scalars(&lagfix, &acc_group);
-      a.points = s.points, a.nacc = std::max(s.st.nacc, 1), a.c0_words = layer * s.points * D;
-      if ((int)lagfix.size() > MAXPTS * MAXACC || !s.setup_deferred) {
+    memcpy(a.lagfix, lagfix.data(), lagfix.size() * 4);
+    for (int e = 0; e < a.nacc; e++) {
+      const Group *g = acc_group[e] >= 0 ? &s.st.groups[acc_group[e]] : nullptr;
+      if (!g || g->parts.size() != 1 || g->parts[0].coeff != 1 || g->parts[0].consts.size() != 1 ||
+          g->parts[0].consts[0] >= GLUE_MAXCONST) {
         set_error("invalid-parameter: layer statement beyond the chained layers' limits");
         return E_PARAM;
       }
-      memcpy(a.lagfix, lagfix.data(), lagfix.size() * 4);
-      for (int e = 0; e < a.nacc; e++) {
-        const Group *g = acc_group[e] >= 0 ? &s.st.groups[acc_group[e]] : nullptr;
-        if (!g || g->parts.size() != 1 || g->parts[0].coeff != 1 || g->parts[0].consts.size() != 1 ||
-            g->parts[0].consts[0] >= GLUE_MAXCONST) {
-          set_error("invalid-parameter: layer statement beyond the chained layers' limits");
-          return E_PARAM;
-        }
-        a.acc_const[e] = (uint8_t)g->parts[0].consts[0];
-      }
-      a.factors = s.d_weights, a.mtilde = s.d_mtilde, a.c0 = s.d_c0, a.ctrl = s.d_ctrl;
-      // (the step of this layer rides on the last launch of the layer before, when that was held back)
-      std::vector<uint8_t> held_now;
-      s.chain_hook = [&]() { return launch_glue<D>(a, &held, held_kernels); };
-      if (fuse) s.held_tail = &held_now;
-      if ((status = s.run_device(unused_state, nullptr, nullptr, nullptr))) return status;
-      held.swap(held_now);
-      held_kernels = s.kernels;
-      prev_ctrl = s.d_ctrl;
+      a.acc_const[e] = (uint8_t)g->parts[0].consts[0];
     }
-    prev_tabs = tabs;
+    a.factors = s.d_weights, a.mtilde = s.d_mtilde, a.c0 = s.d_c0, a.ctrl = s.d_ctrl;
+    if (step.kind == LAYER && K > 1) a.bw = s.d_weights + (size_t)2 * step.rounds * D;  // (the block weights follow the factors)
+    if (step.kind == BLOCKS) s.valid_entries = (uint64_t)K;
+    // (the step that opens this sumcheck rides on the last launch of the one before, when that was held back)
+    std::vector<uint8_t> held_now;
+    s.chain_hook = [&]() { return launch_glue<D>(a, &held, held_kernels); };
+    if (fuse) s.held_tail = &held_now;
+    if ((status = s.run_device(unused_state, nullptr, nullptr, nullptr))) return status;
+    held.swap(held_now);
+    held_kernels = s.kernels;
+    prev_ctrl = s.d_ctrl;
+    prev_tabs = s.cur;
   }
   // ---- one wait, then the log
   std::vector<uint32_t> log(words);
@@ -368,16 +438,16 @@ static int prove_upper_chained(Transcript &tr, int n, int L, const std::vector<s
   uint64_t dims[2] = {2, (uint64_t)D};
   for (int l = 0; l < L; l++)
     if ((status = tr.send(&log[(size_t)l * 2 * D], 2, dims, nullptr, false))) return status;
-  const uint32_t *fin = nullptr, *tt = nullptr, *rho = nullptr;
-  for (int layer = 0; layer < n - 1; layer++) {
-    const int points = layer > 0 ? 2 : 1;
-    const uint32_t *msg = &log[log_off[layer]];
-    rho = msg + (size_t)layer * points * D;
-    fin = rho + (size_t)layer * D;
+  const uint32_t *fin = nullptr, *tt = nullptr, *rho = nullptr, *block_rho = nullptr;
+  for (const Step &step : steps) {
+    const uint32_t *msg = &log[step.log_at], *chal = msg + (size_t)step.rounds * step.points * D;
+    (step.kind == BLOCKS ? block_rho : rho) = chal;
+    dims[0] = (uint64_t)step.points;
+    for (int j = 0; j < step.rounds; j++)
+      if ((status = tr.send(msg + (size_t)j * step.points * D, 2, dims, nullptr, false))) return status;
+    if (!step.finals) continue;
+    fin = chal + (size_t)step.rounds * D;
     tt = fin + (size_t)NT * D;
-    dims[0] = (uint64_t)points;
-    for (int j = 0; j < layer; j++)
-      if ((status = tr.send(msg + (size_t)j * points * D, 2, dims, nullptr, false))) return status;
     dims[0] = 1;
     for (int t = 0; t < NT; t++)
       if ((status = tr.send(fin + (size_t)t * D, 2, dims, nullptr, false))) return status;
@@ -387,6 +457,7 @@ static int prove_upper_chained(Transcript &tr, int n, int L, const std::vector<s
     memcpy(out_ri, rho, (size_t)(n - 2) * D * 4);
     memcpy(out_ri + (size_t)(n - 2) * D, tt, (size_t)D * 4);
   }
+  if (out_rb && K > 1) memcpy(out_rb, block_rho, (size_t)lk * D * 4);
   std::vector<hf::E> cp(L), cq(L);
   next_claims(D, L, fin, hf::from(tt, D), cp, cq);
   for (int l = 0; l < L; l++) {
@@ -416,7 +487,7 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
   // one allocation holds every layer above the leaves: 2 L K (2^n - 1) entries
   if ((status = c.tree.reserve(((((uint64_t)K << n) - K) * 2 * L * D + 64) * 4))) return status;
   uint32_t *next = (uint32_t *)c.tree.ptr;
-  const int m_top = K == 1 ? std::min(n - 1, REDUCE_TOP_LAYERS - 1) : -1;  // these layers in one launch per lookup
+  const int m_top = std::min(n - 1, REDUCE_TOP_LAYERS - 1);  // these layers in one launch
   for (int m = n - 1; m >= 0; m--)
     for (int l = 0; l < L; l++) {
       uint64_t words = ((uint64_t)K << m) * D;
@@ -428,28 +499,86 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
       layers[m][2 * l] = pp;
       layers[m][2 * l + 1] = qq;
     }
-  for (int l = 0; l < L && m_top >= 0; l++) {
+  auto reduce_top = [&](const ReduceTopArgs &a, int blocks) {
+    if (D == 4)
+      hipLaunchKernelGGL(gkr_reduce_top_kernel<4>, dim3(blocks, L), dim3(BLOCK), 0, c.stream, a);
+    else
+      hipLaunchKernelGGL(gkr_reduce_top_kernel<8>, dim3(blocks, L), dim3(BLOCK), 0, c.stream, a);
+  };
+  if (m_top >= 0) {
     ReduceTopArgs a;
     memset(&a, 0, sizeof(a));
-    a.p = layers[m_top + 1][2 * l], a.q = layers[m_top + 1][2 * l + 1], a.m_top = m_top;
-    for (int m = m_top; m >= 0; m--)
-      a.pp[m] = const_cast<uint32_t *>(layers[m][2 * l]), a.qq[m] = const_cast<uint32_t *>(layers[m][2 * l + 1]);
-    if (D == 4)
-      hipLaunchKernelGGL(gkr_reduce_top_kernel<4>, dim3(1), dim3(BLOCK), 0, c.stream, a);
-    else
-      hipLaunchKernelGGL(gkr_reduce_top_kernel<8>, dim3(1), dim3(BLOCK), 0, c.stream, a);
+    a.m_top = m_top;
+    for (int l = 0; l < L; l++) {
+      a.p[l] = layers[m_top + 1][2 * l], a.q[l] = layers[m_top + 1][2 * l + 1];
+      for (int m = m_top; m >= 0; m--)
+        a.pp[l][m] = const_cast<uint32_t *>(layers[m][2 * l]), a.qq[l][m] = const_cast<uint32_t *>(layers[m][2 * l + 1]);
+    }
+    reduce_top(a, K);
     EXH_HIP(hipGetLastError());
   }
-  {  // one block: the layers chained on the device, one wait for the whole proof
-    const char *host_rounds = getenv("EXACTA_HIP_HOST_ROUNDS"), *no_chain = getenv("EXACTA_HIP_NO_GKR_CHAIN");
-    const bool off = (host_rounds && host_rounds[0] == '1') || (no_chain && no_chain[0] == '1');
-    if (K == 1 && n >= 2 && n - 2 <= MAXROUNDS && L * D <= 12 && 2 * L <= GLUE_MAXCONST && !off) {
-      status = D == 4 ? prove_upper_chained<4>(tr, n, L, layers, label, out_ri, out_cp, out_cq)
-                      : prove_upper_chained<8>(tr, n, L, layers, label, out_ri, out_cp, out_cq);
-      if (status) return status;
-      EXH_HIP(hipStreamSynchronize(c.stream));
-      return OK;
+  const char *host_rounds = getenv("EXACTA_HIP_HOST_ROUNDS"), *no_chain = getenv("EXACTA_HIP_NO_GKR_CHAIN");
+  const bool chains = L * D <= 12 && 2 * L <= GLUE_MAXCONST && !(host_rounds && host_rounds[0] == '1') &&
+                      !(no_chain && no_chain[0] == '1');
+  // All layers chained on the device, one wait for the whole proof.  With several blocks as long as a lane holds a block in
+  // the step that forms their weights, and the one-workgroup launch the last round's pairs (and the tables over the block
+  // index): beyond that a layer is two device-driven sumchecks with a wait each, as below.  That way and this one, us: three
+  // blocks of 2^14 and two lookups 1900 and 1310, five of 2^10 1100 and 745, 64 of 2^8 1130 and 830, 33 of 2^10 and three
+  // lookups 3900 and 2330.
+  if (chains && n >= 2 && n - 2 <= MAXROUNDS && (K == 1 || blocks_chain(K, L, D))) {
+    ChainTables tables;
+    auto halves = [&](const std::vector<const uint32_t *> &vectors, uint64_t size) {  // with one block they are views
+      std::vector<const uint32_t *> tabs(NT);
+      for (int i = 0; i < 2 * L; i++) tabs[2 * i] = vectors[i], tabs[2 * i + 1] = vectors[i] + size * D;
+      return tabs;
+    };
+    if (K == 1) {
+      tables.roots = layers[0];
+      for (int layer = 0; layer < n - 1; layer++) tables.layers.push_back(halves(layers[layer + 1], (uint64_t)1 << layer));
+    } else {
+      // the tree over the block index, its lowest layer padded with 0 / 1 (2^lk roots)
+      uint32_t *d_top = bufs.alloc(2 * Kp * 2 * L * D), *d_halves = bufs.alloc((uint64_t)NT * K * (((uint64_t)1 << (n - 1)) - 1) * D);
+      if (!d_top || !d_halves) {
+        set_error("device-out-of-memory: the layers' tables");
+        return E_NOMEM;
+      }
+      ReduceTopArgs a;
+      memset(&a, 0, sizeof(a));
+      a.m_top = lk - 1, a.valid = (uint32_t)K;
+      std::vector<std::vector<const uint32_t *>> top(lk + 1, std::vector<const uint32_t *>(2 * L));
+      for (int l = 0; l < L; l++) {
+        a.p[l] = layers[0][2 * l], a.q[l] = layers[0][2 * l + 1];
+        for (int m = lk; m >= 0; m--) {
+          uint32_t *pp = d_top, *qq = pp + ((uint64_t)D << m);
+          d_top = qq + ((uint64_t)D << m);
+          (m == lk ? a.pad_p[l] : a.pp[l][m]) = pp, (m == lk ? a.pad_q[l] : a.qq[l][m]) = qq;
+          top[m][2 * l] = pp, top[m][2 * l + 1] = qq;
+        }
+      }
+      reduce_top(a, 1);
+      EXH_HIP(hipGetLastError());
+      tables.roots = top[0];
+      for (int j = 0; j < lk; j++) tables.top.push_back(halves(top[j + 1], (uint64_t)1 << j));
+      const uint64_t entries = (uint64_t)K * (((uint64_t)1 << (n - 1)) - 1);
+      const dim3 grid((uint32_t)((entries + BLOCK - 1) / BLOCK), 2 * L);
+      const uint32_t *tree = (const uint32_t *)c.tree.ptr;
+      if (D == 4)
+        hipLaunchKernelGGL(all_halves_kernel<4>, grid, dim3(BLOCK), 0, c.stream, tree, d_halves, (uint32_t)K, n, entries);
+      else
+        hipLaunchKernelGGL(all_halves_kernel<8>, grid, dim3(BLOCK), 0, c.stream, tree, d_halves, (uint32_t)K, n, entries);
+      EXH_HIP(hipGetLastError());
+      for (int layer = 0; layer < n - 1; layer++) {
+        const uint64_t n_out = (uint64_t)K << layer;
+        std::vector<const uint32_t *> tabs(NT);
+        for (int t = 0; t < NT; t++) tabs[t] = d_halves + ((uint64_t)NT * (n_out - K) + t * n_out) * D;
+        tables.layers.push_back(tabs);
+      }
     }
+    status = D == 4 ? prove_upper_chained<4>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq)
+                    : prove_upper_chained<8>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq);
+    if (status) return status;
+    EXH_HIP(hipStreamSynchronize(c.stream));
+    return OK;
   }
   // the per-block roots, and the top tree over the block index on the host (2^lk entries)
   std::vector<std::vector<std::vector<uint32_t>>> top(lk + 1, std::vector<std::vector<uint32_t>>(2 * L));
@@ -488,35 +617,35 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
   // The top tree is a tree of one block over the block index: its roots and layers are PROVE-UPPER's with one
   // block under the label's "-top", so the chain above serves it as well (one wait instead of one per layer).
   bool top_chained = false;
-  {
-    const char *host_rounds = getenv("EXACTA_HIP_HOST_ROUNDS"), *no_chain = getenv("EXACTA_HIP_NO_GKR_CHAIN");
-    const bool off = (host_rounds && host_rounds[0] == '1') || (no_chain && no_chain[0] == '1');
-    if (lk >= 1 && lk - 1 <= MAXROUNDS && L * D <= 12 && 2 * L <= GLUE_MAXCONST && !off) {
-      // every level of every lookup's top tree in one buffer, one copy
-      std::vector<std::vector<const uint32_t *>> top_layers(lk + 1, std::vector<const uint32_t *>(2 * L));
-      std::vector<uint32_t> all;
-      std::vector<std::vector<size_t>> at(lk + 1, std::vector<size_t>(2 * L));
-      for (int j = 0; j <= lk; j++)
-        for (int i = 0; i < 2 * L; i++) {
-          at[j][i] = all.size();
-          all.insert(all.end(), top[j][i].begin(), top[j][i].end());
-        }
-      uint32_t *d_top = bufs.alloc(all.size());
-      if (!d_top) return E_NOMEM;
-      EXH_HIP(hipMemcpyAsync(d_top, all.data(), all.size() * 4, hipMemcpyHostToDevice, c.stream));
-      for (int j = 0; j <= lk; j++)
-        for (int i = 0; i < 2 * L; i++) top_layers[j][i] = d_top + at[j][i];
-      r.assign((size_t)lk * D, 0);
-      std::vector<uint32_t> ocp((size_t)L * D), ocq((size_t)L * D);
-      status = D == 4 ? prove_upper_chained<4>(tr, lk + 1, L, top_layers, label + "-top", r.data(), ocp.data(), ocq.data())
-                      : prove_upper_chained<8>(tr, lk + 1, L, top_layers, label + "-top", r.data(), ocp.data(), ocq.data());
-      if (status) return status;
-      for (int l = 0; l < L; l++) {
-        cp[l] = hf::from(&ocp[(size_t)l * D], D);
-        cq[l] = hf::from(&ocq[(size_t)l * D], D);
+  if (chains && lk >= 1 && lk - 1 <= MAXROUNDS) {
+    // every level of every lookup's top tree in one buffer, one copy
+    ChainTables tables;
+    std::vector<uint32_t> all;
+    std::vector<std::vector<size_t>> at(lk + 1, std::vector<size_t>(2 * L));
+    for (int j = 0; j <= lk; j++)
+      for (int i = 0; i < 2 * L; i++) {
+        at[j][i] = all.size();
+        all.insert(all.end(), top[j][i].begin(), top[j][i].end());
       }
-      top_chained = true;
+    uint32_t *d_top = bufs.alloc(all.size());
+    if (!d_top) return E_NOMEM;
+    EXH_HIP(hipMemcpyAsync(d_top, all.data(), all.size() * 4, hipMemcpyHostToDevice, c.stream));
+    for (int i = 0; i < 2 * L; i++) tables.roots.push_back(d_top + at[0][i]);
+    for (int j = 0; j < lk; j++) {
+      std::vector<const uint32_t *> tabs(NT);
+      for (int i = 0; i < 2 * L; i++) tabs[2 * i] = d_top + at[j + 1][i], tabs[2 * i + 1] = tabs[2 * i] + ((size_t)D << j);
+      tables.layers.push_back(tabs);
     }
+    r.assign((size_t)lk * D, 0);
+    std::vector<uint32_t> ocp((size_t)L * D), ocq((size_t)L * D);
+    status = D == 4 ? prove_upper_chained<4>(tr, lk + 1, 1, 0, L, tables, label + "-top", r.data(), nullptr, ocp.data(), ocq.data())
+                    : prove_upper_chained<8>(tr, lk + 1, 1, 0, L, tables, label + "-top", r.data(), nullptr, ocp.data(), ocq.data());
+    if (status) return status;
+    for (int l = 0; l < L; l++) {
+      cp[l] = hf::from(&ocp[(size_t)l * D], D);
+      cq[l] = hf::from(&ocq[(size_t)l * D], D);
+    }
+    top_chained = true;
   }
   if (!top_chained) {
     for (int l = 0; l < L; l++) {  // the roots

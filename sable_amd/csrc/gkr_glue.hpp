@@ -6,33 +6,48 @@
 namespace exh {
 
 // ------------------------------------------------------------------ the layers chained on the device
-// With one block, the layers' sumchecks run back to back without the host: between two of them one small launch
+// The layers' sumchecks run back to back without the host: between two of them one small launch
 // (one wavefront) does what PROVE-UPPER does on the host there (src/gkr.lisp:248-271) -- it sends the finished
 // layer's finals and draws the fresh point (SEND-FINALS), forms the next layer's point, draws the layer's
 // challenges (LAYER-CHALLENGES), absorbs the next sumcheck's header and writes that sumcheck's constants where its
 // launches expect them: the eq point's factors, the message map, the head of the control block with the
 // transcript's state.  Everything the host needs afterwards goes to a log it reads once at the end.
+// With several blocks the layers of the tree over the block index come first, and then a layer is two sumchecks, its own
+// with the block weights as HIGH table and the one over the block index: the step between those two only records the
+// first one's rounds and opens the second, with the layer's challenges kept from the step before; the step behind the
+// second one sends the finals, and forms the next layer's block weights (eq of the block point, src/gkr.lisp:73-77).
+constexpr int GLUE_MAXBLOCKS = 64, GLUE_BLOCK_BITS = 6;  // a lane per block in the step that forms their weights
+constexpr int GLUE_MAXCONST = 8;  // constants of a layer statement the launch can form: a_l and a_l lambda, l < 4
 struct GkrChainState {
   DevB3S tr;                       // the transcript between launches
   uint32_t point[MAXROUNDS + 1][8];  // the next layer's eq point (canonical)
+  uint32_t consts[GLUE_MAXCONST][8];  // the layer's a_l and a_l lambda, kept for its sumcheck over the block index
   // sticky: a chained layer's sumcheck did not complete (a workgroup of a grid launch gave up, or the control
   // block does not count the layer's rounds); the host reads it after its one wait and voids the proof
   uint32_t failed;
 };
 
-constexpr int GLUE_MAXCONST = 8;  // constants of a layer statement the launch can form: a_l and a_l lambda, l < 4
-
 template <int D>
 struct GlueArgs {
   GkrChainState *chain;
-  int close_kind;  // 0: nothing to close, 1: send the roots, 2: a layer's finals from its control block, 3: from tables
+  // 0: nothing to close, 1: send the roots, 2: a layer's finals from its control block, 3: from tables, 4: the rounds of a
+  // layer's own sumcheck (its finals are those of the one over the block index)
+  int close_kind;
   const Ctrl *prev_ctrl;
   int prev_rounds, prev_points;
+  int fin_skip;  // kind 2: the first tables in the control block's finals that are not sent (the block weights)
+  // kind 2, a sumcheck over the block index (blocks_closed): its challenges are the block point, and the fresh point is
+  // coordinate tt_at of the layer's point, whose others an earlier step left in the chain's state
+  int blocks_closed, tt_at;
   const uint32_t *tabs[MAXT];  // kind 1: the root of p and of q per lookup; kind 3: the layer's tables (one entry each)
   int NT, L;
   uint32_t *log;  // kind 1: the roots (2 L D words); kinds 2, 3: the layer's messages, challenges, finals, fresh point
-  int open;       // open the next layer's sumcheck
+  int open;       // 1: open the next layer's sumcheck, 2: the one over the block index
   int n;          // its rounds
+  // a layer of several blocks: the weights of blocks 0 .. K - 1, eq of the block point of lk coordinates, go to bw (the
+  // sumcheck's HIGH table; null without rounds) and to bw_table (the first table of the one over the block index)
+  int K, lk;
+  uint32_t *bw, *bw_table;
   uint32_t header[16];  // its header's bytes (src/sumcheck.lisp:24-27), as little-endian words
   int header_len;
   uint32_t *factors, *mtilde, *c0;
@@ -68,10 +83,12 @@ __device__ __forceinline__ void gkr_glue_body(const GlueArgs<D> &a) {
   __shared__ uint32_t fin[MAXT * 8];
   __shared__ uint32_t consts[GLUE_MAXCONST][8];
   __shared__ uint32_t point[MAXROUNDS + 1][8];
+  __shared__ uint32_t block_point[GLUE_BLOCK_BITS][8];
   const uint32_t lane = threadIdx.x;
+  const bool from_ctrl = a.close_kind == 2 || a.close_kind == 4;
   RunB3S tr;
   {  // the transcript's state where the last launch (or this one's rounds) left it
-    const uint32_t *g = reinterpret_cast<const uint32_t *>(a.close_kind == 2 ? &a.prev_ctrl->tr : &a.chain->tr);
+    const uint32_t *g = reinterpret_cast<const uint32_t *>(from_ctrl ? &a.prev_ctrl->tr : &a.chain->tr);
     if (lane < sizeof(DevB3S) / 4) buf[lane] = fresh_word(g + lane);
     __builtin_amdgcn_wave_barrier();
     rb3s_load(tr, ring, reinterpret_cast<const DevB3S *>(buf));
@@ -88,50 +105,82 @@ __device__ __forceinline__ void gkr_glue_body(const GlueArgs<D> &a) {
   } else if (a.close_kind != 0) {
     const int R = a.prev_rounds, mw = a.prev_points * D;
     uint32_t *log_msg = a.log, *log_chal = log_msg + R * mw, *log_fin = log_chal + R * D, *log_tt = log_fin + a.NT * D;
-    if (a.close_kind == 2) {
+    if (from_ctrl) {
       if (lane == 0 && (fresh_word(&a.prev_ctrl->gave_up) != 0 || fresh_word(&a.prev_ctrl->round) != (uint32_t)R))
         a.chain->failed = 1;
       for (int u = lane; u < R * mw; u += 64) log_msg[u] = fresh_word(&a.prev_ctrl->msg[u / mw][u % mw]);
       for (int u = lane; u < R * D; u += 64) {
         const uint32_t v = fresh_word(&a.prev_ctrl->chal[u / D][u % D]);
         log_chal[u] = v;
-        point[u / D][u % D] = v;  // the layer's challenges open the next layer's point
+        if (a.blocks_closed)
+          block_point[u / D][u % D] = v;
+        else
+          point[u / D][u % D] = v;  // the layer's challenges open the next layer's point
       }
     }
-    // SEND-FINALS: one message (1, D) per table, then the fresh point (the finals fetched in one trip)
-    for (int u = lane; u < a.NT * D; u += 64) {
-      const uint32_t v = a.close_kind == 2 ? fresh_word(&a.prev_ctrl->finals[u]) : a.tabs[u / D][u % D];
-      fin[u] = v;
-      log_fin[u] = v;
+    if (a.close_kind != 4) {
+      // SEND-FINALS: one message (1, D) per table, then the fresh point (the finals fetched in one trip)
+      for (int u = lane; u < a.NT * D; u += 64) {
+        const uint32_t v = a.close_kind == 2 ? fresh_word(&a.prev_ctrl->finals[a.fin_skip * D + u]) : a.tabs[u / D][u % D];
+        fin[u] = v;
+        log_fin[u] = v;
+      }
+      if (a.blocks_closed)
+        for (int u = lane; u < a.tt_at * D; u += 64) point[u / D][u % D] = fresh_word(&a.chain->point[u / D][u % D]);
+      __builtin_amdgcn_wave_barrier();
+      for (int t = 0; t < a.NT; t++) dev_absorb_words(tr, fin + t * D, D);
+      dev_challenge(tr, D, chal);
+      __builtin_amdgcn_wave_barrier();
+      if (lane < D) {
+        log_tt[lane] = chal[lane];
+        point[a.blocks_closed ? a.tt_at : R][lane] = chal[lane];
+      }
     }
     __builtin_amdgcn_wave_barrier();
-    for (int t = 0; t < a.NT; t++) dev_absorb_words(tr, fin + t * D, D);
-    dev_challenge(tr, D, chal);
-    __builtin_amdgcn_wave_barrier();
-    if (lane < D) {
-      log_tt[lane] = chal[lane];
-      point[R][lane] = chal[lane];
+    const int coords = a.close_kind == 4 ? R : a.blocks_closed ? a.tt_at + 1 : R + 1;
+    for (int u = lane; u < coords * D; u += 64) a.chain->point[u / D][u % D] = point[u / D][u % D];
+  }
+  if (a.open == 1 && a.K > 1) {
+    // the block weights from the block point: the challenges just closed, or the point that the tree over the block
+    // index left; then the layer's own point starts empty
+    Ext<D> e = ext_lift<D>(1);
+    for (int v = 0; v < a.lk; v++) {
+      const uint32_t *r = a.blocks_closed ? block_point[v] : point[v];
+      const bool set = (lane >> v) & 1;
+      Ext<D> f;
+#pragma unroll
+      for (int c = 0; c < D; c++) f.c[c] = to_mont(set ? r[c] : fsub(c == 0 ? 1u : 0u, r[c]));
+      e = ext_mul_mont<D>(e, f);
     }
-    __builtin_amdgcn_wave_barrier();
-    for (int u = lane; u < (R + 1) * D; u += 64) a.chain->point[u / D][u % D] = point[u / D][u % D];
+    if (lane < (uint32_t)a.K) {
+      store_ext<D>(a.bw_table + lane * D, e);
+      if (a.bw) store_ext<D>(a.bw + lane * D, e);
+    }
   }
   if (a.open) {
-    if (a.close_kind == 0 || a.close_kind == 1)
+    if (a.open == 1 && (a.close_kind == 0 || a.close_kind == 1))
       for (int u = lane; u < a.n * D; u += 64) point[u / D][u % D] = a.chain->point[u / D][u % D];
-    // LAYER-CHALLENGES: a_l from one stream of L D base challenges, then lambda
-    dev_challenge(tr, a.L * D, chal);
-    __builtin_amdgcn_wave_barrier();
-    if (lane < (uint32_t)(a.L * D)) consts[2 * (lane / D)][lane % D] = chal[lane];
-    __builtin_amdgcn_wave_barrier();
-    dev_challenge(tr, D, chal);
-    __builtin_amdgcn_wave_barrier();
-    if (lane < (uint32_t)a.L) {  // a_l lambda, exact: one factor carries R
-      Ext<D> x, y;
+    if (a.open == 2) {
+      for (int u = lane; u < 2 * a.L * D; u += 64) consts[u / D][u % D] = fresh_word(&a.chain->consts[u / D][u % D]);
+    } else {
+      // LAYER-CHALLENGES: a_l from one stream of L D base challenges, then lambda
+      dev_challenge(tr, a.L * D, chal);
+      __builtin_amdgcn_wave_barrier();
+      if (lane < (uint32_t)(a.L * D)) consts[2 * (lane / D)][lane % D] = chal[lane];
+      __builtin_amdgcn_wave_barrier();
+      dev_challenge(tr, D, chal);
+      __builtin_amdgcn_wave_barrier();
+      if (lane < (uint32_t)a.L) {  // a_l lambda, exact: one factor carries R
+        Ext<D> x, y;
 #pragma unroll
-      for (int c = 0; c < D; c++) x.c[c] = consts[2 * lane][c], y.c[c] = to_mont(chal[c]);
-      const Ext<D> z = ext_mul_mont<D>(x, y);
+        for (int c = 0; c < D; c++) x.c[c] = consts[2 * lane][c], y.c[c] = to_mont(chal[c]);
+        const Ext<D> z = ext_mul_mont<D>(x, y);
 #pragma unroll
-      for (int c = 0; c < D; c++) consts[2 * lane + 1][c] = z.c[c];
+        for (int c = 0; c < D; c++) consts[2 * lane + 1][c] = z.c[c];
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (a.K > 1)
+        for (int u = lane; u < 2 * a.L * D; u += 64) a.chain->consts[u / D][u % D] = consts[u / D][u % D];
     }
     __builtin_amdgcn_wave_barrier();
     if (lane < 16) buf[lane] = a.header[lane];
@@ -139,7 +188,7 @@ __device__ __forceinline__ void gkr_glue_body(const GlueArgs<D> &a) {
     dev_absorb_bytes(tr, buf, (uint32_t)a.header_len);
     if (a.n > 0) {
       // the eq point's factors r_v R and (1 - r_v) R, variable by variable
-      for (int u = lane; u < a.n * D; u += 64) {
+      for (int u = lane; a.open == 1 && u < a.n * D; u += 64) {
         const uint32_t v = u / D, k = u % D, r = point[v][k];
         a.factors[(2 * v) * D + k] = to_mont(r);
         a.factors[(2 * v + 1) * D + k] = to_mont(fsub(k == 0 ? 1u : 0u, r));

@@ -935,6 +935,8 @@ static uint64_t tail_pairs(int T, int D) {
   return p;
 }
 
+uint64_t SumcheckSession::one_workgroup_pairs(int T, int D) { return tail_pairs(T, D); }
+
 // the Lagrange basis of the group's node e over its nodes at wire point k (0, 2, 3, ...), times the power of R the
 // group's sums carry (R^-degree)
 static uint32_t map_scalar(const Group &grp, size_t e, int k, int points, bool direct) {
@@ -1017,11 +1019,19 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   }
   // A session whose every round runs in the one-workgroup launch needs no set-up launch: that launch builds the
   // weight tables itself from the eq point's factors, which lead the session's constants (EXACTA_HIP_NO_OWN_WEIGHTS=1:
-  // never)
+  // never).  In a chain, whose constants are on the device already, also the all-ones tables of a session without an eq
+  // point, and it reads the block weights, which follow the factors, where they lie; where the constants come from the host
+  // such a session's set-up launch is cheaper than the copy that brings them without it (two points' reduction of 2^9: 66
+  // and 69 us; layers of 64 blocks driven by the host, 2^8 entries: 1108 and 1367 us a tree).
   {
     const char *no_own = getenv("EXACTA_HIP_NO_OWN_WEIGHTS");
-    own_weights = setup_deferred && has_eq && !has_bw && setup.total_eq > 0 && !setup.ones_len &&
-                  size / 2 <= tail_pairs(T, D) && n <= MAXTAIL && !(no_own && no_own[0] == '1');
+    const bool one_launch = size / 2 <= tail_pairs(T, D) && n <= MAXTAIL;
+    own_weights = setup_deferred && one_launch && (chain_hook ? has_bw || K == 1 : has_eq && !has_bw) &&
+                  !(no_own && no_own[0] == '1');
+    if (valid_entries && (!one_launch || cur_base)) {
+      set_error("invalid-parameter: padded tables are extension elements for the one-workgroup launch");
+      return E_PARAM;
+    }
   }
   if (chain_hook) {  // the chain's launch writes what the copy below would bring
     if (!setup_deferred) {
@@ -1197,7 +1207,7 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   device_loop = false;
   if (status) return status;
   if (chain_hook) {  // nothing comes back here: the chain reads the control block on the device
-    if (!tail_done || size != 1) {
+    if (!tail_done || size != (uint64_t)K) {
       set_error("device-error: a chained sumcheck did not end in the one-workgroup launch");
       return E_DEVICE;
     }
@@ -1298,10 +1308,12 @@ int SumcheckSession::launch_tail(int j, int rounds, uint32_t grid, bool first_fo
       a.high_off[jj] = high_off[j + jj];
       a.low_bits[jj] = (uint32_t)low_bits[j + jj];
     }
+    if (j == 0) a.valid = (uint32_t)valid_entries;
     if (own_weights && grid == 1 && j == 0 && rounds == n) {  // the launch builds the weight tables behind its tables
       uint64_t own_entries = (uint64_t)2 * n;
-      for (int jj = 0; jj < n; jj++) own_entries += ((uint64_t)1 << low_bits[jj]) + n_high[jj];
-      a.factors = d_weights, a.n_vars = (uint32_t)n;
+      for (int jj = 0; jj < n; jj++)  // (the HIGH table of all variables but the round's and those of LOW: one entry with block weights)
+        own_entries += ((uint64_t)1 << low_bits[jj]) + ((uint64_t)1 << (n - (jj + 1) - low_bits[jj]));
+      a.own = 1, a.factors = has_eq ? d_weights : nullptr, a.n_vars = (uint32_t)n, a.block_high = has_bw ? 1 : 0;
       a.lds_bytes += (uint32_t)(own_entries * D * 4);
     }
   };

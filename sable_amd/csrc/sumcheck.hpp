@@ -102,6 +102,9 @@ struct SumcheckSession {
   // workgroup, the last rounds) is then not enqueued; its arguments are left here (a TailArgs<D>) for the caller to
   // launch, after this session has returned and even after the next one has begun (they are plain addresses).
   std::vector<uint8_t> *held_tail = nullptr;
+  // Set before run_device: the tables in memory hold this many entries (extension elements), zeros beyond them up to the
+  // session's size; for sessions whose every round runs in the one-workgroup launch (0: all entries are there).
+  uint64_t valid_entries = 0;
   // the scalar (Lagrange basis times the power of R the sums carry) that maps accumulator `acc` to wire point k in
   // the message map: lagfix[k * nacc + acc], and the group each accumulator belongs to
   void message_map_scalars(std::vector<uint32_t> *lagfix, std::vector<int> *acc_group) const;
@@ -131,6 +134,8 @@ struct SumcheckSession {
   // was sent and drawn, final_state (optional) the transcript's hash state after the last challenge, and the
   // session is ready for finish().  Needs points <= MAXPTS.
   int run_device(const DevB3S &state, uint32_t *messages, uint32_t *challenges, DevB3S *final_state = nullptr);
+  // pairs of a round of T tables that the one-workgroup launch takes
+  static uint64_t one_workgroup_pairs(int T, int D);
   // rounds first_round .. first_round + rounds - 1 with the tables in LDS, over `grid` workgroups
   int launch_tail(int first_round, int rounds, uint32_t grid, bool first_fold);
   // the device-driven loop fits this session: rounds, wire points, and its constants in the pinned staging area

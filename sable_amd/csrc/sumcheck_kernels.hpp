@@ -118,12 +118,13 @@ struct TailArgs {
   uint32_t *host_log;
   uint32_t host_flag_at, host_seq;
   const uint32_t *consts;  // a statement in direct form: its constant slots (EXTs, Montgomery form)
-  // A session whose every round runs in this one launch builds its weight tables itself, in LDS behind the tables
-  // (no set-up launch): `factors` holds (r_v R, (1 - r_v) R) for the eq point's n_vars variables; round jj's LOW
-  // table covers the low_bits[jj] variables from first_round + jj + 1 on, its HIGH table the rest.  Null: the
-  // tables are read from `weights`.
+  // A session whose every round runs in this one launch builds its weight tables itself (`own`), in LDS behind the
+  // tables (no set-up launch): `factors` holds (r_v R, (1 - r_v) R) for the eq point's n_vars variables; round jj's LOW
+  // table covers the low_bits[jj] variables from first_round + jj + 1 on, its HIGH table the rest.  Without an eq point
+  // (factors null) the entries are ones; with block weights (block_high) the HIGH entries are those, read from `weights`.
   const uint32_t *factors;
-  uint32_t n_vars;
+  uint32_t n_vars, own, block_high;
+  uint32_t valid;  // entries that the tables in memory hold, zeros beyond them (0: all of them; unfolded extension tables)
 };
 
 template <int D>
@@ -1174,6 +1175,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
             }
           } else if (args.first_fold) {
             v = fold_ext<D>(load_ext<D>(in + 2 * gx * D), load_ext<D>(in + (2 * gx + 1) * D), r);
+          } else if (args.valid && gx >= args.valid) {
+            v = ext_zero<D>();
           } else {
             v = load_ext<D>(in + gx * D);
           }
@@ -1197,7 +1200,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // The session's own weight tables (see TailArgs::factors), in LDS behind the tables: the factors first, then
   // per round its LOW and its HIGH table.  An entry is a chain of at most n_vars products, one entry per thread
   // and trip: entry x of a table over the variables [first, first + bits) is prod_b (x_b ? r_b : 1 - r_b).
-  const bool own_weights = args.factors != nullptr;
+  const bool own_weights = args.own != 0;
   uint32_t *const own_factors = tail_tables + (size_t)d.T * cap * D;
   uint32_t *const own_tables = own_factors + (size_t)2 * args.n_vars * D;
   auto own_high_bits = [&](uint32_t jj) { return args.n_vars - (args.first_round + jj + 1) - args.low_bits[jj]; };
@@ -1207,7 +1210,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     return high ? at + (1u << args.low_bits[jj]) : at;
   };
   if (own_weights) {
-    for (uint32_t u = tid; u < 2 * args.n_vars * D; u += BLOCK) own_factors[u] = args.factors[u];
+    if (args.factors)
+      for (uint32_t u = tid; u < 2 * args.n_vars * D; u += BLOCK) own_factors[u] = args.factors[u];
     __syncthreads();
     const uint32_t total = own_at(args.rounds, false);
     for (uint32_t u = tid; u < total; u += BLOCK) {
@@ -1227,7 +1231,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
       }
       const uint32_t x = u - start;
       Ext<D> e = ext_lift<D>(1);
-      for (uint32_t b = 0; b < bits; b++)
+      for (uint32_t b = 0; args.factors && b < bits; b++)
         e = ext_mul_mont<D>(e, load_ext<D>(own_factors + ((size_t)(first + b) * 2 + (((x >> b) & 1) ? 0 : 1)) * D));
       store_ext<D>(own_tables + (size_t)u * D, e);
     }
@@ -1245,7 +1249,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     const uint64_t i = (uint64_t)wg * pairs + (me < pairs ? me : pairs - 1);
     if (own_weights) {
       wl = load_ext<D>(own_tables + (size_t)(own_at(jj, false) + (uint32_t)(i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
-      wh = load_ext<D>(own_tables + (size_t)(own_at(jj, true) + (uint32_t)(i >> args.low_bits[jj])) * D);
+      wh = args.block_high ? load_ext<D>(args.weights + (args.high_off[jj] + (i >> args.low_bits[jj])) * D)
+                           : load_ext<D>(own_tables + (size_t)(own_at(jj, true) + (uint32_t)(i >> args.low_bits[jj])) * D);
       return;
     }
     wl = load_ext<D>(args.weights + (args.low_off[jj] + (i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
@@ -1300,7 +1305,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     for (int j = 0; j < SPREAD_FACTORS; j++) unit_table[j] = unit.table[j];
     const uint64_t i = (uint64_t)wg * pairs + (on ? unit_pair : pairs - 1);
     const uint32_t *low = own_weights ? own_tables + (size_t)own_at(jj, false) * D : args.weights + args.low_off[jj] * D;
-    const uint32_t *high = own_weights ? own_tables + (size_t)own_at(jj, true) * D : args.weights + args.high_off[jj] * D;
+    const uint32_t *high = own_weights && !args.block_high ? own_tables + (size_t)own_at(jj, true) * D
+                                                           : args.weights + args.high_off[jj] * D;
     const Ext<D> l = load_ext<D>(low + (i & (((uint64_t)1 << args.low_bits[jj]) - 1)) * D);
     const Ext<D> h = load_ext<D>(high + (i >> args.low_bits[jj]) * D);
     unit_w = ext_scale_mont<D>(ext_mul_mont<D>(l, h), on ? R2 : 0u);  // (times R for the product that takes it in below)

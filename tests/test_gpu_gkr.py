@@ -119,6 +119,35 @@ def test_the_chained_layers_and_the_host_driven_layers_send_the_same_bytes(n, lo
         p.free(), q.free()
 
 
+@pytest.mark.parametrize("n,k,lookups,d", [
+    (2, 2, 1, 4), (2, 5, 3, 4),  # one layer in the blocks, without rounds of its own
+    (3, 64, 1, 4), (3, 65, 1, 4),  # as many blocks as the step between two layers has lanes, and one more
+    (4, 33, 2, 4), (9, 7, 3, 4),  # an odd part that no grid of slices takes; many tables
+    (5, 12, 1, 8),  # kernels of a statement's own are there at degree 4 only: the steps are launches of their own
+    (13, 2, 2, 4), (12, 5, 1, 4),  # rounds on slices and streaming rounds in the chain
+])
+def test_layers_of_several_blocks_chained_and_host_driven(n, k, lookups, d, monkeypatch):
+    """With several blocks a layer's two sumchecks and the tree over the block index are one chain on the device: the
+    oracle's proof, outputs and transcript state, as when the host drives every layer."""
+    rng = np.random.default_rng(1000 * n + k)
+    leaves = random_leaves(rng, lookups, n, k, d)
+    dev = [(sa.Table.upload(p), sa.Table.upload(q)) for p, q in leaves]
+    otr = orc.Transcript("gkr-test", d)
+    want = orc.gkr_prove_upper(otr, n, k, leaves)
+    states = []
+    for off in ("0", "1"):
+        monkeypatch.setenv("EXACTA_HIP_NO_GKR_CHAIN", off)
+        tr = sa.Transcript("gkr-test", d)
+        got = sa.prove_upper(tr, n, k, dev)
+        assert tr.proof() == otr.proof()
+        for a, b in zip(got, want):
+            assert same(a, b)
+        states.append(tr.state_digest())
+    assert states[0] == states[1]
+    for p, q in dev:
+        p.free(), q.free()
+
+
 # two trees side by side (a second host thread, stream and workspace): each proof's bytes, outputs and final
 # transcript state are those of the call on its own; pairs of different sizes, both chained, one host-driven
 # (several blocks), both large enough for the grids of slices that must share the device
