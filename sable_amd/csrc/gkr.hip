@@ -3,6 +3,7 @@
 
 #include <string.h>
 
+#include <atomic>
 #include <vector>
 
 #include "context.hpp"
@@ -14,29 +15,62 @@
 
 namespace exh {
 
-// parent (b, x) of children (b, x) and (b, x + 2^m): p = p0 q1 + p1 q0, q = q0 q1
+constexpr int REDUCE_MAXL = MAXT / 4;  // lookups proved together: four tables each
+// the parent of two children: p = p0 q1 + p1 q0, q = q0 q1 (products carry 1/R; multiplying one factor of each product by
+// R^2 first makes them exact)
 template <int D>
-__global__ __launch_bounds__(BLOCK) void gkr_reduce_kernel(const uint32_t *p, const uint32_t *q, uint32_t *pp,
-                                                           uint32_t *qq, uint32_t m, uint64_t n_out) {
-  uint64_t o = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-  if (o >= n_out) return;
-  uint64_t half = (uint64_t)1 << m, b = o >> m, x = o & (half - 1);
-  uint64_t c0 = (b << (m + 1)) + x, c1 = c0 + half;
-  Ext<D> p0 = load_ext<D>(p + c0 * D), p1 = load_ext<D>(p + c1 * D);
-  Ext<D> q0 = load_ext<D>(q + c0 * D), q1 = load_ext<D>(q + c1 * D);
-  // products carry 1/R; multiplying one factor of each product by R^2 first makes them exact
-  Ext<D> q1r, q0r;
-#pragma unroll
-  for (int c = 0; c < D; c++) q1r.c[c] = mont_mul(q1.c[c], R2), q0r.c[c] = mont_mul(q0.c[c], R2);
-  store_ext<D>(pp + o * D, ext_add<D>(ext_mul_mont<D>(p0, q1r), ext_mul_mont<D>(p1, q0r)));
-  store_ext<D>(qq + o * D, ext_mul_mont<D>(q0, q1r));
+struct Fraction {
+  Ext<D> p, q;
+};
+template <int D>
+__device__ __forceinline__ Fraction<D> load_fraction(const uint32_t *p, const uint32_t *q, uint64_t at) {
+  return {load_ext<D>(p + at * D), load_ext<D>(q + at * D)};
+}
+template <int D>
+__device__ __forceinline__ Fraction<D> add_fractions(const Fraction<D> &a, const Fraction<D> &b) {
+  const Ext<D> q1r = ext_scale_mont<D>(b.q, R2), q0r = ext_scale_mont<D>(a.q, R2);
+  return {ext_add<D>(ext_mul_mont<D>(a.p, q1r), ext_mul_mont<D>(b.p, q0r)), ext_mul_mont<D>(a.q, q1r)};
+}
+template <int D>
+__device__ __forceinline__ void store_fraction(uint32_t *p, uint32_t *q, uint64_t at, const Fraction<D> &f) {
+  store_ext<D>(p + at * D, f.p);
+  store_ext<D>(q + at * D, f.q);
+}
+
+// A layer from the one below, parent (b, x) of children (b, x) and (b, x + 2^m), for every lookup (blockIdx.y); TWO: and the
+// layer above that, whose parent (b, x) has the parents (b, x) and (b, x + 2^(m-1)): a thread per parent of the last layer.
+// Two layers in a launch take the middle one from registers: trees of 2^22 and 2^16 leaves, above the last nine
+// layers, 117 us in 20 launches one at a time, 94 in 11.
+struct ReduceArgs {
+  const uint32_t *p[REDUCE_MAXL], *q[REDUCE_MAXL];
+  uint32_t *pp[REDUCE_MAXL][2], *qq[REDUCE_MAXL][2];
+  uint32_t m;
+  uint64_t n_out;  // parents of the last layer, over all blocks
+};
+template <int D, bool TWO>
+__global__ __launch_bounds__(BLOCK) void gkr_reduce_kernel(ReduceArgs a) {
+  const uint64_t o = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+  const uint32_t l = blockIdx.y;
+  if (o >= a.n_out) return;
+  const uint32_t top = TWO ? a.m - 1 : a.m;  // the last layer's
+  const uint64_t half = (uint64_t)1 << a.m, b = o >> top, x = o & (((uint64_t)1 << top) - 1), c0 = (b << (a.m + 1)) + x;
+  const Fraction<D> f0 = load_fraction<D>(a.p[l], a.q[l], c0), f1 = load_fraction<D>(a.p[l], a.q[l], c0 + half);
+  if constexpr (TWO) {
+    const uint64_t quarter = half / 2, at = (b << a.m) + x;
+    const Fraction<D> f2 = load_fraction<D>(a.p[l], a.q[l], c0 + quarter), f3 = load_fraction<D>(a.p[l], a.q[l], c0 + half + quarter);
+    const Fraction<D> g0 = add_fractions<D>(f0, f1), g1 = add_fractions<D>(f2, f3);
+    store_fraction<D>(a.pp[l][0], a.qq[l][0], at, g0);
+    store_fraction<D>(a.pp[l][0], a.qq[l][0], at + quarter, g1);
+    store_fraction<D>(a.pp[l][1], a.qq[l][1], o, add_fractions<D>(g0, g1));
+  } else {
+    store_fraction<D>(a.pp[l][0], a.qq[l][0], o, add_fractions<D>(f0, f1));
+  }
 }
 
 // The layers m_top .. 0 of a block of a lookup's tree, in one workgroup (block blockIdx.x of lookup blockIdx.y): layer m
 // has 2^m <= BLOCK parents, a thread takes one, and the workgroup's barrier stands between a layer's writes and the next
 // one's reads.  (A launch per layer is 4 us each for a few hundred products.)
 constexpr int REDUCE_TOP_LAYERS = 9;     // m_top <= 8: 256 parents
-constexpr int REDUCE_MAXL = MAXT / 4;    // lookups: four tables each
 struct ReduceTopArgs {
   // layer m_top + 1; where the tree over the block index begins, `valid` roots (the others are 0 / 1) that go to pad_p,
   // pad_q with them (else null: every child is there)
@@ -64,13 +98,8 @@ __global__ __launch_bounds__(BLOCK) void gkr_reduce_top_kernel(ReduceTopArgs a) 
     const uint32_t half = 1u << m, x = threadIdx.x;
     const uint64_t o = ((uint64_t)b << m) + x, c0 = ((uint64_t)b << (m + 1)) + x;
     if (x < half) {
-      Ext<D> p0 = load_ext<D>(p + c0 * D), p1 = load_ext<D>(p + (c0 + half) * D);
-      Ext<D> q0 = load_ext<D>(q + c0 * D), q1 = load_ext<D>(q + (c0 + half) * D);
-      Ext<D> q1r, q0r;
-#pragma unroll
-      for (int c = 0; c < D; c++) q1r.c[c] = mont_mul(q1.c[c], R2), q0r.c[c] = mont_mul(q0.c[c], R2);
-      store_ext<D>(a.pp[l][m] + o * D, ext_add<D>(ext_mul_mont<D>(p0, q1r), ext_mul_mont<D>(p1, q0r)));
-      store_ext<D>(a.qq[l][m] + o * D, ext_mul_mont<D>(q0, q1r));
+      const Fraction<D> f0 = load_fraction<D>(p, q, c0), f1 = load_fraction<D>(p, q, c0 + half);
+      store_fraction<D>(a.pp[l][m], a.qq[l][m], o, add_fractions<D>(f0, f1));
     }
     __threadfence();
     __syncthreads();
@@ -78,18 +107,24 @@ __global__ __launch_bounds__(BLOCK) void gkr_reduce_top_kernel(ReduceTopArgs a) 
   }
 }
 
-int gkr_reduce_layer(int D, int K, int m, const uint32_t *p, const uint32_t *q, uint32_t *pp, uint32_t *qq) {
+static int launch_reduce(int D, int K, int L, bool two, ReduceArgs &a) {
   Context &c = ctx();
-  int status = c.require();
-  if (status) return status;
-  uint64_t n_out = (uint64_t)K << m;
-  uint32_t grid = (uint32_t)((n_out + BLOCK - 1) / BLOCK);
+  a.n_out = (uint64_t)K << (two ? a.m - 1 : a.m);
+  const dim3 grid((uint32_t)((a.n_out + BLOCK - 1) / BLOCK), (uint32_t)L);
   if (D == 4)
-    hipLaunchKernelGGL(gkr_reduce_kernel<4>, dim3(grid), dim3(BLOCK), 0, c.stream, p, q, pp, qq, (uint32_t)m, n_out);
+    hipLaunchKernelGGL((two ? gkr_reduce_kernel<4, true> : gkr_reduce_kernel<4, false>), grid, dim3(BLOCK), 0, c.stream, a);
   else
-    hipLaunchKernelGGL(gkr_reduce_kernel<8>, dim3(grid), dim3(BLOCK), 0, c.stream, p, q, pp, qq, (uint32_t)m, n_out);
+    hipLaunchKernelGGL((two ? gkr_reduce_kernel<8, true> : gkr_reduce_kernel<8, false>), grid, dim3(BLOCK), 0, c.stream, a);
   EXH_HIP(hipGetLastError());
   return OK;
+}
+int gkr_reduce_layer(int D, int K, int m, const uint32_t *p, const uint32_t *q, uint32_t *pp, uint32_t *qq) {
+  int status = ctx().require();
+  if (status) return status;
+  ReduceArgs a;
+  memset(&a, 0, sizeof(a));
+  a.p[0] = p, a.q[0] = q, a.pp[0][0] = pp, a.qq[0][0] = qq, a.m = (uint32_t)m;
+  return launch_reduce(D, K, 1, false, a);
 }
 
 // the lower and upper halves of each block, as K contiguous blocks each (HALVES-PER-BLOCK,
@@ -326,9 +361,9 @@ static int prove_upper_chained(Transcript &tr, int n, int K, int lk, int L, cons
     return E_NOMEM;
   }
   const DevB3S first = device_state(tr);
-  EXH_HIP(hipMemcpyAsync(&chain->tr, &first, sizeof(first), hipMemcpyHostToDevice, c.stream));
-  // (a fill kernel would do as well; the chain is never captured into a graph)
-  EXH_HIP(hipMemsetAsync(&chain->failed, 0, sizeof(chain->failed), c.stream));
+  // the log comes to the host as the loop's logs of a single sumcheck do (three copies and a wait on the stream are 40 us)
+  const bool deliver = c.host_pinned_dev && !c.profiling && words + sizeof(DevB3S) / 4 + 2 <= PIN_DOWN_WORDS;
+  volatile uint32_t *flag = c.host_pinned + PIN_DOWN + words + sizeof(DevB3S) / 4 + 1;
   const std::vector<int> strides(NT + 1, D);
   const std::vector<uint32_t> no_point((size_t)std::max(n, lk) * D, 0), no_consts((size_t)2 * L * D, 0), no_bw((size_t)K * D, 0);
   std::vector<const uint32_t *> blk_tabs(NT + 1, nullptr);
@@ -362,7 +397,7 @@ static int prove_upper_chained(Transcript &tr, int n, int K, int lk, int L, cons
     memset(&a, 0, sizeof(a));
     a.chain = chain, a.L = L, a.NT = NT, a.K = 1;
     if (i == 0) {
-      a.close_kind = 1, a.log = d_log;
+      a.close_kind = 1, a.log = d_log, a.start = first;
       for (int t = 0; t < 2 * L; t++) a.tabs[t] = tables.roots[t];
     } else {
       const Step &prev = steps[i - 1];
@@ -376,6 +411,11 @@ static int prove_upper_chained(Transcript &tr, int n, int K, int lk, int L, cons
       if (prev.kind == BLOCKS) a.fin_skip = 1, a.blocks_closed = 1, a.tt_at = prev.layer;
     }
     if (i == steps.size()) {
+      if (deliver) {
+        if (++c.log_seq == 0) ++c.log_seq;  // 0 is what the flag is reset to
+        a.log_all = d_log, a.log_words = (uint32_t)words, a.host_log = c.host_pinned_dev + PIN_DOWN, a.host_seq = c.log_seq;
+        *flag = 0;
+      }
       if ((status = launch_glue<D>(a, &held, held_kernels))) return status;
       break;
     }
@@ -425,14 +465,33 @@ static int prove_upper_chained(Transcript &tr, int n, int K, int lk, int L, cons
     prev_ctrl = s.d_ctrl;
     prev_tabs = s.cur;
   }
-  // ---- one wait, then the log
+  // ---- one wait, then the log: polled in pinned memory, where the last step wrote it, or copied
   std::vector<uint32_t> log(words);
   DevB3S last;
   uint32_t failed = 0;
-  EXH_HIP(hipMemcpyAsync(log.data(), d_log, words * 4, hipMemcpyDeviceToHost, c.stream));
-  EXH_HIP(hipMemcpyAsync(&last, &chain->tr, sizeof(last), hipMemcpyDeviceToHost, c.stream));
-  EXH_HIP(hipMemcpyAsync(&failed, &chain->failed, sizeof(failed), hipMemcpyDeviceToHost, c.stream));
-  EXH_HIP(hipStreamSynchronize(c.stream));
+  if (deliver) {
+    // (a stream that ends without raising the flag, or is in an error state, ends the polling)
+    uint32_t spins = 0;
+    while (*flag != c.log_seq)
+      if ((++spins & 1023) == 0 && hipStreamQuery(c.stream) != hipErrorNotReady) break;
+    if (*flag != c.log_seq) {
+      EXH_HIP(hipStreamSynchronize(c.stream));
+      if (*flag != c.log_seq) {
+        set_error("device-error: the chained layers ended without delivering their log");
+        return E_DEVICE;
+      }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    const uint32_t *down = c.host_pinned + PIN_DOWN;
+    memcpy(log.data(), down, words * 4);
+    memcpy(&last, down + words, sizeof(last));
+    failed = down[words + sizeof(last) / 4];
+  } else {
+    EXH_HIP(hipMemcpyAsync(log.data(), d_log, words * 4, hipMemcpyDeviceToHost, c.stream));
+    EXH_HIP(hipMemcpyAsync(&last, &chain->tr, sizeof(last), hipMemcpyDeviceToHost, c.stream));
+    EXH_HIP(hipMemcpyAsync(&failed, &chain->failed, sizeof(failed), hipMemcpyDeviceToHost, c.stream));
+    EXH_HIP(hipStreamSynchronize(c.stream));
+  }
   if ((status = chain_outcome(failed))) return status;
   // the messages as they were sent, recorded without hashing them again; the transcript takes the device's state
   uint64_t dims[2] = {2, (uint64_t)D};
@@ -493,12 +552,22 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
       uint64_t words = ((uint64_t)K << m) * D;
       uint32_t *pp = next, *qq = next + words;
       next += 2 * words;
-      if (m > m_top &&
-          (status = gkr_reduce_layer(D, K, m, layers[m + 1][2 * l], layers[m + 1][2 * l + 1], pp, qq)))
-        return status;
       layers[m][2 * l] = pp;
       layers[m][2 * l + 1] = qq;
     }
+  for (int m = n - 1; m > m_top;) {
+    const bool two = m - 1 > m_top;
+    ReduceArgs a;
+    memset(&a, 0, sizeof(a));
+    a.m = (uint32_t)m;
+    for (int l = 0; l < L; l++) {
+      a.p[l] = layers[m + 1][2 * l], a.q[l] = layers[m + 1][2 * l + 1];
+      for (int k = 0; k < (two ? 2 : 1); k++)
+        a.pp[l][k] = const_cast<uint32_t *>(layers[m - k][2 * l]), a.qq[l][k] = const_cast<uint32_t *>(layers[m - k][2 * l + 1]);
+    }
+    if ((status = launch_reduce(D, K, L, two, a))) return status;
+    m -= two ? 2 : 1;
+  }
   auto reduce_top = [&](const ReduceTopArgs &a, int blocks) {
     if (D == 4)
       hipLaunchKernelGGL(gkr_reduce_top_kernel<4>, dim3(blocks, L), dim3(BLOCK), 0, c.stream, a);
@@ -576,9 +645,7 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
     }
     status = D == 4 ? prove_upper_chained<4>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq)
                     : prove_upper_chained<8>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq);
-    if (status) return status;
-    EXH_HIP(hipStreamSynchronize(c.stream));
-    return OK;
+    return status;
   }
   // the per-block roots, and the top tree over the block index on the host (2^lk entries)
   std::vector<std::vector<std::vector<uint32_t>>> top(lk + 1, std::vector<std::vector<uint32_t>>(2 * L));

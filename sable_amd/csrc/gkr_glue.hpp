@@ -53,6 +53,12 @@ struct GlueArgs {
   uint32_t *factors, *mtilde, *c0;
   Ctrl *ctrl;
   int points, nacc, c0_words;
+  DevB3S start;  // kind 1: the transcript's state
+  // the last step of a chain: the whole log (log_words at log_all), the transcript's state and the sticky word go to pinned
+  // host memory, then host_seq to the word behind them (null: the host copies them)
+  const uint32_t *log_all;
+  uint32_t log_words, host_seq;
+  uint32_t *host_log;
   uint32_t lagfix[MAXPTS * MAXACC];
   uint8_t acc_const[MAXACC];  // the constant (a_l: 2 l, a_l lambda: 2 l + 1) that is the accumulator's group coefficient
 };
@@ -89,12 +95,14 @@ __device__ __forceinline__ void gkr_glue_body(const GlueArgs<D> &a) {
   RunB3S tr;
   {  // the transcript's state where the last launch (or this one's rounds) left it
     const uint32_t *g = reinterpret_cast<const uint32_t *>(from_ctrl ? &a.prev_ctrl->tr : &a.chain->tr);
-    if (lane < sizeof(DevB3S) / 4) buf[lane] = fresh_word(g + lane);
+    if (lane < sizeof(DevB3S) / 4)
+      buf[lane] = a.close_kind == 1 ? reinterpret_cast<const uint32_t *>(&a.start)[lane] : fresh_word(g + lane);
     __builtin_amdgcn_wave_barrier();
     rb3s_load(tr, ring, reinterpret_cast<const DevB3S *>(buf));
   }
   __builtin_amdgcn_wave_barrier();
   if (a.close_kind == 1) {  // the roots: one message (2, D) per lookup
+    if (lane == 0) a.chain->failed = 0;
     for (int l = 0; l < a.L; l++) {
       if (lane < 2 * D) buf[lane] = a.tabs[2 * l + lane / D][lane % D];
       __builtin_amdgcn_wave_barrier();
@@ -206,6 +214,28 @@ __device__ __forceinline__ void gkr_glue_body(const GlueArgs<D> &a) {
     }
   }
   rb3s_store(tr, &a.chain->tr);
+  if (a.host_log) {
+    // (sixteen words a lane and trip to memory; what this wavefront stored a moment ago is read back through the L2)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const uint32_t state_words = sizeof(DevB3S) / 4, total = a.log_words + state_words + 1;
+    const uint32_t *state = reinterpret_cast<const uint32_t *>(&a.chain->tr);
+    for (uint32_t base = 0; base < total; base += 16 * 64) {
+      uint32_t w[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        const uint32_t u = base + 64 * k + lane;
+        w[k] = fresh_word(u < a.log_words                 ? a.log_all + u
+                          : u < a.log_words + state_words ? state + (u - a.log_words)
+                                                          : &a.chain->failed);
+      }
+#pragma unroll
+      for (int k = 0; k < 16; k++)
+        if (base + 64 * k + lane < total) a.host_log[base + 64 * k + lane] = w[k];
+    }
+    __threadfence_system();
+    if (lane == 0)
+      __hip_atomic_store(a.host_log + total, a.host_seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 template <int D>

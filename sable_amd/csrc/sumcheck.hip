@@ -144,7 +144,7 @@ constexpr uint32_t SLICE_GROUPS = 16;  // rows of totals per round of a grid lau
 constexpr uint32_t ROUND_GROUPS = 32;  // rows of totals of a streaming round (its workgroups' atomics spread over them)
 constexpr size_t PIN_BEGIN = 16384, PIN_BEGIN_WORDS = 4096;
 constexpr size_t PIN_LOOP = PIN_BEGIN + PIN_BEGIN_WORDS, PIN_LOOP_WORDS = 12288;
-constexpr size_t PIN_DOWN = PIN_LOOP + PIN_LOOP_WORDS, PIN_DOWN_WORDS = 32768;
+static_assert(PIN_DOWN == PIN_LOOP + PIN_LOOP_WORDS, "the regions follow one another");
 static inline uint32_t next_pow2(uint64_t v) {
   uint32_t p = 1;
   while (p < v) p <<= 1;

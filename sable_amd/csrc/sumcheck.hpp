@@ -27,6 +27,8 @@ struct KernelSet {  // the launchers generated for one statement and one degree 
   // the step between two layers (TailArgs<D>, GlueArgs<D>)
   std::function<void(const void *tail_args, const void *step_args, hipStream_t stream)> launch_tail_glue;
 };
+// the part of the context's pinned buffer (in words) where a device-driven loop's logs land
+constexpr size_t PIN_DOWN = 32768, PIN_DOWN_WORDS = 32768;
 // EQ-TABLE of k coordinates (canonical, host) into 2^k elements of device memory
 int eq_table_device(int D, int k, const uint32_t *r, uint32_t *d_out);
 // eq tables over ranges of a point's variables in one launch (see sumcheck.hip)
