@@ -13,6 +13,7 @@
 #include "blake3.hpp"
 #include "context.hpp"
 #include "hostfield.hpp"
+#include "prover.hpp"
 #include "sumcheck.hpp"
 #include "sumcheck_kernels.hpp"
 
@@ -1095,6 +1096,21 @@ int open_queries_device(const uint32_t *d_codewords, int ncols, int c, const uin
 // pass; the others fold the codeword (RS:FOLD, src/rs.lisp:93-101).  The sums meet in counted totals (RoundTotals)
 // and the last summing workgroup to arrive writes them into pinned host memory and raises a flag there, so the
 // host neither copies nor waits on the stream: it polls the flag while the codeword's workgroups still run.
+// A round whose message and challenge the device takes care of: what the elected workgroup's first wavefront needs for
+// that, and where it leaves the results.
+struct BfRound {
+  DevB3S state;        // the transcript before the message
+  uint32_t c[3][8];    // message k = c_k (h_k + ysum), h_2 = 2 h_1 - h_0; times R
+  uint32_t ysum[8];
+  uint32_t *r_out;     // the challenge times R, for the launches behind this one (device memory; null: the host's round)
+  // pinned host memory: the message's 24 words, the challenge's 8, the transcript's state behind it, and a status word
+  // (1: the totals did not complete), as 64-bit words (host_seq << 32 | value)
+  unsigned long long *host_log;
+  uint32_t host_seq;
+};
+constexpr uint32_t BF_LOG_WORDS = 24 + 8 + sizeof(DevB3S) / 4 + 1;
+static_assert(BF_LOG_WORDS <= 64, "a word a lane");
+
 struct BfStepArgs {
   // the message table's part: workgroups [0, tt_blocks)
   const uint32_t *tt_in;  // 4 entries per pair when folding, else 2
@@ -1103,7 +1119,9 @@ struct BfStepArgs {
   uint64_t n_pairs;  // pairs after the fold
   uint32_t low_bits, pairs_per_thread, fold, do_sums, tt_blocks;
   uint32_t r_mont[8];
+  const uint32_t *r_dev;  // the fold's challenge, times R, where the device's round left it (null: r_mont)
   RoundTotals totals;
+  BfRound round;
   // 17 64-bit words in pinned host memory, each (host_seq << 32 | value): h0, h1, then 1 when the totals never
   // completed.  Every word says itself that it has arrived, so no fence orders them: a release at system scope
   // writes back the whole L2 of the elected workgroup's XCD, which the fold's stores of the other workgroups keep
@@ -1116,20 +1134,89 @@ struct BfStepArgs {
   uint64_t cw_m;  // elements after the fold
 };
 
-// The sums of a step's workgroup -> totals -> (last workgroup) pinned host memory.  `mine`: the workgroup's `width`
-// words; host_out receives them and a status word, see BfStepArgs.
-__device__ __forceinline__ void bf_deliver_sums(const RoundTotals &totals, const uint32_t *mine, uint32_t width,
-                                                uint32_t workgroups, unsigned long long *host_out, uint32_t host_seq) {
+// the challenge that a step folds by
+__device__ __forceinline__ Ext<8> bf_challenge(const BfStepArgs &a) {
+  Ext<8> r;
+  const uint32_t *from = a.r_dev ? a.r_dev : a.r_mont;
+#pragma unroll
+  for (int c = 0; c < 8; c++) r.c[c] = from[c];
+  return r;
+}
+
+// What the first wavefront fetches for a device's round before the sums' exchange, which hides the trip.
+struct BfRoundWords {
+  uint32_t c, ysum, state;
+};
+__device__ __forceinline__ BfRoundWords bf_round_fetch(const BfRound &r) {
+  const uint32_t lane = threadIdx.x & 63;
+  return {(&r.c[0][0])[lane < 24 ? lane : 0], r.ysum[lane % 8],
+          reinterpret_cast<const uint32_t *>(&r.state)[lane < sizeof(DevB3S) / 4 ? lane : 0]};
+}
+// A round's end on the device (the elected workgroup's first wavefront; sums: h0 and h1 in LDS, 16 words): its message from
+// the sums, through the transcript, to the challenge, which goes to device memory for the launches that are already queued
+// behind this one and with the message and the transcript's state to the host, which records them.
+__device__ __forceinline__ void bf_round_end(const BfRound &r, const BfRoundWords &words, const uint32_t *sums) {
+  struct Lds {
+    uint32_t chal[8], r_mont[8];
+  };
+  __shared__ Lds lds;
+  __shared__ uint32_t ring[RING_WORDS], map[24], value[3][16];  // map and values in powers of w; the values' triples behind them
+  __shared__ DevB3S state;
+  const uint32_t lane = threadIdx.x, power = __brev(lane % 8) >> 29;
+  if (lane < 24) {
+    map[lane / 8 * 8 + power] = words.c;
+    const uint32_t h0 = sums[lane % 8], h1 = sums[8 + lane % 8], k = lane / 8;
+    const uint32_t v = fadd(k == 0 ? h0 : k == 1 ? h1 : fsub(fdbl(h1), h0), words.ysum);
+    value[k][power] = v, value[k][8 + power] = times3(v);
+  }
+  if (lane < sizeof(DevB3S) / 4) reinterpret_cast<uint32_t *>(&state)[lane] = words.state;
+  __builtin_amdgcn_wave_barrier();
+  RunB3S tr;
+  PendingAppend pending{0, 0, 0};
+  rb3s_load(tr, ring, &state);
+  const MessageLane<8> ml = message_lane<8>(3);
+  const uint32_t o = ml.o < 24 ? ml.o : 23, e = __brev(o % 8) >> 29;
+  uint64_t t = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < 8; i++) {
+    if (i >= 4 && i % 2 == 0) t = mont_lazy(t);
+    t += (uint64_t)map[o / 8 * 8 + i] * value[o / 8][((e - i) & 7) + (i > e ? 8 : 0)];
+  }
+  const uint32_t word = mont_reduce4(t);
+  transcript_step<8>(tr, nullptr, 0, 3, &lds, ml, word, pending, false, false, [&] {
+    __builtin_amdgcn_wave_barrier();
+    if (lane < 8) r.r_out[lane] = lds.r_mont[lane];
+  });
+  rb3s_flush(tr, pending);
+  rb3s_store(tr, &state);
+  if (ml.part == 0 && ml.o < 24) map[ml.o] = word;
+  __builtin_amdgcn_wave_barrier();
+  const uint32_t out = lane < 24   ? map[lane]
+                       : lane < 32 ? lds.chal[lane - 24]
+                       : lane < BF_LOG_WORDS - 1 ? reinterpret_cast<const uint32_t *>(&state)[lane - 32] : 0u;
+  if (lane < BF_LOG_WORDS)
+    __hip_atomic_store(r.host_log + lane, ((unsigned long long)r.host_seq << 32) | out, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The sums of a step's workgroup -> totals; the sums over all workgroups (LDS) in the one that arrives last, null in the
+// others.  `mine`: the workgroup's `width` words; *ok is false when the totals did not complete.
+__device__ __forceinline__ const uint32_t *bf_elect(const RoundTotals &totals, const uint32_t *mine, uint32_t width,
+                                                    uint32_t workgroups, bool *ok) {
   __shared__ uint32_t sums[64];
   __shared__ uint32_t scratch[TOTALS_POLLS * BLOCK];
+  *ok = true;
+  if (workgroups == 1) return mine;  // nobody to wait for
+  return add_and_elect(totals, mine, width, scratch, sums, ok, 0, width, workgroups - 1, workgroups) ? sums : nullptr;
+}
+
+// ... and to pinned host memory; host_out receives the words and a status word, see BfStepArgs.
+__device__ __forceinline__ void bf_deliver_sums(const RoundTotals &totals, const uint32_t *mine, uint32_t width,
+                                                uint32_t workgroups, unsigned long long *host_out, uint32_t host_seq) {
   const uint32_t tid = threadIdx.x;
-  bool ok = true;
-  const uint32_t *from = sums;
-  if (workgroups == 1)
-    from = mine;  // nobody to wait for
-  else if (!add_and_elect(totals, mine, width, scratch, sums, &ok, 0, width, workgroups - 1, workgroups))
-    return;
-  if (tid <= width) {
+  bool ok;
+  const uint32_t *from = bf_elect(totals, mine, width, workgroups, &ok);
+  if (from && tid <= width) {
     const uint32_t value = tid < width ? (ok ? from[tid] : 0u) : (ok ? 0u : 1u);
     __hip_atomic_store(host_out + tid, ((unsigned long long)host_seq << 32) | value, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1141,6 +1228,8 @@ __device__ __forceinline__ void bf_finish_sums(const BfStepArgs &a, AccLazy (*ac
   __shared__ uint32_t lds[BLOCK / 64][16];
   __shared__ uint32_t mine[16];
   const uint32_t tid = threadIdx.x, lane = tid & 63;
+  BfRoundWords words{0, 0, 0};
+  if (a.round.r_out) words = bf_round_fetch(a.round);
   const uint32_t total = wave_sums_transposed<16>([&](int k) -> uint32_t { return acc_reduce(acc[k / 8][k % 8]); });
   if (transposed_writer<16>(lane)) lds[tid >> 6][transposed_word<16>(lane)] = total;
   __syncthreads();
@@ -1159,7 +1248,18 @@ __device__ __forceinline__ void bf_finish_sums(const BfStepArgs &a, AccLazy (*ac
     for (int c = 0; c < 8; c++) mine[tid * 8 + c] = mont_mul(t.c[c], R2);
   }
   __syncthreads();
-  bf_deliver_sums(a.totals, mine, 16, a.tt_blocks, a.host_out, a.host_seq);
+  if (!a.round.r_out) {
+    bf_deliver_sums(a.totals, mine, 16, a.tt_blocks, a.host_out, a.host_seq);
+    return;
+  }
+  bool ok;
+  const uint32_t *sums = bf_elect(a.totals, mine, 16, a.tt_blocks, &ok);
+  if (!sums || tid >= 64) return;
+  if (ok)
+    bf_round_end(a.round, words, sums);
+  else if (tid < BF_LOG_WORDS)
+    __hip_atomic_store(a.round.host_log + tid, ((unsigned long long)a.round.host_seq << 32) | (tid == BF_LOG_WORDS - 1 ? 1u : 0u),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // RS:FOLD of one element: pair (a, b) at twiddle x: f0 = (a + b)/2, f1 = (a - b)/(2x), f0 + r (f1 - f0)
@@ -1174,9 +1274,7 @@ __device__ __forceinline__ void bf_fold_codeword(const BfStepArgs &a, const Ext<
 template <bool FOLD>
 __global__ __launch_bounds__(BLOCK) void bf_step_kernel(BfStepArgs a) {
   const uint32_t tid = threadIdx.x;
-  Ext<8> r;
-#pragma unroll
-  for (int c = 0; c < 8; c++) r.c[c] = a.r_mont[c];
+  const Ext<8> r = bf_challenge(a);
   if (blockIdx.x >= a.tt_blocks) {
     bf_fold_codeword(a, r, (uint64_t)(blockIdx.x - a.tt_blocks) * BLOCK + tid);
     return;
@@ -1468,7 +1566,9 @@ static_assert(BF_PIN + BF_MAX_ROUNDS * BF_ROUND_SLOT + BF_MAX_ORACLES * BF_CAP_S
 constexpr size_t BF_CLASS_PIN = 65536, BF_CLASS_SLOT = 136, BF_MAX_CLASSES = 32;
 constexpr size_t BF_FACTOR_PIN = BF_CLASS_PIN + BF_MAX_CLASSES * BF_CLASS_SLOT, BF_FACTOR_WORDS = 512;
 constexpr size_t GATHER_PIN = BF_FACTOR_PIN + BF_FACTOR_WORDS, GATHER_QUADS = 8192;
-static_assert(GATHER_PIN + 10 * GATHER_QUADS <= ((size_t)1 << 18), "the pinned buffer");
+constexpr size_t BF_LOG_PIN = GATHER_PIN + 10 * GATHER_QUADS, BF_LOG_SLOT = 128;  // a slot per round that the device ends
+static_assert(BF_LOG_PIN + BF_MAX_ROUNDS * BF_LOG_SLOT <= ((size_t)1 << 18) && 2 * BF_LOG_WORDS <= BF_LOG_SLOT, "the pinned buffer");
+static_assert(BF_LOG_PIN % 2 == 0, "64-bit words");
 static_assert(GATHER_PIN % 2 == 0 && BF_CLASS_SLOT % 2 == 0, "64-bit words");
 constexpr uint32_t BF_GROUPS = 32;  // rows of totals of a round's sums (16 words each) and of a class's (64 words)
 
@@ -1698,6 +1798,23 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     dom = d;
   }
   std::vector<OracleTree> oracles;
+  // Odd rounds end on the device: their message waits for no oracle's cap, so the launch that sums round i can send it and
+  // draw the challenge, and the launches of level i + 1, its oracle's tree among them, are queued behind it at once -- one
+  // trip to the host for two rounds.  (A cap is 4 KiB for the transcript, 64 compressions one after the other: 38 us on a
+  // wavefront, so the rounds behind a cap stay the host's.)  An opening with every round on the host (EXACTA_HIP_HOST_ROUNDS=1)
+  // and this way, us: two columns of 2^23 and one of 2^19 969 and 922, two of 2^18 478 and 425, three classes up to 2^14
+  // with the verification 629 and 583.
+  const char *host_rounds = getenv("EXACTA_HIP_HOST_ROUNDS");
+  const bool device_rounds = !(host_rounds && host_rounds[0] == '1');
+  auto on_device = [&](int i) { return device_rounds && i % 2 == 1 && i >= std::max(BB, 1) && i < fl; };
+  uint32_t *challenges = mem.alloc((uint64_t)std::max(fl, 1) * 8);
+  if (!challenges) return E_NOMEM;
+  hf::E prf = hf::lift(1, 8), claim = hf::from(v, 8), ysum = hf::zero(8);  // ysum: the classes still to join, :593-595
+  // eq of round i's coordinate at X = 0, 1, 2
+  auto eq_at = [&](int i, hf::E eqx[3]) {
+    const hf::E ri = hf::from(rr + 8 * (size_t)i, 8);
+    eqx[0] = hf::sub(hf::lift(1, 8), ri), eqx[1] = ri, eqx[2] = hf::sub(hf::scale(ri, 2), eqx[0]);
+  };
   auto launch_step = [&](int i, bool fold, bool do_sums, uint32_t *cw_out) -> int {
     BfBaseArgs b;
     memset(&b, 0, sizeof(b));
@@ -1715,8 +1832,23 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     }
     a.pairs_per_thread = std::max<uint32_t>(1, (uint32_t)(tile / BLOCK));
     a.tt_blocks = tt_part ? (uint32_t)((n_pairs + tile - 1) / tile) : 0;
-    if (!xs.empty())
+    if (fold && on_device(i - 1))
+      a.r_dev = challenges + 8 * (size_t)(i - 1);
+    else if (fold)
       for (int k = 0; k < 8; k++) a.r_mont[k] = to_mont(xs.back()[k]);
+    if (a.do_sums && on_device(i)) {
+      hf::E eqx[3];
+      eq_at(i, eqx);
+      BfRound &r = a.round;
+      r.state = device_state(tr);
+      for (int q = 0; q < 3; q++) {
+        const hf::E m = hf::mul(prf, eqx[q]);
+        for (int k = 0; k < 8; k++) r.c[q][k] = to_mont(m[k]);
+      }
+      for (int k = 0; k < 8; k++) r.ysum[k] = ysum[k];
+      r.r_out = challenges + 8 * (size_t)i, r.host_seq = seq;
+      r.host_log = reinterpret_cast<unsigned long long *>(c.host_pinned_dev + BF_LOG_PIN + (size_t)i * BF_LOG_SLOT);
+    }
     if (a.do_sums) {
       a.totals = RoundTotals{totals64 + (uint64_t)i * BF_GROUPS * 16, arrivals + i, groups_of(a.tt_blocks), 16, 200000};
       a.host_out = reinterpret_cast<unsigned long long *>(pin_dev + (size_t)i * BF_ROUND_SLOT), a.host_seq = seq;
@@ -1782,9 +1914,8 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
   } else if (fl > 0 && (status = launch_step(0, false, true, nullptr))) {
     return status;
   }
-  // y_c = H_c at the point's last c coordinates, for the classes still to join; ysum their sum (:593-595)
+  // y_c = H_c at the point's last c coordinates, for the classes still to join
   std::vector<hf::E> yc(ncls, hf::zero(8));
-  hf::E ysum = hf::zero(8);
   auto small_table = [&](int k) { return src[k].h && nv - cls[k] >= fl; };  // no round has its weights: 2^5 elements at most
   for (int k = 0; k + 1 < ncls; k++)
     if (!small_table(k) && (status = launch_class_sums(k))) return status;
@@ -1808,52 +1939,57 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     ysum = hf::add(ysum, yc[k]);
   }
 
-  hf::E prf = hf::lift(1, 8), claim = hf::from(v, 8);
   std::vector<hf::E> open_t;  // the sums over the open variables, folded by the challenges so far
   if (base && (status = open_sums(ncls - 1, &open_t))) return status;
   size_t cap_slots = 0;
-  for (int i = 0; i < fl; i++) {
-    // ---- the round's message from h0, h1
-    hf::E h0, h1;
-    if (i < BB) {
-      std::vector<hf::E> even, odd;
-      for (size_t q = 0; q < open_t.size(); q += 2) even.push_back(open_t[q]), odd.push_back(open_t[q + 1]);
-      h0 = eq_fold(even, rr + 8 * (size_t)(i + 1)), h1 = eq_fold(odd, rr + 8 * (size_t)(i + 1));
-    } else {
-      uint32_t hh[17];
-      if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(pin + (size_t)i * BF_ROUND_SLOT), 17, seq,
-                       hh) ||
-          hh[16]) {
-        set_error("device-error: a basefold round's sums did not arrive");
-        return E_DEVICE;
-      }
-      h0 = hf::from(hh, 8), h1 = hf::from(hh + 8, 8);
-    }
-    const hf::E ri = hf::from(rr + 8 * (size_t)i, 8), one_r = hf::sub(hf::lift(1, 8), ri);
-    const hf::E eqx[3] = {one_r, ri, hf::sub(hf::scale(ri, 2), one_r)};
-    const hf::E hx[3] = {h0, h1, hf::sub(hf::scale(h1, 2), h0)};
-    uint32_t ev[24], x[8];
-    const hf::E a_term = ncls > 1 ? hf::mul(prf, ysum) : hf::zero(8);  // the classes still to join, :607-612
-    for (int parity = 0; parity < 3; parity++) {
-      hf::E t = hf::mul(hf::mul(prf, eqx[parity]), hx[parity]);
-      if (ncls > 1) t = hf::add(t, hf::mul(a_term, eqx[parity]));
-      memcpy(ev + 8 * parity, t.data(), 32);
-    }
-    uint64_t dims[2] = {3, 8};
-    if ((status = tr.send(ev, 2, dims, nullptr))) return status;
-    if (hf::add(hf::from(ev, 8), hf::from(ev + 8, 8)) != claim) {
-      set_error("verification-failure: pcs: basefold sumcheck round " + std::to_string(i) + " failed");
-      return E_REJECT;
-    }
-    tr.challenge(8, x);
+  // the round's claim, and what its message and challenge leave for the next
+  auto end_round = [&](int i, const uint32_t *ev, const uint32_t *x) {
     xs.push_back(hf::from(x, 8));
     if (out_chal) memcpy(out_chal + 8 * i, x, 32);
     claim = hf::lagrange({hf::from(ev, 8), hf::from(ev + 8, 8), hf::from(ev + 16, 8)}, xs.back());
     prf = hf::mul(prf, hf::eq1(hf::from(rr + 8 * i, 8), xs.back()));
-    if (i < BB) {
-      for (size_t q = 0; q < open_t.size() / 2; q++)
-        open_t[q] = hf::add(open_t[2 * q], hf::mul(xs.back(), hf::sub(open_t[2 * q + 1], open_t[2 * q])));
-      open_t.resize(open_t.size() / 2);
+  };
+  const uint64_t dims38[2] = {3, 8};
+  auto refuse_round = [&](int i) {
+    set_error("verification-failure: pcs: basefold sumcheck round " + std::to_string(i) + " failed");
+    return E_REJECT;
+  };
+  auto claim_holds = [&](const uint32_t *ev) { return hf::add(hf::from(ev, 8), hf::from(ev + 8, 8)) == claim; };
+  for (int i = 0; i < fl; i++) {
+    if (!on_device(i)) {
+      // ---- the round's message from h0, h1
+      hf::E h0, h1;
+      if (i < BB) {
+        std::vector<hf::E> even, odd;
+        for (size_t q = 0; q < open_t.size(); q += 2) even.push_back(open_t[q]), odd.push_back(open_t[q + 1]);
+        h0 = eq_fold(even, rr + 8 * (size_t)(i + 1)), h1 = eq_fold(odd, rr + 8 * (size_t)(i + 1));
+      } else {
+        uint32_t hh[17];
+        if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(pin + (size_t)i * BF_ROUND_SLOT), 17, seq,
+                         hh) ||
+            hh[16]) {
+          set_error("device-error: a basefold round's sums did not arrive");
+          return E_DEVICE;
+        }
+        h0 = hf::from(hh, 8), h1 = hf::from(hh + 8, 8);
+      }
+      hf::E eqx[3];
+      eq_at(i, eqx);
+      const hf::E hx[3] = {h0, h1, hf::sub(hf::scale(h1, 2), h0)};
+      uint32_t ev[24], x[8];
+      for (int parity = 0; parity < 3; parity++) {  // with the classes still to join, :607-612
+        const hf::E t = hf::mul(hf::mul(prf, eqx[parity]), hf::add(hx[parity], ysum));
+        memcpy(ev + 8 * parity, t.data(), 32);
+      }
+      if ((status = tr.send(ev, 2, dims38, nullptr))) return status;
+      if (!claim_holds(ev)) return refuse_round(i);
+      tr.challenge(8, x);
+      end_round(i, ev, x);
+      if (i < BB) {
+        for (size_t q = 0; q < open_t.size() / 2; q++)
+          open_t[q] = hf::add(open_t[2 * q], hf::mul(xs.back(), hf::sub(open_t[2 * q + 1], open_t[2 * q])));
+        open_t.resize(open_t.size() / 2);
+      }
     }
     // ---- level l: fold the table and the codeword by x; an oracle tree over the folded codeword; the joins
     const int l = i + 1;
@@ -1878,6 +2014,8 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     // the next round's sums ride on the fold unless a class joins in between
     const bool more = l < fl;
     if ((status = launch_step(l, true, more && !joins, cw_out))) return status;
+    size_t cap_at = 0;
+    uint64_t rows = 0;
     if (oracle) {  // an oracle tree over the folded codeword, its cap to the host behind a flag
       OracleTree o;
       o.level = l;
@@ -1887,12 +2025,31 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
       o.cw = cw_out;
       o.levels = mem.alloc((2 * o.nleaves) * 8);
       if (!o.levels) return E_NOMEM;
-      uint64_t rows = 0, cap_off = 0;
-      const size_t cap_at = BF_MAX_ROUNDS * BF_ROUND_SLOT + cap_slots * BF_CAP_SLOT;
+      uint64_t cap_off = 0;
+      cap_at = BF_MAX_ROUNDS * BF_ROUND_SLOT + cap_slots * BF_CAP_SLOT;
       if ((status = merkle_tree_launch(o.levels, o.nleaves, 2, o.cw, 1, o.cw_len, &rows, &cap_off,
                                        reinterpret_cast<unsigned long long *>(pin_dev + cap_at), seq)))
         return status;
       cap_slots++;
+      oracles.push_back(o);
+    }
+    if (on_device(i)) {  // its message and challenge, recorded as they were sent
+      uint32_t w[BF_LOG_WORDS];
+      const size_t at = BF_LOG_PIN + (size_t)i * BF_LOG_SLOT;
+      if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(c.host_pinned + at), BF_LOG_WORDS, seq, w) ||
+          w[BF_LOG_WORDS - 1]) {
+        set_error("device-error: a basefold round did not arrive");
+        return E_DEVICE;
+      }
+      const bool holds = claim_holds(w);
+      if ((status = tr.send(w, 2, dims38, nullptr, !holds))) return status;
+      if (!holds) return refuse_round(i);  // (the transcript as it stands on the host: the message sent, nothing drawn)
+      DevB3S state;
+      memcpy(&state, w + 32, sizeof(state));
+      if ((status = adopt_device_state(tr, state))) return status;
+      end_round(i, w, w + 24);
+    }
+    if (oracle) {
       std::vector<uint32_t> cap_words(8 * rows);
       if (!await_words(c, reinterpret_cast<const volatile unsigned long long *>(pin + cap_at), 8 * rows, seq,
                        cap_words.data())) {
@@ -1901,7 +2058,6 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
       }
       if ((status = tr.send_bytes(reinterpret_cast<const uint8_t *>(cap_words.data()), (int64_t)(32 * rows), nullptr)))
         return status;
-      oracles.push_back(o);
     }
     if (joins) {
       static const uint32_t one8[8] = {1, 0, 0, 0, 0, 0, 0, 0};

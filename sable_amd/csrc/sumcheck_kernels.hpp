@@ -742,9 +742,9 @@ __device__ __forceinline__ void triple_sums(uint32_t *sums, uint32_t width) {
 
 // The first wavefront's step: send the message whose words the lanes hold (what the last squeeze left to absorb and
 // the message's length go first, unless `prefixed` says that they went already), draw the challenge into e->chal and,
-// times R, e->r_mont, call `ready`, then log both.  What this squeeze leaves to absorb stays in `pending`.
-template <int D, class F>
-__device__ __forceinline__ void transcript_step(RunB3S &tr, Ctrl *ctrl, uint32_t round, uint32_t points, EpilogueLds *e,
+// times R, e->r_mont (LDS), call `ready`, then log both.  What this squeeze leaves to absorb stays in `pending`.
+template <int D, class Lds, class F>
+__device__ __forceinline__ void transcript_step(RunB3S &tr, Ctrl *ctrl, uint32_t round, uint32_t points, Lds *e,
                                                 const MessageLane<D> &ml, uint32_t word, PendingAppend &pending,
                                                 bool prefixed, bool log, F ready) {
   const uint32_t lane = threadIdx.x & 63, words = points * D;

@@ -59,6 +59,33 @@ def test_opening_matches_the_oracle_and_verifies(classes):
     free(dev)
 
 
+@pytest.mark.parametrize("classes", [
+    [(7, 1)], [(8, 1)],  # two rounds and three: a device's round that is the last one, and one before a last oracle
+    [(8, 9)], [(7, 9), (8, 9)], [(6, 1), (10, 9)],  # combined columns: the device's from round 1 on, joins on odd and even levels
+    [(6, 1), (7, 9), (11, 1)]])
+def test_rounds_that_end_on_the_device_and_on_the_host(classes, monkeypatch):
+    """Odd rounds end on the device, or all of them on the host: the oracle's proof and query positions, and the
+    transcript goes on the same way."""
+    nv = max(c for c, _ in classes)
+    both = [committed(c, ncols, 700 + 10 * c + ncols) for c, ncols in classes]
+    dev, host = [d for d, _ in both], [h for _, h in both]
+    rr = orc.splitmix_field(23 + nv, nv * 8).reshape(nv, 8)
+    v = np.zeros(8, np.uint32)
+    for key in host:
+        v = orc.ext_add(v, orc.mle_eval(key["h"], rr[nv - key["c"]:], 8))
+    otr = orc.Transcript("open", 4)
+    want = orc.pcs_open(otr, nv, host, rr, v, queries=5)
+    states = []
+    for on_host in ("0", "1"):
+        monkeypatch.setenv("EXACTA_HIP_HOST_ROUNDS", on_host)
+        tr = sa.Transcript("open", 4)
+        assert sa.pcs_open(tr, nv, dev, rr, v, queries=5) == want
+        assert tr.proof() == otr.proof()
+        states.append(tr.state_digest())
+    assert states[0] == states[1]
+    free(dev)
+
+
 def test_verify_queries_rejects_every_perturbed_message():
     classes = [(6, 2), (9, 2)]
     nv = 9
