@@ -45,7 +45,7 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "c5349eb646db9b036050b2b07e06e9fd638c42d707c8208d7d17e75f04878838",
+    "kernel_sources_sha256": "9789e8c2b7edc37f9afb2778e9d9fa4ad326f1ba3dfcb835616e9fbf0faa4d5d",
     "traffic": {("round_nodes_base", 24): 204089568, ("round_fold2_base", 24): 202987904, ("round_fold3_base", 24): 303140608},
     # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), and multiply-adds and multiplies of the
     # reductions of 344 in round 2 (2^21 pairs), 440 in round 3 (2^20) and 368 in the extension rounds (2^19 + 2^18 + ...)

@@ -348,7 +348,6 @@ long plan_groups(std::vector<Group> *groups, int points, int *nacc) {
   *nacc = 0;
   for (Group &g : *groups) {
     g.evalx.clear();
-    g.acc_base = *nacc;
     int d = (int)g.tabs.size();
     if (d == 0) continue;  // its sum is the sum of the weights: no device work
     if (points < 0)
@@ -359,9 +358,24 @@ long plan_groups(std::vector<Group> *groups, int points, int *nacc) {
     } else {  // degree d: d + 1 cheap points, extrapolated on the host
       for (int x = 0; x <= d; x++) g.evalx.push_back(x);
     }
-    *nacc += (int)g.evalx.size();
     cost += (long)g.evalx.size() * d;
   }
+  // groups of one coefficient and degree one after the other, as many as share accumulators
+  std::vector<Group> ordered;
+  std::vector<bool> taken(groups->size(), false);
+  for (size_t i = 0; i < groups->size(); i++) {
+    if (taken[i]) continue;
+    const int base = *nacc;
+    int terms = 0;
+    for (size_t k = i; k < groups->size() && terms < MAXTERMS; k++) {
+      Group &g = (*groups)[k];
+      if (taken[k] || g.tabs.size() != (*groups)[i].tabs.size() || !(g.parts == (*groups)[i].parts)) continue;
+      taken[k] = true, g.acc_base = base, g.follows = terms++ > 0;
+      ordered.push_back(g);
+    }
+    *nacc += (int)(*groups)[i].evalx.size();
+  }
+  groups->swap(ordered);
   return cost;
 }
 
@@ -473,7 +487,7 @@ std::string Statement::key() const {
     for (size_t i = 0; i < g.tabs.size(); i++) k += (i ? "," : "") + std::to_string(g.tabs[i]);
     k += "]@";
     for (size_t i = 0; i < g.evalx.size(); i++) k += (i ? "," : "") + std::to_string(g.evalx[i]);
-    k += ";";
+    k += g.follows ? "+" + std::to_string(g.acc_base) + ";" : ";";
   }
   return k;
 }
@@ -541,6 +555,9 @@ bool make_desc(const Statement &st, StmtDesc *out) {
       d.ev[g][k] = grp.evalx[k];
       if (grp.evalx[k] > maxx) maxx = grp.evalx[k];
     }
+    d.acc[g] = grp.acc_base, d.lead[g] = g;
+    for (int e = 0; e < g && grp.follows; e++)
+      if (d.lead[e] == e && d.acc[e] == grp.acc_base) d.lead[g] = e;
     g++;
   }
   d.G = g, d.nacc = st.nacc, d.maxx = maxx;
@@ -586,6 +603,10 @@ std::string desc_source(const StmtDesc &d, const std::string &name) {
   }
   o << "},\n    {";
   for (int v = 0; v < MAXV; v++) o << d.vconst[v] << "u" << (v + 1 < MAXV ? "," : "");
+  o << "},\n    {";
+  for (int g = 0; g < MAXG; g++) o << d.lead[g] << (g + 1 < MAXG ? "," : "");
+  o << "},\n    {";
+  for (int g = 0; g < MAXG; g++) o << d.acc[g] << (g + 1 < MAXG ? "," : "");
   o << "}};\n};\n";
   return o.str();
 }

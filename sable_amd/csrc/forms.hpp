@@ -30,12 +30,18 @@ struct Group {
   struct Part {
     uint32_t coeff;
     std::vector<int> consts;  // constant indices (with repetition)
+    bool operator==(const Part &o) const { return coeff == o.coeff && consts == o.consts; }
   };
   std::vector<Part> parts;
   // evaluation points of the group's round polynomial computed on the device (X values); the host
   // extrapolates to the wire points when the group's degree is below the statement's
   std::vector<int> evalx;
   int acc_base = 0;  // index of its first accumulator
+  // A group with the coefficient and the degree of the one before it shares that one's accumulators (as many as MAXTERMS in
+  // a row): the products are added up before they are reduced and weighed, and fewer words are summed and exchanged.  Two
+  // points' reduction of 2^19 at F_p^4 183 -> 175 us, of 2^21 267 -> 251; three blocks' trees of 2^14 and two lookups, whose
+  // layers have two products in three of one coefficient, 1245 -> 1215.
+  bool follows = false;
 };
 
 // A factor that is not a single table: sum of integer multiples of tables plus an integer, as in

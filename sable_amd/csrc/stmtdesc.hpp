@@ -9,12 +9,14 @@ constexpr int MAXVT = 4;    // tables per linear form
 constexpr int MAXG = 16;    // table groups per statement
 constexpr int MAXDEG = 6;   // tables per group
 constexpr int MAXEV = 6;    // evaluation points per group
+constexpr int MAXTERMS = 4; // groups that share accumulators
 constexpr int MAXACC = 36;  // accumulators (group, point) per statement
 constexpr int MAXX = 7;     // largest evaluation point
 constexpr int BLOCK = 256;  // threads per workgroup
 
 // A statement as the kernels see it: G groups, group g the product of the deg[g] factors tab[g][..],
-// evaluated at the nev[g] points ev[g][..]; accumulators are numbered group by group, point by point.
+// evaluated at the nev[g] points ev[g][..]; accumulators are numbered group by group, point by point, a group that
+// follows another (lead) having none of its own.
 // Factor t < T is table t; factor T + v is the linear form sum_k vcoef[v][k] * table vtab[v][k] + vconst[v]
 // (vcoef canonical and, for the kernels' products, in Montgomery form in vcoefm).
 struct StmtDesc {
@@ -28,6 +30,10 @@ struct StmtDesc {
   int vtab[MAXV][MAXVT];
   unsigned vcoef[MAXV][MAXVT], vcoefm[MAXV][MAXVT];
   unsigned vconst[MAXV];
+  // the first group with group g's accumulators (g itself, or one whose products g's are added to: at most MAXTERMS groups
+  // of one coefficient and degree, one after the other), and the first of those accumulators
+  int lead[MAXG];
+  int acc[MAXG];
 };
 
 #if defined(__HIPCC__)
@@ -36,6 +42,22 @@ struct StmtDesc {
 #define EXH_DESC_FN
 #endif
 
+// no group behind g shares g's accumulators (those that do follow one another)
+template <class Desc>
+EXH_DESC_FN constexpr bool group_is_last(const Desc &d, int g) {
+  return !(g + 1 < d.G && g + 1 < MAXG && d.lead[g + 1 < MAXG ? g + 1 : g] == d.lead[g]);
+}
+// the most groups that share an accumulator
+template <class Desc>
+EXH_DESC_FN constexpr int desc_terms(const Desc &d) {
+  int m = 1;
+  for (int g = 0; g < d.G; g++) {
+    int n = 0;
+    for (int h = g; h < d.G; h++) n += d.lead[h] == g ? 1 : 0;
+    m = n > m ? n : m;
+  }
+  return m;
+}
 // the largest number of factors in a group
 template <class Desc>
 EXH_DESC_FN constexpr int desc_maxdeg(const Desc &d) {
@@ -53,10 +75,11 @@ EXH_DESC_FN constexpr int ev_index(const Desc &d, int g, int x) {
     if (e < d.nev[g] && d.ev[g][e] == x) at = e;
   return at;
 }
-// per group: nev * (deg + 1) slots of round 1, then nev extras unless X = 1 is an evaluation point anyway
+// per group: nev * (deg + 1) slots of round 1, then nev extras unless X = 1 is an evaluation point anyway; a group that
+// follows another has none of its own
 template <class Desc>
 EXH_DESC_FN constexpr int group_slots(const Desc &d, int g) {
-  return d.nev[g] * (d.deg[g] + 1) + (ev_index(d, g, 1) < 0 ? d.nev[g] : 0);
+  return d.lead[g] != g ? 0 : d.nev[g] * (d.deg[g] + 1) + (ev_index(d, g, 1) < 0 ? d.nev[g] : 0);
 }
 template <class Desc>
 EXH_DESC_FN constexpr int node_slots(const Desc &d) {

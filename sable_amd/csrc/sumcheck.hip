@@ -662,10 +662,12 @@ static int launch_nodes_round(SumcheckSession &s, uint64_t n_pairs) {
   e.e.points = (uint32_t)s.points, e.e.mtilde = s.d_mtilde, e.e.c0 = s.d_c0;
   e.e.ctrl = s.d_ctrl;
   e.eq1 = s.has_eq ? s.d_weights + (size_t)2 * D : nullptr;  // the eq factors lead the arena: (w_v, 1 - w_v) per variable
-  e.groups = (uint32_t)s.desc.G, e.slots = (uint32_t)s.node_slots_n;
+  e.slots = (uint32_t)s.node_slots_n;
   for (int g = 0; g < s.desc.G; g++) {
-    e.deg[g] = (uint32_t)s.desc.deg[g], e.nev[g] = (uint32_t)s.desc.nev[g];
-    for (int k = 0; k < s.desc.nev[g]; k++) e.ev[g][k] = (uint8_t)s.desc.ev[g][k];
+    if (s.desc.lead[g] != g) continue;  // (its products are in the sums of the group it follows)
+    e.deg[e.groups] = (uint32_t)s.desc.deg[g], e.nev[e.groups] = (uint32_t)s.desc.nev[g];
+    for (int k = 0; k < s.desc.nev[g]; k++) e.ev[e.groups][k] = (uint8_t)s.desc.ev[g][k];
+    e.groups++;
   }
   fill_inv_den(e.inv_den);
   {
@@ -771,6 +773,7 @@ int SumcheckSession::round_sums(uint32_t *out) {
     hf::E total = hf::zero(D), one = hf::lift(1, D);
     for (size_t g = 0; g < st.groups.size(); g++) {
       const Group &grp = st.groups[g];
+      if (grp.follows) continue;
       hf::E coef(group_coef.begin() + g * D, group_coef.begin() + (g + 1) * D);
       if (grp.tabs.empty()) {
         total = hf::add(total, hf::mul(coef, has_eq ? wsum : hf::scale(wsum, 2)));
@@ -791,6 +794,7 @@ int SumcheckSession::round_sums(uint32_t *out) {
   std::vector<hf::E> rows(points, hf::zero(D));
   for (size_t g = 0; g < st.groups.size(); g++) {
     const Group &grp = st.groups[g];
+    if (grp.follows) continue;
     hf::E coef(group_coef.begin() + g * D, group_coef.begin() + (g + 1) * D);
     if (grp.tabs.empty()) {
       hf::E v = hf::mul(coef, wsum);

@@ -321,26 +321,43 @@ __device__ __forceinline__ void accumulate_groups(const Desc &d, const V *lo, co
         for (int g = 0; g < MAXG; g++)
           if (g < d.G && EXT && d.nev[g] >= 3 && d.deg[g] >= 2) wcur[g] = v_add<D>(wcur[g], wslope[g]);
       }
-      int a = 0;
+      AccLazy sum[D];  // (the unreduced sum of the products of groups that share an accumulator, which follow one another)
+      V total;
 #pragma unroll
       for (int g = 0; g < MAXG; g++) {
         if (g < d.G) {
+          const bool pre = EXT && d.nev[g] >= 3 && d.deg[g] >= 2, first = d.lead[g] == g, last = group_is_last(d, g);
+          const bool shared = EXT && !pre && d.deg[g] >= 2 && !(first && last);
 #pragma unroll
           for (int k = 0; k < MAXEV; k++) {
             if (k < d.nev[g]) {
+              const int a = d.acc[g] + k;
               if (d.ev[g][k] == x && (PARTS == 1 || a % PARTS == PART)) {
-                // the product of the factors but the last; the last goes with the accumulation
-                const bool pre = EXT && d.nev[g] >= 3 && d.deg[g] >= 2;
+                // the product of the factors but the last; the last goes with the accumulation or the sum
                 V prod = pre ? wcur[g] : cur[d.tab[g][0]];
 #pragma unroll
                 for (int j = 1; j < MAXDEG; j++)
-                  if (j < d.deg[g] - (pre ? 1 : 0)) prod = v_mul<D>(prod, cur[d.tab[g][j]]);
-                if constexpr (EXT)
-                  v_mul_acc<D>(acc[a], prod, pre ? cur[d.tab[g][d.deg[g] - 1]] : v_of<D, V>(w));
-                else
-                  v_weigh<D>(acc[a], w, prod);
+                  if (j < d.deg[g] - (pre || shared ? 1 : 0)) prod = v_mul<D>(prod, cur[d.tab[g][j]]);
+                if constexpr (EXT) {
+                  if (shared) {
+                    if (first) {
+#pragma unroll
+                      for (int c = 0; c < D; c++) acc_zero(sum[c]);
+                    }
+                    ext_mul_acc<D>(sum, prod, cur[d.tab[g][d.deg[g] - 1]]);
+                    if (last) {
+#pragma unroll
+                      for (int c = 0; c < D; c++) total.c[c] = mont_reduce4(sum[c].v);
+                    }
+                  } else {
+                    total = pre || first ? prod : v_add<D>(total, prod);
+                  }
+                  if (pre || last) v_mul_acc<D>(acc[a], total, pre ? cur[d.tab[g][d.deg[g] - 1]] : v_of<D, V>(w));
+                } else {
+                  total = first ? prod : v_add<D>(total, prod);
+                  if (last) v_weigh<D>(acc[a], w, total);
+                }
               }
-              a++;
             }
           }
         }
@@ -1112,9 +1129,10 @@ __device__ __forceinline__ void small_round_sums(const Desc &d, const Ext<D> *lo
   part_wave_sums<D, PART, PARTS>(d, acc, sums);
 }
 
-// An accumulator as a lane walks it in a spread round (see tail_body): its degree, its evaluation point, and where in
-// LDS its factors' tables begin.
+// A product of an accumulator as a lane walks it in a spread round (see tail_body): its degree (0: the accumulator has no
+// such product), its evaluation point, and where in LDS its factors' tables begin.
 constexpr int SPREAD_FACTORS = MAXDEG;
+constexpr int SPREAD_UNITS = MAXACC + MAXG;  // accumulators times the most products of one, as far as rounds run spread
 struct SpreadUnit {
   uint32_t deg, x, table[SPREAD_FACTORS];
 };
@@ -1139,7 +1157,9 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   __shared__ uint32_t c0s[MAXTAIL * MAXPTS * D];
   // (a statement in direct form, or with linear forms among its factors, keeps a pair's accumulators on one lane)
   constexpr bool SPREAD = !is_direct<Desc>::value;
-  __shared__ SpreadUnit units[SPREAD ? MAXACC : 1];
+  __shared__ SpreadUnit units[SPREAD ? SPREAD_UNITS : 1];
+  // (products of an accumulator: as many lanes each as the next power of two)
+  const uint32_t term_bits = SPREAD ? lane_bits((uint32_t)desc_terms(d)) : 0;
   const uint32_t tid = threadIdx.x, cap = args.capacity, G = gridDim.x, wg = blockIdx.x;
   const uint32_t width = (uint32_t)d.nacc * D;
   if (args.ctrl->round != args.first_round) return;  // an earlier launch gave up: leave the count as it is
@@ -1187,15 +1207,17 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     for (uint32_t u = tid; u < args.points * width; u += BLOCK) epi.mtilde[u] = args.mtilde[u];
     for (uint32_t u = tid; u < args.rounds * args.points * D; u += BLOCK) c0s[u] = args.c0[u];
   }
-  if (SPREAD && tid < (uint32_t)d.nacc) {
-    uint32_t a = 0;
+  if (SPREAD && ((uint32_t)d.nacc << term_bits) <= (uint32_t)SPREAD_UNITS && tid < ((uint32_t)d.nacc << term_bits)) {
+    const uint32_t a = tid >> term_bits, term = tid & ((1u << term_bits) - 1);
+    units[tid].deg = 0, units[tid].x = 0;
+    for (int j = 0; j < SPREAD_FACTORS; j++) units[tid].table[j] = 0;
+    uint32_t met = 0;  // the accumulator's products so far
     for (int g = 0; g < d.G; g++)
-      for (int k = 0; k < d.nev[g]; k++, a++)
-        if (a == tid) {
-          units[tid].deg = (uint32_t)d.deg[g], units[tid].x = (uint32_t)d.ev[g][k];
-          for (int j = 0; j < SPREAD_FACTORS; j++)
-            units[tid].table[j] = (uint32_t)d.tab[g][j < d.deg[g] ? j : 0] * cap * D;
-        }
+      if (a >= (uint32_t)d.acc[g] && a < (uint32_t)(d.acc[g] + d.nev[g]) && met++ == term) {
+        units[tid].deg = (uint32_t)d.deg[g], units[tid].x = (uint32_t)d.ev[g][a - (uint32_t)d.acc[g]];
+        for (int j = 0; j < SPREAD_FACTORS; j++)
+          units[tid].table[j] = (uint32_t)d.tab[g][j < d.deg[g] ? j : 0] * cap * D;
+      }
   }
   // The session's own weight tables (see TailArgs::factors), in LDS behind the tables: the factors first, then
   // per round its LOW and its HIGH table.  An entry is a chain of at most n_vars products, one entry per thread
@@ -1289,18 +1311,21 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // kernels of a statement's own are about even (a launch over GKR layers: one lookup 28.2 and 27.6, two 34.2 and 34.7,
   // three 52.6 and 53.4 with the glue, 57.0 and 51.2 without; over the blocks of two lookups 21.5 and 25.3).
   auto spreads = [&](uint32_t pairs) {
-    return SPREAD && BLOCK == 256 && d.NV == 0 && pairs <= 64 && ((uint32_t)d.nacc << lane_bits(pairs)) <= 192;
+    const uint32_t bits = lane_bits(pairs) + term_bits;
+    return SPREAD && BLOCK == 256 && d.NV == 0 && bits <= 6 && ((uint32_t)d.nacc << bits) <= 192 &&
+           ((uint32_t)d.nacc << term_bits) <= (uint32_t)SPREAD_UNITS;
   };
-  uint32_t unit_a = 0, unit_pair = 0, unit_deg = 0, unit_x = 0, unit_table[SPREAD_FACTORS];
+  uint32_t unit_a = 0, unit_lane = 0, unit_pair = 0, unit_deg = 0, unit_x = 0, unit_table[SPREAD_FACTORS];
   Ext<D> unit_w = ext_zero<D>();
   // a lane's unit of a round and its weight, which wait for nothing that the round before computes
   auto prepare_unit = [&](uint32_t jj, uint32_t pairs) {
     const uint32_t u = tid < 64 ? 0 : tid - 64;
-    const uint32_t bits = lane_bits(pairs);
-    unit_a = u >> bits, unit_pair = u & ((1u << bits) - 1);
-    const bool on = unit_pair < pairs;  // (a lane without a pair takes the last one with no weight)
-    const SpreadUnit &unit = units[unit_a < (uint32_t)d.nacc ? unit_a : 0];
+    // (an accumulator's lanes: the pairs of its first product, of its second, ...)
+    const uint32_t pair_bits = lane_bits(pairs), bits = pair_bits + term_bits;
+    unit_a = u >> bits, unit_lane = u & ((1u << bits) - 1), unit_pair = unit_lane & ((1u << pair_bits) - 1);
+    const SpreadUnit &unit = units[unit_a < (uint32_t)d.nacc ? (unit_a << term_bits) + (unit_lane >> pair_bits) : 0];
     unit_deg = unit.deg, unit_x = unit.x;
+    const bool on = unit_pair < pairs && unit_deg != 0;  // (a lane without a pair takes the last one with no weight)
 #pragma unroll
     for (int j = 0; j < SPREAD_FACTORS; j++) unit_table[j] = unit.table[j];
     const uint64_t i = (uint64_t)wg * pairs + (on ? unit_pair : pairs - 1);
@@ -1341,7 +1366,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     f = ext_mul_mont<D>(f, unit_w);
     // Over the pairs, the low lane bits of a unit: the words are halved as long as there are several.  Bit 2 comes first:
     // its partner is the opposite lane of a group of 8, which still holds the same words then (see lane_partner).
-    const uint32_t lanes = 1u << lane_bits(pairs);
+    const uint32_t lanes = 1u << (lane_bits(pairs) + term_bits);
     uint32_t v[D], word = 0, count = D, keys = 0;
 #pragma unroll
     for (int c = 0; c < D; c++) v[c] = f.c[c];
@@ -1368,7 +1393,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
       }
     };
     step(LaneBit<4>{}), step(LaneBit<1>{}), step(LaneBit<2>{}), step(LaneBit<8>{}), step(LaneBit<16>{}), step(LaneBit<32>{});
-    if (tid >= 64 && unit_a < (uint32_t)d.nacc && (unit_pair & ~keys) == 0) {
+    if (tid >= 64 && unit_a < (uint32_t)d.nacc && (unit_lane & ~keys) == 0) {
 #pragma unroll
       for (int k = 0; k < D; k++)
         if (k < (int)count) {
@@ -1832,11 +1857,14 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
                 cu[t] += du[t], cv[t] += dv[t];
             }
         }
-        int base = 0;  // first slot of group g
+        int base = 0, lead_base = 0;  // first slot of group g, and of the group whose slots it shares
+        double shared_sum[MAXDEG + 1];
 #pragma unroll
         for (int g = 0; g < MAXG; g++) {
           if (g < d.G) {
             const int e = ev_index(d, g, x);  // an evaluation point's row, or at X1 = 1 the row of extras
+            const bool first = d.lead[g] == g, last = group_is_last(d, g);
+            if (first) lead_base = base;
             if (e >= 0 || x == 1) {
               double val[MAXDEG];
 #pragma unroll
@@ -1846,18 +1874,21 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
               for (int m = 0; m <= MAXDEG; m++) {
                 if (m <= d.deg[g]) {
                   if (e >= 0)
-                    slot = base + e * (d.deg[g] + 1) + m;
+                    slot = lead_base + e * (d.deg[g] + 1) + m;
                   else  // only the nodes that are evaluation points
-                    slot = ev_index(d, g, m) < 0 ? -1 : base + d.nev[g] * (d.deg[g] + 1) + ev_index(d, g, m);
+                    slot = ev_index(d, g, m) < 0 ? -1 : lead_base + d.nev[g] * (d.deg[g] + 1) + ev_index(d, g, m);
                   if (slot >= PASS * SPP && slot < (PASS + 1) * SPP) {
                     double prod = val[0];
 #pragma unroll
                     for (int j = 1; j < MAXDEG; j++)
                       if (j < d.deg[g]) prod = f_mul(prod, val[j]);
-                    if (d.deg[g] == 1) prod = f_reduce(prod);
-                    const uint32_t pv = f_residue32(prod);
+                    shared_sum[m] = first ? prod : shared_sum[m] + prod;  // (groups that share the slot follow one another)
+                    if (last) {
+                      const double total = d.deg[g] == 1 || !first ? f_reduce(shared_sum[m]) : shared_sum[m];
+                      const uint32_t pv = f_residue32(total);
 #pragma unroll
-                    for (int c = 0; c < D; c++) lazy_mad(acc[slot - PASS * SPP][c], we.c[c], pv);
+                      for (int c = 0; c < D; c++) lazy_mad(acc[slot - PASS * SPP][c], we.c[c], pv);
+                    }
                   }
 #pragma unroll
                   for (int j = 0; j < MAXDEG; j++)
@@ -1899,7 +1930,7 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
     // carry 1/R per multiplication, which the epilogue's constants expect: times R^(1 - degree) here.
     int base = 0, deg = 1;
     for (int g = 0; g < d.G; g++) {
-      if (PASS * SPP + (int)tid >= base) deg = d.deg[g];
+      if (d.lead[g] == g && PASS * SPP + (int)tid >= base) deg = d.deg[g];
       base += group_slots(d, g);
     }
     uint32_t fix = R1;  // mont_mul(v, fix) = v R^(1 - degree)

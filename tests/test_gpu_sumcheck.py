@@ -334,6 +334,37 @@ def test_round_three_from_the_base_tables(form, names, cnames, d, n, monkeypatch
     prove_both("bind3", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames)
 
 
+T4 = ["t0", "t1", "t2", "t3"]
+
+
+@pytest.mark.parametrize("form,names,cnames,d,n,base", [
+    ("(+ (* e0 g0) (* e1 g1) (* e2 g2))", ["e0", "g0", "e1", "g1", "e2", "g2"], [], 4, 7, False),  # three products of one sum
+    ("(+ (* e0 g0) (* e1 g1))", ["e0", "g0", "e1", "g1"], [], 4, 13, True),  # ... in the base-field sweep's slots
+    (*GKR2, 4, 5, False),  # sums of two products beside sums of one
+    # on the interpreter: five products, more than one sum takes; sums of single tables; cubes evaluated at three points
+    ("(+ (* a t0 t1) (* a t2 t3) (* a t1 t2) (* a t0 t3) (* a t0 t2))", T4, ["a"], 4, 9, True),
+    ("(+ (* a t0) (* a t1) (* a t2) (* t0 t1) (* t2 t3))", T4, ["a"], 8, 8, False),
+    ("(+ (* a t0 t1 t2) (* a t1 t2 t3) (* 5 t0 t1) (* 5 t2 t3))", T4, ["a"], 4, 6, True),
+])
+def test_products_that_share_a_sum(form, names, cnames, d, n, base, monkeypatch):
+    """Table monomials of one coefficient and degree share their accumulators: the oracle's proof from the rounds in LDS,
+    from streaming rounds, and with the host's rounds; the claim is the oracle's."""
+    rng = np.random.default_rng(n * 23 + d)
+    tables = [rng.integers(0, P, 1 << n, dtype=np.uint32) if base else rand_ext(rng, (1 << n,), d) for _ in names]
+    tables[-1][...] = P - 1
+    eq = rand_ext(rng, (n,), d)
+    consts = rand_ext(rng, (len(cnames),), d) if cnames else None
+    for switch, value in (("EXACTA_HIP_MAX_SLICE_PAIRS", "100000"), ("EXACTA_HIP_MAX_SLICE_PAIRS", "0"),
+                          ("EXACTA_HIP_HOST_ROUNDS", "1")):
+        monkeypatch.setenv(switch, value)
+        st, ost, *_ = prove_both("shared", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames)
+    dev = [sa.Table.upload(t) for t in tables]
+    assert same(sa.hypercube_sum(st, n, dev, d, eq=eq, constants=consts),
+                orc.hypercube_sum(ost, n, tables, d, eq=eq, constants=consts))
+    for t in dev:
+        t.free()
+
+
 @pytest.mark.parametrize("form,names,cnames,d,n,K,base", [
     (*GKR2, 4, 8, 3, False),  # eight tables, four held ahead; 384 and 192 pairs: a last workgroup with half its lanes
     (*GKR2, 4, 10, 1, True),
