@@ -606,6 +606,110 @@ __global__ __launch_bounds__(BLOCK) void subtree_kernel(uint32_t *level, uint64_
   }
 }
 
+// The same for trees of few leaves and for the upper levels of large ones, a compression on the four lanes of a quad
+// (dev_transcript.hpp): a thread hashing alone is a chain of 678 instructions five cycles apart, 1.4 us, and a leaf of many
+// columns or a level above another is one such chain after the other while most of the device idles; on four lanes it is
+// 0.6 us, for a third more instructions in all.  A workgroup of THREADS takes THREADS / 4 leaves or twice as many digests;
+// both levels of a step lie in LDS, two digests -- one message -- a row.  Arguments as above; height at most the levels of
+// the workgroup's own tree.  256 threads over the leaves: with 1024 (256 leaves, eight levels, fewer workgroups) 2^13
+// leaves of 70 columns took 97 us for 79, 2^14 of 30 columns 77 for 68, and 2^16 of two 62 for 66.
+constexpr int QUAD_LEAF_THREADS = 256, QUAD_LEAF_HEIGHT = 6;     // 64 leaves
+constexpr int QUAD_NODE_THREADS = 1024, QUAD_NODE_HEIGHT = 9;    // 512 digests
+constexpr uint64_t QUAD_LEAVES = 1 << 16, QUAD_DIGESTS = 1 << 17;  // trees and levels up to here (merkle_tree_launch)
+constexpr int QUAD_ROW = 20;  // words of a row: rows begin on 16 bytes and four lanes' words of different quads meet on few banks
+template <int LEAVES, int THREADS>
+__global__ __launch_bounds__(THREADS) void quad_tree_kernel(uint32_t *level, uint64_t n, int height, const uint32_t *cw,
+                                                            int ncols, uint64_t cw_len, unsigned long long *cap_out,
+                                                            uint32_t seq) {
+  constexpr int QUADS = THREADS / 4, BOTTOM = LEAVES ? QUADS : 2 * QUADS;
+  __shared__ __align__(16) uint32_t rows[2][QUADS * QUAD_ROW];
+  const uint32_t tid = threadIdx.x, quad = tid / 4, i = tid % 4;
+  const uint32_t iva = i == 0 ? EXH_B3_IV0 : i == 1 ? EXH_B3_IV1 : i == 2 ? EXH_B3_IV2 : EXH_B3_IV3;
+  const uint32_t ivb = i == 0 ? EXH_B3_IV4 : i == 1 ? EXH_B3_IV5 : i == 2 ? EXH_B3_IV6 : EXH_B3_IV7;
+  uint32_t at[28];
+  b3_quad_offsets(at);
+  auto compress = [&](const uint32_t *row, uint32_t &a, uint32_t &b, uint32_t len, uint32_t flags) {
+    uint32_t m[28], w2, w3;
+#pragma unroll
+    for (int k = 0; k < 28; k++) m[k] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(row) + at[k]);
+    b3_quad_rounds(m, a, b, i == 2 ? len : i == 3 ? flags : 0u, a, b, w2, w3);
+  };
+  auto digest_at = [&](int buffer, uint32_t d) { return rows[buffer] + (d >> 1) * QUAD_ROW + (d & 1) * 8; };
+  uint64_t first = (uint64_t)blockIdx.x * BOTTOM, count = n;  // this workgroup's first node of the level at hand
+  uint32_t *out = level;
+  if constexpr (LEAVES != 0) {
+    const uint64_t l = first + quad < n ? first + quad : n - 1;
+    uint32_t *row = rows[1] + quad * QUAD_ROW, ha = 0, hb = 0;  // (the other buffer is free until the first level is done)
+    if constexpr (LEAVES == 1) {
+      for (int start = 0; start < ncols; start += 64) {
+        const int have = ncols - start < 64 ? ncols - start : 64, nblocks = (have + 3) / 4;
+        auto fetch = [&](int b) {
+          const int k = 4 * b + (int)i;
+          return k < have ? *reinterpret_cast<const uint4 *>(cw + (uint64_t)(start + k) * cw_len + 4 * l) : make_uint4(0, 0, 0, 0);
+        };
+        uint32_t da = iva, db = ivb;
+        uint4 v = fetch(0);
+        for (int b = 0; b < nblocks; b++) {
+          __builtin_amdgcn_wave_barrier();
+          *reinterpret_cast<uint4 *>(row + 4 * i) = v;
+          __builtin_amdgcn_wave_barrier();
+          if (b + 1 < nblocks) v = fetch(b + 1);
+          const int here = have - 4 * b < 4 ? have - 4 * b : 4;
+          compress(row, da, db, 16u * (uint32_t)here,
+                   (b == 0 ? B3_CHUNK_START : 0u) | (b == nblocks - 1 ? (B3_CHUNK_END | B3_ROOT) : 0u));
+        }
+        if (start == 0) {
+          ha = da, hb = db;
+        } else {  // h = BLAKE3(h || d)
+          __builtin_amdgcn_wave_barrier();
+          row[i] = ha, row[4 + i] = hb, row[8 + i] = da, row[12 + i] = db;
+          __builtin_amdgcn_wave_barrier();
+          ha = iva, hb = ivb;
+          compress(row, ha, hb, 64, B3_CHUNK_START | B3_CHUNK_END | B3_ROOT);
+        }
+      }
+    } else {  // lane s holds symbol 4 l + s: word 4 k + s of block b is its coordinate 4 b + k
+      const uint4 *sym = reinterpret_cast<const uint4 *>(cw + (4 * l + i) * 8);
+      const uint4 v[2] = {sym[0], sym[1]};
+      ha = iva, hb = ivb;
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        __builtin_amdgcn_wave_barrier();
+        row[i] = v[b].x, row[4 + i] = v[b].y, row[8 + i] = v[b].z, row[12 + i] = v[b].w;
+        __builtin_amdgcn_wave_barrier();
+        compress(row, ha, hb, 64, b == 0 ? B3_CHUNK_START : (B3_CHUNK_END | B3_ROOT));
+      }
+    }
+    uint32_t *to = digest_at(0, quad);
+    to[i] = ha, to[4 + i] = hb;
+    if (first + quad < n) out[8 * (first + quad) + i] = ha, out[8 * (first + quad) + 4 + i] = hb;
+  } else {
+    const uint64_t q = 2 * first + tid;  // two quads of words a digest, a row of four to two digests
+    if (q < 2 * n) *reinterpret_cast<uint4 *>(rows[0] + (tid >> 2) * QUAD_ROW + (tid & 3) * 4) = reinterpret_cast<const uint4 *>(level)[q];
+  }
+  uint32_t width = BOTTOM;
+  for (int s = 1; s <= height; s++) {
+    __syncthreads();
+    out += 8 * count;
+    count /= 2, first /= 2, width /= 2;
+    if (quad < width && first + quad < count) {
+      uint32_t a = iva, b = ivb;
+      compress(rows[(s - 1) & 1] + quad * QUAD_ROW, a, b, 64, B3_CHUNK_START | B3_CHUNK_END | B3_ROOT);
+      uint32_t *to = digest_at(s & 1, quad);
+      to[i] = a, to[4 + i] = b;
+      out[8 * (first + quad) + i] = a, out[8 * (first + quad) + 4 + i] = b;
+    }
+  }
+  if (cap_out) {
+    __syncthreads();
+    for (uint32_t w = tid; w < 8 * width; w += THREADS)
+      if (first + w / 8 < count)
+        __hip_atomic_store(cap_out + 8 * first + w, ((unsigned long long)seq << 32) | digest_at(height & 1, w / 8)[w % 8],
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+static_assert(1 << QUAD_LEAF_HEIGHT == QUAD_LEAF_THREADS / 4 && 1 << QUAD_NODE_HEIGHT == QUAD_NODE_THREADS / 2, "a workgroup's own tree");
+
 // a tree of a single leaf: its digest is the whole tree
 template <int LEAVES>
 __global__ void single_leaf_kernel(uint32_t *level, const uint32_t *cw, int ncols, uint64_t cw_len) {
@@ -653,14 +757,28 @@ static int merkle_tree_launch(uint32_t *d_levels, uint64_t nleaves, int leaves, 
     // 2^22 leaves: 246 us with nine levels in the first launch, 198 us with five, 175 us with three; five leaves the
     // fewest launches above -- over digests only, nine levels each -- and the shortest commit, 0.51 against 0.55 ms).
     static const int leaf_height = getenv("EXH_MERKLE_LEAF_HEIGHT") ? atoi(getenv("EXH_MERKLE_LEAF_HEIGHT")) : 5;
-    // (a workgroup to a compute unit or fewer leave no other work to idle beside: one launch climbs all it can)
-    const int max_height = leaves != 0 && !(cap_out && n / 2 <= 128 * BLOCK) ? leaf_height : 9;
+    // Four lanes a compression while that is what fills the device.  Whole commitments, a thread against four lanes:
+    // 2^13 leaves of 70 columns 126 against 79 us, 2^16 leaves of 100 columns 240 against 195 and of 2 columns 73
+    // against 66; 2^17 leaves 72 and 72, 2^18 91 against 97, 2^20 156 against 214 (the third more instructions).
+    // Digests: under 2^22 leaves of two columns, 2^17 digests and fewer, 435 against 426; 2^18 to 2^20 digests level.
+    const bool quads = n <= (leaves ? QUAD_LEAVES : QUAD_DIGESTS);
+    const int max_height = quads ? (leaves ? QUAD_LEAF_HEIGHT : QUAD_NODE_HEIGHT) : leaves ? leaf_height : 9;
     for (uint64_t v = n; v > stop && height < max_height; v >>= 1) height++;
     unsigned long long *const out = n >> height == stop ? cap_out : nullptr;
-    uint32_t grid = (uint32_t)((n / 2 + BLOCK - 1) / BLOCK);
+    const uint64_t bottom = quads ? (leaves ? QUAD_LEAF_THREADS / 4 : QUAD_NODE_THREADS / 2) : 2 * BLOCK;
+    uint32_t grid = (uint32_t)((n + bottom - 1) / bottom);
     c.prof_begin(leaves == 1 ? "merkle_leaves" : leaves == 2 ? "merkle_oracle_leaves" : "merkle_levels", 0,
                  (leaves == 1 ? (uint64_t)ncols * 16 * n : leaves == 2 ? 128 * n : 0) + 64 * n);
-    if (leaves == 1)
+    if (quads && leaves == 1)
+      hipLaunchKernelGGL((quad_tree_kernel<1, QUAD_LEAF_THREADS>), dim3(grid), dim3(QUAD_LEAF_THREADS), 0, c.stream, level, n,
+                         height, cw, ncols, cw_len, out, seq);
+    else if (quads && leaves == 2)
+      hipLaunchKernelGGL((quad_tree_kernel<2, QUAD_LEAF_THREADS>), dim3(grid), dim3(QUAD_LEAF_THREADS), 0, c.stream, level, n,
+                         height, cw, ncols, cw_len, out, seq);
+    else if (quads)
+      hipLaunchKernelGGL((quad_tree_kernel<0, QUAD_NODE_THREADS>), dim3(grid), dim3(QUAD_NODE_THREADS), 0, c.stream, level, n,
+                         height, cw, ncols, cw_len, out, seq);
+    else if (leaves == 1)
       hipLaunchKernelGGL(subtree_kernel<1>, dim3(grid), dim3(BLOCK), 0, c.stream, level, n, height, cw, ncols, cw_len, out,
                          seq);
     else if (leaves == 2)

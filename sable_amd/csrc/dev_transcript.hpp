@@ -49,19 +49,23 @@ struct RunB3S {
   uint32_t at[28];      // where in a block (bytes) this lane's message words of each round lie: columns x, y, diagonals x, y
 };
 
-__device__ __forceinline__ void rb3s_init(RunB3S &s, uint32_t *ring) {
-  const uint32_t i = threadIdx.x & 3, di = (i + 3) & 3;  // (the diagonal G that runs on this lane, see b3_compress_quad)
-  s.ring = ring;
+// where in a block (bytes) a lane's message words of each round lie
+__device__ __forceinline__ void b3_quad_offsets(uint32_t at[28]) {
+  const uint32_t i = threadIdx.x & 3, di = (i + 3) & 3;  // (the diagonal G that runs on this lane, see b3_quad_rounds)
 #pragma unroll
   for (int r = 0; r < 7; r++) {
     // the four lanes' word numbers sit in the nibbles of a compile-time constant: no table in memory to read
-    s.at[4 * r] = 4 * ((b3_lane_words(r, 0) >> (4 * i)) & 15u), s.at[4 * r + 1] = 4 * ((b3_lane_words(r, 1) >> (4 * i)) & 15u);
-    s.at[4 * r + 2] = 4 * ((b3_lane_words(r, 8) >> (4 * di)) & 15u);
-    s.at[4 * r + 3] = 4 * ((b3_lane_words(r, 9) >> (4 * di)) & 15u);
+    at[4 * r] = 4 * ((b3_lane_words(r, 0) >> (4 * i)) & 15u), at[4 * r + 1] = 4 * ((b3_lane_words(r, 1) >> (4 * i)) & 15u);
+    at[4 * r + 2] = 4 * ((b3_lane_words(r, 8) >> (4 * di)) & 15u);
+    at[4 * r + 3] = 4 * ((b3_lane_words(r, 9) >> (4 * di)) & 15u);
   }
 }
+__device__ __forceinline__ void rb3s_init(RunB3S &s, uint32_t *ring) {
+  s.ring = ring;
+  b3_quad_offsets(s.at);
+}
 
-// The compression of the pending half with the state's columns spread over the lanes of a quad; d: the state's last
+// The compression with the state's columns spread over the lanes of a quad (of the pending half, below); d: the state's last
 // row (counter low, counter high, block length, flags on lanes 0 to 3).  Lane i of each quad returns w0 = out[i],
 // w1 = out[4+i], w2 = out[8+i], w3 = out[12+i].
 // For the diagonals row b, the last one a half-round computes, stays where it is and rows a, c and d come to it: a
@@ -69,20 +73,11 @@ __device__ __forceinline__ void rb3s_init(RunB3S &s, uint32_t *ring) {
 // two instructions for its source, and the compiler counts every operand of such an instruction: permuting c and d
 // inside the addition and the exclusive-or put two waits into every half-round).  With the chaining value and the
 // word offsets in registers a compression takes 600 ns on a lone wavefront; rotating b, c and d, from LDS, 675 ns.
-__device__ __forceinline__ void b3_compress_quad(const RunB3S &s, uint32_t d, uint32_t &w0, uint32_t &w1, uint32_t &w2,
-                                                 uint32_t &w3) {
+// m: the lane's message words; cva, cvb: words i and 4 + i of the chaining value.
+__device__ __forceinline__ void b3_quad_rounds(const uint32_t m[28], uint32_t cva, uint32_t cvb, uint32_t d, uint32_t &w0,
+                                               uint32_t &w1, uint32_t &w2, uint32_t &w3) {
   const uint32_t i = threadIdx.x & 3;
-  uint32_t m[28];
-  const uint8_t *block = reinterpret_cast<const uint8_t *>(s.ring);
-  // (the half as a constant in either branch: it then is part of the instructions' offsets)
-  if (s.half == 0) {
-#pragma unroll
-    for (int k = 0; k < 28; k++) m[k] = *reinterpret_cast<const uint32_t *>(block + s.at[k]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 28; k++) m[k] = *reinterpret_cast<const uint32_t *>(block + 64 + s.at[k]);
-  }
-  uint32_t a = s.cva, b = s.cvb, c = i == 0 ? EXH_B3_IV0 : i == 1 ? EXH_B3_IV1 : i == 2 ? EXH_B3_IV2 : EXH_B3_IV3;
+  uint32_t a = cva, b = cvb, c = i == 0 ? EXH_B3_IV0 : i == 1 ? EXH_B3_IV1 : i == 2 ? EXH_B3_IV2 : EXH_B3_IV3;
 #define EXH_B3_HALF(A, C, D, x, y)                  \
   {                                                 \
     uint32_t t = (A) + (x), cq = (C), dq = (D);     \
@@ -107,7 +102,21 @@ __device__ __forceinline__ void b3_compress_quad(const RunB3S &s, uint32_t d, ui
   }
 #undef EXH_B3_HALF
   a = EXH_QUAD(a, 0x39), c = EXH_QUAD(c, 0x93), d = EXH_QUAD(d, 0x4E);
-  w0 = a ^ c, w1 = b ^ d, w2 = c ^ s.cva, w3 = d ^ s.cvb;
+  w0 = a ^ c, w1 = b ^ d, w2 = c ^ cva, w3 = d ^ cvb;
+}
+__device__ __forceinline__ void b3_compress_quad(const RunB3S &s, uint32_t d, uint32_t &w0, uint32_t &w1, uint32_t &w2,
+                                                 uint32_t &w3) {
+  uint32_t m[28];
+  const uint8_t *block = reinterpret_cast<const uint8_t *>(s.ring);
+  // (the half as a constant in either branch: it then is part of the instructions' offsets)
+  if (s.half == 0) {
+#pragma unroll
+    for (int k = 0; k < 28; k++) m[k] = *reinterpret_cast<const uint32_t *>(block + s.at[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 28; k++) m[k] = *reinterpret_cast<const uint32_t *>(block + 64 + s.at[k]);
+  }
+  b3_quad_rounds(m, s.cva, s.cvb, d, w0, w1, w2, w3);
 }
 
 // lane i of a quad: the i-th of four uniform values

@@ -94,6 +94,25 @@ def test_merkle_commit_matches_the_oracle(c, ncols):
         x.free()
 
 
+# trees hashed on four lanes a compression: a workgroup takes 64 leaves (six levels) or 512 digests (nine), a leaf four
+# columns a block, 64 a hash; 2^16 leaves are the most of the leaf kernel, 2^17 digests of the other
+@pytest.mark.parametrize("c,ncols", [(2, 3), (6, 4), (7, 1), (7, 5), (8, 64), (9, 65), (10, 128), (10, 130), (11, 6), (16, 7),
+                                     (17, 3), (18, 2), (19, 1)])
+def test_small_trees_match_the_oracle(c, ncols):
+    rng = np.random.default_rng(7 * c + ncols)
+    cols = [rng.integers(0, P, 1 << c, dtype=np.uint32) for _ in range(ncols)]
+    ocw, olevels, ocap = orc.commit_columns(cols, c)
+    tr, otr = sa.Transcript("commit", 4), orc.Transcript("commit", 4)
+    t = sa.Table.upload(np.concatenate(cols))
+    cw, levels = sa.pcs_commit(tr, t, ncols, c)
+    otr.send_bytes(ocap.tobytes())
+    assert tr.proof() == otr.proof()
+    got = levels.download().reshape(-1, 8).astype("<u4").view(np.uint8).reshape(-1, 32)
+    assert same(got, np.concatenate(olevels))
+    for x in (t, cw, levels):
+        x.free()
+
+
 def test_commit_full_size_paths_open_to_the_cap():
     """Config 5's commitment at full size: two 2^23-coefficient columns -> 2^22 leaves -> cap of 128; a few
     leaves are recomputed on the host from the downloaded codeword symbols and opened against the cap."""
@@ -135,6 +154,22 @@ def test_basefold_matches_the_oracle(nv):
     assert sa.basefold_verify(sa.Transcript("bf", 4, proof=tr.proof()), nv, rr, v) == got[0]
     with pytest.raises(sa.VerificationFailure):
         sa.basefold_verify(sa.Transcript("bf", 4, proof=tr.proof()), nv, rr, orc.ext_add(v, orc.base_to_ext(1, 8)))
+    t.free()
+
+
+@pytest.mark.parametrize("nv", [1, 2, 5, 6, 8, 15, 17])
+def test_basefold_whose_trees_are_small_matches_the_oracle(nv):
+    """The oracles' trees, hashed on four lanes a compression: one leaf up to more than the leaf kernel's 2^16."""
+    rng = np.random.default_rng(300 + nv)
+    h = rng.integers(0, P, (1 << nv, 8), dtype=np.uint32)
+    rr = rng.integers(0, P, (nv, 8), dtype=np.uint32)
+    v = orc.mle_eval(h, rr, 8)
+    tr, otr = sa.Transcript("bf", 4), orc.Transcript("bf", 4)
+    t = sa.Table.upload(h)
+    got = sa.basefold_prove(tr, nv, rr, v, t)
+    want = orc.basefold_prove(otr, nv, rr, v, h)
+    assert tr.proof() == otr.proof()
+    assert got[0] == want[0] and same(got[1], want[1]) and same(got[2], want[2])
     t.free()
 
 
