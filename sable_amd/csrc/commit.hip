@@ -1810,10 +1810,13 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     return w;
   };
   std::vector<Split> round_w(std::max(fl, 1)), class_w(ncls);
-  for (int i = BB; i < fl; i++)
-    // (tiles of 2^10 to 2^12 pairs, at least a thousand of them while the table is that large: long tiles in few
-    // workgroups trail their loads one after another, short ones pay the reduction and the atomics per tile)
-    round_w[i] = split(i + 1, std::min(std::max(nv - 1 - i - 10, 10), 12));
+  // (tiles of 2^10 to 2^12 pairs, at least a thousand of them while the table is that large: long tiles in few
+  // workgroups trail their loads one after another, short ones pay the reduction and the atomics per tile.  Tables of
+  // under 2^18 pairs leave most of the device idle either way and take as many tiles as it has compute units, down to a
+  // pair a thread: four pairs one after the other are 2 us of a round, an opening of 2^23 x 2 and 2^19 825 against
+  // 787 us, of 2^18 x 2 359 against 328; twice or four times as many tiles made no difference.)
+  auto tile_bits = [](int pair_bits) { return std::min(std::max(pair_bits - 10, std::min(std::max(pair_bits - 8, 8), 10)), 12); };
+  for (int i = BB; i < fl; i++) round_w[i] = split(i + 1, tile_bits(nv - 1 - i));
   auto open_bits = [&](int k) { return k + 1 == ncls ? BB : BF_BASE_BITS; };
   for (int k = 0; k < ncls; k++)
     if (!src[k].h && (k + 1 < ncls || base)) {
@@ -1942,7 +1945,7 @@ int basefold_prove_classes(Transcript &tr, int nv, int ncls, const int *cls, con
     const bool from_base = fold && tt_base, cw_base = from_base && cw_out && i == CB;
     a.tt_in = tt, a.fold = fold ? 1 : 0, a.do_sums = do_sums && tt_part ? 1 : 0, a.n_pairs = n_pairs;
     if (fold && tt_part) a.tt_out = (tt == tt_a) ? tt_b : tt_a;
-    uint64_t tile = std::min<uint64_t>(std::max<uint64_t>(n_pairs, 1), 4 * BLOCK);
+    uint64_t tile = n_pairs < (uint64_t)1 << 18 ? BLOCK : 4 * BLOCK;
     if (a.do_sums) {
       const Split &w = round_w[i];
       a.low = weights + w.low * 8, a.high = weights + w.high * 8, a.low_bits = (uint32_t)w.low_bits;

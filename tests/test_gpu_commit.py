@@ -157,9 +157,10 @@ def test_basefold_matches_the_oracle(nv):
     t.free()
 
 
-@pytest.mark.parametrize("nv", [1, 2, 5, 6, 8, 15, 17])
+@pytest.mark.parametrize("nv", [1, 2, 5, 6, 8, 15, 17, 19])
 def test_basefold_whose_trees_are_small_matches_the_oracle(nv):
-    """The oracles' trees, hashed on four lanes a compression: one leaf up to more than the leaf kernel's 2^16."""
+    """The oracles' trees, hashed on four lanes a compression: one leaf up to more than the leaf kernel's 2^16; and
+    rounds of 2^8, 2^9 and 2^10 pairs to a workgroup (tables of fewer than 2^17, 2^18 and 2^19 pairs)."""
     rng = np.random.default_rng(300 + nv)
     h = rng.integers(0, P, (1 << nv, 8), dtype=np.uint32)
     rr = rng.integers(0, P, (nv, 8), dtype=np.uint32)
