@@ -190,6 +190,8 @@ typedef struct {
 /* TABLE-VALUES (src/domain.lisp:311-321): the sumcheck table of a column's half (0 or 1; -1 for a column with one
    table, which does not depend on the top in-block variable): K blocks of 2^(n-1) base values -> a new table */
 int exh_domain_table(const exh_domain_column *column, int half, int n, int K, exh_table *out);
+/* `count` such tables in one call and one launch: out[t] from columns[t] and halves[t]. */
+int exh_domain_tables(const exh_domain_column *columns, const int *halves, int count, int n, int K, exh_table *out);
 /* DOMAIN-LEAVES (src/domain.lisp:298-309) of one lookup: the forms tag, values[0..n_values) and num (NULL: the
    numerator 1) over the columns' names; z and betas (n_values * D) canonical.  out_p, out_q: new tables of
    K * 2^n EXTs, p = num, q = Z - tag - sum_i beta_i v_i, as PROVE-UPPER takes them */

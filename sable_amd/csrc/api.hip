@@ -664,21 +664,30 @@ int domain_column_of(const exh_domain_column *in, int n, int K, DomainColumn *ou
 }
 }  // namespace
 
-int exh_domain_table(const exh_domain_column *column, int half, int n, int K, exh_table *out) {
+int exh_domain_tables(const exh_domain_column *columns, const int *halves, int count, int n, int K, exh_table *out) {
   ApiLock api_lock;
-  DomainColumn col;
-  int status = domain_column_of(column, n, K, &col);
-  if (status) return status;
-  if (n < 2 || n > 40 || K < 1) {
+  std::vector<DomainColumn> cols((size_t)(count > 0 ? count : 0));
+  int status;
+  for (int t = 0; t < count; t++)
+    if ((status = domain_column_of(columns + t, n, K, &cols[(size_t)t]))) return status;
+  if (n < 2 || n > 40 || K < 1 || count < 0) {
     set_error("invalid-parameter: domain table arguments");
     return E_PARAM;
   }
-  if ((status = exh_table_alloc((uint64_t)K << (n - 1), 1, out))) return status;
-  if ((status = domain_table(col, half, n, K, table_of(*out)->ptr))) {
-    exh_table_free(*out);
-    *out = 0;
-  }
+  std::vector<uint32_t *> ptrs((size_t)count);
+  int made = 0;
+  for (status = OK; made < count && status == OK; made += status == OK)
+    if (!(status = exh_table_alloc((uint64_t)K << (n - 1), 1, out + made))) ptrs[(size_t)made] = table_of(out[made])->ptr;
+  if (status || (status = domain_tables(cols, halves, n, K, ptrs.data())))
+    for (int t = 0; t < made; t++) {
+      exh_table_free(out[t]);
+      out[t] = 0;
+    }
   return status;
+}
+
+int exh_domain_table(const exh_domain_column *column, int half, int n, int K, exh_table *out) {
+  return exh_domain_tables(column, &half, 1, n, K, out);
 }
 
 int exh_domain_leaves(int D, int n, int K, const exh_domain_column *columns, int n_columns, const char *tag,

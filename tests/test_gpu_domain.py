@@ -87,6 +87,17 @@ def test_leaves_and_tables_of_the_toy_domain(n, k, d):
         assert mt[0] == tt[0] and np.array_equal(sd.table_values(mt, k, n).download(), od.table_values(tt, k, n))
 
 
+@pytest.mark.parametrize("count", [1, 16, 17, 33])
+@pytest.mark.parametrize("n,k", [(2, 1), (10, 3)])
+def test_tables_of_one_launch(n, k, count):
+    """Sixteen tables to a launch: a table alone, the most of one launch, and the rest in the next ones."""
+    theirs = toy_domain(n=n, k=k, seed=n + k)
+    tables, want = sd.domain_tables(device_toy(theirs)), od.domain_tables(theirs)
+    order = [(7 * i) % len(want) for i in range(count)]
+    for got, i in zip(sd.tables_values([tables[i] for i in order], k, n), order):
+        assert np.array_equal(got.download(), od.table_values(want[i], k, n))
+
+
 CASES = [("products", dict(n=6, k=1, seed=1)), ("products", dict(n=8, k=3, seed=2)), ("products", dict(n=12, k=2, seed=3)),
          ("products", dict(n=16, k=1, seed=4)), ("products", dict(n=5, k=4, seed=5, merge=True, lookups=False)),
          ("products", dict(n=4, k=3, seed=6, merge=True, constraints=False)), ("products", dict(n=3, k=1, seed=7, merge=True)),
