@@ -474,7 +474,7 @@ int eq_tables_launch(int D, int count, const int *first, const int *bits, const 
   return OK;
 }
 
-static uint64_t tail_pairs(int T, int D);
+static uint64_t whole_pairs(int T, int D);
 
 int SumcheckSession::launch_setup(const uint32_t *staged, size_t staged_words) {
   Context &c = ctx();
@@ -483,7 +483,7 @@ int SumcheckSession::launch_setup(const uint32_t *staged, size_t staged_words) {
   memcpy(&eqt, setup.eqt, sizeof(eqt));
   // a session whose first round fits the one-workgroup launch never takes the grid launch
   uint32_t *zero = reinterpret_cast<uint32_t *>(d_slice_totals);
-  uint64_t zero_words = size / 2 > tail_pairs(st.T(), D) ? zeroed_words : 0;
+  uint64_t zero_words = size / 2 > whole_pairs(st.T(), D) ? zeroed_words : 0;
   const uint32_t zero_grid = (uint32_t)((zero_words + 4 * BLOCK - 1) / (4 * BLOCK));  // four words a thread
   bool cleared = false;
   c.prof_begin("weights", 0, 0);
@@ -939,6 +939,16 @@ static uint64_t tail_pairs(int T, int D) {
   return p;
 }
 
+// A session that begins with at most this many pairs runs in that launch as a whole: at F_p^4 twice as many (two pairs a
+// thread in round 0, 64 KiB of tables), which saves the set-up launch and a grid of two workgroups for one round.  With it
+// and without, us: a product of two base tables of 2^10 79.7 and 82.4, two points' reduction of 2^10 79.5 and 84.9, three
+// factors of 2^10 94.6 and 96.2, layers of a fraction tree even; four pairs a thread lose (2^11: 95 and 89), and so do two
+// at F_p^8 (2^10: 111 and 103).
+static uint64_t whole_pairs(int T, int D) {
+  const bool streaming = getenv("EXACTA_HIP_MAX_SLICE_PAIRS") != nullptr;  // tests: keep more rounds on the streaming kernels
+  return (D == 4 && !streaming ? 2 : 1) * tail_pairs(T, D);
+}
+
 uint64_t SumcheckSession::one_workgroup_pairs(int T, int D) { return tail_pairs(T, D); }
 
 // the Lagrange basis of the group's node e over its nodes at wire point k (0, 2, 3, ...), times the power of R the
@@ -1023,15 +1033,13 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   }
   // A session whose every round runs in the one-workgroup launch needs no set-up launch: that launch builds the
   // weight tables itself from the eq point's factors, which lead the session's constants (EXACTA_HIP_NO_OWN_WEIGHTS=1:
-  // never).  In a chain, whose constants are on the device already, also the all-ones tables of a session without an eq
-  // point, and it reads the block weights, which follow the factors, where they lie; where the constants come from the host
-  // such a session's set-up launch is cheaper than the copy that brings them without it (two points' reduction of 2^9: 66
-  // and 69 us; layers of 64 blocks driven by the host, 2^8 entries: 1108 and 1367 us a tree).
+  // never), or all ones without an eq point, and reads block weights, which follow the factors, where they lie.  Outside a
+  // chain it brings the constants from pinned memory itself, as the set-up launch does (a product of two tables of 2^9:
+  // 67.7 us, 71.2 with a copy on the stream before it).
   {
     const char *no_own = getenv("EXACTA_HIP_NO_OWN_WEIGHTS");
-    const bool one_launch = size / 2 <= tail_pairs(T, D) && n <= MAXTAIL;
-    own_weights = setup_deferred && one_launch && (chain_hook ? has_bw || K == 1 : has_eq && !has_bw) &&
-                  !(no_own && no_own[0] == '1');
+    const bool one_launch = size / 2 <= whole_pairs(T, D) && n <= MAXTAIL;
+    own_weights = setup_deferred && one_launch && (has_bw || K == 1) && !(no_own && no_own[0] == '1');
     if (valid_entries && (!one_launch || cur_base)) {
       set_error("invalid-parameter: padded tables are extension elements for the one-workgroup launch");
       return E_PARAM;
@@ -1051,9 +1059,11 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
     // which reads them where they lie; with one copy on the stream when there is no such launch
     // (EXACTA_HIP_COPY_CONSTANTS=1: always by that copy, the set-up launch behind it)
     const char *copy_constants = getenv("EXACTA_HIP_COPY_CONSTANTS");
-    const bool by_launch = !own_weights && (setup.total_eq || setup.ones_len) && c.host_pinned_dev &&
+    const bool by_launch = (own_weights || setup.total_eq || setup.ones_len) && c.host_pinned_dev &&
                            !(copy_constants && copy_constants[0] == '1');
-    if (!by_launch)
+    if (by_launch && own_weights)
+      staged_words = setup_words + up_words;
+    else if (!by_launch)
       EXH_HIP(hipMemcpyAsync(d_weights, c.host_pinned + PIN_BEGIN, (setup_words + up_words) * 4, hipMemcpyHostToDevice,
                              c.stream));
     setup_deferred = false;
@@ -1107,7 +1117,7 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
       tail_done = false;
       continue;
     }
-    if (n_pairs <= tail_pairs(T, D) && n - j <= MAXTAIL) break;
+    if (n_pairs <= (j == 0 ? whole_pairs(T, D) : tail_pairs(T, D)) && n - j <= MAXTAIL) break;
     round = j;
     // once every workgroup of a resident grid can hold its slice of the tables in LDS, the rounds down
     // to where one workgroup suffices run in one launch
@@ -1295,7 +1305,7 @@ int SumcheckSession::launch_tail(int j, int rounds, uint32_t grid, bool first_fo
     a.first_fold = first_fold ? 1 : 0;
     a.rounds = (uint32_t)rounds;
     a.first_round = (uint32_t)j;
-    a.capacity = (uint32_t)(grid > 1 ? slice_entries : 2 * tail_pairs(T, D));
+    a.capacity = (uint32_t)(grid > 1 ? slice_entries : std::max(slice_entries, 2 * tail_pairs(T, D)));
     a.lds_bytes = (uint32_t)(T * a.capacity * D * 4);
     a.points = (uint32_t)points;
     a.ctrl = d_ctrl;
@@ -1319,6 +1329,7 @@ int SumcheckSession::launch_tail(int j, int rounds, uint32_t grid, bool first_fo
         own_entries += ((uint64_t)1 << low_bits[jj]) + ((uint64_t)1 << (n - (jj + 1) - low_bits[jj]));
       a.own = 1, a.factors = has_eq ? d_weights : nullptr, a.n_vars = (uint32_t)n, a.block_high = has_bw ? 1 : 0;
       a.lds_bytes += (uint32_t)(own_entries * D * 4);
+      if (staged_words) a.staged = c.host_pinned_dev + PIN_BEGIN, a.staged_dst = d_weights, a.staged_words = (uint32_t)staged_words;
     }
   };
   if (grid > 1 && !slice_totals_clear)  // the rounds' totals start at zero (64-bit words)

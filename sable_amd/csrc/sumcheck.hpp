@@ -121,6 +121,7 @@ struct SumcheckSession {
   int owns_arenas() const;
   bool setup_deferred = false;
   bool own_weights = false;  // the one launch that runs every round builds the weight tables itself
+  size_t staged_words = 0;   // and brings this many words of constants from the pinned staging area
   size_t setup_words = 0;
   struct {
     uint64_t total_eq = 0, ones_off = 0, ones_len = 0;

@@ -125,6 +125,11 @@ struct TailArgs {
   const uint32_t *factors;
   uint32_t n_vars, own, block_high;
   uint32_t valid;  // entries that the tables in memory hold, zeros beyond them (0: all of them; unfolded extension tables)
+  // ... and brings its constants itself: staged_words words from pinned host memory to staged_dst, where the control block,
+  // the message map, the factors and the block weights are then read (null: they are there already)
+  const uint32_t *staged;
+  uint32_t *staged_dst;
+  uint32_t staged_words;
 };
 
 template <int D>
@@ -1162,6 +1167,10 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   const uint32_t term_bits = SPREAD ? lane_bits((uint32_t)desc_terms(d)) : 0;
   const uint32_t tid = threadIdx.x, cap = args.capacity, G = gridDim.x, wg = blockIdx.x;
   const uint32_t width = (uint32_t)d.nacc * D;
+  if (args.staged) {  // (a trip over the bus for all of them)
+    for (uint32_t u = tid; u < args.staged_words; u += BLOCK) args.staged_dst[u] = args.staged[u];
+    __syncthreads();
+  }
   if (args.ctrl->round != args.first_round) return;  // an earlier launch gave up: leave the count as it is
   RunB3S tr;
   PendingAppend pending{0, 0, 0};  // (the first wavefront's)
@@ -1266,9 +1275,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   const uint32_t lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   // (every thread loads, from a clamped index: a load under a condition has to be merged with the old value as soon
   // as it is issued, which turns the prefetch into a wait for memory at the end of every round)
-  auto fetch_weight = [&](uint32_t jj, uint32_t pairs) {
-    const uint32_t me = pairs <= 64 ? lane : tid;
-    const uint64_t i = (uint64_t)wg * pairs + (me < pairs ? me : pairs - 1);
+  auto load_weight = [&](uint32_t jj, uint64_t i) {
     if (own_weights) {
       wl = load_ext<D>(own_tables + (size_t)(own_at(jj, false) + (uint32_t)(i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
       wh = args.block_high ? load_ext<D>(args.weights + (args.high_off[jj] + (i >> args.low_bits[jj])) * D)
@@ -1277,6 +1284,10 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     }
     wl = load_ext<D>(args.weights + (args.low_off[jj] + (i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
     wh = load_ext<D>(args.weights + (args.high_off[jj] + (i >> args.low_bits[jj])) * D);
+  };
+  auto fetch_weight = [&](uint32_t jj, uint32_t pairs) {
+    const uint32_t me = pairs <= 64 ? lane : tid;
+    load_weight(jj, (uint64_t)wg * pairs + (me < pairs ? me : pairs - 1));
   };
   // A fold of `count` outputs by r, in place: the lanes run in lockstep, so every read of a chunk of 64 comes before
   // its writes, and those land below what later chunks read.  `spread`: wavefronts 1 to 3, an output per lane (a
@@ -1460,12 +1471,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
               lo[t] = load_ext<D>(p);
               hi[t] = load_ext<D>(p + D);
             }
-          if (i >= BLOCK) {  // beyond the prefetched pair (never with the session's own tables: one launch's
-                             // rounds have a pair per thread at most)
-            const uint64_t gi = (uint64_t)wg * pairs + i;
-            wl = load_ext<D>(args.weights + (args.low_off[jj] + (gi & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
-            wh = load_ext<D>(args.weights + (args.high_off[jj] + (gi >> args.low_bits[jj])) * D);
-          }
+          if (i >= BLOCK) load_weight(jj, (uint64_t)wg * pairs + i);  // beyond the prefetched pair
           accumulate_pair<D, Ext<D>>(d, lo, hi, ext_mul_mont<D>(wl, wh), acc, args.consts);
         }
         if (more && !next_spread) fetch_weight(jj + 1, pairs / 2);

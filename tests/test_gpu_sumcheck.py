@@ -425,6 +425,40 @@ def test_a_small_session_builds_its_weight_tables_in_its_one_launch(form, names,
         t.free()
 
 
+@pytest.mark.parametrize("form,names,cnames,d,n,K,base,with_eq", [
+    ("(* t0 t1)", ["t0", "t1"], [], 4, 10, 1, True, True),   # 512 pairs: two a thread
+    ("(* t0 t1)", ["t0", "t1"], [], 4, 10, 1, False, False),
+    ("(* t0 t1)", ["t0", "t1"], [], 4, 11, 1, False, False),  # one more: a grid for the first rounds
+    ("(* t0 t1)", ["t0", "t1"], [], 4, 8, 3, False, True),    # 384 pairs, block weights
+    ("(* t0 t1)", ["t0", "t1"], [], 4, 6, 9, True, False),    # 288 pairs, 31 of a wavefront's lanes in the second trip idle
+    (*GKR2, 4, 9, 1, False, True),  # eight tables: 256 pairs and 64 KiB of them
+    (*GKR2, 4, 7, 3, False, True),
+    ("(+ (* a t0 t1) (* a t2 t3) (* a t1 t2) (* 3 t0))", T4, ["a"], 4, 10, 1, True, True),  # on the interpreter
+    ("(* t0 t1)", ["t0", "t1"], [], 8, 9, 1, False, False),   # 256 pairs at F_p^8, all ones
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 5, 4, True, True),
+])
+def test_a_session_of_one_launch(form, names, cnames, d, n, K, base, with_eq, monkeypatch):
+    """The most pairs that a session's one launch takes, two a thread at F_p^4, with an eq point or all ones, with block
+    weights or without, its constants brought by the launch or by a copy: the oracle's proof."""
+    rng = np.random.default_rng(n * 37 + d + K)
+    tables = [rng.integers(0, P, K << n, dtype=np.uint32) if base else rand_ext(rng, (K << n,), d) for _ in names]
+    eq = rand_ext(rng, (n,), d) if with_eq else None
+    consts = rand_ext(rng, (len(cnames),), d) if cnames else None
+    bw = rand_ext(rng, (K,), d) if K > 1 else None
+    for copy in ("0", "1"):
+        monkeypatch.setenv("EXACTA_HIP_COPY_CONSTANTS", copy)
+        st, _, proof, _ = prove_both("whole", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames,
+                                     block_weights=bw)
+    monkeypatch.setenv("EXACTA_HIP_COPY_CONSTANTS", "0")
+    dev = [sa.Table.upload(t) for t in tables]
+    out = {}
+    launched = launch_names(lambda: out.setdefault("got", sa.prove(sa.Transcript("whole", d), n, st, dev, eq=eq,
+                                                                   constants=consts, block_weights=bw)))
+    assert (len(launched) == 1) == (n < 11), launched
+    for t in dev:
+        t.free()
+
+
 @pytest.mark.parametrize("form,names,d,n,base,with_eq", [
     ("(* t0 t1 t2)", ["t0", "t1", "t2"], 4, 17, True, True),
     ("(* t0 t1)", ["t0", "t1"], 8, 12, False, True),
