@@ -5,8 +5,8 @@
 // F_p[w]/(w^D - 3).  Products go through 32-bit Montgomery reduction (R = 2^32): mont_mul(a, b) is
 // a b / R, so a caller that wants the exact product passes one operand pre-multiplied by R, or
 // corrects a whole sum afterwards by a power of R.  Sums of products are accumulated unreduced
-// (four products below p^2 fit 64 bits, as in src/field.lisp:213-218; longer sums use a 96-bit
-// accumulator) and reduced once.
+// (four products below p^2 fit 64 bits, as in src/field.lisp:213-218; longer sums are kept below
+// p 2^32 a step at a time, or in a 96-bit accumulator where base values are weighed) and reduced once.
 #pragma once
 // (a run-time compilation of these kernels has the runtime's declarations built in and no host headers)
 #if !defined(__HIPCC_RTC__)

@@ -2,10 +2,11 @@
 //
 // One launch does, for every pair i of the tables being summed,
 //   [FOLD]  bind the previous round's variable: read four entries per table, write the two folded
-//           entries lo + r (hi - lo) (src/sumcheck.lisp:84-104), and use them as the pair;
+//           entries lo + r (hi - lo) (src/sumcheck.lisp:84-104), and use them as the pair (or bind two
+//           or three variables of the base tables at once, src/sumcheck.lisp:496-510);
 //   sums    for every group g of the statement (a product of tables) and each of its evaluation
 //           points X:  acc[g, X] += LOW[l] * prod_{t in g} line_t(X),  line_t(X) = lo + X (hi - lo),
-//           i = h |LOW| + l  (src/sumcheck.lisp:230-257), unreduced in 96-bit accumulators;
+//           i = h |LOW| + l  (src/sumcheck.lisp:230-257), in lazily reduced 64-bit accumulators;
 //   then reduces the accumulators over the workgroup (cross-lane, then LDS), multiplies by HIGH[h]
 //   and writes one partial per workgroup.  A second small kernel adds the partials.
 //
