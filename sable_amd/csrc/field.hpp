@@ -315,9 +315,10 @@ __device__ __forceinline__ double f_mul(double a, double b) {
 __device__ __forceinline__ double f_scale(double x, uint32_t c) {
   return c == 1 ? x : c == P - 1 ? -x : f_mul(x, c > P / 2 ? (double)c - F_P : (double)c);
 }
-// a residue of v below 2^32 as an integer, for |v| < p + 2^28: v + p sits in the low word of v + p + 1.5 * 2^52
-__device__ __forceinline__ uint32_t f_residue32(double v) {
-  return (uint32_t)__double_as_longlong(v + (F_P + F_MAGIC));
+// the canonical residue of an integer |v| < p: the low word of v + MAGIC is v mod 2^32, and p above it wraps below it when v < 0
+__device__ __forceinline__ uint32_t f_small_canonical(double v) {
+  const uint32_t r = (uint32_t)__double_as_longlong(v + F_MAGIC);
+  return umin32(r, r + P);
 }
 // the canonical residue of an integer |v| < 2^80
 __device__ __forceinline__ uint32_t f_canonical(double v) {
