@@ -593,8 +593,12 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
   // the step that forms their weights, and the one-workgroup launch the last round's pairs (and the tables over the block
   // index): beyond that a layer is two device-driven sumchecks with a wait each, as below.  That way and this one, us: three
   // blocks of 2^14 and two lookups 1900 and 1310, five of 2^10 1100 and 745, 64 of 2^8 1130 and 830, 33 of 2^10 and three
-  // lookups 3900 and 2330.
+  // lookups 3900 and 2330.  The chain holds every layer's tables at once, as many bytes as the tree again: where there is no
+  // room for them the layers go one at a time as well (nothing has been sent by then).
   if (chains && n >= 2 && n - 2 <= MAXROUNDS && (K == 1 || blocks_chain(K, L, D))) {
+    DeviceBuffers held;
+    uint32_t *d_top = K > 1 ? held.alloc(2 * Kp * 2 * L * D) : nullptr;
+    uint32_t *d_halves = K > 1 ? held.alloc((uint64_t)NT * K * (((uint64_t)1 << (n - 1)) - 1) * D) : nullptr;
     ChainTables tables;
     auto halves = [&](const std::vector<const uint32_t *> &vectors, uint64_t size) {  // with one block they are views
       std::vector<const uint32_t *> tabs(NT);
@@ -604,13 +608,10 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
     if (K == 1) {
       tables.roots = layers[0];
       for (int layer = 0; layer < n - 1; layer++) tables.layers.push_back(halves(layers[layer + 1], (uint64_t)1 << layer));
+    } else if (!d_top || !d_halves) {
+      status = E_NOMEM;
     } else {
       // the tree over the block index, its lowest layer padded with 0 / 1 (2^lk roots)
-      uint32_t *d_top = bufs.alloc(2 * Kp * 2 * L * D), *d_halves = bufs.alloc((uint64_t)NT * K * (((uint64_t)1 << (n - 1)) - 1) * D);
-      if (!d_top || !d_halves) {
-        set_error("device-out-of-memory: the layers' tables");
-        return E_NOMEM;
-      }
       ReduceTopArgs a;
       memset(&a, 0, sizeof(a));
       a.m_top = lk - 1, a.valid = (uint32_t)K;
@@ -643,9 +644,15 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
         tables.layers.push_back(tabs);
       }
     }
-    status = D == 4 ? prove_upper_chained<4>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq)
-                    : prove_upper_chained<8>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq);
-    return status;
+    if (status == OK)
+      status = D == 4 ? prove_upper_chained<4>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq)
+                      : prove_upper_chained<8>(tr, n, K, lk, L, tables, label, out_ri, out_rb, out_cp, out_cq);
+    if (status != E_NOMEM || K == 1) return status;
+  }
+  if (status == E_NOMEM) {
+    (void)hipGetLastError();  // (the refused allocation's)
+    c.pool.trim();
+    status = OK;
   }
   // the per-block roots, and the top tree over the block index on the host (2^lk entries)
   std::vector<std::vector<std::vector<uint32_t>>> top(lk + 1, std::vector<std::vector<uint32_t>>(2 * L));
