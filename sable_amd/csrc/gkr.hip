@@ -257,19 +257,28 @@ int send_finals(Transcript &tr, int D, int ntables, const uint32_t *finals, hf::
   return OK;
 }
 
-struct DeviceBuffers {  // frees what it allocated when the proof ends
+// Frees what it allocated when the proof, or the part of it that the object belongs to, ends.
+// (EXACTA_HIP_GKR_BUFFER_LIMIT=<bytes>, for tests: a thread's proof holds no more than that at a time, as if the device
+// had no room for more.)
+struct DeviceBuffers {
+  static thread_local uint64_t live;  // bytes that the thread's objects hold
+  uint64_t bytes = 0;
   std::vector<void *> owned;
   ~DeviceBuffers() {
     for (void *p : owned) ctx().pool.release(p);
+    live -= bytes;
   }
   uint32_t *alloc(uint64_t words) {
+    const char *limit = getenv("EXACTA_HIP_GKR_BUFFER_LIMIT");
+    if (limit && live + words * 4 > strtoull(limit, nullptr, 10)) return nullptr;
     void *p = ctx().pool.alloc(words * 4);
     if (!p) return nullptr;
     owned.push_back(p);
+    bytes += words * 4, live += words * 4;
     return (uint32_t *)p;
   }
 };
-
+thread_local uint64_t DeviceBuffers::live = 0;
 
 constexpr size_t GKR_BW_PIN = 8192, GKR_BW_PIN_WORDS = 1024;  // words of the context's pinned buffer (see below)
 
@@ -594,7 +603,8 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
   // index): beyond that a layer is two device-driven sumchecks with a wait each, as below.  That way and this one, us: three
   // blocks of 2^14 and two lookups 1900 and 1310, five of 2^10 1100 and 745, 64 of 2^8 1130 and 830, 33 of 2^10 and three
   // lookups 3900 and 2330.  The chain holds every layer's tables at once, as many bytes as the tree again: where there is no
-  // room for them the layers go one at a time as well (nothing has been sent by then).
+  // room for them the layers go one at a time as well (nothing has been sent by then), in the largest one's memory, half of
+  // that.
   if (chains && n >= 2 && n - 2 <= MAXROUNDS && (K == 1 || blocks_chain(K, L, D))) {
     DeviceBuffers held;
     uint32_t *d_top = K > 1 ? held.alloc(2 * Kp * 2 * L * D) : nullptr;
@@ -653,6 +663,16 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
     (void)hipGetLastError();  // (the refused allocation's)
     c.pool.trim();
     status = OK;
+  }
+  // With several blocks a layer's halves and the blocks' values after its rounds, in memory that the layers take in turn (a
+  // layer's launches are done before the next one's are enqueued); had before anything is sent.
+  uint32_t *d_halves = nullptr, *d_blk = nullptr;
+  if (K > 1 && n >= 2) {
+    d_halves = bufs.alloc(((uint64_t)NT * K << (n - 2)) * D), d_blk = bufs.alloc((uint64_t)(NT + 1) * Kp * D);
+    if (!d_halves || !d_blk) {
+      set_error("device-out-of-memory: the tables of a layer of several blocks");
+      return E_NOMEM;
+    }
   }
   // the per-block roots, and the top tree over the block index on the host (2^lk entries)
   std::vector<std::vector<std::vector<uint32_t>>> top(lk + 1, std::vector<std::vector<uint32_t>>(2 * L));
@@ -772,7 +792,7 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
       const uint64_t n_out = K * size;
       HalvesArgs h;
       memset(&h, 0, sizeof(h));
-      if (!(h.out = bufs.alloc((uint64_t)NT * n_out * D))) return E_NOMEM;
+      h.out = d_halves;
       h.size_bits = (uint32_t)layer, h.n_out = n_out;
       for (int i = 0; i < 2 * L; i++) {
         h.v[i] = layers[layer + 1][i];
@@ -788,10 +808,6 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
     }
     // With several blocks the folded tables (one entry per block) stay on the device, zero padded to 2^lk, as the
     // tables of the sumcheck over the block index; the weights, padded alike, go before them in one copy.
-    uint32_t *d_blk = nullptr;
-    if (lk > 0) {
-      if (!(d_blk = bufs.alloc((uint64_t)(NT + 1) * Kp * D))) return E_NOMEM;
-    }
     status = sumcheck_prove(tr, layer, st, tabs.data(), strides.data(), layer > 0 ? ri.data() : nullptr,
                             consts.data(), label, bw.data(), K, layer > 0 ? 2 : 0, rho.data(),
                             lk > 0 ? nullptr : finals.data(), nullptr, lk > 0 ? d_blk + Kp * D : nullptr, Kp);

@@ -148,6 +148,41 @@ def test_layers_of_several_blocks_chained_and_host_driven(n, k, lookups, d, monk
         p.free(), q.free()
 
 
+@pytest.mark.parametrize("n,k,lookups,d", [(11, 2, 1, 4), (11, 3, 2, 4), (10, 5, 3, 4), (10, 64, 1, 4), (9, 3, 1, 8)])
+def test_layers_of_several_blocks_without_room_for_all_of_them(n, k, lookups, d, monkeypatch):
+    """Room for the largest layer's tables but not for every layer's, as the chain holds them, or for those and not for the
+    chain's own buffers: the oracle's proof all the same.  Without room for a layer the proof is refused before anything is
+    sent, and goes through with the same transcript afterwards."""
+    rng = np.random.default_rng(100 * n + k)
+    leaves = random_leaves(rng, lookups, n, k, d)
+    dev = [(sa.Table.upload(p), sa.Table.upload(q)) for p, q in leaves]
+    otr = orc.Transcript("gkr-test", d)
+    want = orc.gkr_prove_upper(otr, n, k, leaves)
+    padded = 1 << (k - 1).bit_length()
+    largest, every = 16 * lookups * (k << (n - 2)) * d, 16 * lookups * k * ((1 << (n - 1)) - 1) * d
+    top, blocks = 16 * lookups * padded * d, 4 * (4 * lookups + 1) * padded * d
+    most = largest + blocks + 40000  # (and the log and the state of the tree over the block index)
+    assert most < every
+    for limit in (most, top + every + 4):
+        monkeypatch.setenv("EXACTA_HIP_GKR_BUFFER_LIMIT", str(limit))
+        tr = sa.Transcript("gkr-test", d)
+        got = sa.prove_upper(tr, n, k, dev)
+        assert tr.proof() == otr.proof() and tr.state_digest() == otr.state_digest()
+        for a, b in zip(got, want):
+            assert same(a, b)
+    tr = sa.Transcript("gkr-test", d)
+    start = (tr.proof(), tr.state_digest())
+    monkeypatch.setenv("EXACTA_HIP_GKR_BUFFER_LIMIT", str(largest - 4))
+    with pytest.raises(sa.ExactaError):
+        sa.prove_upper(tr, n, k, dev)
+    assert (tr.proof(), tr.state_digest()) == start
+    monkeypatch.delenv("EXACTA_HIP_GKR_BUFFER_LIMIT")
+    sa.prove_upper(tr, n, k, dev)
+    assert tr.proof() == otr.proof()
+    for p, q in dev:
+        p.free(), q.free()
+
+
 # two trees side by side (a second host thread, stream and workspace): each proof's bytes, outputs and final
 # transcript state are those of the call on its own; pairs of different sizes, both chained, one host-driven
 # (several blocks), both large enough for the grids of slices that must share the device
