@@ -69,8 +69,13 @@ __global__ __launch_bounds__(BLOCK) void gkr_reduce_kernel(ReduceArgs a) {
 
 // The layers m_top .. 0 of a block of a lookup's tree, in one workgroup (block blockIdx.x of lookup blockIdx.y): layer m
 // has 2^m <= BLOCK parents, a thread takes one, and the workgroup's barrier stands between a layer's writes and the next
-// one's reads.  (A launch per layer is 4 us each for a few hundred products.)
+// one's reads: nobody else reads them in this launch, so they need not leave the compute unit's XCD.  (With a device-wide
+// fence every workgroup writes back its L2 behind every layer: blocks of 2^8, 64 of them 47 us and 16.5 without, 1024 of them
+// 546 and 13.6; 16384 blocks of 2^4 3860 and 50.)  A launch per layer is 4 us each for a few hundred products; blocks beyond
+// what the device holds at once are enough to fill it and leave most of a workgroup idle: 4096 of 2^4 16.6 us here and 8.5 in
+// two launches, 16384 50 and 10, but 1024 of 2^8 13.6 here and 18.2 in four launches (REDUCE_TOP_BLOCKS).
 constexpr int REDUCE_TOP_LAYERS = 9;     // m_top <= 8: 256 parents
+constexpr int REDUCE_TOP_BLOCKS = 2048;  // eight workgroups a compute unit
 struct ReduceTopArgs {
   // layer m_top + 1; where the tree over the block index begins, `valid` roots (the others are 0 / 1) that go to pad_p,
   // pad_q with them (else null: every child is there)
@@ -90,7 +95,6 @@ __global__ __launch_bounds__(BLOCK) void gkr_reduce_top_kernel(ReduceTopArgs a) 
       store_ext<D>(a.pad_p[l] + o * D, o < a.valid ? load_ext<D>(p + o * D) : ext_zero<D>());
       store_ext<D>(a.pad_q[l] + o * D, o < a.valid ? load_ext<D>(q + o * D) : ext_lift<D>(1));
     }
-    __threadfence();
     __syncthreads();
     p = a.pad_p[l], q = a.pad_q[l];
   }
@@ -101,7 +105,6 @@ __global__ __launch_bounds__(BLOCK) void gkr_reduce_top_kernel(ReduceTopArgs a) 
       const Fraction<D> f0 = load_fraction<D>(p, q, c0), f1 = load_fraction<D>(p, q, c0 + half);
       store_fraction<D>(a.pp[l][m], a.qq[l][m], o, add_fractions<D>(f0, f1));
     }
-    __threadfence();
     __syncthreads();
     p = a.pp[l][m], q = a.qq[l][m];
   }
@@ -555,7 +558,8 @@ int gkr_prove_upper(Transcript &tr, int n, int K, int L, const uint32_t *const *
   // one allocation holds every layer above the leaves: 2 L K (2^n - 1) entries
   if ((status = c.tree.reserve(((((uint64_t)K << n) - K) * 2 * L * D + 64) * 4))) return status;
   uint32_t *next = (uint32_t *)c.tree.ptr;
-  const int m_top = std::min(n - 1, REDUCE_TOP_LAYERS - 1);  // these layers in one launch
+  // these layers in one launch (-1: none)
+  const int m_top = (uint64_t)K * L <= (uint64_t)REDUCE_TOP_BLOCKS ? std::min(n - 1, REDUCE_TOP_LAYERS - 1) : -1;
   for (int m = n - 1; m >= 0; m--)
     for (int l = 0; l < L; l++) {
       uint64_t words = ((uint64_t)K << m) * D;

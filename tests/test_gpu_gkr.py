@@ -102,6 +102,22 @@ def test_several_blocks_on_the_grid_of_slices_and_on_the_streaming_rounds(n, k, 
         p.free(), q.free()
 
 
+@pytest.mark.parametrize("n,k,lookups,d", [(1, 2048, 1, 4), (3, 2048, 1, 4), (3, 2049, 1, 4), (2, 1024, 2, 4), (2, 1025, 2, 4),
+                                           (1, 2049, 1, 8), (4, 2100, 1, 8)])
+def test_many_small_blocks_match_the_oracle(n, k, lookups, d):
+    """Either side of the most blocks whose trees' upper layers are one launch, odd and even layers in the two-layer launches."""
+    rng = np.random.default_rng(10 * n + k)
+    leaves = random_leaves(rng, lookups, n, k, d)
+    dev = [(sa.Table.upload(p), sa.Table.upload(q)) for p, q in leaves]
+    tr, otr = sa.Transcript("gkr-test", d), orc.Transcript("gkr-test", d)
+    got, want = sa.prove_upper(tr, n, k, dev), orc.gkr_prove_upper(otr, n, k, leaves)
+    assert tr.proof() == otr.proof()
+    for a, b in zip(got, want):
+        assert same(a, b)
+    for p, q in dev:
+        p.free(), q.free()
+
+
 @pytest.mark.parametrize("n,lookups,d", [(9, 1, 4), (6, 2, 4), (8, 1, 8), (7, 3, 4)])
 def test_the_chained_layers_and_the_host_driven_layers_send_the_same_bytes(n, lookups, d, monkeypatch):
     rng = np.random.default_rng(100 + n)
