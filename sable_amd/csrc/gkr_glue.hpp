@@ -249,7 +249,7 @@ __global__ __launch_bounds__(64) void gkr_glue_kernel(GlueArgs<D> a) {
 template <int D, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(1, 1))) void tail_glue_kernel(TailArgs<D> t,
                                                                                                     GlueArgs<D> g) {
-  tail_body<D>(S::d, t);
+  tail_body<D, Tail::WHOLE>(S::d, t);
   __syncthreads();
   if (threadIdx.x < 64) gkr_glue_body<D>(g);
 }

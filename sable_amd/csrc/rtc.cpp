@@ -120,7 +120,8 @@ void compile_part(Job *job, Part *part) {
 // the one-workgroup kernel of a statement: with half the registers for a statement in direct form at F_p^8 (see
 // tail_kernel_narrow)
 std::string tail_expression(int D, bool direct) {
-  return std::string(direct && D == 8 ? "exh::tail_kernel_narrow<" : "exh::tail_kernel<") + std::to_string(D) + ", exh::RtStmt>";
+  return direct && D == 8 ? "exh::tail_kernel_narrow<8, exh::RtStmt>"
+                          : "exh::tail_kernel<" + std::to_string(D) + ", exh::RtStmt, exh::Tail::EITHER>";
 }
 
 // the kernel behind launcher arguments passed by value as one struct

@@ -1150,11 +1150,21 @@ struct LaneBit {
   static constexpr int value = M;
 };
 
+// A launch of LDS-resident rounds is part of a proof -- the grid of slices, or one workgroup with the last rounds -- or a
+// session as a whole in one workgroup, which brings its constants, builds its weight tables and pads its tables.  A
+// statement's own kernels are two, one for each: the launches of a chain wait for their instructions, and the parts of a
+// proof without the session's code are 2 to 5 % shorter (us, one kernel for both and two: slices of 2^16 50.8 and 49.9, of
+// 2^19 at four tables 103.6 and 101.3, of a fraction tree's layers 51.0 and 49.9 on average; a layer's last launch with the
+// step behind it 44.2 and 42.5; a session of 2^10 55.8 and 53.6).  Not the grid and the one workgroup behind it as two: its
+// instructions then come from memory when the streaming rounds before have used up the caches (last rounds of three tables of
+// 2^24 47.5 and 53.4).  EITHER: one kernel for both, where it is compiled at run time or runs any statement.
+enum class Tail { ROUNDS, WHOLE, EITHER };
+
 // Load (folding or lifting on the way in) into LDS, then per round sums -> message -> challenge -> fold
 // on the slice this workgroup holds: entries [w * E, (w + 1) * E) of every table, E = entries / grid.
 // A grid launch ends when its rounds are done and leaves the slices in `out` for the one-workgroup
 // launch that follows; that one ends with the finals.
-template <int D, class Desc>
+template <int D, Tail KIND, class Desc>
 __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args) {
   extern __shared__ __align__(16) uint32_t tail_tables[];  // [T][capacity][D]
   __shared__ uint32_t lds[BLOCK / 64][MAXACC * D];
@@ -1166,9 +1176,11 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   __shared__ SpreadUnit units[SPREAD ? SPREAD_UNITS : 1];
   // (products of an accumulator: as many lanes each as the next power of two)
   const uint32_t term_bits = SPREAD ? lane_bits((uint32_t)desc_terms(d)) : 0;
-  const uint32_t tid = threadIdx.x, cap = args.capacity, G = gridDim.x, wg = blockIdx.x;
+  constexpr bool SESSION = KIND != Tail::ROUNDS;
+  const uint32_t tid = threadIdx.x, cap = args.capacity, G = KIND == Tail::WHOLE ? 1 : gridDim.x,
+                 wg = KIND == Tail::WHOLE ? 0 : blockIdx.x;
   const uint32_t width = (uint32_t)d.nacc * D;
-  if (args.staged) {  // (a trip over the bus for all of them)
+  if (SESSION && args.staged) {  // (a trip over the bus for all of them)
     for (uint32_t u = tid; u < args.staged_words; u += BLOCK) args.staged_dst[u] = args.staged[u];
     __syncthreads();
   }
@@ -1205,7 +1217,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
             }
           } else if (args.first_fold) {
             v = fold_ext<D>(load_ext<D>(in + 2 * gx * D), load_ext<D>(in + (2 * gx + 1) * D), r);
-          } else if (args.valid && gx >= args.valid) {
+          } else if (SESSION && args.valid && gx >= args.valid) {
             v = ext_zero<D>();
           } else {
             v = load_ext<D>(in + gx * D);
@@ -1232,7 +1244,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // The session's own weight tables (see TailArgs::factors), in LDS behind the tables: the factors first, then
   // per round its LOW and its HIGH table.  An entry is a chain of at most n_vars products, one entry per thread
   // and trip: entry x of a table over the variables [first, first + bits) is prod_b (x_b ? r_b : 1 - r_b).
-  const bool own_weights = args.own != 0;
+  const bool own_weights = SESSION && args.own != 0;
   uint32_t *const own_factors = tail_tables + (size_t)d.T * cap * D;
   uint32_t *const own_tables = own_factors + (size_t)2 * args.n_vars * D;
   auto own_high_bits = [&](uint32_t jj) { return args.n_vars - (args.first_round + jj + 1) - args.low_bits[jj]; };
@@ -1986,16 +1998,16 @@ template <int D, bool IN_BASE, bool FOLD, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel(RoundArgs<D> args) {
   round_body<D, IN_BASE, FOLD ? 1 : 0, decltype(S::d), true>(S::d, args);
 }
-template <int D, class S>
+template <int D, class S, Tail KIND>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(1, 1))) void tail_kernel(TailArgs<D> args) {
-  tail_body<D>(S::d, args);
+  tail_body<D, KIND>(S::d, args);
 }
 // (the same with half the registers: a statement in direct form at F_p^8 needs more than the 512 either way, and the
 // compiler's use of the upper half of the register file for 64-bit values that it also spills has been seen to end
 // in registers it then rejects)
 template <int D, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void tail_kernel_narrow(TailArgs<D> args) {
-  tail_body<D>(S::d, args);
+  tail_body<D, Tail::EITHER>(S::d, args);
 }
 // base tables folded by the first FOLDS = 2 or 3 challenges at once, see round_core; without tables to write (out[0] null)
 // only the sums are taken
@@ -2015,7 +2027,7 @@ __global__ __launch_bounds__(BLOCK) void round_kernel_interp(RoundArgs<D> args, 
 }
 template <int D>
 __global__ __launch_bounds__(BLOCK) void tail_kernel_interp(TailArgs<D> args, StmtDesc d) {
-  tail_body<D>(d, args);
+  tail_body<D, Tail::EITHER>(d, args);
 }
 
 }  // namespace exh
