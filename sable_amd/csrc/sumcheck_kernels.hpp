@@ -1646,17 +1646,12 @@ struct NodesArgs {
   NodesEpilogueArgs epi;
 };
 
-// p 2^32 off a 64-bit sum below 2 p 2^32 that has reached it: hi - p wraps above hi when hi < p
-__device__ __forceinline__ uint64_t lazy_lower(uint64_t acc) {
-  const uint32_t hi = (uint32_t)(acc >> 32);
-  return ((uint64_t)umin32(hi, hi - P) << 32) | (uint32_t)acc;
-}
 // A 64-bit accumulator of 32 x 32-bit products kept below p 2^32 by a conditional subtraction of p from its high
 // word after every product: acc < p 2^32, the product of a canonical weight and a residue below 2^32 is below
 // p 2^32 as well, so the sum is below 2^64, and min(hi, hi - p) brings it back (hi < p: hi - p wraps above hi).
 // Eight registers per slot at F_p^4 where the 96-bit form takes twelve, for one more (cheap) instruction per word.
 __device__ __forceinline__ void lazy_mad(uint64_t &acc, uint32_t w, uint32_t v) {
-  acc = lazy_lower((uint64_t)w * v + acc);
+  acc = mont_lazy((uint64_t)w * v + acc);
 }
 __device__ __forceinline__ uint32_t lazy_reduce(uint64_t acc) {
   Acc96 a;
@@ -1931,7 +1926,7 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
 #pragma unroll
       for (int a = 0; a < SPP; a++)
 #pragma unroll
-        for (int c = 0; c < D; c++) acc[a][c] = lazy_lower(acc[a][c]);
+        for (int c = 0; c < D; c++) acc[a][c] = mont_lazy(acc[a][c]);
     }
   }
 
