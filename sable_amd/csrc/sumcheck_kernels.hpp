@@ -1157,8 +1157,8 @@ struct LaneBit {
 // 2^19 at four tables 103.6 and 101.3, of a fraction tree's layers 51.0 and 49.9 on average; a layer's last launch with the
 // step behind it 44.2 and 42.5; a session of 2^10 55.8 and 53.6).  Not the grid and the one workgroup behind it as two: its
 // instructions then come from memory when the streaming rounds before have used up the caches (last rounds of three tables of
-// 2^24 47.5 and 53.4).  EITHER: one kernel for both, where it is compiled at run time or runs any statement.
-enum class Tail { ROUNDS, WHOLE, EITHER };
+// 2^24 47.5 and 53.4).  EITHER: one kernel for both, where it is compiled at run time; INTERPRETER: for any statement.
+enum class Tail { ROUNDS, WHOLE, EITHER, INTERPRETER };
 
 // Load (folding or lifting on the way in) into LDS, then per round sums -> message -> challenge -> fold
 // on the slice this workgroup holds: entries [w * E, (w + 1) * E) of every table, E = entries / grid.
@@ -1334,8 +1334,17 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // the interpreter gains most (six groups, n = 12: 497 and 683; one group of six factors, n = 10: 428 and 767), the
   // kernels of a statement's own are about even (a launch over GKR layers: one lookup 28.2 and 27.6, two 34.2 and 34.7,
   // three 52.6 and 53.4 with the glue, 57.0 and 51.2 without; over the blocks of two lookups 21.5 and 25.3).
-  auto spreads = [&](uint32_t pairs) {
+  // An accumulator's products are on lanes of their own; in the interpreter, where they do not all fit, a lane takes them
+  // one after the other: a round beyond that costs it 25 us (three products of one coefficient and a table, a proof of 2^8
+  // 175 us and 237 without, of 2^15 469 and 597; 203 and 552 when every product had an accumulator of its own).  The kernels
+  // of a statement's own lose by it (three products of two tables, slices of 2^12 33.2 us and 31.6 without).
+  constexpr bool WALK = KIND == Tail::INTERPRETER;
+  auto term_lanes = [&](uint32_t pairs) {
     const uint32_t bits = lane_bits(pairs) + term_bits;
+    return bits > 6 || ((uint32_t)d.nacc << bits) > 192 ? 0 : term_bits;
+  };
+  auto spreads = [&](uint32_t pairs) {
+    const uint32_t bits = lane_bits(pairs) + (WALK ? term_lanes(pairs) : term_bits);
     return SPREAD && BLOCK == 256 && d.NV == 0 && bits <= 6 && ((uint32_t)d.nacc << bits) <= 192 &&
            ((uint32_t)d.nacc << term_bits) <= (uint32_t)SPREAD_UNITS;
   };
@@ -1345,7 +1354,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   auto prepare_unit = [&](uint32_t jj, uint32_t pairs) {
     const uint32_t u = tid < 64 ? 0 : tid - 64;
     // (an accumulator's lanes: the pairs of its first product, of its second, ...)
-    const uint32_t pair_bits = lane_bits(pairs), bits = pair_bits + term_bits;
+    const uint32_t pair_bits = lane_bits(pairs), bits = pair_bits + (WALK ? term_lanes(pairs) : term_bits);
     unit_a = u >> bits, unit_lane = u & ((1u << bits) - 1), unit_pair = unit_lane & ((1u << pair_bits) - 1);
     const SpreadUnit &unit = units[unit_a < (uint32_t)d.nacc ? (unit_a << term_bits) + (unit_lane >> pair_bits) : 0];
     unit_deg = unit.deg, unit_x = unit.x;
@@ -1387,10 +1396,20 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
       if (j < maxdeg) {
         if ((uint32_t)j < unit_deg) f = ext_mul_mont<D>(f, factor(unit_table[j]));
       }
+    if constexpr (WALK) {
+      if (term_lanes(pairs) < term_bits && unit_a < (uint32_t)d.nacc)  // (of one degree and one evaluation point)
+        for (uint32_t term = 1; term < 1u << term_bits; term++) {
+          const SpreadUnit &unit = units[(unit_a << term_bits) + term];
+          if (unit.deg == 0) break;
+          Ext<D> g = factor(unit.table[0]);
+          for (uint32_t j = 1; j < unit.deg; j++) g = ext_mul_mont<D>(g, factor(unit.table[j]));
+          f = ext_add<D>(f, g);
+        }
+    }
     f = ext_mul_mont<D>(f, unit_w);
     // Over the pairs, the low lane bits of a unit: the words are halved as long as there are several.  Bit 2 comes first:
     // its partner is the opposite lane of a group of 8, which still holds the same words then (see lane_partner).
-    const uint32_t lanes = 1u << (lane_bits(pairs) + term_bits);
+    const uint32_t lanes = 1u << (lane_bits(pairs) + (WALK ? term_lanes(pairs) : term_bits));
     uint32_t v[D], word = 0, count = D, keys = 0;
 #pragma unroll
     for (int c = 0; c < D; c++) v[c] = f.c[c];
@@ -2022,7 +2041,7 @@ __global__ __launch_bounds__(BLOCK) void round_kernel_interp(RoundArgs<D> args, 
 }
 template <int D>
 __global__ __launch_bounds__(BLOCK) void tail_kernel_interp(TailArgs<D> args, StmtDesc d) {
-  tail_body<D, Tail::EITHER>(d, args);
+  tail_body<D, Tail::INTERPRETER>(d, args);
 }
 
 }  // namespace exh

@@ -365,6 +365,24 @@ def test_products_that_share_a_sum(form, names, cnames, d, n, base, monkeypatch)
         t.free()
 
 
+@pytest.mark.parametrize("d,n,K", [(4, 5, 3), (4, 6, 1), (4, 4, 17), (8, 5, 3), (8, 7, 1)])
+@pytest.mark.parametrize("form", [
+    "(+ (* a t0 t1) (* a t2 t3) (* a t1 t2) (* 3 t0))",  # three products of one sum, and a sum of one
+    "(+ (* a t0 t1) (* a t2 t3) (* a t1 t2) (* a t0 t3) (* a t0 t2))",  # four, the most of one sum, and one
+    "(+ (* t0 t1 t2) (* t1 t2 t3) (* 5 t2 t3) (* 5 t0 t3))"])
+def test_the_interpreter_walks_the_products_of_a_sum(form, d, n, K):
+    """Rounds whose products of shared sums are more than the lanes of three wavefronts, but not their sums: a lane takes the
+    products one after the other; then the rounds where they have lanes of their own.  Pairs that are no power of two."""
+    rng = np.random.default_rng(n * 29 + d + K)
+    cnames = ["a"] if "(* a" in form else []
+    tables = [rand_ext(rng, (K << n,), d) for _ in T4]
+    tables[0][...] = P - 1
+    st, *_ = prove_both("walk", d, n, form, T4, tables, eq=rand_ext(rng, (n,), d), cnames=cnames,
+                        constants=rand_ext(rng, (len(cnames),), d) if cnames else None,
+                        block_weights=rand_ext(rng, (K,), d) if K > 1 else None)
+    assert not st.has_generated_kernel(d)
+
+
 @pytest.mark.parametrize("form,names,cnames,d,n,K,base", [
     (*GKR2, 4, 8, 3, False),  # eight tables, four held ahead; 384 and 192 pairs: a last workgroup with half its lanes
     (*GKR2, 4, 10, 1, True),
