@@ -140,7 +140,7 @@ const KernelSet *find_kernels(const std::string &key, int D) {
 // ------------------------------------------------------------------ the session
 // regions of the context's pinned host buffer (in words): per-round results | the session's eq point
 // and block weights | the device loop's constants | the device loop's logs and final tables
-constexpr uint32_t SLICE_GROUPS = 16;  // rows of totals per round of a grid launch of LDS-resident slices
+constexpr uint32_t SLICE_GROUPS = 8;   // rows of totals per round of a grid launch of LDS-resident slices (see launch_tail)
 constexpr uint32_t ROUND_GROUPS = 32;  // rows of totals of a streaming round (its workgroups' atomics spread over them)
 constexpr size_t PIN_BEGIN = 16384, PIN_BEGIN_WORDS = 4096;
 constexpr size_t PIN_LOOP = PIN_BEGIN + PIN_BEGIN_WORDS, PIN_LOOP_WORDS = 12288;
@@ -1291,8 +1291,12 @@ int SumcheckSession::launch_tail(int j, int rounds, uint32_t grid, bool first_fo
   int status = dst.reserve((size_t)T * final_size * D * 4);
   if (status) return status;
   const uint64_t slice_entries = (first_fold ? size / 2 : size) / grid;
-  // groups of workgroups share a row of totals: few enough that a workgroup polls all the rows' words at
-  // once, one per thread (a second pass of polls is a second trip to memory in every round)
+  // Groups of workgroups share a row of totals: few enough that a workgroup polls all the rows' words at once, one per thread
+  // (a second pass of polls is a second trip to memory in every round), and at most eight: the more words every workgroup
+  // polls, the longer each takes to arrive, and statements of few sums would take more rows.  Slices with 16, 8 and 4 rows at
+  // most, us: two tables of 2^16 50.3, 41.8 and 42.6; two points' reduction of 2^19 101.9, 86.6 and 88.3; three points' of
+  // 2^17 78.2, 60.1 and 61.3; the layers of a fraction tree of 2^22 50.0, 46.9 and 46.6 on average; statements of 32 words and
+  // more have eight rows or fewer either way.
   uint32_t groups = 1;
   while (groups * 2 <= SLICE_GROUPS && grid % (groups * 2) == 0 && groups * 2 * (uint32_t)st.nacc * D <= BLOCK) groups *= 2;
   auto fill = [&](auto &a) {
