@@ -359,7 +359,12 @@ def domain_leaves(dom, z, betas):
 
 def table_values(table, k, n):
     """TABLE-VALUES on the device: the Table of K 2^(n-1) base values of one sumcheck table."""
-    return tables_values([table], k, n)[0]
+    _, col, half, _, _ = table
+    keep = []
+    cs = col.c_struct(keep)
+    h = C.c_uint64()
+    check(load().exh_domain_table(C.byref(cs), -1 if half is None else half, n, k, C.byref(h)))
+    return sa.Table(h.value, k << (n - 1), 1)
 
 
 def tables_values(tables, k, n):
