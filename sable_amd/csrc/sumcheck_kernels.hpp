@@ -926,9 +926,13 @@ __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const 
   // (64 registers of words: two tables at a time of extension elements at D = 8, four at D = 4, all of them in base tables.
   // Without it, at D = 8, a table's loads waited behind the store of the table before: the largest fold round of a
   // four-table statement, 1.6 GB, took 530 us, 440 this way; more or fewer slots, 32 or 96 registers, make no difference
-  // beyond the runs'.  Whole pairs held twice, as D = 4 did, are 96 registers for three tables and spill for eight.
+  // beyond the runs'.  Whole pairs held twice are 96 registers for three tables at D = 4 and spill for eight; fold rounds of
+  // three tables and 2^21, 2^20 and 2^19 pairs one behind the other 149, 77.1 and 43.2 us that way with the arithmetic of
+  // then, 147, 74.6 and 40.6 now.  (The first launch of a kernel in a proof fetches its instructions from memory: behind the
+  // bind by three a fold round of 2^19 pairs takes 49 us, with either way of fetching.)
   // A lane without a next pair fetches the tile's first one: a load under a condition would have to be merged with
-  // what the slot held as soon as it is issued.)
+  // what the slot held as soon as it is issued.  Left out by a condition on the pair's number, which is the same for all
+  // lanes, that round takes 49.2 us for 48.6, and the fold rounds of four tables at D = 8 399 for 229 on average.)
   // The interpreter, and a statement in direct form, which is wide and calls its evaluator in a loop, keep the plain order.
   constexpr bool AHEAD = GENERATED && !is_direct<Desc>::value;
   if constexpr (AHEAD) {
@@ -1145,6 +1149,15 @@ struct SpreadUnit {
 __device__ __forceinline__ uint32_t lane_bits(uint32_t n) {  // 2^bits: the next power of two from n up
   return n <= 1 ? 0 : 32 - __builtin_clz(n - 1);
 }
+// An accumulator's products are on lanes of their own (2^term_bits); in the interpreter, where they do not all fit, a lane
+// takes them one after the other: a round beyond that costs it 25 us (three products of one coefficient and a table, a proof
+// of 2^8 175 us and 237 without, of 2^15 469 and 597; 203 and 552 when every product had an accumulator of its own).  The
+// kernels of a statement's own lose by it (three products of two tables, slices of 2^12 33.2 us and 31.6 without).  The lanes
+// of an accumulator in the interpreter:
+__device__ __forceinline__ uint32_t unit_bits(uint32_t pairs, uint32_t nacc, uint32_t term_bits) {
+  const uint32_t bits = lane_bits(pairs) + term_bits;
+  return bits > 6 || (nacc << bits) > 192 ? lane_bits(pairs) : bits;
+}
 template <int M>
 struct LaneBit {
   static constexpr int value = M;
@@ -1334,17 +1347,11 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // the interpreter gains most (six groups, n = 12: 497 and 683; one group of six factors, n = 10: 428 and 767), the
   // kernels of a statement's own are about even (a launch over GKR layers: one lookup 28.2 and 27.6, two 34.2 and 34.7,
   // three 52.6 and 53.4 with the glue, 57.0 and 51.2 without; over the blocks of two lookups 21.5 and 25.3).
-  // An accumulator's products are on lanes of their own; in the interpreter, where they do not all fit, a lane takes them
-  // one after the other: a round beyond that costs it 25 us (three products of one coefficient and a table, a proof of 2^8
-  // 175 us and 237 without, of 2^15 469 and 597; 203 and 552 when every product had an accumulator of its own).  The kernels
-  // of a statement's own lose by it (three products of two tables, slices of 2^12 33.2 us and 31.6 without).
+  // (WALK: see unit_bits.)
   constexpr bool WALK = KIND == Tail::INTERPRETER;
-  auto term_lanes = [&](uint32_t pairs) {
-    const uint32_t bits = lane_bits(pairs) + term_bits;
-    return bits > 6 || ((uint32_t)d.nacc << bits) > 192 ? 0 : term_bits;
-  };
   auto spreads = [&](uint32_t pairs) {
-    const uint32_t bits = lane_bits(pairs) + (WALK ? term_lanes(pairs) : term_bits);
+    uint32_t bits = lane_bits(pairs) + term_bits;
+    if constexpr (WALK) bits = unit_bits(pairs, (uint32_t)d.nacc, term_bits);
     return SPREAD && BLOCK == 256 && d.NV == 0 && bits <= 6 && ((uint32_t)d.nacc << bits) <= 192 &&
            ((uint32_t)d.nacc << term_bits) <= (uint32_t)SPREAD_UNITS;
   };
@@ -1354,7 +1361,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   auto prepare_unit = [&](uint32_t jj, uint32_t pairs) {
     const uint32_t u = tid < 64 ? 0 : tid - 64;
     // (an accumulator's lanes: the pairs of its first product, of its second, ...)
-    const uint32_t pair_bits = lane_bits(pairs), bits = pair_bits + (WALK ? term_lanes(pairs) : term_bits);
+    uint32_t pair_bits = lane_bits(pairs), bits = pair_bits + term_bits;
+    if constexpr (WALK) bits = unit_bits(pairs, (uint32_t)d.nacc, term_bits);
     unit_a = u >> bits, unit_lane = u & ((1u << bits) - 1), unit_pair = unit_lane & ((1u << pair_bits) - 1);
     const SpreadUnit &unit = units[unit_a < (uint32_t)d.nacc ? (unit_a << term_bits) + (unit_lane >> pair_bits) : 0];
     unit_deg = unit.deg, unit_x = unit.x;
@@ -1397,7 +1405,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
         if ((uint32_t)j < unit_deg) f = ext_mul_mont<D>(f, factor(unit_table[j]));
       }
     if constexpr (WALK) {
-      if (term_lanes(pairs) < term_bits && unit_a < (uint32_t)d.nacc)  // (of one degree and one evaluation point)
+      if (unit_bits(pairs, (uint32_t)d.nacc, term_bits) < lane_bits(pairs) + term_bits &&
+          unit_a < (uint32_t)d.nacc)  // (of one degree and one evaluation point)
         for (uint32_t term = 1; term < 1u << term_bits; term++) {
           const SpreadUnit &unit = units[(unit_a << term_bits) + term];
           if (unit.deg == 0) break;
@@ -1409,7 +1418,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     f = ext_mul_mont<D>(f, unit_w);
     // Over the pairs, the low lane bits of a unit: the words are halved as long as there are several.  Bit 2 comes first:
     // its partner is the opposite lane of a group of 8, which still holds the same words then (see lane_partner).
-    const uint32_t lanes = 1u << (lane_bits(pairs) + (WALK ? term_lanes(pairs) : term_bits));
+    uint32_t lanes = 1u << (lane_bits(pairs) + term_bits);
+    if constexpr (WALK) lanes = 1u << unit_bits(pairs, (uint32_t)d.nacc, term_bits);
     uint32_t v[D], word = 0, count = D, keys = 0;
 #pragma unroll
     for (int c = 0; c < D; c++) v[c] = f.c[c];
