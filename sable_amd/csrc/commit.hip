@@ -903,7 +903,7 @@ int merkle_levels_injected_device(const uint32_t *d_leaves, uint64_t nleaves, in
 // ------------------------------------------------------------------ BaseFold
 // DOT-PAIRS (src/pcs.lisp:473-483) for the three parities at once: sums over pairs of
 // pick(tt) pick(et), pick = even entry, odd entry, 2 odd - even.  Partials per workgroup.
-// Bound by memory: a wavefront's loads of a pair touch 16 KiB a quarter of a line at a time, and with more of them on a
+// Bound by memory: a wavefront's loads of a pair touch 8 KiB a quarter of a line at a time, and with more of them on a
 // compute unit than its L1 holds lines for, the quarters come from L2 again.  Three wavefronts a SIMD, tables of 2^22 and
 // 2^24: 51.7 and 213 us; five, as many as the registers allow, 58.7 and 266; four 75 and 278; two 54.3 and 214.
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) void dot_pairs_kernel(const uint32_t *tt, const uint32_t *et, uint64_t n_pairs,

@@ -299,8 +299,8 @@ int chain_outcome(uint32_t failed) {
   return E_DEVICE;
 }
 
-// PROVE-UPPER's in-block layers with one block, chained on the device (see gkr_glue_kernel): every launch of every
-// layer's sumcheck is enqueued at once, the host waits once and reads the log.
+// PROVE-UPPER's layers, and with several blocks the tree over the block index before them, chained on the device (see
+// gkr_glue.hpp): every launch of every sumcheck is enqueued at once, the host waits once and reads the log.
 // `held`: the finished layer's last launch (its rounds in one workgroup), not enqueued yet: the step rides on it
 // (tail_glue_kernel); empty: the step is a launch of its own.
 template <int D>
