@@ -928,8 +928,8 @@ __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const 
   // four-table statement, 1.6 GB, took 530 us, 440 this way; more or fewer slots, 32 or 96 registers, make no difference
   // beyond the runs'.  Whole pairs held twice are 96 registers for three tables at D = 4 and spill for eight; fold rounds of
   // three tables and 2^21, 2^20 and 2^19 pairs one behind the other 149, 77.1 and 43.2 us that way with the arithmetic of
-  // then, 147, 74.6 and 40.6 now.  (The first launch of a kernel in a proof fetches its instructions from memory: behind the
-  // bind by three a fold round of 2^19 pairs takes 49 us, with either way of fetching.)
+  // then, 147, 74.6 and 40.6 now.  (Behind the bind by three, the first of its kernel in a proof, a fold round of 2^19 pairs
+  // takes 49 us with either way of fetching.)
   // A lane without a next pair fetches the tile's first one: a load under a condition would have to be merged with
   // what the slot held as soon as it is issued.  Left out by a condition on the pair's number, which is the same for all
   // lanes, that round takes 49.2 us for 48.6, and the fold rounds of four tables at D = 8 399 for 229 on average.)
