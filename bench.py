@@ -45,8 +45,8 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "a33278ad9a8efe8a61d0160ab58a8dd73407036b992eb2e555812f000b421e21",
-    "traffic": {("round_nodes_base", 24): 204020103, ("round_fold2_base", 24): 202936694, ("round_fold3_base", 24): 303098916},
+    "kernel_sources_sha256": "231a00fb2cee641286b99b93aa3e3877ea67932f9a1fb3c2ae20907df886f4d1",
+    "traffic": {("round_nodes_base", 24): 204020487, ("round_fold2_base", 24): 202949492, ("round_fold3_base", 24): 303107363},
     # per pair: 76 multiply-adds in the sweep (2^22 pairs of four entries), and multiply-adds and multiplies of the
     # reductions of 344 in round 2 (2^21 pairs), 440 in round 3 (2^20) and 344 in the extension rounds (2^19 + 2^18 + ...)
     "int32_mul_per_prove": 76 * (1 << 22) + 344 * (1 << 21) + 440 * (1 << 20) + 344 * (1 << 20),
