@@ -157,6 +157,12 @@ constexpr int brev(int i, int D) {
   return r;
 }
 
+// the same for an index known at run time
+template <int D>
+EXH_HD uint32_t brev_bits(uint32_t i) {
+  return D == 8 ? (i & 2) | (i >> 2 & 1) | (i & 1) << 2 : (i >> 1 & 1) | (i & 1) << 1;
+}
+
 template <int D>
 struct Ext {
   uint32_t c[D];
@@ -315,10 +321,9 @@ __device__ __forceinline__ double f_mul(double a, double b) {
 __device__ __forceinline__ double f_scale(double x, uint32_t c) {
   return c == 1 ? x : c == P - 1 ? -x : f_mul(x, c > P / 2 ? (double)c - F_P : (double)c);
 }
-// the canonical residue of an integer |v| < p: the low word of v + MAGIC is v mod 2^32, and p above it wraps below it when v < 0
-__device__ __forceinline__ uint32_t f_small_canonical(double v) {
-  const uint32_t r = (uint32_t)__double_as_longlong(v + F_MAGIC);
-  return umin32(r, r + P);
+// the word whose bytes are the four signed digits of an integer |v| < p / 2 + 2^28: v + 0x80808080 has the digits plus 128
+__device__ __forceinline__ uint32_t f_signed_digits(double v) {
+  return (uint32_t)__double_as_longlong(v + (F_MAGIC + 2155905152.0)) ^ 0x80808080u;
 }
 // the canonical residue of an integer |v| < 2^80
 __device__ __forceinline__ uint32_t f_canonical(double v) {

@@ -88,11 +88,19 @@ EXH_DESC_FN constexpr int node_slots(const Desc &d) {
   return n;
 }
 
+// the pairs of factors that the sweep takes as quadratics: where a row of slots costs fewer products that way and their
+// values stay small
+template <class Desc>
+EXH_DESC_FN constexpr int sweep_quads(const Desc &d, int g) {
+  return d.maxx > 4 ? 0 : d.deg[g] == 4 ? 2 : d.deg[g] == 3 ? 1 : 0;
+}
+
 // the launches per round of the base-field sweep for degree D and the slots each takes: the slots are split
-// evenly over launches of at most NODES_CAP4 (F_p^4) or NODES_CAP8 (F_p^8) slots, what two wavefronts per SIMD
-// have the registers for at two registers a slot and coordinate; no launches when the slot sums do not fit the
-// accumulators' buffers
-constexpr int NODES_CAP4 = 20, NODES_CAP8 = 8;
+// evenly over launches of at most NODES_CAP4 (F_p^4) or NODES_CAP8 (F_p^8) slots, a slot taking D registers of sums; no
+// launches when the slot sums do not fit the accumulators' buffers
+constexpr int NODES_CAP4 = 20, NODES_CAP8 = 24;
+// wavefronts a SIMD: two, one where the sums and what a lane holds of its pairs take more than half the registers
+EXH_DESC_FN constexpr int sweep_waves(int D, int slots) { return slots * (D + 1) > 128 ? 1 : 2; }
 template <class Desc>
 EXH_DESC_FN constexpr int nodes_slots_per_pass(const Desc &d, int D) {
   int slots = node_slots(d), cap = D == 4 ? NODES_CAP4 : NODES_CAP8, passes = (slots + cap - 1) / cap;

@@ -20,10 +20,12 @@ namespace exh {
 // eq weights for every round in one launch.  Table k covers the eq point's variables
 // [first, first + bits): entry x = prod_b (x_b ? r_b : 1 - r_b) (src/field.lisp:354-363: bit b of the
 // index pairs with the b-th variable).  factors[v] = (r_v R, (1 - r_v) R): each product is exact.
+// Table `digits` (-1: none) is written in the digit form of the base-field sweep's weights (store_sweep_digits), a
+// quarter of the coordinates a thread.
 struct EqTables {
-  int count;
-  uint64_t off[64];  // in EXTs
-  int first[64], bits[64];
+  int count, digits;
+  uint64_t off[67];  // in EXTs
+  int first[67], bits[67];
 };
 
 // (both set-up kernels also clear the totals of the grid launch of LDS-resident slices: the first launch of a
@@ -55,7 +57,9 @@ __global__ __launch_bounds__(BLOCK) void eq_tables_kernel(EqTables tabs, const u
     start += (uint64_t)1 << tabs.bits[k];
     k++;
   }
-  uint64_t x = gid - start;
+  uint64_t x = gid - start;  // (the digit form's table comes last: four threads an entry)
+  const uint32_t quarter = (uint32_t)x & 3;
+  if (k == tabs.digits) x >>= 2;
   Ext<D> e = ext_lift<D>(1);
   for (int b = 0; b < tabs.bits[k]; b++) {
     const uint32_t *f = lds_factors + ((size_t)(tabs.first[k] + b) * 2 + (((x >> b) & 1) ? 0 : 1)) * D;
@@ -64,7 +68,10 @@ __global__ __launch_bounds__(BLOCK) void eq_tables_kernel(EqTables tabs, const u
     for (int c = 0; c < D; c++) fe.c[c] = f[c];
     e = ext_mul_mont<D>(e, fe);
   }
-  store_ext<D>(out + (tabs.off[k] + x) * D, e);
+  if (k == tabs.digits)
+    store_sweep_digits<D>(out + tabs.off[k] * D, x, e, quarter);
+  else
+    store_ext<D>(out + (tabs.off[k] + x) * D, e);
 }
 
 template <int D>
@@ -225,6 +232,7 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
   low_off.assign(n, 0), high_off.assign(n, 0), low_bits.assign(n, 0), n_high.assign(n, 0);
   EqTables eqt;
   memset(&eqt, 0, sizeof(eqt));
+  eqt.digits = -1;
   uint64_t pos = (uint64_t)2 * n;  // in EXTs: the eq factors come first
   uint64_t bw_off = 0, ones_off = 0, ones_len = 0, total_eq = 0;
   if (has_bw) {
@@ -266,6 +274,31 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
     }
     if (has_bw) high_off[j] = bw_off;
   }
+  // round 1's weights once more for the base-field sweep, where the rounds may open with it: by the pair index's low four
+  // bits, by the bits from there to sweep_bits in digit form, and by the rest
+  node_slots_n = node_slots(desc);  // grid sums of the sweep that serves rounds 0 and 1
+  bool all_stride_1 = true;
+  for (int t = 0; t < T; t++) all_stride_1 = all_stride_1 && strides[t] == 1;
+  sweep_ready = all_stride_1 && (has_bw || K == 1) && !claim_mode && !private_buffers && sweep_fits();
+  sweep_bits = 0, sweep_columns = sweep_digits = sweep_high = 0;
+  if (sweep_ready) {
+    // a tile of the pairs for every workgroup that is resident at once; HIGH covers the bits above it, or the blocks
+    while (((uint64_t)1 << sweep_bits) * sweep_grid() < size / 4) sweep_bits++;
+    sweep_bits = std::min(std::max(sweep_bits, 8), 8 + SWEEP_PPT_BITS);
+    if (has_bw) sweep_bits = n - 2;
+  }
+  if (sweep_ready && has_eq) {
+    const int first[3] = {2 + sweep_bits, 2, 6}, bits[3] = {n - 2 - sweep_bits, 4, sweep_bits - 4};
+    uint64_t *const where[3] = {&sweep_high, &sweep_columns, &sweep_digits};
+    for (int k = has_bw ? 1 : 0; k < 3; k++) {
+      *where[k] = pos;
+      eqt.off[eqt.count] = pos, eqt.first[eqt.count] = first[k], eqt.bits[eqt.count] = bits[k];
+      eqt.count++;
+      pos += (uint64_t)(k == 2 ? 4 : 1) << bits[k];
+      total_eq += (uint64_t)(k == 2 ? 4 : 1) << bits[k];
+    }
+    eqt.digits = eqt.count - 1;
+  }
   if (!has_eq && n > 0) {
     ones_off = pos;
     pos += ones_len;
@@ -281,7 +314,6 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
   // prove, 256 lose 15 %)
   const uint64_t grid_cap = std::min<uint64_t>(1024, 2 * (uint64_t)std::max(c.compute_units, 1));
   if (max_grid > grid_cap) max_grid = grid_cap;
-  node_slots_n = node_slots(desc);  // grid sums of the sweep that serves rounds 0 and 1 from the base tables
   pstride = next_pow2((uint64_t)std::max(std::max(st.nacc, 1), node_slots_n <= MAXACC ? node_slots_n : 0) * D);
   uint64_t partial_off = pos * D;  // from here in words
   // (a workgroup's partial row per workgroup of the largest grid a round can take: tiles stop growing at the span
@@ -430,6 +462,7 @@ int eq_table_device(int D, int k, const uint32_t *r, uint32_t *d_out) {
   EXH_HIP(hipMemcpyAsync(d_factors, factors.data(), factors.size() * 4, hipMemcpyHostToDevice, c.stream));
   EqTables eqt;
   memset(&eqt, 0, sizeof(eqt));
+  eqt.digits = -1;
   eqt.count = 1, eqt.off[0] = 0, eqt.first[0] = 0, eqt.bits[0] = k;
   const uint64_t total = (uint64_t)1 << k;
   uint32_t grid = (uint32_t)((total + BLOCK - 1) / BLOCK);
@@ -457,6 +490,7 @@ int eq_tables_launch(int D, int count, const int *first, const int *bits, const 
   }
   EqTables eqt;
   memset(&eqt, 0, sizeof(eqt));
+  eqt.digits = -1;
   eqt.count = count;
   uint64_t total = 0;
   for (int k = 0; k < count; k++) {
@@ -475,6 +509,32 @@ int eq_tables_launch(int D, int count, const int *first, const int *bits, const 
 }
 
 static uint64_t whole_pairs(int T, int D);
+
+// pairs of T tables in a workgroup's LDS in the grid of slices, and the workgroups that grid may have
+static uint64_t slice_pairs(int T, int D) {
+  uint64_t most = SLICE_LDS_BYTES / ((uint64_t)T * 2 * D * 4);
+  if (const char *cap = getenv("EXACTA_HIP_MAX_SLICE_PAIRS"))  // tests: keep more rounds on the streaming kernels
+    most = std::min<uint64_t>(most, strtoull(cap, nullptr, 10));
+  return most;
+}
+static uint64_t slice_grid() {
+  Context &c = ctx();
+  // (proofs running side by side share the device: each one's grid takes its part, a power of two)
+  return std::min<uint64_t>(256, c.compute_units > 0 ? c.compute_units : 1) / (c.share > 1 ? 2 : 1);
+}
+
+// Rounds 0 and 1 of the session's base tables can come from one sweep of them, when round 2 is a streaming round as well.
+// (Its tiles, of 2^8 pairs and more, lie within one block: blocks of under 2^10 entries take the ordinary rounds.)
+bool SumcheckSession::sweep_fits() const {
+  return generated && kernels->nodes_passes > 0 && node_slots_n <= MAXACC && n >= 10 &&
+         (size & (size - 1)) == 0 && size / 8 > slice_pairs(st.T(), D) * slice_grid();
+}
+
+// Its workgroups: as many as are resident at once.
+uint64_t SumcheckSession::sweep_grid() const {
+  const int waves = sweep_waves(D, nodes_slots_per_pass(desc, D));
+  return (uint64_t)waves * (uint64_t)std::max(ctx().compute_units, 1);
+}
 
 int SumcheckSession::launch_setup(const uint32_t *staged, size_t staged_words) {
   Context &c = ctx();
@@ -645,16 +705,19 @@ static int launch_nodes_round(SumcheckSession &s, uint64_t n_pairs) {
   memset(&a, 0, sizeof(a));
   int T = s.st.T();
   for (int t = 0; t < T; t++) a.in[t] = s.cur[t];
-  a.low = s.d_weights + s.low_off[1] * D;  // round 1's weights; round 0's extra factor goes in by the epilogue
-  a.high = s.d_weights + s.high_off[1] * D;
-  a.low_bits = (uint32_t)s.low_bits[1];
+  // round 1's weights; round 0's extra factor goes in by the epilogue
+  a.columns = s.has_eq ? s.d_weights + s.sweep_columns * D : nullptr;
+  a.digits = s.has_eq ? s.d_weights + s.sweep_digits * D : nullptr;
+  a.high = s.has_bw ? s.d_weights + s.high_off[1] * D : s.has_eq ? s.d_weights + s.sweep_high * D : nullptr;
+  a.low_bits = (uint32_t)s.sweep_bits;
   a.n_pairs = n_pairs;
-  // (two workgroups fit a compute unit beside the accumulators: the session's grid cap has them all resident
-  // at once, which spreads each workgroup's fixed work -- first loads, the reduction over lanes -- over the most pairs)
+  // (every workgroup is resident at once, which spreads its fixed work -- first loads, the reduction over lanes -- over
+  // the most pairs)
   uint32_t ppt = 1;
-  ppt = tile_pairs_per_thread(n_pairs, s.max_grid, (uint64_t)1 << a.low_bits);
+  while ((uint64_t)BLOCK * ppt * s.sweep_grid() < n_pairs && (uint64_t)BLOCK * ppt * 2 <= ((uint64_t)1 << s.sweep_bits) &&
+         ppt * 2 <= (1u << SWEEP_PPT_BITS))
+    ppt *= 2;
   a.pairs_per_thread = ppt;
-  a.deferred = (uint64_t)BLOCK * ppt <= ((uint64_t)1 << a.low_bits) ? 1 : 0;
   uint32_t grid = (uint32_t)((n_pairs + (uint64_t)BLOCK * ppt - 1) / ((uint64_t)BLOCK * ppt));
   // the two rounds' epilogue, run by the last workgroup of the last pass (see RoundTotals)
   NodesEpilogueArgs &e = a.epi;
@@ -1080,11 +1143,7 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   int status = OK, j = 0;
   int folds_due = 0;  // folds by the last challenges drawn that the tables still await (2 after the base-field sweep for rounds 0 and 1)
   const char *no_nodes = getenv("EXACTA_HIP_NO_BASE_ROUND1");
-  uint64_t slice_max = SLICE_LDS_BYTES / ((uint64_t)T * 2 * D * 4);
-  if (const char *cap = getenv("EXACTA_HIP_MAX_SLICE_PAIRS"))  // tests: keep more rounds on the streaming kernels
-    slice_max = std::min<uint64_t>(slice_max, strtoull(cap, nullptr, 10));
-  // (proofs running side by side share the device: each one's grid takes its part, a power of two)
-  const uint64_t grid_max = std::min<uint64_t>(256, c.compute_units > 0 ? c.compute_units : 1) / (c.share > 1 ? 2 : 1);
+  const uint64_t slice_max = slice_pairs(T, D), grid_max = slice_grid();
   // pairs that the grid of LDS-resident slices can take, and the one-workgroup launch: more of them are a streaming round
   auto slices_max = [&]() { return std::max(slice_max * grid_max, tail_pairs(T, D)); };
   for (; j < n && status == OK; j++) {
@@ -1121,7 +1180,6 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
     round = j;
     // once every workgroup of a resident grid can hold its slice of the tables in LDS, the rounds down
     // to where one workgroup suffices run in one launch
-    const bool pow2 = (size & (size - 1)) == 0;
     // (several blocks: the pairs are an odd multiple of a power of two, and the grid that multiple of one, so that
     // every workgroup's slice is a power of two of pairs and halves with the rounds; a fold pairs neighbours, so a
     // slice need not lie in one block)
@@ -1170,8 +1228,7 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
     }
     // rounds 0 and 1 from one sweep of the base tables, when round 2 is a streaming round as well: their sums
     // come from base-field products on a grid of (X0, X1) and the tables are not folded until round 2
-    const bool nodes_rounds = j == 0 && cur_base && folds_due == 0 && n >= 3 && generated && kernels->nodes_passes > 0 &&
-                              node_slots_n <= MAXACC && pow2 && (n_pairs / 4) > slice_max * grid_max &&
+    const bool nodes_rounds = j == 0 && cur_base && folds_due == 0 && sweep_ready && (n_pairs / 4) > slice_max * grid_max &&
                               !(no_nodes && no_nodes[0] == '1');
     if (nodes_rounds) {
       status = D == 4 ? launch_nodes_round<4>(*this, n_pairs / 2) : launch_nodes_round<8>(*this, n_pairs / 2);

@@ -67,6 +67,11 @@ struct SumcheckSession {
   uint64_t max_grid = 0;
   uint32_t pstride = 0;  // words per workgroup partial
   int node_slots_n = 0;  // slot sums of the base-field sweep that serves rounds 0 and 1
+  bool sweep_ready = false;                     // its weights are laid out: the rounds may open with it
+  int sweep_bits = 0;                            // its pairs' index below HIGH
+  uint64_t sweep_columns = 0, sweep_digits = 0, sweep_high = 0;  // where the weights are (with an eq point), in EXTs
+  bool sweep_fits() const;
+  uint64_t sweep_grid() const;
   bool device_loop = false;
   Ctrl *d_ctrl = nullptr;
   std::vector<uint32_t> final_cache;  // the tables as the device loop's tail left them, when read back with its logs

@@ -1648,7 +1648,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
 //   (extra e):          X1 = 1, X0 = the e-th evaluation point                     -- round 0: its sum at X0 is
 //                       eq(w1, 0) * slot(X1 = 0, X0) + eq(w1, 1) * slot(X1 = 1, X0), the weight of variable 1
 //                       being the one factor round 0's weights have beyond round 1's.
-// All products are base-field; no folded table is written; round 2 folds twice.  A launch covers the slots
+// All products are base-field; no folded table is written; rounds 2 and 3 read the base tables.  A launch covers the slots
 // [PASS * SPP, (PASS + 1) * SPP) so the accumulators stay in registers.
 // The epilogue of that sweep, both rounds by one workgroup: slot sums -> round 0's accumulator sums -> its
 // message, through the transcript, to r0 -> the Lagrange basis at r0 -> round 1's accumulator sums -> its
@@ -1665,9 +1665,11 @@ struct NodesEpilogueArgs {
 template <int D>
 struct NodesArgs {
   const uint32_t *in[MAXT];  // base tables
-  const uint32_t *low, *high;
-  uint64_t n_pairs;          // pairs of round 1: four base entries each
-  uint32_t low_bits, pairs_per_thread, deferred;
+  // round 1's weights in three factors: the pair index's low four bits (16 EXTs), the bits from there to low_bits in digit
+  // form (SWEEP_* below), and HIGH for the rest (null: ones)
+  const uint32_t *columns, *digits, *high;
+  uint64_t n_pairs;          // pairs of round 1, four base entries each: a multiple of BLOCK
+  uint32_t low_bits, pairs_per_thread;  // a workgroup's tile stays within 2^low_bits pairs
   // the slot sums of all passes meet in one set of counted totals (slot s at word s * D), and the last workgroup
   // of the last pass to arrive runs the two rounds' epilogue itself (see RoundTotals)
   RoundTotals totals;
@@ -1678,7 +1680,6 @@ struct NodesArgs {
 // A 64-bit accumulator of 32 x 32-bit products kept below p 2^32 by a conditional subtraction of p from its high
 // word after every product: acc < p 2^32, the product of a canonical weight and a residue below 2^32 is below
 // p 2^32 as well, so the sum is below 2^64, and min(hi, hi - p) brings it back (hi < p: hi - p wraps above hi).
-// Eight registers per slot at F_p^4 where the 96-bit form takes twelve, for one more (cheap) instruction per word.
 __device__ __forceinline__ void lazy_mad(uint64_t &acc, uint32_t w, uint32_t v) {
   acc = mont_lazy((uint64_t)w * v + acc);
 }
@@ -1687,6 +1688,56 @@ __device__ __forceinline__ uint32_t lazy_reduce(uint64_t acc) {
   a.lo = acc, a.hi = 0;
   return acc_reduce(a);
 }
+
+// The sweep's weighted sums are matrix products.  A wavefront's step is 128 pairs: lane n + 16 g takes pairs 64 t + 16 g + n
+// (t = 0, 1), so that column n holds the pairs whose index ends in n, and along a column only the index above the low four
+// bits varies: sum over k of mid[k] v[k][n] for all sixteen columns at once, with the sixteen columns' own weights applied
+// once a workgroup.  In bytes: a value is written in four signed digits v = sum_j v_j 2^(8 j), a weight's coordinate w as the
+// four digits of each of w 2^(8 j) mod p, and w v is congruent to sum_i 2^(8 i) sum_j digit_i(w 2^(8 j)) v_j, so that row
+// (coordinate, i) of the product's result, an exact 32-bit sum, is that coordinate's i-th digit sum.  Sixteen rows
+// at F_p^4 and thirty-two at F_p^8, eight pairs' four bytes along the contraction: v_mfma_i32_16x16x32_i8 with the value's
+// word as it is for the right operand and digit words made once per proof (store_sweep_digits) for the left.
+// What that takes from the vector units, which bound the sweep: a slot's weighted sum is two instructions a pair (its digits)
+// where a multiply-add a coordinate, their reductions and a canonical value are eleven at F_p^4 and nineteen at F_p^8, and
+// half the registers, so that F_p^8 needs one pass for the 24 slots of a product of four, not three.  With the quadratics
+// below: 283 instructions a pair for 559 with three tables at F_p^4 (2^24 entries: 100 -> 70 us), 480 for 1455 with four at
+// F_p^8 (2^26: 860 -> 385 us).
+constexpr int SWEEP_STEP = 128;         // pairs of a wavefront's step
+constexpr int SWEEP_MIDS = SWEEP_STEP / 16;
+constexpr uint32_t DIGIT_BIAS = 0x80808080u;
+// A digit sum grows by at most 4 * 128 * 128 a pair of its column, a column has a sixteenth of a wavefront's share of the
+// tile, and the sums of four digits are put together below 2^54.02.
+constexpr int SWEEP_PPT_BITS = 12;
+static_assert(((uint64_t)64 / 16 * 4 * 128 * 128) << SWEEP_PPT_BITS <= (uint64_t)1 << 30, "a digit sum stays within 2^30");
+// the word whose bytes are the signed digits of a canonical value
+EXH_HD uint32_t signed_digits(uint32_t v) { return (v + DIGIT_BIAS) ^ DIGIT_BIAS; }
+
+#if defined(__HIPCC__)
+typedef int digit_sums __attribute__((ext_vector_type(4)));
+// a quarter of weight k's coordinates into place: [k / 8][coordinate / 4][lane (coordinate % 4) * 4 + i + 16 (k % 4)][k / 4 % 2], byte j = digit i of
+// w 2^(8 j)
+template <int D>
+__device__ __forceinline__ void store_sweep_digits(uint32_t *out, uint64_t k, const Ext<D> &e, uint32_t quarter) {
+  constexpr uint32_t SHIFT[4] = {R1, (uint32_t)(((uint64_t)R1 << 8) % P), (uint32_t)(((uint64_t)R1 << 16) % P),
+                                 (uint32_t)(((uint64_t)R1 << 24) % P)};  // 2^(8 j) R
+#pragma unroll
+  for (uint32_t tile = 0; tile < D / 4; tile++) {
+    const uint32_t w = quarter == 0 ? e.c[4 * tile] : quarter == 1 ? e.c[4 * tile + 1] : quarter == 2 ? e.c[4 * tile + 2]
+                                                                                                   : e.c[4 * tile + 3];
+    uint32_t dig[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) dig[j] = signed_digits(mont_mul(w, SHIFT[j]));
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      uint32_t word = 0;
+#pragma unroll
+      for (int j = 0; j < 4; j++) word |= ((dig[j] >> (8 * i)) & 255u) << (8 * j);
+      const uint32_t lane = quarter * 4 + i + 16u * (uint32_t)(k & 3);
+      out[(((k >> 3) * (D / 4) + tile) * 64 + lane) * 2 + ((k >> 2) & 1)] = word;
+    }
+  }
+}
+#endif
 
 // the LDS of the two rounds' epilogue
 template <int D>
@@ -1817,163 +1868,267 @@ __device__ __forceinline__ void nodes_epilogue_body(const NodesEpilogueArgs &arg
   }
 }
 
-// the slot sums: lines and products in double precision (field.hpp), weighted sums in integers
+// the slot sums: lines and products in double precision (field.hpp), weighted sums on the matrix cores (above)
 template <int D, int PASS, int SPP, class Desc>
 __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &args) {
   // magnitudes, in units of p: a table line's ends < 1, a linear form < 5 (MAXVT terms and the constant),
   // the step between X points < 10, so at X <= 7 a line's end < 65 and its slope < 52, a node's value
   // < 65 + 6 * 52 = 377; a product of two < 377^2 p^2 < 2^80 and its quotient by p < 2^49.
+  // A quadratic's reduced values and coefficient are within 0.57 p; at X <= 4 it is within 19 times that, and in X0 <= 4
+  // within 19 times that again: 206 p.
   static_assert(MAXVT <= 4 && MAXX <= 7 && MAXDEG <= 6, "the bounds of the double-precision products");
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint64_t tile = (uint64_t)BLOCK * args.pairs_per_thread, tile_start = (uint64_t)blockIdx.x * tile;
+  const uint64_t tile_end = tile_start + tile < args.n_pairs ? tile_start + tile : args.n_pairs;
   const uint64_t low_mask = ((uint64_t)1 << args.low_bits) - 1;
-  // the weighted sums themselves are integer: one 32 x 32 -> 64 multiply-add per word into a lazily reduced 64-bit sum.
-  // The sum takes the products of two pairs, both factors canonical, before it is lowered (one instruction more to make a
-  // value canonical, one a word and pair less): a proof of four tables of 2^26 at F_p^8 3607 -> 3540 us, of three of 2^24 at
-  // F_p^4 480 -> 477.
-  static_assert(2 * (uint64_t)(P - 1) * (P - 1) < (uint64_t)P << 32, "two products above a lowered sum stay below 2 p 2^32");
-  uint64_t acc[SPP][D];
+  constexpr int TILES = D / 4, STEPS = SWEEP_STEP / 64;
+  digit_sums acc[SPP][TILES];
+  uint32_t held[SPP];  // the digits of a step's first pairs, until its second ones complete the product's operand
 #pragma unroll
   for (int a = 0; a < SPP; a++)
 #pragma unroll
-    for (int c = 0; c < D; c++) acc[a][c] = 0;
+    for (int q = 0; q < TILES; q++) acc[a][q] = digit_sums{0, 0, 0, 0};
 
-  // the loads run PREFETCH pairs ahead of the arithmetic: few waves fit beside the accumulators
-  constexpr int PREFETCH = 2;
-  uint4 ahead[PREFETCH][MAXT];
-  Ext<D> wahead[PREFETCH];
-  auto fetch = [&](uint32_t k, uint4 *e, Ext<D> &w) {
-    const uint64_t i = tile_start + (uint64_t)k * BLOCK + tid;
-    if (k < args.pairs_per_thread && i < args.n_pairs) {
+  // the loads run a step ahead of the arithmetic: few waves fit beside the accumulators
+  uint4 ahead[STEPS][MAXT];
+  uint2 wahead[TILES];
+  const uint64_t first = tile_start + wave * SWEEP_STEP;
+  // (a wavefront's step lies in its tile as a whole; behind the last one the first is fetched again, and not used)
+  auto fetch = [&](int t, uint64_t base) {
 #pragma unroll
-      for (int t = 0; t < MAXT; t++)
-        if (t < d.T) e[t] = *reinterpret_cast<const uint4 *>(args.in[t] + 4 * i);
-      w = load_ext<D>(args.low + (i & low_mask) * D);
+    for (int q = 0; q < MAXT; q++)
+      if (q < d.T) ahead[t][q] = reinterpret_cast<const uint4 *>(args.in[q] + 4 * (base + 64 * t))[lane];
+  };
+  auto fetch_digits = [&](uint64_t base) {
+    if (args.digits) {
+      const uint32_t *const at = args.digits + ((base & low_mask) / SWEEP_STEP) * (TILES * 128);
+#pragma unroll
+      for (int q = 0; q < TILES; q++) wahead[q] = reinterpret_cast<const uint2 *>(at)[q * 64 + lane];
     }
   };
+  // without an eq point every weight is one: coordinate 0's row i has digit i of 2^(8 j), one at j = i
 #pragma unroll
-  for (int a = 0; a < PREFETCH; a++) fetch(a, ahead[a], wahead[a]);
-
-  for (uint32_t k = 0; k < args.pairs_per_thread; k++) {
-    const uint64_t i = tile_start + (uint64_t)k * BLOCK + tid;
-    if (i >= args.n_pairs) break;
-    // per factor: the line in r0 at X = 0 (u0 + r0 v0) and at X = 1 (u1 + r0 v1)
-    double cu[MAXT], cv[MAXT], du[MAXT], dv[MAXT], u1[MAXT], v1[MAXT];
+  for (int q = 0; q < TILES; q++)
+    wahead[q].x = wahead[q].y = q == 0 && (lane & 15) < 4 ? 1u << (8 * (lane & 15)) : 0u;
+  if (first < tile_end) {
 #pragma unroll
-    for (int t = 0; t < MAXT; t++)
-      if (t < d.T) {
-        const uint4 e = ahead[0][t];
-        cu[t] = (double)e.x, cv[t] = (double)e.y - cu[t], u1[t] = (double)e.z, v1[t] = (double)e.w - u1[t];
-      }
-    Ext<D> we = wahead[0];
+    for (int t = 0; t < STEPS; t++) fetch(t, first);
+    fetch_digits(first);
+  }
+  for (uint64_t base = first; base < tile_end; base += (BLOCK / 64) * SWEEP_STEP) {
+    const uint64_t next = base + (BLOCK / 64) * SWEEP_STEP < tile_end ? base + (BLOCK / 64) * SWEEP_STEP : first;
+    uint2 weights[TILES];
 #pragma unroll
-    for (int a = 0; a + 1 < PREFETCH; a++) {
+    for (int q = 0; q < TILES; q++) weights[q] = wahead[q];
+    fetch_digits(next);
+#pragma unroll
+    for (int step_pairs = 0; step_pairs < STEPS; step_pairs++) {
+      // per factor: the line in r0 at X = 0 (u0 + r0 v0) and at X = 1 (u1 + r0 v1)
+      double cu[MAXT], cv[MAXT], du[MAXT], dv[MAXT], u1[MAXT], v1[MAXT];
 #pragma unroll
       for (int t = 0; t < MAXT; t++)
-        if (t < d.T) ahead[a][t] = ahead[a + 1][t];
-      wahead[a] = wahead[a + 1];
-    }
-    fetch(k + PREFETCH, ahead[PREFETCH - 1], wahead[PREFETCH - 1]);
-#pragma unroll
-    for (int v = 0; v < MAXV; v++)
-      if (v < d.NV) {  // a linear form of the tables: the same combination of the lines
-        double a0 = (double)d.vconst[v], b0 = 0, a1 = a0, b1 = 0;
-#pragma unroll
-        for (int q = 0; q < MAXVT; q++)
-          if (q < d.vn[v]) {
-            const int t = d.vtab[v][q];
-            a0 += f_scale(cu[t], d.vcoef[v][q]), b0 += f_scale(cv[t], d.vcoef[v][q]);
-            a1 += f_scale(u1[t], d.vcoef[v][q]), b1 += f_scale(v1[t], d.vcoef[v][q]);
-          }
-        cu[d.T + v] = a0, cv[d.T + v] = b0, u1[d.T + v] = a1, v1[d.T + v] = b1;
-      }
-#pragma unroll
-    for (int t = 0; t < MAXT; t++)
-      if (t < d.T + d.NV) du[t] = u1[t] - cu[t], dv[t] = v1[t] - cv[t];
-    if (!args.deferred) we = ext_mul_mont<D>(we, load_ext<D>(args.high + (i >> args.low_bits) * D));
-
-    int slot = 0;  // numbered group by group (point by point, node by node, then the extras) -- visited X1-major
-#pragma unroll
-    for (int x = 0; x <= MAXX; x++) {
-      if (x <= d.maxx || x == 1) {
-        if (x >= 1) {
-#pragma unroll
-          for (int t = 0; t < MAXT; t++)
-            if (t < d.T + d.NV) {
-              if (x == 1)
-                cu[t] = u1[t], cv[t] = v1[t];
-              else
-                cu[t] += du[t], cv[t] += dv[t];
-            }
+        if (t < d.T) {
+          const uint4 e = ahead[step_pairs][t];
+          cu[t] = (double)e.x, cv[t] = (double)e.y - cu[t], u1[t] = (double)e.z, v1[t] = (double)e.w - u1[t];
         }
-        int base = 0, lead_base = 0;  // first slot of group g, and of the group whose slots it shares
-        double shared_sum[MAXDEG + 1];
+      fetch(step_pairs, next);
 #pragma unroll
-        for (int g = 0; g < MAXG; g++) {
-          if (g < d.G) {
-            const int e = ev_index(d, g, x);  // an evaluation point's row, or at X1 = 1 the row of extras
-            const bool first = d.lead[g] == g, last = group_is_last(d, g);
-            if (first) lead_base = base;
-            if (e >= 0 || x == 1) {
-              double val[MAXDEG];
+      for (int v = 0; v < MAXV; v++)
+        if (v < d.NV) {  // a linear form of the tables: the same combination of the lines
+          double a0 = (double)d.vconst[v], b0 = 0, a1 = a0, b1 = 0;
 #pragma unroll
-              for (int j = 0; j < MAXDEG; j++)
-                if (j < d.deg[g]) val[j] = cu[d.tab[g][j]];
+          for (int q = 0; q < MAXVT; q++)
+            if (q < d.vn[v]) {
+              const int t = d.vtab[v][q];
+              a0 += f_scale(cu[t], d.vcoef[v][q]), b0 += f_scale(cv[t], d.vcoef[v][q]);
+              a1 += f_scale(u1[t], d.vcoef[v][q]), b1 += f_scale(v1[t], d.vcoef[v][q]);
+            }
+          cu[d.T + v] = a0, cv[d.T + v] = b0, u1[d.T + v] = a1, v1[d.T + v] = b1;
+        }
 #pragma unroll
-              for (int m = 0; m <= MAXDEG; m++) {
-                if (m <= d.deg[g]) {
-                  if (e >= 0)
-                    slot = lead_base + e * (d.deg[g] + 1) + m;
-                  else  // only the nodes that are evaluation points
-                    slot = ev_index(d, g, m) < 0 ? -1 : lead_base + d.nev[g] * (d.deg[g] + 1) + ev_index(d, g, m);
-                  if (slot >= PASS * SPP && slot < (PASS + 1) * SPP) {
-                    double prod = val[0];
+      for (int t = 0; t < MAXT; t++)
+        if (t < d.T + d.NV) du[t] = u1[t] - cu[t], dv[t] = v1[t] - cv[t];
+
+      // A group of three or four factors takes two of them (or two and two) as one quadratic in X1 and in X0: nine products
+      // give its values at X1 = 0 and 1 and its coefficient of X1^2, each of them at X0 = 0 and 1 and as the coefficient of
+      // X0^2, and the others follow by differences; a slot is then one product, where a factor at a time takes two or three.
+      double qcur[MAXG][2][3], qstep[MAXG][2][3], qtwo[MAXG][2][3], qnext[MAXG][2][3];
 #pragma unroll
-                    for (int j = 1; j < MAXDEG; j++)
-                      if (j < d.deg[g]) prod = f_mul(prod, val[j]);
-                    shared_sum[m] = first ? prod : shared_sum[m] + prod;  // (groups that share the slot follow one another)
-                    if (last) {
-                      const double total = d.deg[g] == 1 || !first ? f_reduce(shared_sum[m]) : shared_sum[m];
-                      const uint32_t pv = f_small_canonical(total);
+      for (int g = 0; g < MAXG; g++)
+        if (g < d.G && sweep_quads(d, g) > 0) {
 #pragma unroll
-                      for (int c = 0; c < D; c++) acc[slot - PASS * SPP][c] += (uint64_t)we.c[c] * pv;
-                    }
-                  }
+          for (int h = 0; h < 2; h++)
+            if (h < sweep_quads(d, g)) {
+              const int a = d.tab[g][2 * h], b = d.tab[g][2 * h + 1];
+              const double va[3][3] = {
+                  {cu[a], u1[a], du[a]}, {cu[a] + cv[a], u1[a] + v1[a], du[a] + dv[a]}, {cv[a], v1[a], dv[a]}};
+              const double vb[3][3] = {
+                  {cu[b], u1[b], du[b]}, {cu[b] + cv[b], u1[b] + v1[b], du[b] + dv[b]}, {cv[b], v1[b], dv[b]}};
 #pragma unroll
-                  for (int j = 0; j < MAXDEG; j++)
-                    if (j < d.deg[g]) val[j] += cv[d.tab[g][j]];
-                }
+              for (int k = 0; k < 3; k++) {
+                qcur[g][h][k] = f_mul(va[k][0], vb[k][0]);
+                qnext[g][h][k] = f_mul(va[k][1], vb[k][1]);
+                const double square = f_mul(va[k][2], vb[k][2]);
+                qtwo[g][h][k] = square + square;
+                qstep[g][h][k] = qnext[g][h][k] - qcur[g][h][k];
               }
             }
-            base += group_slots(d, g);
+        }
+      int slot = 0;  // numbered group by group (point by point, node by node, then the extras) -- visited X1-major
+#pragma unroll
+      for (int x = 0; x <= MAXX; x++) {
+        if (x <= d.maxx || x == 1) {
+          if (x >= 1) {
+#pragma unroll
+            for (int t = 0; t < MAXT; t++)
+              if (t < d.T + d.NV) {
+                if (x == 1)
+                  cu[t] = u1[t], cv[t] = v1[t];
+                else
+                  cu[t] += du[t], cv[t] += dv[t];
+              }
+#pragma unroll
+            for (int g = 0; g < MAXG; g++)
+#pragma unroll
+              for (int h = 0; h < 2; h++)
+                if (g < d.G && h < sweep_quads(d, g))
+#pragma unroll
+                  for (int k = 0; k < 3; k++) {
+                    if (x == 1) {
+                      qcur[g][h][k] = qnext[g][h][k];
+                    } else {
+                      qstep[g][h][k] += qtwo[g][h][k];
+                      qcur[g][h][k] += qstep[g][h][k];
+                    }
+                  }
+          }
+          int base = 0, lead_base = 0;  // first slot of group g, and of the group whose slots it shares
+          double shared_sum[MAXDEG + 1];
+#pragma unroll
+          for (int g = 0; g < MAXG; g++) {
+            if (g < d.G) {
+              const int e = ev_index(d, g, x);  // an evaluation point's row, or at X1 = 1 the row of extras
+              const bool first = d.lead[g] == g, last = group_is_last(d, g);
+              if (first) lead_base = base;
+              if (e >= 0 || x == 1) {
+                // the row's factors at X0 = 0, the quadratics first
+                const int quads = sweep_quads(d, g), factors = d.deg[g] - quads;
+                double val[MAXDEG], step[2];
+#pragma unroll
+                for (int j = 0; j < MAXDEG; j++) {
+                  if (j < quads)
+                    val[j] = qcur[g][j < 2 ? j : 0][0], step[j < 2 ? j : 0] = qcur[g][j < 2 ? j : 0][1] - val[j];
+                  else if (j < factors)
+                    val[j] = cu[d.tab[g][j + quads]];
+                }
+#pragma unroll
+                for (int m = 0; m <= MAXDEG; m++) {
+                  if (m <= d.deg[g]) {
+                    if (e >= 0)
+                      slot = lead_base + e * (d.deg[g] + 1) + m;
+                    else  // only the nodes that are evaluation points
+                      slot = ev_index(d, g, m) < 0 ? -1 : lead_base + d.nev[g] * (d.deg[g] + 1) + ev_index(d, g, m);
+                    if (slot >= PASS * SPP && slot < (PASS + 1) * SPP) {
+                      double prod = val[0];
+#pragma unroll
+                      for (int j = 1; j < MAXDEG; j++)
+                        if (j < factors) prod = f_mul(prod, val[j]);
+                      shared_sum[m] = first ? prod : shared_sum[m] + prod;  // (groups that share the slot follow one another)
+                      if (last) {
+                        const double total = d.deg[g] == 1 || !first ? f_reduce(shared_sum[m]) : shared_sum[m];
+                        const uint32_t digits = f_signed_digits(total);
+                        const int at = slot - PASS * SPP;
+                        if (step_pairs == 0) {
+                          held[at] = digits;
+                        } else {
+                          const long value = (long)((uint64_t)digits << 32 | held[at]);
+#pragma unroll
+                          for (int q = 0; q < TILES; q++)
+                            acc[at][q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                                (long)((uint64_t)weights[q].y << 32 | weights[q].x), value, acc[at][q], 0, 0, 0);
+                        }
+                      }
+                    }
+#pragma unroll
+                    for (int j = 0; j < MAXDEG; j++) {
+                      if (j < quads) {
+                        if (m > 0) step[j < 2 ? j : 0] += 2.0 * qcur[g][j < 2 ? j : 0][2];
+                        val[j] = val[j] + step[j < 2 ? j : 0];
+                      } else if (j < factors) {
+                        val[j] += cv[d.tab[g][j + quads]];
+                      }
+                    }
+                  }
+                }
+              }
+              base += group_slots(d, g);
+            }
           }
         }
       }
-    }
-    (void)slot;
-    if (k & 1) {  // (a last pair by itself stays as it is: the reduction takes any 64-bit sum)
-#pragma unroll
-      for (int a = 0; a < SPP; a++)
-#pragma unroll
-        for (int c = 0; c < D; c++) acc[a][c] = mont_lazy(acc[a][c]);
+      (void)slot;
     }
   }
 
-  // the workgroup's sums of this launch's slots, HIGH applied once when deferred
-  constexpr int WORDS = SPP * D, CHUNKS = (WORDS + 31) / 32;
-  __shared__ uint32_t lds[BLOCK / 64][CHUNKS * 32];
+  // the workgroup's sums of this launch's slots, the columns' weights and HIGH applied once
+  constexpr int OWN = (SPP + 3) / 4, WORDS = OWN * D;  // slots and words that a wavefront sees to
+  static_assert(BLOCK == 256, "four wavefronts share the slots");
+  __shared__ uint32_t by_wave[BLOCK / 64][SPP * TILES][64];
+  __shared__ uint32_t lds[BLOCK / 64][(WORDS + 31) / 32 * 32];
   __shared__ NodesEpilogueLds<D> L;
-  const uint32_t lane = tid & 63, wave = tid >> 6;
   nodes_epilogue_stage<D>(args.epi, L);  // (the loads' trip hides behind the reduction below)
-  {  // the wavefront's sums, 32 words at a time by the transposing reduction
+  // This lane holds coordinates 4 q + g of its column's sums: the sum over a column's coordinates c of w^brev(c) times the
+  // column's weight, so of the weight's words moved up by brev(c) powers of w, those that wrap tripled; times R^2, since the
+  // digit sums come out over R and the product takes another.
+  uint32_t weight[TILES][D];
+#pragma unroll
+  for (int q = 0; q < TILES; q++) {
+    const uint32_t c = 4 * q + (lane >> 4), power = brev_bits<D>(c);
+#pragma unroll
+    for (int e = 0; e < D; e++) {
+      const uint32_t from = brev_bits<D>((brev(e, D) - power) & (D - 1));
+      uint32_t v = args.columns ? args.columns[(lane & 15) * D + from] : from == 0 ? 1u : 0u;
+      if ((uint32_t)brev(e, D) < power) v = times3(v);
+      weight[q][e] = mont_mul(v, R3);
+    }
+  }
+  // the four wavefronts' columns added up, a quarter of the slots by each
+#pragma unroll
+  for (int a = 0; a < SPP; a++)
+#pragma unroll
+    for (int q = 0; q < TILES; q++) {
+      const digit_sums &v = acc[a][q];
+      const int64_t t = (int64_t)v[0] + (int64_t)v[1] * 256 + (int64_t)v[2] * 65536 + (int64_t)v[3] * 16777216;
+      by_wave[wave][a * TILES + q][lane] = mont_reduce((uint64_t)(t + (int64_t)((uint64_t)P << 24)));  // (below 2^54.02 + 2^55)
+    }
+  __syncthreads();
+  uint32_t column[OWN][TILES];
+#pragma unroll
+  for (int a = 0; a < OWN; a++) {
+    const uint32_t at = wave * OWN + a;
+#pragma unroll
+    for (int q = 0; q < TILES; q++) {
+      uint32_t v = 0;
+      if (at < (uint32_t)SPP) {
+        v = by_wave[0][at * TILES + q][lane];
+#pragma unroll
+        for (int w = 1; w < BLOCK / 64; w++) v = fadd(v, by_wave[w][at * TILES + q][lane]);
+      }
+      column[a][q] = v;
+    }
+  }
+  {  // and added up across the lanes, 32 words at a time by the transposing reduction
     const uint32_t idx = transposed_word<32>(lane);
 #pragma unroll
-    for (int first = 0; first < WORDS; first += 32) {
+    for (int first_word = 0; first_word < WORDS; first_word += 32) {
       const uint32_t total = wave_sums_transposed<32>([&](int k) -> uint32_t {
-        const int o = first + k;
-        return o < WORDS ? lazy_reduce(acc[o / D][o % D]) : 0u;
+        const int o = first_word + k;
+        if (o >= WORDS) return 0u;
+        const uint64_t t = (uint64_t)column[o / D][0] * weight[0][o % D];
+        if constexpr (TILES == 2) return mont_reduce4(t + (uint64_t)column[o / D][TILES - 1] * weight[TILES - 1][o % D]);
+        return mont_reduce(t);
       });
-      if (transposed_writer<32>(lane)) lds[wave][first + idx] = total;
+      if (transposed_writer<32>(lane)) lds[wave][first_word + idx] = total;
     }
   }
   __syncthreads();
@@ -1992,12 +2147,10 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
     for (int q = 1; q < deg; q++) fix = mont_mul(fix, 1u);
 #pragma unroll
     for (int c = 0; c < D; c++) {
-      uint32_t v = lds[0][tid * D + c];
-#pragma unroll
-      for (int wv = 1; wv < BLOCK / 64; wv++) v = fadd(v, lds[wv][tid * D + c]);
-      sum.c[c] = mont_mul(v, fix);
+      sum.c[c] = mont_mul(lds[tid / OWN][tid % OWN * D + c], fix);
     }
-    if (args.deferred) sum = ext_mul_mont<D>(sum, load_ext<D>(args.high + (tile_start >> args.low_bits) * D));
+    // (the product's 1/R is one that the epilogue's constants expect)
+    sum = args.high ? ext_mul_mont<D>(sum, load_ext<D>(args.high + (tile_start >> args.low_bits) * D)) : ext_scale_mont<D>(sum, 1u);
   }
   // the slot sums of all workgroups and passes, and in the last workgroup of the last pass both rounds' epilogue
   if (mine) {
@@ -2039,8 +2192,10 @@ template <int D, class S, int FOLDS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel_bind(RoundArgs<D> args) {
   round_body<D, true, FOLDS, decltype(S::d), true>(S::d, args);
 }
+// (one wavefront a SIMD for 24 slots at F_p^8: two passes of twelve with two a SIMD repeat the tables' part of the work,
+// 500 us for 440)
 template <int D, class S, int PASS, int SPP>
-__global__ __launch_bounds__(BLOCK) void nodes_kernel(NodesArgs<D> args) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sweep_waves(D, SPP), sweep_waves(D, SPP)))) void nodes_kernel(NodesArgs<D> args) {
   nodes_body<D, PASS, SPP>(S::d, args);
 }
 

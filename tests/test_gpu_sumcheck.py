@@ -414,6 +414,36 @@ def test_base_field_sweep_with_block_weights(K, n, d, with_eq, monkeypatch):
                block_weights=bw)
 
 
+@pytest.mark.parametrize("form,names,cnames,d,n,K,with_eq", [
+    # one tile of the sweep, its last wavefronts without pairs; 2^8 pairs a tile, several tiles; two steps a wavefront and tile
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 10, 1, True),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 20, 1, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 10, 1, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 19, 1, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 18, 1, False),
+    # a degree's slots without and with quadratics; blocks, whose weights are HIGH
+    ("(* t0 t1)", ["t0", "t1"], [], 8, 11, 4, True),
+    ("(* t0 t1 t2)", ["t0", "t1", "t2"], [], 4, 12, 2, False),
+    ("(* t0 t1 t2)", ["t0", "t1", "t2"], [], 8, 13, 2, True),
+])
+def test_the_sweeps_sums_on_the_matrix_cores(form, names, cnames, d, n, K, with_eq, monkeypatch):
+    """Rounds 0 and 1 from the sweep whose weighted sums are products of signed digits: the oracle's proof, with values and
+    weights whose digits and words are the largest and the smallest there are."""
+    monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
+    rng = np.random.default_rng(n * 31 + d + K)
+    tables = [rng.integers(0, P, K << n, dtype=np.uint32) for _ in names]
+    tables[0][:] = P - 1
+    edges = np.array([0, 1, P - 1, P // 2, P // 2 + 1, 0x80, 0x7f7f7f7f % P, 0x80808080 % P], dtype=np.uint32)
+    tables[-1][: K << (n - 1)] = edges[rng.integers(0, len(edges), K << (n - 1))]
+    eq = rand_ext(rng, (n,), d) if with_eq else None
+    if with_eq:
+        eq[2:6] = P - 1  # (the columns' weights, and some of the digits')
+        eq[6, 1:] = 0
+    consts = rand_ext(rng, (len(cnames),), d) if cnames else None
+    bw = rand_ext(rng, (K,), d) if K > 1 else None
+    prove_both("sweep", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames, block_weights=bw)
+
+
 @pytest.mark.parametrize("form,names,cnames,d,n,base", [
     (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 8, True),
     (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 3, False),
