@@ -129,7 +129,7 @@ struct SumcheckSession {
   size_t staged_words = 0;   // and brings this many words of constants from the pinned staging area
   size_t setup_words = 0;
   struct {
-    uint64_t total_eq = 0, ones_off = 0, ones_len = 0;
+    uint64_t eq_blocks = 0, ones_off = 0, ones_len = 0;
     unsigned char eqt[1536];  // the EqTables argument of eq_tables_kernel
   } setup;
   int launch_setup(const uint32_t *staged = nullptr, size_t staged_words = 0);
