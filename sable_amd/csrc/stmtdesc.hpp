@@ -88,11 +88,23 @@ EXH_DESC_FN constexpr int node_slots(const Desc &d) {
   return n;
 }
 
-// the pairs of factors that the sweep takes as quadratics: where a row of slots costs fewer products that way and their
-// values stay small
+// The pairs of factors that the sweep takes as quadratics, where a row of slots costs fewer products that way and their
+// values stay small: one of three factors, two of four, in the first groups that have them (each is eighteen registers).
+constexpr int MAXQUADS = 4;
+template <class Desc>
+EXH_DESC_FN constexpr int group_quads(const Desc &d, int g) {
+  return d.maxx > 4 ? 0 : d.deg[g] == 4 ? 2 : d.deg[g] == 3 ? 1 : 0;
+}
+// those of group g's that are taken, and the first one's number
+template <class Desc>
+EXH_DESC_FN constexpr int first_quad(const Desc &d, int g) {
+  int n = 0;
+  for (int h = 0; h < g; h++) n += n + group_quads(d, h) <= MAXQUADS ? group_quads(d, h) : 0;
+  return n;
+}
 template <class Desc>
 EXH_DESC_FN constexpr int sweep_quads(const Desc &d, int g) {
-  return d.maxx > 4 ? 0 : d.deg[g] == 4 ? 2 : d.deg[g] == 3 ? 1 : 0;
+  return first_quad(d, g) + group_quads(d, g) <= MAXQUADS ? group_quads(d, g) : 0;
 }
 
 // the launches per round of the base-field sweep for degree D and the slots each takes: the slots are split

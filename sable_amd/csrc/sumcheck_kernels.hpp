@@ -1714,8 +1714,8 @@ EXH_HD uint32_t signed_digits(uint32_t v) { return (v + DIGIT_BIAS) ^ DIGIT_BIAS
 
 #if defined(__HIPCC__)
 typedef int digit_sums __attribute__((ext_vector_type(4)));
-// a quarter of weight k's coordinates into place: [k / 8][coordinate / 4][lane (coordinate % 4) * 4 + i + 16 (k % 4)][k / 4 % 2], byte j = digit i of
-// w 2^(8 j)
+// a quarter of weight k's coordinates into place: [k / 8][coordinate / 4][lane (coordinate % 4) * 4 + i + 16 (k % 4)][k / 4 % 2],
+// byte j = digit i of w 2^(8 j)
 template <int D>
 __device__ __forceinline__ void store_sweep_digits(uint32_t *out, uint64_t k, const Ext<D> &e, uint32_t quarter) {
   constexpr uint32_t SHIFT[4] = {R1, (uint32_t)(((uint64_t)R1 << 8) % P), (uint32_t)(((uint64_t)R1 << 16) % P),
@@ -1952,118 +1952,112 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
       // A group of three or four factors takes two of them (or two and two) as one quadratic in X1 and in X0: nine products
       // give its values at X1 = 0 and 1 and its coefficient of X1^2, each of them at X0 = 0 and 1 and as the coefficient of
       // X0^2, and the others follow by differences; a slot is then one product, where a factor at a time takes two or three.
-      double qcur[MAXG][2][3], qstep[MAXG][2][3], qtwo[MAXG][2][3], qnext[MAXG][2][3];
+      double qcur[MAXQUADS][3], qstep[MAXQUADS][3], qtwo[MAXQUADS][3], qnext[MAXQUADS][3];
+      int quads_n = 0;
 #pragma unroll
       for (int g = 0; g < MAXG; g++)
-        if (g < d.G && sweep_quads(d, g) > 0) {
+        if (g < d.G) {
 #pragma unroll
           for (int h = 0; h < 2; h++)
             if (h < sweep_quads(d, g)) {
-              const int a = d.tab[g][2 * h], b = d.tab[g][2 * h + 1];
+              const int a = d.tab[g][2 * h], b = d.tab[g][2 * h + 1], q = first_quad(d, g) + h;
               const double va[3][3] = {
                   {cu[a], u1[a], du[a]}, {cu[a] + cv[a], u1[a] + v1[a], du[a] + dv[a]}, {cv[a], v1[a], dv[a]}};
               const double vb[3][3] = {
                   {cu[b], u1[b], du[b]}, {cu[b] + cv[b], u1[b] + v1[b], du[b] + dv[b]}, {cv[b], v1[b], dv[b]}};
 #pragma unroll
               for (int k = 0; k < 3; k++) {
-                qcur[g][h][k] = f_mul(va[k][0], vb[k][0]);
-                qnext[g][h][k] = f_mul(va[k][1], vb[k][1]);
+                qcur[q][k] = f_mul(va[k][0], vb[k][0]);
+                qnext[q][k] = f_mul(va[k][1], vb[k][1]);
                 const double square = f_mul(va[k][2], vb[k][2]);
-                qtwo[g][h][k] = square + square;
-                qstep[g][h][k] = qnext[g][h][k] - qcur[g][h][k];
+                qtwo[q][k] = square + square;
+                qstep[q][k] = qnext[q][k] - qcur[q][k];
               }
+              quads_n = q + 1;
             }
         }
       int slot = 0;  // numbered group by group (point by point, node by node, then the extras) -- visited X1-major
 #pragma unroll
-      for (int x = 0; x <= MAXX; x++) {
-        if (x <= d.maxx || x == 1) {
-          if (x >= 1) {
+      for (int x = 0; x <= (d.maxx > 1 ? d.maxx : 1); x++) {
+        if (x >= 1) {
 #pragma unroll
-            for (int t = 0; t < MAXT; t++)
-              if (t < d.T + d.NV) {
-                if (x == 1)
-                  cu[t] = u1[t], cv[t] = v1[t];
-                else
-                  cu[t] += du[t], cv[t] += dv[t];
-              }
+          for (int t = 0; t < MAXT; t++)
+            if (t < d.T + d.NV) {
+              if (x == 1)
+                cu[t] = u1[t], cv[t] = v1[t];
+              else
+                cu[t] += du[t], cv[t] += dv[t];
+            }
 #pragma unroll
-            for (int g = 0; g < MAXG; g++)
+          for (int q = 0; q < MAXQUADS; q++)
+            if (q < quads_n)
 #pragma unroll
-              for (int h = 0; h < 2; h++)
-                if (g < d.G && h < sweep_quads(d, g))
-#pragma unroll
-                  for (int k = 0; k < 3; k++) {
-                    if (x == 1) {
-                      qcur[g][h][k] = qnext[g][h][k];
-                    } else {
-                      qstep[g][h][k] += qtwo[g][h][k];
-                      qcur[g][h][k] += qstep[g][h][k];
-                    }
-                  }
-          }
-          int base = 0, lead_base = 0;  // first slot of group g, and of the group whose slots it shares
-          double shared_sum[MAXDEG + 1];
-#pragma unroll
-          for (int g = 0; g < MAXG; g++) {
-            if (g < d.G) {
-              const int e = ev_index(d, g, x);  // an evaluation point's row, or at X1 = 1 the row of extras
-              const bool first = d.lead[g] == g, last = group_is_last(d, g);
-              if (first) lead_base = base;
-              if (e >= 0 || x == 1) {
-                // the row's factors at X0 = 0, the quadratics first
-                const int quads = sweep_quads(d, g), factors = d.deg[g] - quads;
-                double val[MAXDEG], step[2];
-#pragma unroll
-                for (int j = 0; j < MAXDEG; j++) {
-                  if (j < quads)
-                    val[j] = qcur[g][j < 2 ? j : 0][0], step[j < 2 ? j : 0] = qcur[g][j < 2 ? j : 0][1] - val[j];
-                  else if (j < factors)
-                    val[j] = cu[d.tab[g][j + quads]];
+              for (int k = 0; k < 3; k++) {
+                if (x == 1) {
+                  qcur[q][k] = qnext[q][k];
+                } else {
+                  qstep[q][k] += qtwo[q][k];
+                  qcur[q][k] += qstep[q][k];
                 }
+              }
+        }
+        int base = 0, lead_base = 0;  // first slot of group g, and of the group whose slots it shares
+        double shared_sum[MAXDEG + 1];
 #pragma unroll
-                for (int m = 0; m <= MAXDEG; m++) {
-                  if (m <= d.deg[g]) {
-                    if (e >= 0)
-                      slot = lead_base + e * (d.deg[g] + 1) + m;
-                    else  // only the nodes that are evaluation points
-                      slot = ev_index(d, g, m) < 0 ? -1 : lead_base + d.nev[g] * (d.deg[g] + 1) + ev_index(d, g, m);
-                    if (slot >= PASS * SPP && slot < (PASS + 1) * SPP) {
-                      double prod = val[0];
+        for (int g = 0; g < d.G; g++) {
+          const int e = ev_index(d, g, x);  // an evaluation point's row, or at X1 = 1 the row of extras
+          const bool first = d.lead[g] == g, last = group_is_last(d, g);
+          if (first) lead_base = base;
+          if (e >= 0 || x == 1) {
+            // the row's factors at X0 = 0, the quadratics first
+            const int quads = sweep_quads(d, g), factors = d.deg[g] - quads, q0 = first_quad(d, g);
+            double val[MAXDEG], step[2];
 #pragma unroll
-                      for (int j = 1; j < MAXDEG; j++)
-                        if (j < factors) prod = f_mul(prod, val[j]);
-                      shared_sum[m] = first ? prod : shared_sum[m] + prod;  // (groups that share the slot follow one another)
-                      if (last) {
-                        const double total = d.deg[g] == 1 || !first ? f_reduce(shared_sum[m]) : shared_sum[m];
-                        const uint32_t digits = f_signed_digits(total);
-                        const int at = slot - PASS * SPP;
-                        if (step_pairs == 0) {
-                          held[at] = digits;
-                        } else {
-                          const long value = (long)((uint64_t)digits << 32 | held[at]);
+            for (int j = 0; j < MAXDEG; j++) {
+              if (j < quads)
+                val[j] = qcur[q0 + (j & 1)][0], step[j & 1] = qcur[q0 + (j & 1)][1] - val[j];
+              else if (j < factors)
+                val[j] = cu[d.tab[g][j + quads]];
+            }
 #pragma unroll
-                          for (int q = 0; q < TILES; q++)
-                            acc[at][q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
-                                (long)((uint64_t)weights[q].y << 32 | weights[q].x), value, acc[at][q], 0, 0, 0);
-                        }
-                      }
-                    }
+            for (int m = 0; m <= d.deg[g]; m++) {
+              if (e >= 0)
+                slot = lead_base + e * (d.deg[g] + 1) + m;
+              else  // only the nodes that are evaluation points
+                slot = ev_index(d, g, m) < 0 ? -1 : lead_base + d.nev[g] * (d.deg[g] + 1) + ev_index(d, g, m);
+              if (slot >= PASS * SPP && slot < (PASS + 1) * SPP) {
+                double prod = val[0];
 #pragma unroll
-                    for (int j = 0; j < MAXDEG; j++) {
-                      if (j < quads) {
-                        if (m > 0) step[j < 2 ? j : 0] += 2.0 * qcur[g][j < 2 ? j : 0][2];
-                        val[j] = val[j] + step[j < 2 ? j : 0];
-                      } else if (j < factors) {
-                        val[j] += cv[d.tab[g][j + quads]];
-                      }
-                    }
+                for (int j = 1; j < MAXDEG; j++)
+                  if (j < factors) prod = f_mul(prod, val[j]);
+                shared_sum[m] = first ? prod : shared_sum[m] + prod;  // (groups that share the slot follow one another)
+                if (last) {
+                  const double total = d.deg[g] == 1 || !first ? f_reduce(shared_sum[m]) : shared_sum[m];
+                  const uint32_t digits = f_signed_digits(total);
+                  const int at = slot - PASS * SPP;
+                  if (step_pairs == 0) {
+                    held[at] = digits;
+                  } else {
+                    const long value = (long)((uint64_t)digits << 32 | held[at]);
+#pragma unroll
+                    for (int q = 0; q < TILES; q++)
+                      acc[at][q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                          (long)((uint64_t)weights[q].y << 32 | weights[q].x), value, acc[at][q], 0, 0, 0);
                   }
                 }
               }
-              base += group_slots(d, g);
+#pragma unroll
+              for (int j = 0; j < MAXDEG; j++) {
+                if (j < quads) {
+                  if (m > 0) step[j & 1] += 2.0 * qcur[q0 + (j & 1)][2];
+                  val[j] += step[j & 1];
+                } else if (j < factors) {
+                  val[j] += cv[d.tab[g][j + quads]];
+                }
+              }
             }
           }
+          base += group_slots(d, g);
         }
       }
       (void)slot;
@@ -2195,7 +2189,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 // (one wavefront a SIMD for 24 slots at F_p^8: two passes of twelve with two a SIMD repeat the tables' part of the work,
 // 500 us for 440)
 template <int D, class S, int PASS, int SPP>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sweep_waves(D, SPP), sweep_waves(D, SPP)))) void nodes_kernel(NodesArgs<D> args) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sweep_waves(D, SPP), sweep_waves(D, SPP)))) void
+nodes_kernel(NodesArgs<D> args) {
   nodes_body<D, PASS, SPP>(S::d, args);
 }
 
