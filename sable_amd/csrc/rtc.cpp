@@ -176,7 +176,9 @@ int load_job(Job *job) {
     for (int fold = 0; fold < 2; fold++)
       round[base][fold] = fn["exh::round_kernel<" + d + ", " + (base ? "true" : "false") + ", " + (fold ? "true" : "false") +
                              ", " + st + ">"];
-  hipFunction_t bind2 = fn["exh::round_kernel_bind<" + d + ", " + st + ", 2>"], bind3 = fn["exh::round_kernel_bind<" + d + ", " + st + ", 3>"];
+  hipFunction_t bind2 = fn["exh::round_kernel_bind<" + d + ", " + st + ", 2>"];
+  hipFunction_t bind3 = fn["exh::round_kernel_bind<" + d + ", " + st + ", 3>"];
+  hipFunction_t bind4 = job->D == 8 ? fn["exh::round_kernel_bind<8, " + st + ", 4>"] : nullptr;
   hipFunction_t tail = fn[tail_expression(job->D, !job->source.empty())];
   int passes = node_slots(job->desc) <= MAXACC ? nodes_launches(job->desc, job->D) : 0;
   std::vector<hipFunction_t> nodes;
@@ -189,7 +191,7 @@ int load_job(Job *job) {
     launch_module(round[in_base ? 1 : 0][fold ? 1 : 0], args, grid, 0, s);
   };
   set.launch_bind = [=](const void *args, int folds, uint32_t grid, hipStream_t s) {
-    launch_module(folds == 3 ? bind3 : bind2, args, grid, 0, s);
+    launch_module(folds == 4 ? bind4 : folds == 3 ? bind3 : bind2, args, grid, 0, s);
   };
   set.launch_nodes = [=](const void *args, int pass, uint32_t grid, hipStream_t s) {
     launch_module(nodes[(size_t)pass], args, grid, 0, s);
@@ -287,8 +289,8 @@ void rtc_request(const std::string &key, const StmtDesc &desc, int D, const std:
     for (const char *fold : {"true", "false"})
       exprs.push_back("exh::round_kernel<" + d + ", " + base + ", " + fold + ", " + st + ">");
   // (the double fold follows the base-field sweep, which a statement in direct form does not take)
-  for (const char *folds : {", 2>", ", 3>"})
-    if (source.empty()) exprs.push_back("exh::round_kernel_bind<" + d + ", " + st + folds);
+  for (const char *folds : {", 2>", ", 3>", ", 4>"})
+    if (source.empty() && (folds[2] != '4' || D == 8)) exprs.push_back("exh::round_kernel_bind<" + d + ", " + st + folds);
   exprs.push_back(tail_expression(D, !source.empty()));
   int passes = node_slots(desc) <= MAXACC ? nodes_launches(desc, D) : 0;
   for (int p = 0; p < passes; p++)

@@ -618,7 +618,7 @@ static uint32_t tile_pairs_per_thread(uint64_t n_pairs, uint64_t max_grid, uint6
   return ppt;
 }
 
-// `folds`: the folds before the sums, 0 or 1, or 2 or 3 of base tables at once; outs: the folded tables (empty: not kept)
+// `folds`: the folds before the sums, 0 or 1, or 2 to 4 of base tables at once; outs: the folded tables (empty: not kept)
 template <int D>
 static int launch_round(SumcheckSession &s, int folds, bool do_sums, const std::vector<uint32_t *> &outs,
                         uint64_t n_pairs, int j) {
@@ -668,7 +668,8 @@ static int launch_round(SumcheckSession &s, int folds, bool do_sums, const std::
   {
     // bytes this launch must move: every table read once, the folded tables written once
     uint64_t in_words = ((uint64_t)2 << folds) * n_pairs * (s.cur_base ? 1 : D), out_words = a.out[0] ? 2 * n_pairs * D : 0;
-    const char *name = folds == 3   ? "round_fold3_base"
+    const char *name = folds == 4   ? "round_fold4_base"
+                       : folds == 3 ? "round_fold3_base"
                        : folds == 2 ? "round_fold2_base"
                        : folds      ? (s.cur_base ? "round_fold_base" : "round_fold_ext")
                                     : (s.cur_base ? "round_base" : "round_ext");
@@ -1172,14 +1173,16 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   for (; j < n && status == OK; j++) {
     const bool fold_due = folds_due > 0;
     uint64_t n_pairs = (size >> folds_due) / 2;  // pairs summed in round j (after the pending folds)
-    // Rounds 2 and 3 after the base-field sweep read the base tables once more, bound by two and by three challenges at
-    // once.  When round 3 is a streaming round too, nothing of generation 2 is written: generation 3 comes from as many
-    // bytes of the base tables as generation 2 has (half as many at F_p^8), and takes fewer instructions than a fold.
+    // Rounds 2 and 3 after the base-field sweep, at F_p^8 round 4 as well, read the base tables once more, bound by two, three
+    // and four challenges at once.  When the round behind one of them is a streaming round too, it writes nothing: generation 3
+    // comes from as many bytes of the base tables as generation 2 has (half as many at F_p^8), and takes fewer instructions
+    // than a fold; generation 4 from half of generation 3's bytes at F_p^8, in the instructions of a fold.
     // A proof this way and with generation 2 kept, us: four tables of 2^26 at F_p^8 3508 and 4004, of 2^23 765 and 822;
-    // three of 2^24 at F_p^4 479 and 503.  (Where the rounds from 3 on run on slices they take generation 2 as it is.)
+    // three of 2^24 at F_p^4 479 and 503; four of 2^26 at F_p^8 2835 where 2955 with generation 3 kept.
+    // (Where the next rounds run on slices they take the generation as it is.)
     if (folds_due >= 2) {
       round = j;
-      const bool keep = folds_due == 3 || n_pairs / 2 <= slices_max();
+      const bool keep = folds_due == (D == 8 ? 4 : 3) || n_pairs / 2 <= slices_max();
       if (keep) {
         const uint64_t out_size = size >> folds_due;
         Arena &dst = ((generation + folds_due - 1) % 2 == 0) ? arena_a() : arena_b();
@@ -1193,8 +1196,9 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
         generation += folds_due;
         folds_due = 1;
       } else {
-        status = D == 4 ? launch_round<4>(*this, 2, true, {}, n_pairs, j) : launch_round<8>(*this, 2, true, {}, n_pairs, j);
-        folds_due = 3;
+        status = D == 4 ? launch_round<4>(*this, folds_due, true, {}, n_pairs, j)
+                        : launch_round<8>(*this, folds_due, true, {}, n_pairs, j);
+        folds_due++;
       }
       tail_done = false;
       continue;

@@ -372,6 +372,88 @@ __device__ __forceinline__ void accumulate_groups(const Desc &d, const V *lo, co
   }
 }
 
+// A product of four factors, as two products of two: factors 0 and 1 (with the weight on factor 0) and factors 2 and 3 are
+// quadratics in X, known from their values at 0 and 1 and their coefficient of X^2 -- a pair costs twelve products where a
+// factor at a time takes fourteen (2867 instructions for 3135 at F_p^8), and the first quadratic needs the first tables alone.
+// Registers are what it must not cost: with 25 words of it spilled the bind by three took 740 us, 559 with two.
+// (`h`: which two)
+template <class Desc>
+__device__ __forceinline__ bool product_of_four(const Desc &d) {
+  return d.G == 1 && d.deg[0] == 4 && d.nev[0] == 4;
+}
+// the last table that factors 0 and 1 are made of
+template <class Desc>
+__device__ __forceinline__ int first_half_table(const Desc &d) {
+  int last = 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int f = d.tab[0][j];
+    if (f < d.T) {
+      last = f > last ? f : last;
+    } else {
+#pragma unroll
+      for (int k = 0; k < MAXVT; k++)
+        if (k < d.vn[f - d.T]) last = d.vtab[f - d.T][k] > last ? d.vtab[f - d.T][k] : last;
+    }
+  }
+  return last;
+}
+template <int D, class Desc>
+__device__ __forceinline__ void factor_line(const Desc &d, int f, const Ext<D> *lo, const Ext<D> *hi, Ext<D> &at0, Ext<D> &slope) {
+  at0 = ext_zero<D>(), slope = ext_zero<D>();
+#pragma unroll
+  for (int t = 0; t < MAXT; t++)
+    if (t < d.T && f == t) at0 = lo[t], slope = ext_sub<D>(hi[t], lo[t]);
+#pragma unroll
+  for (int v = 0; v < MAXV; v++)
+    if (v < d.NV && f == d.T + v) {
+#pragma unroll
+      for (int k = 0; k < MAXVT; k++)
+        if (k < d.vn[v]) {
+          const int t = d.vtab[v][k];
+          const Ext<D> a = v_scale<D>(lo[t], d.vcoef[v][k], d.vcoefm[v][k]);
+          const Ext<D> b = v_scale<D>(ext_sub<D>(hi[t], lo[t]), d.vcoef[v][k], d.vcoefm[v][k]);
+          at0 = k == 0 ? a : ext_add<D>(at0, a), slope = k == 0 ? b : ext_add<D>(slope, b);
+        }
+      at0 = v_offset<D>(at0, d.vconst[v]);
+    }
+}
+template <int D>
+struct Quadratic {
+  Ext<D> at0, at1, square;  // values at 0 and 1, coefficient of X^2
+};
+template <int D, class Desc>
+__device__ __forceinline__ Quadratic<D> quadratic(const Desc &d, int h, const Ext<D> *lo, const Ext<D> *hi, const Ext<D> &w) {
+  Ext<D> a, da, b, db;
+  factor_line<D>(d, d.tab[0][2 * h], lo, hi, a, da);
+  factor_line<D>(d, d.tab[0][2 * h + 1], lo, hi, b, db);
+  if (h == 0) a = ext_mul_mont<D>(a, w), da = ext_mul_mont<D>(da, w);
+  Quadratic<D> q;
+  q.at0 = ext_mul_mont<D>(a, b);
+  q.square = ext_mul_mont<D>(da, db);
+  q.at1 = ext_mul_mont<D>(ext_add<D>(a, da), ext_add<D>(b, db));
+  return q;
+}
+template <int D, class Desc>
+__device__ __forceinline__ void accumulate_quadratics(const Desc &d, const Quadratic<D> &p, const Quadratic<D> &q, AccLazy (*acc)[D]) {
+  Ext<D> x = p.at0, y = q.at0, dx = ext_sub<D>(p.at1, p.at0), dy = ext_sub<D>(q.at1, q.at0);
+  const Ext<D> ddx = ext_add<D>(p.square, p.square), ddy = ext_add<D>(q.square, q.square);
+#pragma unroll
+  for (int at = 0; at <= MAXX; at++) {
+    if (at <= d.maxx) {
+      if (at == 1) {
+        x = p.at1, y = q.at1;
+      } else if (at > 1) {
+        dx = ext_add<D>(dx, ddx), dy = ext_add<D>(dy, ddy);
+        x = ext_add<D>(x, dx), y = ext_add<D>(y, dy);
+      }
+#pragma unroll
+      for (int k = 0; k < MAXEV; k++)
+        if (k < d.nev[0] && d.ev[0][k] == at) ext_mul_acc<D>(acc[d.acc[0] + k], x, y);
+    }
+  }
+}
+
 template <int D, class V, class Desc, int PARTS = 1, int PART = 0, class Acc>
 __device__ __forceinline__ void accumulate_pair(const Desc &d, const V *lo, const V *hi, const Ext<D> &w,
                                                 Acc (*acc)[D], const uint32_t *kc = nullptr) {
@@ -399,23 +481,17 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
   return fadd(fadd(a, b), fadd(c, d));
 }
 
-// eq((r0, .., r_(F-1)), b) for b < 2^F, F = 2 or 3 (bit k of b goes with r_k), in Montgomery form: the weights that bind
-// the first F variables of a base table at once, entry <- sum_b e[b] * T[2^F x + b] (BIND-PREFIX, src/sumcheck.lisp:496-510)
+// eq((r0, .., r_(F-1)), b) for b < 2^F, F = 2 to 4 (bit k of b goes with r_k), in Montgomery form: the weights that bind
+// the first F variables of a base table at once, entry <- sum_b e[b] * T[2^F x + b] (BIND-PREFIX, src/sumcheck.lisp:496-510).
+// Of challenges 0 to F - 1 (the last one also lies in ctrl->r_mont), a coefficient a lane, into e in powers of w: every
+// workgroup forms them for itself, and as straight code on values that are the same for all lanes the 2 or 6 products run on
+// the scalar unit, some 1,200 dependent instructions at D = 8 and F = 2 before a workgroup's first pair.  All threads call.
 template <int D, int F>
-struct BindWeights {
-  Ext<D> e[1 << F];
-};
-// The weights of challenges 0 to F - 1 (the last one also lies in ctrl->r_mont), a coefficient a lane: every workgroup
-// forms them for itself, and as straight code on values that are the same for all lanes the 2 or 6 products run on the
-// scalar unit, some 1,200 dependent instructions at D = 8 and F = 2 before a workgroup's first pair.  All threads call;
-// the words end up in scalar registers.
-template <int D, int F>
-__device__ __forceinline__ BindWeights<D, F> bind_weights(const Ctrl *ctrl) {
-  __shared__ uint32_t r[F][2 * D];           // the challenges in powers of w, times R; then their triples
-  __shared__ uint32_t e[(1 << F) * D];       // the weights, in powers of w
+__device__ __forceinline__ void bind_weights_lds(const Ctrl *ctrl, uint32_t *e) {
+  __shared__ uint32_t r[F][2 * D];  // the challenges in powers of w, times R; then their triples
   const uint32_t tid = threadIdx.x, k = tid % D;
   if (tid < (uint32_t)(F * D)) {
-    const uint32_t v = to_mont(ctrl->chal[tid / D][brev(k, D)]);
+    const uint32_t v = to_mont(ctrl->chal[tid / D][brev_bits<D>(k)]);
     r[tid / D][k] = v, r[tid / D][D + k] = times3(v);
     if (tid < (uint32_t)D) {
       const uint32_t one = k == 0 ? R1 : 0u;
@@ -441,6 +517,16 @@ __device__ __forceinline__ BindWeights<D, F> bind_weights(const Ctrl *ctrl) {
     if (tid < (uint32_t)(D << f)) e[at + k] = rest, e[(D << f) + at + k] = v;
   }
   __syncthreads();
+}
+template <int D, int F>
+struct BindWeights {
+  Ext<D> e[1 << F];
+};
+// the words end up in scalar registers
+template <int D, int F>
+__device__ __forceinline__ BindWeights<D, F> bind_weights(const Ctrl *ctrl) {
+  __shared__ uint32_t e[(1 << F) * D];
+  bind_weights_lds<D, F>(ctrl, e);
   BindWeights<D, F> w;
 #pragma unroll
   for (int b = 0; b < 1 << F; b++)
@@ -465,6 +551,145 @@ __device__ __forceinline__ Ext<D> bind(const BindWeights<D, F> &w, const uint32_
   }
   return o;
 }
+
+// ---- folds of extension elements of degree 8 on the matrix cores.  A folded entry's coordinates are fixed combinations, the
+// same for every entry of a launch, of the words it comes from: out[c] = sum_k M[c][k] in[k] mod p, of the two entries' 16
+// words when an extension table is folded (1 - r and r times the powers of w), of 2^F words when F variables of a base table
+// are bound at once.  Both sides are written in signed bytes.  A table word is four digits, in[k] = sum_j v_j 2^(8 j); a
+// coefficient is the digits of each of M[c][k] 2^(8 j) mod p; and out[c] is congruent to sum_i 2^(8 i) of its row i's sum,
+// over k and j, of digit_i(M[c][k] 2^(8 j)) v_j, an exact 32-bit sum: 32 rows, 32 entries a product.  The left operand is made
+// once by a workgroup and stays in registers; the right one is the tables' words as they lie in memory, sixteen bytes a lane;
+// what is left to the vector units is two instructions for the digits of a word read and eight to put four digit sums together
+// (digit_sums_value), 12 a coordinate of a fold where a product and the subtraction and addition about it are 25.
+// Four tables of 2^26, with the quadratics of accumulate_quadratics: the rounds bound by two and by three challenges 973 -> 862
+// and 620 -> 559 us (469 where it writes nothing), by four 415, the largest fold round 440 -> 420 (1.6 GB, 3.8 TB/s).
+// At F_p^4, where those 25 are 17, the rounds took as long one way as the other: 78.8 and 83.3 us, 62.3 and 62, 48.8 and 48.7.
+constexpr uint32_t DIGIT_BIAS = 0x80808080u;
+// the word whose bytes are the signed digits of a canonical value
+EXH_HD uint32_t signed_digits(uint32_t v) { return (v + DIGIT_BIAS) ^ DIGIT_BIAS; }
+#if defined(__HIPCC__)
+typedef int digit_sums __attribute__((ext_vector_type(4)));
+typedef int digit_sums16 __attribute__((ext_vector_type(16)));
+// sum_i 2^(8 i) d_i mod p, canonical, for |d_i| <= 2^20 (64 products of signed bytes): with a = d_0 + 2^8 d_1 and
+// b = d_2 + 2^8 d_3 within 2^28.01 the quotient's estimate from b alone leaves less than 0.64 p.
+__device__ __forceinline__ uint32_t digit_sums_value(int d0, int d1, int d2, int d3) {
+  const int a = d0 + d1 * 256, b = d2 + d3 * 256;
+  const int q = (int)(((int64_t)b * 132104 + 0x80000000ll) >> 32);  // b 2^16 / p, rounded: 132104 = rint(2^48 / p)
+  const uint32_t r = ((uint32_t)b << 16) + (uint32_t)a - (uint32_t)q * P;
+  return umin32(r, r + P);
+}
+
+// FOLDS = 1: an extension table folded by one challenge; 2 to 4: base tables bound at once.  A wavefront's 64 pairs go in two
+// batches of 32; the results have a lane hold four coordinates of an entry, and exchanges between the lanes' halves bring a
+// pair's words to its own lane.
+template <int FOLDS>
+struct FoldMap {
+  static constexpr int WORDS = FOLDS == 1 ? 16 : 1 << FOLDS;  // of memory, per folded entry
+  static constexpr int PARTS = WORDS / 4;                     // quads a lane holds of a batch (a pair's 2 WORDS, by two lanes)
+  digit_sums op[2];
+};
+// The map of a launch: of the challenge r_mont (FOLDS = 1), or of challenges 0 to FOLDS - 1.  All threads call.
+template <int FOLDS>
+__device__ __forceinline__ FoldMap<FOLDS> fold_map(const Ext<8> &r_mont, const Ctrl *ctrl) {
+  constexpr int D = 8;
+  typedef FoldMap<FOLDS> Map;
+  __shared__ uint32_t e[FOLDS == 1 ? D : D << FOLDS];  // the challenge in tower order, or a bind's weights in powers of w
+  __shared__ uint4 rows[Map::WORDS * D];               // coordinate c's four rows of word k at k * D + c
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  if constexpr (FOLDS == 1) {
+    if (tid == 0) {
+#pragma unroll
+      for (int q = 0; q < D; q++) e[q] = r_mont.c[q];
+    }
+    __syncthreads();
+  } else {
+    bind_weights_lds<D, FOLDS>(ctrl, e);
+  }
+  if (tid < (uint32_t)(Map::WORDS * D)) {
+    const uint32_t k = tid / D, to = brev_bits<D>(tid % D), up = brev_bits<D>(k % D);
+    uint32_t v;  // M[c][k] R
+    if constexpr (FOLDS == 1) {
+      const uint32_t from = brev_bits<D>((to - up) & (D - 1));
+      v = e[from];
+      if (k < (uint32_t)D) v = fsub(from == 0 ? R1 : 0u, v);
+      if (to < up) v = times3(v);
+    } else {
+      v = e[k * D + to];
+    }
+    uint32_t dig[4], row[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; j++) dig[j] = signed_digits(mont_mul(v, 1u << (8 * j)));
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) row[i] |= (dig[j] >> (8 * i) & 255u) << (8 * j);
+    rows[tid] = make_uint4(row[0], row[1], row[2], row[3]);
+  }
+  __syncthreads();
+  // this lane's row of the left operand is digit i of coordinate c, so that a lane of the result has coordinates 4 g + 0 .. 3
+  const uint32_t i = lane & 3, c = 4 * (lane >> 2 & 1) + ((lane & 31) >> 3), g = lane >> 5;
+  auto digits = [&](uint32_t k) { return (int)reinterpret_cast<const uint32_t *>(rows)[(k * D + c) * 4 + i]; };
+  Map m;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    if constexpr (FOLDS == 2) {  // a product holds the pair: its first half is the first entry's, its second half the other's
+      m.op[0][t] = g == 0 ? digits(t) : 0;
+      m.op[1][t] = g == 0 ? 0 : digits(t);
+    } else {  // an entry's words fill a product, or two
+      m.op[0][t] = digits(4 * g + t);
+      m.op[1][t] = Map::WORDS == 16 ? digits(8 + 4 * g + t) : 0;
+    }
+  }
+  return m;
+}
+// the words of a wavefront's pairs base .. base + 63 as the products take them; pairs beyond `last` are `last` again
+template <int FOLDS>
+__device__ __forceinline__ void fetch_mapped(const uint32_t *in, uint64_t base, uint32_t last, uint4 *raw) {
+  typedef FoldMap<FOLDS> Map;
+  const uint32_t lane = threadIdx.x & 63, n = lane % 32, g = lane / 32;
+  const char *const from = reinterpret_cast<const char *>(in + base * (2 * Map::WORDS));  // (the same for all lanes)
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    uint32_t at = umin32(32 * b + n, last) * (8 * Map::WORDS) + 16 * g;
+    asm("" : "+v"(at));  // (an offset from a scalar address, not one of many addresses kept in vector registers)
+#pragma unroll
+    for (int part = 0; part < Map::PARTS; part++)
+      raw[b * Map::PARTS + part] = *reinterpret_cast<const uint4 *>(from + at + part * 32);
+  }
+}
+// and the pair of this lane from them
+template <int FOLDS>
+__device__ __forceinline__ void pair_mapped(const FoldMap<FOLDS> &m, const uint4 *raw, Ext<8> &lo, Ext<8> &hi) {
+  auto words = [](const uint4 &q) {
+    return digit_sums{(int)signed_digits(q.x), (int)signed_digits(q.y), (int)signed_digits(q.z), (int)signed_digits(q.w)};
+  };
+  digit_sums16 zero;
+#pragma unroll
+  for (int q = 0; q < 16; q++) zero[q] = 0;
+  uint32_t v[2][2][4];  // [entry][batch][coordinate % 4]
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      digit_sums16 x;
+      if constexpr (FoldMap<FOLDS>::WORDS == 16) {
+        x = __builtin_amdgcn_mfma_i32_32x32x32_i8(m.op[0], words(raw[4 * b + 2 * h]), zero, 0, 0, 0);
+        x = __builtin_amdgcn_mfma_i32_32x32x32_i8(m.op[1], words(raw[4 * b + 2 * h + 1]), x, 0, 0, 0);
+      } else {
+        x = __builtin_amdgcn_mfma_i32_32x32x32_i8(m.op[FOLDS == 2 ? h : 0], words(raw[FOLDS == 2 ? b : 2 * b + h]), zero, 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[h][b][q] = digit_sums_value(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
+    }
+  // the halves of the lanes hold coordinates 0 to 3 and 4 to 7 of a batch's entries
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v[0][0][q], v[0][1][q], false, false);
+    const auto t = __builtin_amdgcn_permlane32_swap(v[1][0][q], v[1][1][q], false, false);
+    lo.c[q] = s[0], lo.c[4 + q] = s[1], hi.c[q] = t[0], hi.c[4 + q] = t[1];
+  }
+}
+#endif
 
 // the pair (lo, hi) of every table at pair index i, folding first when FOLD
 template <int D, bool IN_BASE, bool FOLD, class V, class Desc>
@@ -503,7 +728,7 @@ __device__ __forceinline__ void load_pair(const Desc &d, const uint32_t *const *
 // tables at once by the bind weights.
 template <int D, bool IN_BASE, int FOLDS>
 constexpr int raw_quads() {
-  return IN_BASE ? (FOLDS == 3 ? 4 : FOLDS == 2 ? 2 : 1) : FOLDS == 1 ? D : D / 2;
+  return IN_BASE ? (FOLDS == 4 ? 8 : FOLDS == 3 ? 4 : FOLDS == 2 ? 2 : 1) : FOLDS == 1 ? D : D / 2;
 }
 template <int D, bool IN_BASE, int FOLDS, int Q>
 __device__ __forceinline__ void fetch_raw(const uint32_t *in, uint64_t i, uint4 *raw) {
@@ -526,7 +751,7 @@ __device__ __forceinline__ Ext<D> ext_from_quads(const uint4 *q) {
 }
 template <int D, bool IN_BASE, int FOLDS, class V>
 __device__ __forceinline__ void pair_from_raw(const uint4 *raw, const Ext<D> &r, V &lo, V &hi,
-                                              const BindWeights<D, FOLDS == 3 ? 3 : 2> *bw) {
+                                              const BindWeights<D, FOLDS >= 2 ? FOLDS : 2> *bw) {
   if constexpr (FOLDS >= 2) {
     constexpr int H = FOLDS == 3 ? 2 : 1;  // quads per entry
     uint32_t v[8 * H];
@@ -902,10 +1127,14 @@ struct RoundShape {
   const uint32_t *consts;
 };
 
+// what goes through fold_map (a base table's fold by one challenge, a product a coordinate, does not)
+constexpr bool folds_mapped(int D, bool in_base, int folds) { return D == 8 && (folds >= 2 || (folds == 1 && !in_base)); }
+
 template <int D, bool IN_BASE, int FOLDS, class Desc, bool GENERATED = false>
 __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const *in, uint32_t *const *out,
                                            const RoundShape<D> &sh, const Ext<D> &r, uint32_t block,
-                                           uint32_t *partial_row, const BindWeights<D, FOLDS == 3 ? 3 : 2> *bw = nullptr) {
+                                           uint32_t *partial_row, const BindWeights<D, FOLDS >= 2 ? FOLDS : 2> *bw = nullptr,
+                                           const FoldMap<FOLDS == 0 ? 1 : FOLDS> *map = nullptr) {
   constexpr bool BASE_MODE = IN_BASE && FOLDS == 0;  // the pair's values are base-field
   using V = typename std::conditional<BASE_MODE, uint32_t, Ext<D>>::type;
   const uint32_t tid = threadIdx.x;
@@ -935,7 +1164,56 @@ __device__ __forceinline__ void round_core(const Desc &d, const uint32_t *const 
   // lanes, that round takes 49.2 us for 48.6, and the fold rounds of four tables at D = 8 399 for 229 on average.)
   // The interpreter, and a statement in direct form, which is wide and calls its evaluator in a loop, keep the plain order.
   constexpr bool AHEAD = GENERATED && !is_direct<Desc>::value;
-  if constexpr (AHEAD) {
+  if constexpr (AHEAD && folds_mapped(D, IN_BASE, FOLDS)) {
+    // (the products take a wavefront's pairs together: its lanes stay together, and those beyond the last pair neither store
+    // nor sum)
+    constexpr int Q = raw_quads<D, IN_BASE, FOLDS>(), SLOTS = FETCH_QUADS / Q < MAXT ? FETCH_QUADS / Q : MAXT;
+    const bool store = FOLDS == 1 || out[0] != nullptr;
+    uint4 raw[SLOTS][Q];
+    const uint32_t lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint64_t first = tile_start + wave * 64 < sh.n_pairs ? tile_start + wave * 64 : tile_start;
+    auto last_of = [&](uint64_t base) { return sh.n_pairs - base < 64 ? (uint32_t)(sh.n_pairs - base) - 1 : 63u; };
+#pragma unroll
+    for (int t = 0; t < SLOTS; t++)
+      if (t < d.T) fetch_mapped<FOLDS>(in[t], first, last_of(first), raw[t]);
+    for (uint32_t k = 0; k < sh.pairs_per_thread; k++) {
+      const uint64_t base = tile_start + (uint64_t)k * BLOCK + wave * 64;
+      if (base >= sh.n_pairs) break;
+      const uint64_t next = k + 1 < sh.pairs_per_thread && base + BLOCK < sh.n_pairs ? base + BLOCK : first;
+      const uint32_t last = last_of(base), next_last = last_of(next);
+      Ext<D> w;
+      if (sh.do_sums) {
+        w = load_ext<D>(sh.low + ((uint32_t)(base + lane) & (uint32_t)low_mask) * D);
+        if (!sh.deferred) w = ext_mul_mont<D>(w, load_ext<D>(sh.high + ((base + umin32(lane, last)) >> sh.low_bits) * D));
+      }
+      V lo[MAXT], hi[MAXT];
+      Quadratic<D> half;
+#pragma unroll
+      for (int t = 0; t < MAXT; t++)
+        if (t < d.T) {
+          pair_mapped<FOLDS>(*map, raw[t % SLOTS], lo[t], hi[t]);
+          if (t + SLOTS < d.T)
+            fetch_mapped<FOLDS>(in[t + SLOTS < MAXT ? t + SLOTS : 0], base, last, raw[t % SLOTS]);
+          else
+            fetch_mapped<FOLDS>(in[t % SLOTS], next, next_last, raw[t % SLOTS]);
+          if (store && lane <= last) {
+            char *const to = reinterpret_cast<char *>(out[t] + base * (2 * D));
+            uint32_t at = lane * (8 * D);
+            asm("" : "+v"(at));
+            store_ext<D>(reinterpret_cast<uint32_t *>(to + at), lo[t]);
+            store_ext<D>(reinterpret_cast<uint32_t *>(to + at + 4 * D), hi[t]);
+          }
+          // (what the first tables give by themselves, while the others' words arrive)
+          if (sh.do_sums && product_of_four(d) && t == first_half_table(d)) half = quadratic<D>(d, 0, lo, hi, w);
+        }
+      if (sh.do_sums && lane <= last) {
+        if (product_of_four(d))
+          accumulate_quadratics<D>(d, half, quadratic<D>(d, 1, lo, hi, w), acc);
+        else
+          accumulate_pair<D, V>(d, lo, hi, w, acc, sh.consts);
+      }
+    }
+  } else if constexpr (AHEAD) {
     constexpr int Q = raw_quads<D, IN_BASE, FOLDS>(), SLOTS = FETCH_QUADS / Q < MAXT ? FETCH_QUADS / Q : MAXT;
     const bool store = FOLDS == 1 || (FOLDS >= 2 && out[0] != nullptr);
     uint4 raw[SLOTS][Q];
@@ -1048,15 +1326,18 @@ __device__ __forceinline__ void round_body(const Desc &d, const RoundArgs<D> &ar
                    args.points, args.mtilde, args.c0, args.ctrl, args.consts};
   uint32_t *const partial_row = args.partials + (uint64_t)blockIdx.x * args.pstride;
   Ext<D> r = ext_zero<D>();
-  if constexpr (FOLDS >= 2) {
+  if constexpr (FOLDS == 1) {
+    const uint32_t *rp = args.ctrl ? args.ctrl->r_mont : args.r_mont;
+#pragma unroll
+    for (int c = 0; c < D; c++) r.c[c] = rp[c];
+  }
+  if constexpr (GENERATED && !is_direct<Desc>::value && folds_mapped(D, IN_BASE, FOLDS)) {
+    const FoldMap<FOLDS> map = fold_map<FOLDS>(r, args.ctrl);
+    round_core<D, IN_BASE, FOLDS, Desc, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x, partial_row, nullptr, &map);
+  } else if constexpr (FOLDS >= 2) {
     const BindWeights<D, FOLDS> bw = bind_weights<D, FOLDS>(args.ctrl);
     round_core<D, true, FOLDS, Desc, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x, partial_row, &bw);
   } else {
-    if constexpr (FOLDS == 1) {
-      const uint32_t *rp = args.ctrl ? args.ctrl->r_mont : args.r_mont;
-#pragma unroll
-      for (int c = 0; c < D; c++) r.c[c] = rp[c];
-    }
     round_core<D, IN_BASE, FOLDS, Desc, GENERATED>(d, args.in, args.out, sh, r, blockIdx.x, partial_row);
   }
 }
@@ -1704,16 +1985,11 @@ __device__ __forceinline__ uint32_t lazy_reduce(uint64_t acc) {
 // F_p^8 (2^26: 860 -> 385 us).
 constexpr int SWEEP_STEP = 128;         // pairs of a wavefront's step
 constexpr int SWEEP_MIDS = SWEEP_STEP / 16;
-constexpr uint32_t DIGIT_BIAS = 0x80808080u;
 // A digit sum grows by at most 4 * 128 * 128 a pair of its column, a column has a sixteenth of a wavefront's share of the
 // tile, and the sums of four digits are put together below 2^54.02.
 constexpr int SWEEP_PPT_BITS = 12;
 static_assert(((uint64_t)64 / 16 * 4 * 128 * 128) << SWEEP_PPT_BITS <= (uint64_t)1 << 30, "a digit sum stays within 2^30");
-// the word whose bytes are the signed digits of a canonical value
-EXH_HD uint32_t signed_digits(uint32_t v) { return (v + DIGIT_BIAS) ^ DIGIT_BIAS; }
-
 #if defined(__HIPCC__)
-typedef int digit_sums __attribute__((ext_vector_type(4)));
 // a quarter of weight k's coordinates into place: [k / 8][coordinate / 4][lane (coordinate % 4) * 4 + i + 16 (k % 4)][k / 4 % 2],
 // byte j = digit i of w 2^(8 j)
 template <int D>
@@ -2180,8 +2456,8 @@ template <int D, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void tail_kernel_narrow(TailArgs<D> args) {
   tail_body<D, Tail::EITHER>(S::d, args);
 }
-// base tables folded by the first FOLDS = 2 or 3 challenges at once, see round_core; without tables to write (out[0] null)
-// only the sums are taken
+// base tables folded by the first FOLDS = 2 or 3 (at F_p^8 also 4) challenges at once, see round_core; without tables to write
+// (out[0] null) only the sums are taken
 template <int D, class S, int FOLDS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel_bind(RoundArgs<D> args) {
   round_body<D, true, FOLDS, decltype(S::d), true>(S::d, args);

@@ -401,6 +401,31 @@ def test_streaming_rounds_with_tables_fetched_ahead(form, names, cnames, d, n, K
     assert st.has_generated_kernel(d)
 
 
+@pytest.mark.parametrize("form,names,n,K,base,with_eq", [
+    # base tables bound by two, three and four challenges: the last size whose generation 3 is kept, then those that keep 4
+    (CONFIG3, ["c0", "c1", "c2", "c3"], 12, 1, True, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], 13, 1, True, True),
+    ("(* t0 t1)", ["t0", "t1"], 14, 1, True, False),
+    ("(* t0 t1 t2)", ["t0", "t1", "t2"], 13, 2, True, True),
+    # folds whose pairs end within a wavefront's 64, and within its first half
+    (CONFIG3, ["c0", "c1", "c2", "c3"], 7, 17, False, True),
+    ("(* t0 t1 t2)", ["t0", "t1", "t2"], 6, 37, False, False),
+    ("(* t0 t1)", ["t0", "t1"], 8, 5, False, True),
+])
+def test_folds_on_the_matrix_cores(form, names, n, K, base, with_eq, monkeypatch):
+    """F_p^8: folded entries as products of signed digits, and a product of four factors by quadratics; words and challenges'
+    digits at their bounds among the tables."""
+    monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
+    rng = np.random.default_rng(n * 37 + K)
+    tables = [rng.integers(0, P, K << n, dtype=np.uint32) if base else rand_ext(rng, (K << n,), 8) for _ in names]
+    tables[0][...] = P - 1
+    edges = np.array([0, 1, P - 1, P // 2, P // 2 + 1, 0x80, 0x7f7f7f7f % P, 0x80808080 % P], dtype=np.uint32)
+    tables[-1][...] = edges[rng.integers(0, len(edges), tables[-1].shape)]
+    st, *_ = prove_both("map", 8, n, form, names, tables, eq=rand_ext(rng, (n,), 8) if with_eq else None,
+                        block_weights=rand_ext(rng, (K,), 8) if K > 1 else None)
+    assert st.has_generated_kernel(8)
+
+
 @pytest.mark.parametrize("K,n,d,with_eq", [(2, 8, 4, True), (4, 10, 4, False), (2, 6, 8, True)])
 def test_base_field_sweep_with_block_weights(K, n, d, with_eq, monkeypatch):
     """The same opening sweep when block weights are the HIGH factor (K a power of two, base tables)."""
