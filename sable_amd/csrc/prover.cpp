@@ -226,8 +226,9 @@ int sumcheck_prove(Transcript &tr, int n, const Statement &st, const uint32_t *c
 
 // g(X) at x from the message (g at 0, 2, 3, ...) and the claim, which gives g(1)
 // (NEXT-CLAIM, src/sumcheck.lisp:137-145)
+// (eq_inverse: 1 / eq_rj)
 static int next_claim(int D, int points, hf::E &claim, const uint32_t *message, const uint32_t *eq_rj,
-                      const uint32_t *x) {
+                      const uint32_t *eq_inverse, const uint32_t *x) {
   std::vector<hf::E> vals;
   hf::E g0 = hf::from(message, D), g1;
   if (eq_rj) {  // claim = (1 - r) g(0) + r g(1)
@@ -236,7 +237,7 @@ static int next_claim(int D, int points, hf::E &claim, const uint32_t *message, 
       set_error("field-division-by-zero: ext-inv of the eq point's coordinate");
       return E_DIVZERO;
     }
-    g1 = hf::mul(hf::sub(claim, hf::mul(hf::sub(hf::lift(1, D), r), g0)), hf::inv(r));
+    g1 = hf::mul(hf::sub(claim, hf::mul(hf::sub(hf::lift(1, D), r), g0)), hf::from(eq_inverse, D));
   } else {
     g1 = hf::sub(claim, g0);
   }
@@ -261,6 +262,26 @@ int sumcheck_verify(Transcript &tr, int n, const Statement &st, const uint32_t *
   hf::E claim(D);
   for (int k = 0; k < D; k++) claim[k] = claim_in[k] % P;
   absorb_header(tr, label, n, degree, blocks);
+  // the inverses of the eq point's coordinates (zero's is zero) with one inversion for all of them: running[j] is the product
+  // of those before j
+  std::vector<uint32_t> inverse;
+  if (eq && n > 0) {
+    inverse.assign((size_t)n * D, 0u);
+    std::vector<hf::E> r((size_t)n), running((size_t)n);
+    hf::E all = hf::lift(1, D);
+    for (int j = 0; j < n; j++) {
+      r[j] = hf::from(eq + (size_t)j * D, D);
+      for (uint32_t &w : r[j]) w %= P;
+      running[j] = all;
+      if (!hf::is_zero(r[j])) all = hf::mul(all, r[j]);
+    }
+    hf::E left = hf::inv(all);
+    for (int j = n - 1; j >= 0; j--) {
+      if (hf::is_zero(r[j])) continue;
+      memcpy(&inverse[(size_t)j * D], hf::mul(left, running[j]).data(), 4 * (size_t)D);
+      left = hf::mul(left, r[j]);
+    }
+  }
   for (int j = 0; j < n; j++) {
     uint32_t message[16 * 8];
     uint64_t dims[2] = {(uint64_t)points, (uint64_t)D};
@@ -271,7 +292,8 @@ int sumcheck_verify(Transcript &tr, int n, const Statement &st, const uint32_t *
     }
     uint32_t *r = out_chal + (size_t)j * D;
     tr.challenge(D, r);
-    if ((status = next_claim(D, points, claim, message, eq ? eq + (size_t)j * D : nullptr, r))) return status;
+    if ((status = next_claim(D, points, claim, message, eq ? eq + (size_t)j * D : nullptr,
+                             eq ? &inverse[(size_t)j * D] : nullptr, r))) return status;
   }
   memcpy(out_reduced, claim.data(), 4 * D);
   return OK;

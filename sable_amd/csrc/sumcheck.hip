@@ -790,7 +790,7 @@ static hf::E weight_sum(const SumcheckSession &s, int j) {
   uint64_t nl = (uint64_t)1 << s.low_bits[j];
   if (!s.has_eq) wsum = hf::lift((uint32_t)(nl % P), s.D);
   if (s.has_bw)
-    wsum = hf::mul(wsum, s.bw_sum);
+    wsum = hf::mul(wsum, hf::from(s.bw_sum.data(), s.D));
   else if (!s.has_eq)
     wsum = hf::scale(wsum, (uint32_t)(s.n_high[j] % P));
   return wsum;
@@ -870,7 +870,8 @@ int SumcheckSession::round_sums(uint32_t *out) {
       hf::E g0(c.host_pinned + (size_t)grp.acc_base * D, c.host_pinned + (size_t)(grp.acc_base + 1) * D);
       hf::E g1(c.host_pinned + (size_t)(grp.acc_base + 1) * D, c.host_pinned + (size_t)(grp.acc_base + 2) * D);
       g0 = hf::scale(g0, fix), g1 = hf::scale(g1, fix);
-      hf::E v = has_eq ? hf::add(hf::mul(hf::sub(one, eq0), g0), hf::mul(eq0, g1)) : hf::add(g0, g1);
+      const hf::E w = has_eq ? hf::from(eq0.data(), D) : one;
+      hf::E v = has_eq ? hf::add(hf::mul(hf::sub(one, w), g0), hf::mul(w, g1)) : hf::add(g0, g1);
       total = hf::add(total, hf::mul(coef, v));
     }
     memcpy(out, total.data(), 4 * D);
