@@ -315,7 +315,7 @@ static int launch_glue(const GlueArgs<D> &a, std::vector<uint8_t> *held = nullpt
     return OK;
   }
   c.prof_begin("gkr_glue", a.n, 0);
-  hipLaunchKernelGGL(gkr_glue_kernel<D>, dim3(1), dim3(64), 0, c.stream, a);
+  hipLaunchKernelGGL(gkr_glue_kernel<D>, dim3(1), dim3(BLOCK), 0, c.stream, a);
   c.prof_end();
   EXH_HIP(hipGetLastError());
   return OK;

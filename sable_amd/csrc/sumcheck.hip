@@ -1127,7 +1127,7 @@ int SumcheckSession::run_device(const DevB3S &state, uint32_t *messages, uint32_
   {
     const char *no_own = getenv("EXACTA_HIP_NO_OWN_WEIGHTS");
     const bool one_launch = size / 2 <= whole_pairs(T, D) && n <= MAXTAIL;
-    own_weights = setup_deferred && one_launch && (has_bw || K == 1) && !(no_own && no_own[0] == '1');
+    own_weights = setup_deferred && one_launch && n <= OWN_VARS + 1 && (has_bw || K == 1) && !(no_own && no_own[0] == '1');
     if (valid_entries && (!one_launch || cur_base)) {
       set_error("invalid-parameter: padded tables are extension elements for the one-workgroup launch");
       return E_PARAM;
@@ -1413,9 +1413,7 @@ int SumcheckSession::launch_tail(int j, int rounds, uint32_t grid, bool first_fo
     }
     if (j == 0) a.valid = (uint32_t)valid_entries;
     if (own_weights && grid == 1 && j == 0 && rounds == n) {  // the launch builds the weight tables behind its tables
-      uint64_t own_entries = (uint64_t)2 * n;
-      for (int jj = 0; jj < n; jj++)  // (the HIGH table of all variables but the round's and those of LOW: one entry with block weights)
-        own_entries += ((uint64_t)1 << low_bits[jj]) + ((uint64_t)1 << (n - (jj + 1) - low_bits[jj]));
+      const uint64_t own_entries = (uint64_t)2 * n + ((uint64_t)1 << n);
       a.own = 1, a.factors = has_eq ? d_weights : nullptr, a.n_vars = (uint32_t)n, a.block_high = has_bw ? 1 : 0;
       a.lds_bytes += (uint32_t)(own_entries * D * 4);
       if (staged_words) a.staged = c.host_pinned_dev + PIN_BEGIN, a.staged_dst = d_weights, a.staged_words = (uint32_t)staged_words;

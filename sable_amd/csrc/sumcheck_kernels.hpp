@@ -33,6 +33,7 @@ namespace exh {
 constexpr int MAXROUNDS = 48;  // rounds of one device-driven sumcheck (a count of them fits six bits)
 constexpr int MAXPTS = 7;      // wire points of a device-driven round message
 constexpr int MAXTAIL = 16;    // rounds the tail kernel can take
+constexpr int OWN_VARS = 10;   // variables behind the first of a session whose one launch builds its weight tables
 
 // The control block of a device-driven sumcheck, in device memory: the transcript state, the current
 // fold challenge, the launch's completion counter and the logs the host reads back at the end.
@@ -1454,12 +1455,80 @@ struct LaneBit {
 // 2^24 47.5 and 53.4).  EITHER: one kernel for both, where it is compiled at run time; INTERPRETER: for any statement.
 enum class Tail { ROUNDS, WHOLE, EITHER, INTERPRETER };
 
+// A workgroup's slice of every table into LDS, MODE: entries of base tables (0), folded on the way in (1), of extension tables
+// (2), folded (3).  Every load of a batch is issued before the first is waited for.  With a table's store to LDS between its load
+// and the next table's, a launch opened with a trip to memory for each table and 256 entries: with the state and the constants,
+// which are asked for beside the tables too, 9,900 cycles for nine tables of four entries and 18,200 for four of 2^10, now 5,700
+// and 8,500.  The lanes beyond the slice fetch its last entry again.  `valid`: entries that there are, zeros beyond (0: all).
+template <int D, int MODE, class Desc>
+__device__ __forceinline__ void load_slice(const Desc &d, const uint32_t *const *in, uint32_t *tables, uint32_t cap, uint64_t first,
+                                           uint32_t entries, uint32_t valid, const Ext<D> &r) {
+  constexpr int WORDS = (MODE & 1 ? 2 : 1) * (MODE >= 2 ? D : 1), QUADS = (WORDS + 3) / 4;
+  constexpr int SLOTS = FETCH_QUADS / QUADS;
+  const int chunks = 4 * d.T <= SLOTS ? 4 : 2 * d.T <= SLOTS ? 2 : 1;  // of 256 entries, in a batch
+  const uint64_t last = MODE == 2 && valid && valid < first + entries ? valid - 1 : first + entries - 1;
+  for (uint32_t base = threadIdx.x; base - threadIdx.x < entries; base += BLOCK * chunks)
+#pragma unroll
+    for (int t0 = 0; t0 < MAXT; t0 += SLOTS)
+      if (t0 < d.T) {
+        uint4 raw[SLOTS][QUADS];
+#pragma unroll
+        for (int s = 0; s < SLOTS; s++) {
+          const int t = t0 + s / chunks;
+          if (t < d.T) {
+            uint64_t x = first + base + s % chunks * BLOCK;
+            x = x < last ? x : last;
+            const uint32_t *p = in[t] + x * WORDS;
+            if constexpr (WORDS == 1)
+              raw[s][0].x = *p;
+            else if constexpr (WORDS == 2) {
+              const uint2 e = *reinterpret_cast<const uint2 *>(p);
+              raw[s][0].x = e.x, raw[s][0].y = e.y;
+            } else {
+#pragma unroll
+              for (int q = 0; q < QUADS; q++) raw[s][q] = reinterpret_cast<const uint4 *>(p)[q];
+            }
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < SLOTS; s++) {
+          const int t = t0 + s / chunks;
+          const uint32_t x = base + s % chunks * BLOCK;
+          if (t < d.T && x < entries) {
+            Ext<D> v;
+            if constexpr (MODE == 0) {
+              v = ext_zero<D>();
+              v.c[0] = raw[s][0].x;
+            } else if constexpr (MODE == 1) {
+              v = fold_base<D>(raw[s][0].x, raw[s][0].y, r);
+            } else if constexpr (MODE == 2) {
+              v = ext_from_quads<D>(raw[s]);
+              if (valid && first + x >= valid) v = ext_zero<D>();
+            } else {
+              v = fold_ext<D>(ext_from_quads<D>(raw[s]), ext_from_quads<D>(raw[s] + D / 4), r);
+            }
+            store_ext<D>(tables + ((size_t)t * cap + x) * D, v);
+          }
+        }
+      }
+}
+
+// What a launch of rounds leaves to a step that follows in the same launch (the first wavefront's transcript, in registers
+// and LDS, and the tables).
+struct TailEnd {
+  RunB3S tr;
+  PendingAppend pending{0, 0, 0};
+  const uint32_t *tables;  // table t's one entry at t * capacity * D
+};
+
 // Load (folding or lifting on the way in) into LDS, then per round sums -> message -> challenge -> fold
 // on the slice this workgroup holds: entries [w * E, (w + 1) * E) of every table, E = entries / grid.
 // A grid launch ends when its rounds are done and leaves the slices in `out` for the one-workgroup
 // launch that follows; that one ends with the finals.
-template <int D, Tail KIND, class Desc>
-__device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args) {
+// STEP: a step follows in the launch, which takes the transcript and the finals from `end`; they go nowhere else.  False when
+// an earlier launch had given up.
+template <int D, Tail KIND, bool STEP = false, class Desc>
+__device__ __forceinline__ bool tail_body(const Desc &d, const TailArgs<D> &args, TailEnd &end) {
   extern __shared__ __align__(16) uint32_t tail_tables[];  // [T][capacity][D]
   __shared__ uint32_t lds[BLOCK / 64][MAXACC * D];
   __shared__ uint32_t sums[2 * TRIPLED];
@@ -1474,32 +1543,52 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   const uint32_t tid = threadIdx.x, cap = args.capacity, G = KIND == Tail::WHOLE ? 1 : gridDim.x,
                  wg = KIND == Tail::WHOLE ? 0 : blockIdx.x;
   const uint32_t width = (uint32_t)d.nacc * D;
-  if (SESSION && args.staged) {  // (a trip over the bus for all of them)
-    for (uint32_t u = tid; u < args.staged_words; u += BLOCK) args.staged_dst[u] = args.staged[u];
-    __syncthreads();
-  }
-  if (args.ctrl->round != args.first_round) return;  // an earlier launch gave up: leave the count as it is
-  RunB3S tr;
-  PendingAppend pending{0, 0, 0};  // (the first wavefront's)
+  RunB3S &tr = end.tr;
+  PendingAppend &pending = end.pending;  // (the first wavefront's)
+  end.tables = tail_tables;
   MessageLane<D> ml;
   bool prefixed = false;
-  if (tid < 64) {
-    rb3s_load(tr, epi.ring, &args.ctrl->tr);
-    ml = message_lane<D>(args.points);
-  }
   uint32_t entries = (args.first_fold ? args.entries / 2 : args.entries) / G;  // of this workgroup's slice
-  {
-    Ext<D> r = ext_zero<D>();
-    if (args.first_fold) {
-#pragma unroll
-      for (int c = 0; c < D; c++) r.c[c] = args.ctrl->r_mont[c];
+  const uint32_t my_staged = SESSION && args.staged ? args.staged[tid < args.staged_words ? tid : 0] : 0;
+  auto constants = [&] {  // (a trip over the bus for all of them)
+    if (SESSION && args.staged) {
+      if (tid < args.staged_words) args.staged_dst[tid] = my_staged;
+      for (uint32_t u = tid + BLOCK; u < args.staged_words; u += BLOCK) args.staged_dst[u] = args.staged[u];
+      __syncthreads();
     }
+  };
+  // The session's own weight tables (see TailArgs::factors), in LDS behind the tables: the factors, then an element 1, which is
+  // every round's HIGH table, then the LOW tables as one heap: 2^s + x is the product over the last s variables as x's bits have
+  // it (a session's rounds are few enough that LOW takes all variables behind the round's), the table of the round before s
+  // variables.
+  const bool own_weights = SESSION && args.own != 0;
+  uint32_t *const own_factors = tail_tables + (size_t)d.T * cap * D;
+  uint32_t *const own_tables = own_factors + (size_t)2 * args.n_vars * D;
+  auto own_at = [&](uint32_t jj) { return 1u << (args.n_vars - (args.first_round + jj + 1)); };  // in elements
+  uint32_t done_rounds;
+  {
+    // what the rounds need from memory besides the tables is asked for before them and goes to LDS behind them
+    Ext<D> r = ext_zero<D>();
+    uint32_t my_state = 0, my_map = 0, my_c0 = 0, my_factor = 0;
+    const uint32_t map_words = args.points * width, c0_words = args.rounds * args.points * D, factor_words = 2 * args.n_vars * D;
+    auto ask = [&] {
+      if (args.first_fold) {
 #pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-      if (t < d.T) {
-        const uint32_t *in = args.in[t];
+        for (int c = 0; c < D; c++) r.c[c] = args.ctrl->r_mont[c];
+      }
+      my_state = reinterpret_cast<const uint32_t *>(&args.ctrl->tr)[tid < sizeof(DevB3S) / 4 ? tid : 0];
+      my_map = args.mtilde[tid < map_words ? tid : 0], my_c0 = args.c0[tid < c0_words ? tid : 0];
+      if (own_weights && args.factors) my_factor = args.factors[tid < factor_words ? tid : 0];
+      done_rounds = args.ctrl->round;
+    };
+    const bool early = !(SESSION && args.staged);
+    if (early) ask();
+    const uint64_t first = (uint64_t)wg * entries;
+    if constexpr (KIND == Tail::INTERPRETER) {
+      for (int t = 0; t < d.T; t++)
         for (uint32_t x = tid; x < entries; x += BLOCK) {
-          const uint64_t gx = (uint64_t)wg * entries + x;  // index after the fold on the way in
+          const uint64_t gx = first + x;  // index after the fold on the way in
+          const uint32_t *in = args.in[t];
           Ext<D> v;
           if (args.in_base) {
             if (args.first_fold) {
@@ -1518,60 +1607,78 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
           }
           store_ext<D>(tail_tables + ((size_t)t * cap + x) * D, v);
         }
-      }
+    } else if (args.in_base) {
+      if (args.first_fold)
+        load_slice<D, 1>(d, args.in, tail_tables, cap, first, entries, 0, r);
+      else
+        load_slice<D, 0>(d, args.in, tail_tables, cap, first, entries, 0, r);
+    } else if (args.first_fold) {
+      load_slice<D, 3>(d, args.in, tail_tables, cap, first, entries, 0, r);
+    } else {
+      load_slice<D, 2>(d, args.in, tail_tables, cap, first, entries, SESSION ? args.valid : 0, r);
     }
-    for (uint32_t u = tid; u < args.points * width; u += BLOCK) epi.mtilde[u] = args.mtilde[u];
-    for (uint32_t u = tid; u < args.rounds * args.points * D; u += BLOCK) c0s[u] = args.c0[u];
+    constants();
+    if (!early) ask();
+    if (tid < sizeof(DevB3S) / 4) epi.state[tid] = my_state;
+    if (tid < map_words) epi.mtilde[tid] = my_map;
+    for (uint32_t u = tid + BLOCK; u < map_words; u += BLOCK) epi.mtilde[u] = args.mtilde[u];
+    if (tid < c0_words) c0s[tid] = my_c0;
+    for (uint32_t u = tid + BLOCK; u < c0_words; u += BLOCK) c0s[u] = args.c0[u];
+    if (own_weights && args.factors) {
+      if (tid < factor_words) own_factors[tid] = my_factor;
+      for (uint32_t u = tid + BLOCK; u < factor_words; u += BLOCK) own_factors[u] = args.factors[u];
+    }
   }
-  if (SPREAD && ((uint32_t)d.nacc << term_bits) <= (uint32_t)SPREAD_UNITS && tid < ((uint32_t)d.nacc << term_bits)) {
-    const uint32_t a = tid >> term_bits, term = tid & ((1u << term_bits) - 1);
-    units[tid].deg = 0, units[tid].x = 0;
-    for (int j = 0; j < SPREAD_FACTORS; j++) units[tid].table[j] = 0;
+  __syncthreads();
+  if (tid < 64) {
+    rb3s_load(tr, epi.ring, reinterpret_cast<const DevB3S *>(epi.state));
+    ml = message_lane<D>(args.points);
+  }
+  if (done_rounds != args.first_round) return false;  // an earlier launch gave up: leave the count as it is
+  static_assert(SPREAD_UNITS <= 64 && BLOCK == 256, "the units are made by the last wavefront's lanes");
+  if (const uint32_t u = tid - 192; SPREAD && tid >= 192 && ((uint32_t)d.nacc << term_bits) <= (uint32_t)SPREAD_UNITS &&
+                                    u < ((uint32_t)d.nacc << term_bits)) {
+    const uint32_t a = u >> term_bits, term = u & ((1u << term_bits) - 1);
+    units[u].deg = 0, units[u].x = 0;
+    for (int j = 0; j < SPREAD_FACTORS; j++) units[u].table[j] = 0;
     uint32_t met = 0;  // the accumulator's products so far
     for (int g = 0; g < d.G; g++)
       if (a >= (uint32_t)d.acc[g] && a < (uint32_t)(d.acc[g] + d.nev[g]) && met++ == term) {
-        units[tid].deg = (uint32_t)d.deg[g], units[tid].x = (uint32_t)d.ev[g][a - (uint32_t)d.acc[g]];
+        units[u].deg = (uint32_t)d.deg[g], units[u].x = (uint32_t)d.ev[g][a - (uint32_t)d.acc[g]];
         for (int j = 0; j < SPREAD_FACTORS; j++)
-          units[tid].table[j] = (uint32_t)d.tab[g][j < d.deg[g] ? j : 0] * cap * D;
+          units[u].table[j] = (uint32_t)d.tab[g][j < d.deg[g] ? j : 0] * cap * D;
       }
   }
-  // The session's own weight tables (see TailArgs::factors), in LDS behind the tables: the factors first, then
-  // per round its LOW and its HIGH table.  An entry is a chain of at most n_vars products, one entry per thread
-  // and trip: entry x of a table over the variables [first, first + bits) is prod_b (x_b ? r_b : 1 - r_b).
-  const bool own_weights = SESSION && args.own != 0;
-  uint32_t *const own_factors = tail_tables + (size_t)d.T * cap * D;
-  uint32_t *const own_tables = own_factors + (size_t)2 * args.n_vars * D;
-  auto own_high_bits = [&](uint32_t jj) { return args.n_vars - (args.first_round + jj + 1) - args.low_bits[jj]; };
-  auto own_at = [&](uint32_t jj, bool high) {  // where round jj's LOW (HIGH) table begins, in elements
-    uint32_t at = 0;
-    for (uint32_t q = 0; q < jj; q++) at += (1u << args.low_bits[q]) + (1u << own_high_bits(q));
-    return high ? at + (1u << args.low_bits[jj]) : at;
-  };
   if (own_weights) {
-    if (args.factors)
-      for (uint32_t u = tid; u < 2 * args.n_vars * D; u += BLOCK) own_factors[u] = args.factors[u];
+    // The heap's entries of up to five variables, and beside them, on another wavefront, the products over the variables before
+    // those five (below a factor R: `parts`, a heap as well); every other entry is a product of one of each.  An entry by
+    // itself is a chain of up to nine products of 1,100 cycles and a search for its table: the weights of a session of 2^10 took
+    // 20,000 cycles that way, 3,750 this way, of 2^6 5,000 and 1,850.
+    constexpr uint32_t LAST = 5;
+    __shared__ Ext<D> parts[2 << (OWN_VARS - LAST)];
+    const uint32_t vars = args.n_vars - 1, late = vars < LAST ? vars : LAST, before = vars - late;
+    auto product = [&](uint32_t from, uint32_t bits, uint32_t x) {  // over variables [from, from + bits), times R; bits >= 1
+      auto factor = [&](uint32_t b) { return load_ext<D>(own_factors + ((size_t)(from + b) * 2 + (x >> b & 1 ? 0 : 1)) * D); };
+      Ext<D> e = factor(0);
+      for (uint32_t b = 1; b < bits; b++) e = ext_mul_mont<D>(e, factor(b));
+      return e;
+    };
+    if (!args.factors) {
+      for (uint32_t u = tid; u < 2u << vars; u += BLOCK) store_ext<D>(own_tables + (size_t)u * D, ext_lift<D>(1));
+    } else if (tid >= 64 && tid < 128) {
+      const uint32_t u = tid - 64, bits = u == 0 ? 0 : 31 - __builtin_clz(u);
+      if (u < 2u << late)
+        store_ext<D>(own_tables + (size_t)u * D, bits == 0 ? ext_lift<D>(1)  // (the exact product)
+                                                           : ext_scale_mont<D>(product(args.n_vars - bits, bits, u - (1u << bits)), 1u));
+    } else if (tid >= 128 && tid < 192) {
+      const uint32_t u = tid - 128, bits = u == 0 ? 0 : 31 - __builtin_clz(u);
+      if (bits > 0 && u < 2u << before) parts[u] = product(args.n_vars - late - bits, bits, u - (1u << bits));
+    }
     __syncthreads();
-    const uint32_t total = own_at(args.rounds, false);
-    for (uint32_t u = tid; u < total; u += BLOCK) {
-      uint32_t jj = 0, start = 0, first = 0, bits = 0;
-      for (;; jj++) {  // (u < total: the scan ends inside the rounds)
-        const uint32_t lb = args.low_bits[jj], hb = own_high_bits(jj);
-        if (u < start + (1u << lb)) {
-          first = args.first_round + jj + 1, bits = lb;
-          break;
-        }
-        start += 1u << lb;
-        if (u < start + (1u << hb)) {
-          first = args.first_round + jj + 1 + lb, bits = hb;
-          break;
-        }
-        start += 1u << hb;
-      }
-      const uint32_t x = u - start;
-      Ext<D> e = ext_lift<D>(1);
-      for (uint32_t b = 0; args.factors && b < bits; b++)
-        e = ext_mul_mont<D>(e, load_ext<D>(own_factors + ((size_t)(first + b) * 2 + (((x >> b) & 1) ? 0 : 1)) * D));
-      store_ext<D>(own_tables + (size_t)u * D, e);
+    for (uint32_t u = (2u << late) + tid; args.factors && u < 2u << vars; u += BLOCK) {
+      const uint32_t bits = 31 - __builtin_clz(u), x = u - (1u << bits), s = bits - late;
+      const Ext<D> rest = load_ext<D>(own_tables + (size_t)((1u << late) + (x >> s)) * D);
+      store_ext<D>(own_tables + (size_t)u * D, ext_mul_mont<D>(parts[(1u << s) + (x & ((1u << s) - 1))], rest));
     }
     __syncthreads();
   }
@@ -1584,9 +1691,9 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
   // as it is issued, which turns the prefetch into a wait for memory at the end of every round)
   auto load_weight = [&](uint32_t jj, uint64_t i) {
     if (own_weights) {
-      wl = load_ext<D>(own_tables + (size_t)(own_at(jj, false) + (uint32_t)(i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
+      wl = load_ext<D>(own_tables + (size_t)(own_at(jj) + (uint32_t)(i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
       wh = args.block_high ? load_ext<D>(args.weights + (args.high_off[jj] + (i >> args.low_bits[jj])) * D)
-                           : load_ext<D>(own_tables + (size_t)(own_at(jj, true) + (uint32_t)(i >> args.low_bits[jj])) * D);
+                           : load_ext<D>(own_tables);
       return;
     }
     wl = load_ext<D>(args.weights + (args.low_off[jj] + (i & (((uint64_t)1 << args.low_bits[jj]) - 1))) * D);
@@ -1651,9 +1758,8 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
 #pragma unroll
     for (int j = 0; j < SPREAD_FACTORS; j++) unit_table[j] = unit.table[j];
     const uint64_t i = (uint64_t)wg * pairs + (on ? unit_pair : pairs - 1);
-    const uint32_t *low = own_weights ? own_tables + (size_t)own_at(jj, false) * D : args.weights + args.low_off[jj] * D;
-    const uint32_t *high = own_weights && !args.block_high ? own_tables + (size_t)own_at(jj, true) * D
-                                                           : args.weights + args.high_off[jj] * D;
+    const uint32_t *low = own_weights ? own_tables + (size_t)own_at(jj) * D : args.weights + args.low_off[jj] * D;
+    const uint32_t *high = own_weights && !args.block_high ? own_tables : args.weights + args.high_off[jj] * D;
     const Ext<D> l = load_ext<D>(low + (i & (((uint64_t)1 << args.low_bits[jj]) - 1)) * D);
     const Ext<D> h = load_ext<D>(high + (i >> args.low_bits[jj]) * D);
     unit_w = ext_scale_mont<D>(ext_mul_mont<D>(l, h), on ? R2 : 0u);  // (times R for the product that takes it in below)
@@ -1829,7 +1935,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
           // leave a mark: the others may have seen this workgroup's sums and go on to publish the rounds, but
           // its slice is never written
           if (tid == 0) __hip_atomic_store(&args.ctrl->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          return;
+          return true;
         }
         for (uint32_t o = tid; o < width; o += BLOCK) {
           uint32_t v = 0;
@@ -1884,12 +1990,14 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
     }
     entries = pairs;
   }
+  if (STEP) __syncthreads();  // (the logs' stores are done before the step's other wavefronts read them)
 #pragma unroll
   for (int t = 0; t < MAXT; t++)
     if (t < d.T)
       for (uint32_t x = tid; x < entries; x += BLOCK)
         store_ext<D>(args.out + (((size_t)t * G + wg) * entries + x) * D,
                      load_ext<D>(tail_tables + ((size_t)t * cap + x) * D));
+  if (STEP) return true;
   if (G == 1 && entries == 1 && tid < (uint32_t)d.T * D)  // the finals travel with the logs
     args.ctrl->finals[tid] = tail_tables[(size_t)(tid / D) * cap * D + tid % D];
   if (tid < 64) rb3s_flush(tr, pending);
@@ -1918,6 +2026,7 @@ __device__ __forceinline__ void tail_body(const Desc &d, const TailArgs<D> &args
       __hip_atomic_store(args.host_log + args.host_flag_at, args.host_seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
+  return true;
 }
 
 // ---- rounds 0 and 1 from one sweep of the base tables.  A pair of round 1 is four base entries per table:
@@ -2447,14 +2556,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 }
 template <int D, class S, Tail KIND>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(1, 1))) void tail_kernel(TailArgs<D> args) {
-  tail_body<D, KIND>(S::d, args);
+  TailEnd end;
+  tail_body<D, KIND>(S::d, args, end);
 }
 // (the same with half the registers: a statement in direct form at F_p^8 needs more than the 512 either way, and the
 // compiler's use of the upper half of the register file for 64-bit values that it also spills has been seen to end
 // in registers it then rejects)
 template <int D, class S>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void tail_kernel_narrow(TailArgs<D> args) {
-  tail_body<D, Tail::EITHER>(S::d, args);
+  TailEnd end;
+  tail_body<D, Tail::EITHER>(S::d, args, end);
 }
 // base tables folded by the first FOLDS = 2 or 3 (at F_p^8 also 4) challenges at once, see round_core; without tables to write
 // (out[0] null) only the sums are taken
@@ -2477,7 +2588,8 @@ __global__ __launch_bounds__(BLOCK) void round_kernel_interp(RoundArgs<D> args, 
 }
 template <int D>
 __global__ __launch_bounds__(BLOCK) void tail_kernel_interp(TailArgs<D> args, StmtDesc d) {
-  tail_body<D, Tail::INTERPRETER>(d, args);
+  TailEnd end;
+  tail_body<D, Tail::INTERPRETER>(d, args, end);
 }
 
 }  // namespace exh

@@ -717,3 +717,20 @@ def test_rounds_spread_over_the_lanes(form, nt, d, K, n):
     tables = [rand_ext(rng, (K << n,), d) for _ in range(nt)]
     bw = rand_ext(rng, (K,), d) if K > 1 else None
     prove_both("spread", d, n, form, ["t%d" % t for t in range(nt)], tables, eq=rand_ext(rng, (n,), d), block_weights=bw)
+
+
+@pytest.mark.parametrize("n", range(1, 12))
+@pytest.mark.parametrize("form,names,d,base", [
+    ("(* t0 t1)", ["t0", "t1"], 4, True),    # four chunks of 256 entries a batch of loads
+    ("(* t0 t1)", ["t0", "t1"], 8, False),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], 8, True),
+    (GKR2[0], GKR2[1], 4, False),            # eight tables, one chunk a batch
+])
+def test_sessions_of_every_size_of_one_launch(form, names, d, base, n):
+    """A session's weight heap (variables behind its first: none, up to five, more) and its tables' loads, up to the first
+    size that takes a launch before it."""
+    rng = np.random.default_rng(31 * n + d + base)
+    tables = [rng.integers(0, P, 1 << n, dtype=np.uint32) if base else rand_ext(rng, (1 << n,), d) for _ in names]
+    cnames = GKR2[2] if form == GKR2[0] else []
+    constants = rand_ext(rng, (len(cnames),), d) if cnames else None
+    prove_both("sessions", d, n, form, names, tables, eq=rand_ext(rng, (n,), d), constants=constants, cnames=cnames)
