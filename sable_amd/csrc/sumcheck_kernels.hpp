@@ -1990,7 +1990,8 @@ __device__ __forceinline__ bool tail_body(const Desc &d, const TailArgs<D> &args
     }
     entries = pairs;
   }
-  if (STEP) __syncthreads();  // (the logs' stores are done before the step's other wavefronts read them)
+  const bool delivers = !STEP && args.host_log && G == 1;
+  if (STEP || delivers) __syncthreads();  // (the logs' stores are done before other wavefronts read them)
 #pragma unroll
   for (int t = 0; t < MAXT; t++)
     if (t < d.T)
@@ -1998,33 +1999,53 @@ __device__ __forceinline__ bool tail_body(const Desc &d, const TailArgs<D> &args
         store_ext<D>(args.out + (((size_t)t * G + wg) * entries + x) * D,
                      load_ext<D>(tail_tables + ((size_t)t * cap + x) * D));
   if (STEP) return true;
-  if (G == 1 && entries == 1 && tid < (uint32_t)d.T * D)  // the finals travel with the logs
-    args.ctrl->finals[tid] = tail_tables[(size_t)(tid / D) * cap * D + tid % D];
-  if (tid < 64) rb3s_flush(tr, pending);
-  if (wg == 0 && tid < 64) {
-    rb3s_store(tr, &args.ctrl->tr);
-    if (tid == 0) args.ctrl->round = args.first_round + args.rounds;
+  const uint32_t done = args.first_round + args.rounds;
+  if (G == 1 && entries == 1 && tid < (uint32_t)d.T * D) {  // the finals travel with the logs
+    const uint32_t v = tail_tables[(size_t)(tid / D) * cap * D + tid % D];
+    args.ctrl->finals[tid] = v;
+    if (delivers) args.host_log[offsetof(Ctrl, finals) / 4 + tid] = v;
   }
-  if (args.host_log && G == 1) {
-    __syncthreads();
-    // every word through the L2 (this workgroup wrote some of them a moment ago, other launches the rest); of
-    // the logs only what the rounds filled: the head, points * D words of a round's message, D of its challenge
+  if (tid < 64) {
+    rb3s_flush(tr, pending);
+    if (wg == 0) {
+      // (by way of LDS: with the state stored twice, the compiler reloads a spilled pair of registers -- its 64-bit counter, in the
+      // kernel of a wide statement -- into an odd one, which it then refuses)
+      rb3s_store(tr, reinterpret_cast<DevB3S *>(epi.state));
+      __builtin_amdgcn_wave_barrier();
+      if (tid < sizeof(DevB3S) / 4) {
+        reinterpret_cast<uint32_t *>(&args.ctrl->tr)[tid] = epi.state[tid];
+        if (delivers) args.host_log[tid] = epi.state[tid];
+      }
+      if (tid == 0) args.ctrl->round = done;
+      if (tid == 0 && delivers) args.host_log[offsetof(Ctrl, round) / 4] = done;
+    }
+  } else if (delivers) {
+    // The other wavefronts bring what the rounds filled of the logs -- points * D words of a round's message, D of its
+    // challenge -- and the mark of a grid that gave up, every word through the L2 (this workgroup wrote some of them a moment
+    // ago, other launches the rest), while the first one ends the transcript and sends its state itself.
+    const uint32_t mw = args.points * D, messages = done * mw, total = messages + done * D + 1;
     const uint32_t *words = reinterpret_cast<const uint32_t *>(args.ctrl);
-    auto deliver = [&](uint32_t at) {
-      args.host_log[at] = __hip_atomic_load(words + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    const uint32_t all_rounds = args.first_round + args.rounds, mw = args.points * D;
-    for (uint32_t u = tid; u < offsetof(Ctrl, msg) / 4; u += BLOCK) deliver(u);
-    for (uint32_t u = tid; u < all_rounds * mw; u += BLOCK)
-      deliver((uint32_t)(offsetof(Ctrl, msg) / 4) + (u / mw) * (MAXPTS * 8) + u % mw);
-    for (uint32_t u = tid; u < all_rounds * D; u += BLOCK)
-      deliver((uint32_t)(offsetof(Ctrl, chal) / 4) + (u / D) * 8 + u % D);
-    for (uint32_t u = tid; u < (uint32_t)d.T * D; u += BLOCK) deliver((uint32_t)(offsetof(Ctrl, finals) / 4) + u);
+    constexpr uint32_t TRIP = 4, LANES = BLOCK - 64;
+    for (uint32_t base = tid - 64; base < total; base += TRIP * LANES) {
+      uint32_t at[TRIP], w[TRIP];
+#pragma unroll
+      for (uint32_t k = 0; k < TRIP; k++) {
+        const uint32_t u = base + k * LANES, c = u - messages;
+        at[k] = u < messages    ? (uint32_t)(offsetof(Ctrl, msg) / 4) + u / mw * (MAXPTS * 8) + u % mw
+                : u < total - 1 ? (uint32_t)(offsetof(Ctrl, chal) / 4) + c / D * 8 + c % D
+                                : (uint32_t)(offsetof(Ctrl, gave_up) / 4);
+        w[k] = __hip_atomic_load(words + at[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < TRIP; k++)
+        if (base + k * LANES < total) args.host_log[at[k]] = w[k];
+    }
+  }
+  if (delivers) {
     __threadfence_system();
     __syncthreads();
-    if (tid == 0) {
+    if (tid == 0)
       __hip_atomic_store(args.host_log + args.host_flag_at, args.host_seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
   }
   return true;
 }
