@@ -6,8 +6,8 @@
 namespace exh {
 
 // ------------------------------------------------------------------ the layers chained on the device
-// The layers' sumchecks run back to back without the host: between two of them one small launch
-// (one wavefront) does what PROVE-UPPER does on the host there (src/gkr.lisp:248-271) -- it sends the finished
+// The layers' sumchecks run back to back without the host: between two of them one workgroup
+// does what PROVE-UPPER does on the host there (src/gkr.lisp:248-271) -- it sends the finished
 // layer's finals and draws the fresh point (SEND-FINALS), forms the next layer's point, draws the layer's
 // challenges (LAYER-CHALLENGES), absorbs the next sumcheck's header and writes that sumcheck's constants where its
 // launches expect them: the eq point's factors, the message map, the head of the control block with the
