@@ -21,17 +21,23 @@ namespace exh {
 // [first, first + bits): entry x = prod_b (x_b ? r_b : 1 - r_b) (src/field.lisp:354-363: bit b of the
 // index pairs with the b-th variable).  factors[v] = (r_v R, (1 - r_v) R): each product is exact.
 // Table `digits` (-1: none) is written in the digit form of the base-field sweep's weights (store_sweep_digits), a
-// quarter of the coordinates a thread.
+// quarter of the coordinates a thread.  It has 2^digit_bits entries, entry x that of its variables' bits of x; with `blocks`
+// it is a product with a block weight as well, the one at x >> block_from of those that begin block_weights words behind the
+// first factor.
 struct EqTables {
-  int count, digits;
+  int count, digits, digit_bits, blocks, block_from;
+  uint32_t block_weights;
   uint64_t off[67];  // in EXTs
   int first[67], bits[67];
 };
-// bits of an entry's index within a workgroup, and the workgroups of a table
+// bits of an entry's index, of those within a workgroup, and the workgroups of a table
+static __host__ __device__ inline int eq_index_bits(const EqTables &tabs, int k) {
+  return k == tabs.digits ? tabs.digit_bits : tabs.bits[k];
+}
 static __host__ __device__ inline int eq_block_bits(const EqTables &tabs, int k) { return k == tabs.digits ? 6 : 8; }
 static __host__ __device__ inline uint64_t eq_blocks(const EqTables &tabs, int k) {
-  const int inside = eq_block_bits(tabs, k);
-  return tabs.bits[k] > inside ? (uint64_t)1 << (tabs.bits[k] - inside) : 1;
+  const int bits = eq_index_bits(tabs, k), inside = eq_block_bits(tabs, k);
+  return bits > inside ? (uint64_t)1 << (bits - inside) : 1;
 }
 static uint64_t eq_grid(const EqTables &tabs) {
   uint64_t blocks = 0;
@@ -67,6 +73,8 @@ __global__ __launch_bounds__(BLOCK) void eq_tables_kernel(EqTables tabs, const u
   while (k < tabs.count && block >= eq_blocks(tabs, k)) block -= eq_blocks(tabs, k++);
   if (k == tabs.count) return;  // (a workgroup that only clears)
   const int bits = tabs.bits[k], inside = eq_block_bits(tabs, k), low = bits < inside ? bits : inside;
+  const int here = eq_index_bits(tabs, k) < inside ? eq_index_bits(tabs, k) : inside;  // of the index, in this workgroup
+  const uint32_t *const block_weights = factors + tabs.block_weights;
   // the variables' factors into LDS first: a load from memory inside each link of a chain would be most of the kernel's time
   __shared__ uint32_t lds_factors[2 * MAXROUNDS * 8];
   __shared__ Ext<D> parts[2 * 16 + MAXROUNDS / 4];
@@ -99,14 +107,17 @@ __global__ __launch_bounds__(BLOCK) void eq_tables_kernel(EqTables tabs, const u
   }
   __syncthreads();
   const uint32_t at = k == tabs.digits ? tid >> 2 : tid;
-  if (at >> low) return;
-  Ext<D> e = ext_mul_mont<D>(parts[at & 15], parts[16 + (at >> 4)]);
+  if (at >> here) return;
+  const uint32_t own = at & ((1u << low) - 1);
+  Ext<D> e = ext_mul_mont<D>(parts[own & 15], parts[16 + (own >> 4)]);
   for (int q = 0; q < shared_parts; q++) e = ext_mul_mont<D>(e, parts[32 + q]);
-  const uint64_t x = (block << low) + at;
-  if (k == tabs.digits)
+  const uint64_t x = (block << here) + at;
+  if (k == tabs.digits) {
+    if (tabs.blocks) e = ext_mul_mont<D>(e, ext_scale_mont<D>(load_ext<D>(block_weights + (x >> tabs.block_from) * D), R2));
     store_sweep_digits<D>(out + tabs.off[k] * D, x, e, tid & 3);
-  else
+  } else {
     store_ext<D>(out + (tabs.off[k] + x) * D, e);
+  }
 }
 
 template <int D>
@@ -251,6 +262,8 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
   }
   has_eq = eq != nullptr;
   has_bw = bw != nullptr;
+  const size_t host_words = (size_t)(2 * n + (has_bw ? K : 0)) * D;
+  setup_words = host_words;
   size = (uint64_t)K << n;
   round = 0;
   pending_fold = false;
@@ -308,28 +321,33 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
     if (has_bw) high_off[j] = bw_off;
   }
   // round 1's weights once more for the base-field sweep, where the rounds may open with it: by the pair index's low four
-  // bits, by the bits from there to sweep_bits in digit form, and by the rest
+  // bits, by the bits from there to sweep_bits in digit form, and by the rest.  A tile of the sweep has one weight of the rest,
+  // and 2^8 pairs or more: in shorter blocks the block weights go into the digit form instead, which then covers all pairs.
   node_slots_n = node_slots(desc);  // grid sums of the sweep that serves rounds 0 and 1
   bool all_stride_1 = true;
   for (int t = 0; t < T; t++) all_stride_1 = all_stride_1 && strides[t] == 1;
-  sweep_ready = all_stride_1 && (has_bw || K == 1) && !claim_mode && !private_buffers && sweep_fits();
+  sweep_ready = all_stride_1 && (has_bw || K == 1) && !claim_mode && !private_buffers && device_capable() && sweep_fits();
+  sweep_blocks = false;
   sweep_bits = 0, sweep_columns = sweep_digits = sweep_high = 0;
   if (sweep_ready) {
     // a tile of the pairs for every workgroup that is resident at once; HIGH covers the bits above it, or the blocks
     while (((uint64_t)1 << sweep_bits) * sweep_grid() < size / 4) sweep_bits++;
     sweep_bits = std::min(std::max(sweep_bits, 8), 8 + SWEEP_PPT_BITS);
     if (has_bw) sweep_bits = n - 2;
+    sweep_blocks = has_bw && n < 10;
+    while (sweep_blocks && ((uint64_t)1 << sweep_bits) < size / 4) sweep_bits++;
   }
-  if (sweep_ready && has_eq) {
-    const int first[3] = {2 + sweep_bits, 2, 6}, bits[3] = {n - 2 - sweep_bits, 4, sweep_bits - 4};
+  if (sweep_ready && (has_eq || sweep_blocks)) {
+    const int first[3] = {2 + sweep_bits, 2, 6}, bits[3] = {n - 2 - sweep_bits, 4, !has_eq ? 0 : sweep_blocks ? n - 6 : sweep_bits - 4};
     uint64_t *const where[3] = {&sweep_high, &sweep_columns, &sweep_digits};
-    for (int k = has_bw ? 1 : 0; k < 3; k++) {
+    for (int k = !has_eq ? 2 : has_bw ? 1 : 0; k < 3; k++) {
       *where[k] = pos;
       eqt.off[eqt.count] = pos, eqt.first[eqt.count] = first[k], eqt.bits[eqt.count] = bits[k];
       eqt.count++;
-      pos += (uint64_t)(k == 2 ? 4 : 1) << bits[k];
+      pos += k == 2 ? (uint64_t)4 << (sweep_bits - 4) : (uint64_t)1 << bits[k];
     }
-    eqt.digits = eqt.count - 1;
+    eqt.digits = eqt.count - 1, eqt.digit_bits = sweep_bits - 4;
+    eqt.blocks = sweep_blocks ? 1 : 0, eqt.block_from = n - 6, eqt.block_weights = (uint32_t)(2 * n * D);
   }
   if (!has_eq && n > 0) {
     ones_off = pos;
@@ -426,7 +444,6 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
   // ---- upload the eq factors and block weights, build the weight tables
   // staged in pinned memory when it fits (no wait: the region is not written again before this
   // session's next wait), else in a vector that must outlive the copy
-  const size_t host_words = (size_t)(2 * n + (has_bw ? K : 0)) * D;
   // (a session with buffers of its own may be one of several begun back to back: each waits for its copy)
   const bool staged = host_words <= PIN_BEGIN_WORDS && !private_buffers;
   std::vector<uint32_t> spill(staged ? 0 : host_words, 0);
@@ -443,9 +460,8 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
     for (size_t i = 0; i < (size_t)K * D; i++) host[(size_t)2 * n * D + i] = bw[i] % P;
   static_assert(sizeof(EqTables) <= sizeof(setup.eqt), "EqTables outgrew its stash");
   memcpy(setup.eqt, &eqt, sizeof(eqt));
-  setup.eq_blocks = has_eq ? eq_grid(eqt) : 0;
+  setup.eq_blocks = eq_grid(eqt);
   setup.ones_off = ones_off, setup.ones_len = has_eq ? 0 : ones_len;
-  setup_words = host_words;
   setup_deferred = defer_setup && staged;
   if (!setup_deferred) {
     if (host_words) EXH_HIP(hipMemcpyAsync(base, host, host_words * 4, hipMemcpyHostToDevice, c.stream));
@@ -549,9 +565,10 @@ static uint64_t slice_grid() {
 }
 
 // Rounds 0 and 1 of the session's base tables can come from one sweep of them, when round 2 is a streaming round as well.
-// (Its tiles, of 2^8 pairs and more, lie within one block: blocks of under 2^10 entries take the ordinary rounds.)
+// (Blocks of 2^6 entries and more: a column of sixteen pairs lies in one.  Twelve tables of 2048 blocks of 2^9 at F_p^4, the
+// opening rounds: the ordinary ones 45 + 45 + 37 us, the sweep and the bind behind it 43 + 33.)
 bool SumcheckSession::sweep_fits() const {
-  return generated && kernels->nodes_passes > 0 && node_slots_n <= MAXACC && n >= 10 &&
+  return generated && kernels->nodes_passes > 0 && node_slots_n <= MAXACC && n >= 6 && size >= 4 * (uint64_t)BLOCK &&
          (size & (size - 1)) == 0 && size / 8 > slice_pairs(st.T(), D) * slice_grid();
 }
 
@@ -731,8 +748,11 @@ static int launch_nodes_round(SumcheckSession &s, uint64_t n_pairs) {
   for (int t = 0; t < T; t++) a.in[t] = s.cur[t];
   // round 1's weights; round 0's extra factor goes in by the epilogue
   a.columns = s.has_eq ? s.d_weights + s.sweep_columns * D : nullptr;
-  a.digits = s.has_eq ? s.d_weights + s.sweep_digits * D : nullptr;
-  a.high = s.has_bw ? s.d_weights + s.high_off[1] * D : s.has_eq ? s.d_weights + s.sweep_high * D : nullptr;
+  a.digits = s.has_eq || s.sweep_blocks ? s.d_weights + s.sweep_digits * D : nullptr;
+  a.high = s.sweep_blocks ? nullptr
+           : s.has_bw     ? s.d_weights + s.high_off[1] * D
+           : s.has_eq     ? s.d_weights + s.sweep_high * D
+                          : nullptr;
   a.low_bits = (uint32_t)s.sweep_bits;
   a.n_pairs = n_pairs;
   // (every workgroup is resident at once, which spreads its fixed work -- first loads, the reduction over lanes -- over

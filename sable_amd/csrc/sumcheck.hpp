@@ -69,6 +69,7 @@ struct SumcheckSession {
   int node_slots_n = 0;  // slot sums of the base-field sweep that serves rounds 0 and 1
   bool sweep_ready = false;                     // its weights are laid out: the rounds may open with it
   int sweep_bits = 0;                            // its pairs' index below HIGH
+  bool sweep_blocks = false;                     // the block weights are in its digits
   uint64_t sweep_columns = 0, sweep_digits = 0, sweep_high = 0;  // where the weights are (with an eq point), in EXTs
   bool sweep_fits() const;
   uint64_t sweep_grid() const;

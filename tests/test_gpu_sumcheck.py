@@ -42,6 +42,16 @@ def prove_both(label, d, n, form, names, host_tables, eq=None, constants=None, c
     return st, ost, tr.proof(), got
 
 
+def proof_launches(label, d, n, st, host_tables, **given):
+    """The launches of one proof by their names, and its bytes."""
+    dev = [sa.Table.upload(t) for t in host_tables]
+    tr = sa.Transcript(label, d)
+    names = launch_names(lambda: sa.prove(tr, n, st, dev, **given))
+    for t in dev:
+        t.free()
+    return names, tr.proof()
+
+
 def test_golden_proofs_byte_for_byte(vectors):
     """tests.lisp:277-282: the prover writes the same bytes as the original prover, after the magic."""
     for v in vectors("sumcheck"):
@@ -437,6 +447,32 @@ def test_base_field_sweep_with_block_weights(K, n, d, with_eq, monkeypatch):
     consts = rand_ext(rng, (1,), d)
     prove_both("nodes-bw", d, n, CONFIG2, ["t0", "t1", "t2"], tables, eq=eq, constants=consts, cnames=["alpha"],
                block_weights=bw)
+
+
+@pytest.mark.parametrize("form,names,cnames,d,n,K,with_eq", [
+    # the longest blocks that are no tile by themselves, one and two in a workgroup's, then several in a wavefront's step; the
+    # shortest, of a column's sixteen pairs
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 9, 2, True),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 9, 64, False),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 8, 16, True),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 6, 16, True),
+    ("(* t0 t1)", ["t0", "t1"], [], 4, 6, 1024, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 9, 4, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 7, 32, False),
+    ("(* t0 t1 t2)", ["t0", "t1", "t2"], [], 8, 6, 256, True),
+])
+def test_the_sweep_over_short_blocks(form, names, cnames, d, n, K, with_eq, monkeypatch):
+    """Blocks shorter than a tile of the sweep, whose weights are among its digits: the oracle's proof, from the sweep."""
+    monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
+    rng = np.random.default_rng(n * 41 + d + K)
+    tables = [rng.integers(0, P, K << n, dtype=np.uint32) for _ in names]
+    tables[0][:] = P - 1
+    given = dict(eq=rand_ext(rng, (n,), d) if with_eq else None, block_weights=rand_ext(rng, (K,), d),
+                 constants=rand_ext(rng, (len(cnames),), d) if cnames else None)
+    given["block_weights"][-1] = P - 1
+    st, _, proof, _ = prove_both("short", d, n, form, names, tables, cnames=cnames, **given)
+    launches, again = proof_launches("short", d, n, st, tables, **given)
+    assert "round_nodes_base" in launches and again == proof
 
 
 @pytest.mark.parametrize("form,names,cnames,d,n,K,with_eq", [
