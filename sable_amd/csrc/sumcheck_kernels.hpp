@@ -34,6 +34,10 @@ constexpr int MAXROUNDS = 48;  // rounds of one device-driven sumcheck (a count 
 constexpr int MAXPTS = 7;      // wire points of a device-driven round message
 constexpr int MAXTAIL = 16;    // rounds the tail kernel can take
 constexpr int OWN_VARS = 10;   // variables behind the first of a session whose one launch builds its weight tables
+// A round's LOW table takes all variables behind the round's when they are no more than these, and HIGH is one entry then:
+// what the heap of such a session's weights stands on.
+constexpr int LOW_VARS = 13;
+static_assert(OWN_VARS <= LOW_VARS, "the weights that a session's one launch builds have one HIGH entry");
 
 // The control block of a device-driven sumcheck, in device memory: the transcript state, the current
 // fold challenge, the launch's completion counter and the logs the host reads back at the end.
@@ -121,9 +125,11 @@ struct TailArgs {
   uint32_t host_flag_at, host_seq;
   const uint32_t *consts;  // a statement in direct form: its constant slots (EXTs, Montgomery form)
   // A session whose every round runs in this one launch builds its weight tables itself (`own`), in LDS behind the
-  // tables (no set-up launch): `factors` holds (r_v R, (1 - r_v) R) for the eq point's n_vars variables; round jj's LOW
-  // table covers the low_bits[jj] variables from first_round + jj + 1 on, its HIGH table the rest.  Without an eq point
-  // (factors null) the entries are ones; with block weights (block_high) the HIGH entries are those, read from `weights`.
+  // tables (no set-up launch): `factors` holds (r_v R, (1 - r_v) R) for the eq point's n_vars <= OWN_VARS + 1 variables.
+  // They are one heap of 2^n_vars entries.  Entries [2^s, 2^(s + 1)) are the products over the last s variables, and the LOW
+  // table of the round before those; low_bits is s in that round, so that its HIGH table is one entry, and entry 0, which is
+  // one, serves every round as such.  Without an eq point (factors null) all entries are ones; with block weights (block_high)
+  // the HIGH entries are those, read from `weights`.
   const uint32_t *factors;
   uint32_t n_vars, own, block_high;
   uint32_t valid;  // entries that the tables in memory hold, zeros beyond them (0: all of them; unfolded extension tables)
