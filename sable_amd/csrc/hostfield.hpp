@@ -13,7 +13,7 @@ namespace exh {
 namespace hf {
 
 // D canonical words, tower order, D <= 8 (1 and 2 for the inverse's descent), held in place: a verifier's round is a few dozen
-// of them, and as vectors on the heap they were most of its time
+// of them, and as vectors on the heap they were most of its time.  (Nothing here checks D: the entry points do.)
 class E {
   uint32_t w_[8];
   int n_ = 0;

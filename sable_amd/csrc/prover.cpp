@@ -300,6 +300,10 @@ int sumcheck_verify(Transcript &tr, int n, const Statement &st, const uint32_t *
 }
 
 int check_final(const Statement &st, int D, const uint32_t *reduced, const uint32_t *finals, const uint32_t *consts) {
+  if (D < 1 || D > 8) {
+    set_error("invalid-parameter: degree");
+    return E_PARAM;
+  }
   uint32_t expected[8];
   evaluate_statement(st, D, finals, consts, expected);
   if (memcmp(expected, reduced, 4 * D) != 0) {

@@ -43,6 +43,14 @@ def test_device_entry_points_fail_loudly_without_a_gpu():
     assert sa.load().exh_table_upload(buf.ctypes.data_as(sa.u32p), C.c_uint64(4), 1, C.byref(h)) == sa.lib.E_DEVICE
 
 
+@pytest.mark.parametrize("d", [9, 16, 64])
+def test_the_final_check_refuses_elements_longer_than_the_fields(d):
+    """An element is held in place, eight words of it: a longer one is an error and not written past its end."""
+    st = sa.Statement("(* t0 t1)", ["t0", "t1"])
+    with pytest.raises(sa.InvalidParameter):
+        sa.check_final(np.zeros(d, np.uint32), st, np.zeros((2, d), np.uint32))
+
+
 def test_blake3_and_transcript_vectors(vectors):
     for v in vectors("blake3"):
         data = hx(v["input"])
