@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import sable_amd as sa
+from conftest import launch_names
 from oracle import binding as orc
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +62,18 @@ def test_generate_ahead_of_the_first_proof_d8():
     for n in (3, 12, 18):
         want, tabs, eq, cv = proof_pair(form, tables, [], n, d, 50 + n)
         assert device_proof(st, tabs, eq, cv, n, d) == want
+
+
+@pytest.mark.parametrize("d", [4, 8])
+def test_a_sweep_of_several_launches(d, monkeypatch):
+    """A statement of more slots than one launch of the opening sweep takes: 24 of its product of four, 8 of its product of two,
+    sixteen a launch.  One tile of the sweep, several, and two steps of a wavefront."""
+    form, tables, constants = "(+ (* t0 t1 t2 t3) (* a t0 t1))", ["t0", "t1", "t2", "t3"], ["a"]
+    st = sa.Statement(form, tables, constants)
+    assert st.generate(d, wait=True) and st.has_generated_kernel(d)
+    monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
+    for n in (10, 13, 21 if d == 4 else 20):
+        want, tabs, eq, cv = proof_pair(form, tables, constants, n, d, 70 + n)
+        out = {}
+        launches = launch_names(lambda: out.setdefault("proof", device_proof(st, tabs, eq, cv, n, d)))
+        assert launches.count("round_nodes_base") == 2 and out["proof"] == want, f"n={n}"

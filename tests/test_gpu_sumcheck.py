@@ -296,11 +296,16 @@ def test_rounds_on_a_grid_of_lds_resident_slices(form, names, cnames, d, base, w
     # linear forms with coefficients other than +-1 (a generated kernel exists for this one, too)
     ("(* (+ (* 5 t0) (* -3 t1) 7) (- t2 (* 2 t0)))", ["t0", "t1", "t2"], [], 4, 9),
     ("(* (+ (* 5 t0) (* -3 t1) 7) (- t2 (* 2 t0)))", ["t0", "t1", "t2"], [], 4, 13),
+    # the sweep's smallest size (smaller ones above, which only small grids of slices would leave to it, take ordinary rounds)
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 10),
+    ("(* t0 t1)", ["t0", "t1"], [], 8, 10),
+    ("(* (+ (* 5 t0) (* -3 t1) 7) (- t2 (* 2 t0)))", ["t0", "t1", "t2"], [], 4, 10),
 ])
 def test_round_one_in_the_base_field_and_the_double_fold(form, names, cnames, d, n, monkeypatch):
     """With base tables and streaming rounds 1 and 2 (forced here at small n; the headline sizes take this path
     by themselves) rounds 0 and 1 are summed from base-field products on a grid of (X0, X1) and round 2 folds
-    twice at once: same proof bytes, finals and folded tables as the oracle."""
+    twice at once: same proof bytes, finals and folded tables as the oracle.  From n = 10 on; with fewer variables the
+    ordinary rounds' are."""
     monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
     rng = np.random.default_rng(n * 10 + d)
     tables = [rng.integers(0, P, 1 << n, dtype=np.uint32) for _ in names]
@@ -310,13 +315,11 @@ def test_round_one_in_the_base_field_and_the_double_fold(form, names, cnames, d,
     assert st.has_generated_kernel(d)
     # and without the eq weights
     prove_both("nodes", d, n, form, names, tables, constants=consts, cnames=cnames)
+    launches, again = proof_launches("nodes", d, n, st, tables, eq=eq, constants=consts)
+    assert ("round_nodes_base" in launches) == (n >= 10) and again == proof
     monkeypatch.setenv("EXACTA_HIP_NO_BASE_ROUND1", "1")
-    tr = sa.Transcript("nodes", d)
-    dev = [sa.Table.upload(t) for t in tables]
-    sa.prove(tr, n, st, dev, eq=eq, constants=consts)
-    assert tr.proof() == proof
-    for t in dev:
-        t.free()
+    launches, again = proof_launches("nodes", d, n, st, tables, eq=eq, constants=consts)
+    assert "round_nodes_base" not in launches and again == proof
 
 
 GKR2 = ("(+ (* a p0 q1) (* a p1 q0) (* al q0 q1) (* b r0 s1) (* b r1 s0) (* bl s0 s1))",
@@ -436,7 +439,10 @@ def test_folds_on_the_matrix_cores(form, names, n, K, base, with_eq, monkeypatch
     assert st.has_generated_kernel(8)
 
 
-@pytest.mark.parametrize("K,n,d,with_eq", [(2, 8, 4, True), (4, 10, 4, False), (2, 6, 8, True)])
+@pytest.mark.parametrize("K,n,d,with_eq", [
+    (2, 8, 4, True), (4, 10, 4, False), (2, 6, 8, True),  # (the first and the last: too few pairs for the sweep)
+    (2, 10, 4, True), (4, 11, 4, True), (2, 14, 4, True), (8, 10, 4, False),
+])
 def test_base_field_sweep_with_block_weights(K, n, d, with_eq, monkeypatch):
     """The same opening sweep when block weights are the HIGH factor (K a power of two, base tables)."""
     monkeypatch.setenv("EXACTA_HIP_MAX_SLICE_PAIRS", "0")
@@ -445,8 +451,10 @@ def test_base_field_sweep_with_block_weights(K, n, d, with_eq, monkeypatch):
     bw = rand_ext(rng, (K,), d)
     eq = rand_ext(rng, (n,), d) if with_eq else None
     consts = rand_ext(rng, (1,), d)
-    prove_both("nodes-bw", d, n, CONFIG2, ["t0", "t1", "t2"], tables, eq=eq, constants=consts, cnames=["alpha"],
-               block_weights=bw)
+    st, _, proof, _ = prove_both("nodes-bw", d, n, CONFIG2, ["t0", "t1", "t2"], tables, eq=eq, constants=consts,
+                                 cnames=["alpha"], block_weights=bw)
+    launches, again = proof_launches("nodes-bw", d, n, st, tables, eq=eq, constants=consts, block_weights=bw)
+    assert ("round_nodes_base" in launches) == (n >= 10) and again == proof
 
 
 @pytest.mark.parametrize("form,names,cnames,d,n,K,with_eq", [
@@ -476,16 +484,21 @@ def test_the_sweep_over_short_blocks(form, names, cnames, d, n, K, with_eq, monk
 
 
 @pytest.mark.parametrize("form,names,cnames,d,n,K,with_eq", [
-    # one tile of the sweep, its last wavefronts without pairs; 2^8 pairs a tile, several tiles; two steps a wavefront and tile
+    # one tile of the sweep, its last wavefronts without pairs; a tile of 2^9 pairs on every workgroup, a step a wavefront;
+    # two steps a wavefront and tile
     (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 10, 1, True),
     (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 20, 1, True),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 21, 1, True),
     (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 10, 1, True),
     (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 19, 1, True),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 20, 1, True),
     (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 18, 1, False),
+    (CONFIG3, ["c0", "c1", "c2", "c3"], [], 8, 20, 1, False),
     # a degree's slots without and with quadratics; blocks, whose weights are HIGH
     ("(* t0 t1)", ["t0", "t1"], [], 8, 11, 4, True),
     ("(* t0 t1 t2)", ["t0", "t1", "t2"], [], 4, 12, 2, False),
     ("(* t0 t1 t2)", ["t0", "t1", "t2"], [], 8, 13, 2, True),
+    (CONFIG2, ["t0", "t1", "t2"], ["alpha"], 4, 20, 2, True),  # (two steps of a block's tile)
 ])
 def test_the_sweeps_sums_on_the_matrix_cores(form, names, cnames, d, n, K, with_eq, monkeypatch):
     """Rounds 0 and 1 from the sweep whose weighted sums are products of signed digits: the oracle's proof, with values and
@@ -502,7 +515,18 @@ def test_the_sweeps_sums_on_the_matrix_cores(form, names, cnames, d, n, K, with_
         eq[6, 1:] = 0
     consts = rand_ext(rng, (len(cnames),), d) if cnames else None
     bw = rand_ext(rng, (K,), d) if K > 1 else None
-    prove_both("sweep", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames, block_weights=bw)
+    orc.set_fast(orc.host_threads())
+    try:
+        st, _, proof, _ = prove_both("sweep", d, n, form, names, tables, eq=eq, constants=consts, cnames=cnames,
+                                     block_weights=bw)
+    finally:
+        orc.set_fast(0)
+    given = dict(eq=eq, constants=consts, block_weights=bw)
+    launches, again = proof_launches("sweep", d, n, st, tables, **given)
+    assert "round_nodes_base" in launches and again == proof
+    monkeypatch.setenv("EXACTA_HIP_NO_BASE_ROUND1", "1")
+    launches, again = proof_launches("sweep", d, n, st, tables, **given)
+    assert "round_nodes_base" not in launches and again == proof
 
 
 @pytest.mark.parametrize("form,names,cnames,d,n,base", [
