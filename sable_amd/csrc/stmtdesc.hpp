@@ -109,14 +109,25 @@ EXH_DESC_FN constexpr int sweep_quads(const Desc &d, int g) {
 
 // the launches per round of the base-field sweep for degree D and the slots each takes: the slots are split
 // evenly over launches of at most NODES_CAP4 (F_p^4) or NODES_CAP8 (F_p^8) slots, a slot taking D registers of sums; no
-// launches when the slot sums do not fit the accumulators' buffers
-constexpr int NODES_CAP4 = 20, NODES_CAP8 = 24;
-// wavefronts a SIMD: two, one where the sums and what a lane holds of its pairs take more than half the registers
-EXH_DESC_FN constexpr int sweep_waves(int D, int slots) { return slots * (D + 1) > 128 ? 1 : 2; }
+// launches when the slot sums do not fit the accumulators' buffers.  A launch repeats the tables' part of the work, so that at
+// F_p^4 one takes all slots there can be.  Four tables of 2^24, one launch and two, us: 24 slots 106 and 144, 32 slots 106 and
+// 152; eight tables of 2^22, 32 slots, 48 and 60.  At F_p^8 24 slots have been measured (nodes_kernel), more have not.
+constexpr int NODES_CAP4 = MAXACC, NODES_CAP8 = 24;
 template <class Desc>
 EXH_DESC_FN constexpr int nodes_slots_per_pass(const Desc &d, int D) {
   int slots = node_slots(d), cap = D == 4 ? NODES_CAP4 : NODES_CAP8, passes = (slots + cap - 1) / cap;
   return (slots + passes - 1) / passes;
+}
+// Wavefronts a SIMD: two where 256 registers hold what a lane has of a launch's slots (D sums and a word of digits each), its
+// tables (eight words fetched ahead each), their lines and linear forms' (twelve) and its quadratics.  Tables of 2^24, us of the
+// sweep by one wavefront a SIMD and by two (the words by this count): F_p^8, three tables, 15 slots 92 and 83 (213), 19 slots
+// 95 and 85 (249), 23 slots 103 and 193 (285); four tables, twice 16 slots 185 and 208 (260), 24 slots 123 and 284 (336);
+// F_p^4, four tables, 32 slots 107 and 161 (276).
+template <class Desc>
+EXH_DESC_FN constexpr int sweep_waves(const Desc &d, int D, int slots) {
+  int words = slots * (D + 1) + 8 * d.T + 12 * (d.T + d.NV);
+  for (int g = 0; g < d.G; g++) words += 18 * sweep_quads(d, g);
+  return words > 256 ? 1 : 2;
 }
 template <class Desc>
 EXH_DESC_FN constexpr int nodes_launches(const Desc &d, int D) {

@@ -574,7 +574,7 @@ bool SumcheckSession::sweep_fits() const {
 
 // Its workgroups: as many as are resident at once.
 uint64_t SumcheckSession::sweep_grid() const {
-  const int waves = sweep_waves(D, nodes_slots_per_pass(desc, D));
+  const int waves = sweep_waves(desc, D, nodes_slots_per_pass(desc, D));
   return (uint64_t)waves * (uint64_t)std::max(ctx().compute_units, 1);
 }
 

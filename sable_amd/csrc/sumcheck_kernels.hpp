@@ -2603,7 +2603,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 // (one wavefront a SIMD for 24 slots at F_p^8: two passes of twelve with two a SIMD repeat the tables' part of the work,
 // 500 us for 440)
 template <int D, class S, int PASS, int SPP>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sweep_waves(D, SPP), sweep_waves(D, SPP)))) void
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sweep_waves(S::d, D, SPP), sweep_waves(S::d, D, SPP)))) void
 nodes_kernel(NodesArgs<D> args) {
   nodes_body<D, PASS, SPP>(S::d, args);
 }

@@ -64,10 +64,11 @@ def test_generate_ahead_of_the_first_proof_d8():
         assert device_proof(st, tabs, eq, cv, n, d) == want
 
 
-@pytest.mark.parametrize("d", [4, 8])
-def test_a_sweep_of_several_launches(d, monkeypatch):
-    """A statement of more slots than one launch of the opening sweep takes: 24 of its product of four, 8 of its product of two,
-    sixteen a launch.  One tile of the sweep, several, and two steps of a wavefront."""
+@pytest.mark.parametrize("d,passes", [(4, 1), (8, 2)])
+def test_a_sweep_of_many_slots(d, passes, monkeypatch):
+    """A statement of 32 slots, 24 of its product of four and 8 of its product of two: more than a launch of the opening sweep
+    takes at F_p^8, where it has sixteen, and than two wavefronts a SIMD have the registers for at F_p^4.  One tile of the sweep,
+    several, and two steps of a wavefront."""
     form, tables, constants = "(+ (* t0 t1 t2 t3) (* a t0 t1))", ["t0", "t1", "t2", "t3"], ["a"]
     st = sa.Statement(form, tables, constants)
     assert st.generate(d, wait=True) and st.has_generated_kernel(d)
@@ -76,4 +77,4 @@ def test_a_sweep_of_several_launches(d, monkeypatch):
         want, tabs, eq, cv = proof_pair(form, tables, constants, n, d, 70 + n)
         out = {}
         launches = launch_names(lambda: out.setdefault("proof", device_proof(st, tabs, eq, cv, n, d)))
-        assert launches.count("round_nodes_base") == 2 and out["proof"] == want, f"n={n}"
+        assert launches.count("round_nodes_base") == passes and out["proof"] == want, f"n={n}"
