@@ -17,7 +17,7 @@ namespace exh {
 struct KernelSet {  // the launchers generated for one statement and one degree D, at build time or at run time
   std::function<void(const void *args, bool in_base, bool fold, uint32_t grid, hipStream_t stream)> launch;
   std::function<void(const void *args, uint32_t grid, hipStream_t stream)> launch_tail;
-  // base tables folded two or three times at once (rounds 2 and 3 after the base-field sweep), and that sweep's slot sums
+  // base tables folded two to four times at once (the rounds after the base-field sweep), and that sweep's slot sums
   std::function<void(const void *args, int folds, uint32_t grid, hipStream_t stream)> launch_bind;
   std::function<void(const void *args, int pass, uint32_t grid, hipStream_t stream)> launch_nodes;
   int nodes_passes = 0;  // launches of launch_nodes per round (0: not available)

@@ -2083,7 +2083,7 @@ template <int D>
 struct NodesArgs {
   const uint32_t *in[MAXT];  // base tables
   // round 1's weights in three factors: the pair index's low four bits (16 EXTs), the bits from there to low_bits in digit
-  // form (SWEEP_* below), and HIGH for the rest (null: ones)
+  // form (SWEEP_* below), and HIGH for the rest (null: ones; the weights of blocks shorter than a tile are in the digits)
   const uint32_t *columns, *digits, *high;
   uint64_t n_pairs;          // pairs of round 1, four base entries each: a multiple of BLOCK
   uint32_t low_bits, pairs_per_thread;  // a workgroup's tile stays within 2^low_bits pairs
@@ -2117,10 +2117,9 @@ __device__ __forceinline__ uint32_t lazy_reduce(uint64_t acc) {
 // What that takes from the vector units, which bound the sweep: a slot's weighted sum is two instructions a pair (its digits)
 // where a multiply-add a coordinate, their reductions and a canonical value are eleven at F_p^4 and nineteen at F_p^8, and
 // half the registers, so that F_p^8 needs one pass for the 24 slots of a product of four, not three.  With the quadratics
-// below: 283 instructions a pair for 559 with three tables at F_p^4 (2^24 entries: 100 -> 70 us), 480 for 1455 with four at
-// F_p^8 (2^26: 860 -> 385 us).
+// below, by the counters: 327 vector instructions a pair for 559 with three tables at F_p^4 (2^24 entries: 100 -> 70 us), 517
+// for 1455 with four at F_p^8 (2^26: 860 -> 355 to 385 us).
 constexpr int SWEEP_STEP = 128;         // pairs of a wavefront's step
-constexpr int SWEEP_MIDS = SWEEP_STEP / 16;
 // A digit sum grows by at most 4 * 128 * 128 a pair of its column, a column has a sixteenth of a wavefront's share of the
 // tile, and the sums of four digits are put together below 2^54.02.
 constexpr int SWEEP_PPT_BITS = 12;
@@ -2318,7 +2317,7 @@ __device__ __forceinline__ void nodes_body(const Desc &d, const NodesArgs<D> &ar
       for (int q = 0; q < TILES; q++) wahead[q] = reinterpret_cast<const uint2 *>(at)[q * 64 + lane];
     }
   };
-  // without an eq point every weight is one: coordinate 0's row i has digit i of 2^(8 j), one at j = i
+  // without digits every weight is one: coordinate 0's row i has digit i of 2^(8 j), one at j = i
 #pragma unroll
   for (int q = 0; q < TILES; q++)
     wahead[q].x = wahead[q].y = q == 0 && (lane & 15) < 4 ? 1u << (8 * (lane & 15)) : 0u;
@@ -2600,8 +2599,8 @@ template <int D, class S, int FOLDS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void round_kernel_bind(RoundArgs<D> args) {
   round_body<D, true, FOLDS, decltype(S::d), true>(S::d, args);
 }
-// (one wavefront a SIMD for 24 slots at F_p^8: two passes of twelve with two a SIMD repeat the tables' part of the work,
-// 500 us for 440)
+// (24 slots at F_p^8 by one wavefront a SIMD: two passes of twelve with two a SIMD repeat the tables' part of the work, 487 us
+// for 356 with four tables of 2^26 and 162 for 123 of 2^24; three tables, 15 slots, two passes and one 114 and 81)
 template <int D, class S, int PASS, int SPP>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sweep_waves(S::d, D, SPP), sweep_waves(S::d, D, SPP)))) void
 nodes_kernel(NodesArgs<D> args) {
