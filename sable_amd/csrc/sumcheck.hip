@@ -21,23 +21,20 @@ namespace exh {
 // [first, first + bits): entry x = prod_b (x_b ? r_b : 1 - r_b) (src/field.lisp:354-363: bit b of the
 // index pairs with the b-th variable).  factors[v] = (r_v R, (1 - r_v) R): each product is exact.
 // Table `digits` (-1: none) is written in the digit form of the base-field sweep's weights (store_sweep_digits), a
-// quarter of the coordinates a thread.  It has 2^digit_bits entries, entry x that of its variables' bits of x; with `blocks`
-// it is a product with a block weight as well, the one at x >> block_from of those that begin block_weights words behind the
-// first factor.
+// quarter of the coordinates a thread.  It covers digit_vars variables, the first bits of its index; with `blocks` an entry is
+// a product with a block weight as well, the one at x >> block_from of those that begin block_weights words behind the first
+// factor.
 struct EqTables {
-  int count, digits, digit_bits, blocks, block_from;
+  int count, digits, digit_vars, blocks, block_from;
   uint32_t block_weights;
   uint64_t off[67];  // in EXTs
   int first[67], bits[67];
 };
-// bits of an entry's index, of those within a workgroup, and the workgroups of a table
-static __host__ __device__ inline int eq_index_bits(const EqTables &tabs, int k) {
-  return k == tabs.digits ? tabs.digit_bits : tabs.bits[k];
-}
+// bits of an entry's index within a workgroup, and the workgroups of a table
 static __host__ __device__ inline int eq_block_bits(const EqTables &tabs, int k) { return k == tabs.digits ? 6 : 8; }
 static __host__ __device__ inline uint64_t eq_blocks(const EqTables &tabs, int k) {
-  const int bits = eq_index_bits(tabs, k), inside = eq_block_bits(tabs, k);
-  return bits > inside ? (uint64_t)1 << (bits - inside) : 1;
+  const int inside = eq_block_bits(tabs, k);
+  return tabs.bits[k] > inside ? (uint64_t)1 << (tabs.bits[k] - inside) : 1;
 }
 static uint64_t eq_grid(const EqTables &tabs) {
   uint64_t blocks = 0;
@@ -72,8 +69,8 @@ __global__ __launch_bounds__(BLOCK) void eq_tables_kernel(EqTables tabs, const u
   uint64_t block = blockIdx.x;
   while (k < tabs.count && block >= eq_blocks(tabs, k)) block -= eq_blocks(tabs, k++);
   if (k == tabs.count) return;  // (a workgroup that only clears)
-  const int bits = tabs.bits[k], inside = eq_block_bits(tabs, k), low = bits < inside ? bits : inside;
-  const int here = eq_index_bits(tabs, k) < inside ? eq_index_bits(tabs, k) : inside;  // of the index, in this workgroup
+  const int bits = k == tabs.digits ? tabs.digit_vars : tabs.bits[k], inside = eq_block_bits(tabs, k);
+  const int low = bits < inside ? bits : inside, here = tabs.bits[k] < inside ? tabs.bits[k] : inside;  // (of variables; of the index)
   const uint32_t *const block_weights = factors + tabs.block_weights;
   // the variables' factors into LDS first: a load from memory inside each link of a chain would be most of the kernel's time
   __shared__ uint32_t lds_factors[2 * MAXROUNDS * 8];
@@ -338,15 +335,15 @@ int SumcheckSession::begin(const Statement &statement, int D_, int n_, const uin
     while (sweep_blocks && ((uint64_t)1 << sweep_bits) < size / 4) sweep_bits++;
   }
   if (sweep_ready && (has_eq || sweep_blocks)) {
-    const int first[3] = {2 + sweep_bits, 2, 6}, bits[3] = {n - 2 - sweep_bits, 4, !has_eq ? 0 : sweep_blocks ? n - 6 : sweep_bits - 4};
+    const int first[3] = {2 + sweep_bits, 2, 6}, bits[3] = {n - 2 - sweep_bits, 4, sweep_bits - 4};
     uint64_t *const where[3] = {&sweep_high, &sweep_columns, &sweep_digits};
     for (int k = !has_eq ? 2 : has_bw ? 1 : 0; k < 3; k++) {
       *where[k] = pos;
       eqt.off[eqt.count] = pos, eqt.first[eqt.count] = first[k], eqt.bits[eqt.count] = bits[k];
       eqt.count++;
-      pos += k == 2 ? (uint64_t)4 << (sweep_bits - 4) : (uint64_t)1 << bits[k];
+      pos += (uint64_t)(k == 2 ? 4 : 1) << bits[k];
     }
-    eqt.digits = eqt.count - 1, eqt.digit_bits = sweep_bits - 4;
+    eqt.digits = eqt.count - 1, eqt.digit_vars = !has_eq ? 0 : sweep_blocks ? n - 6 : sweep_bits - 4;
     eqt.blocks = sweep_blocks ? 1 : 0, eqt.block_from = n - 6, eqt.block_weights = (uint32_t)(2 * n * D);
   }
   if (!has_eq && n > 0) {
