@@ -45,7 +45,7 @@ def int32_mul_peak(rate=None):
 # the same counter reads for the plain copy kernel of `--workload copy`), and 32-bit integer multiply instructions
 # per lane and prove from the kernels' instruction streams times their trip counts (profiles/ holds both summaries).
 MEASURED = {
-    "kernel_sources_sha256": "635a4a1a49b1ded03494967a1d00e936fd02dc1c2290dcc01960fdab7e4b07ca",
+    "kernel_sources_sha256": "f0ea83a893d02d3c9b75a1eafbab5453db44419164b12001885840d738e8497f",
     "traffic": {("round_nodes_base", 24): 215074963, ("round_fold2_base", 24): 202947230, ("round_fold3_base", 24): 303094495},
     # per pair: none in the sweep (its weighted sums are matrix products of bytes), and multiply-adds and multiplies of the
     # reductions of 344 in round 2 (2^21 pairs), 440 in round 3 (2^20) and 344 in the extension rounds (2^19 + 2^18 + ...)

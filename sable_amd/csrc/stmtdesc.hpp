@@ -122,7 +122,7 @@ EXH_DESC_FN constexpr int nodes_slots_per_pass(const Desc &d, int D) {
 // tables (eight words fetched ahead each), their lines and linear forms' (twelve) and its quadratics.  Tables of 2^24, us of the
 // sweep by one wavefront a SIMD and by two (the words by this count): F_p^8, three tables, 15 slots 92 and 83 (213), 19 slots
 // 95 and 85 (249), 23 slots 103 and 193 (285); four tables, twice 16 slots 185 and 208 (260), 24 slots 123 and 284 (336);
-// F_p^4, four tables, 32 slots 107 and 161 (276).
+// F_p^4, four tables, 32 slots 107 and 161 (276); twelve tables of 2^20, 8 slots, 35 and 43 (280).
 template <class Desc>
 EXH_DESC_FN constexpr int sweep_waves(const Desc &d, int D, int slots) {
   int words = slots * (D + 1) + 8 * d.T + 12 * (d.T + d.NV);

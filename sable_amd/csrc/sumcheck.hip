@@ -563,7 +563,7 @@ static uint64_t slice_grid() {
 
 // Rounds 0 and 1 of the session's base tables can come from one sweep of them, when round 2 is a streaming round as well.
 // (Blocks of 2^6 entries and more: a column of sixteen pairs lies in one.  Twelve tables of 2048 blocks of 2^9 at F_p^4, the
-// opening rounds: the ordinary ones 45 + 45 + 37 us, the sweep and the bind behind it 43 + 33.)
+// opening rounds: the ordinary ones 45 + 45 + 37 us, the sweep and the bind behind it 35 + 34.)
 bool SumcheckSession::sweep_fits() const {
   return generated && kernels->nodes_passes > 0 && node_slots_n <= MAXACC && n >= 6 && size >= 4 * (uint64_t)BLOCK &&
          (size & (size - 1)) == 0 && size / 8 > slice_pairs(st.T(), D) * slice_grid();
